@@ -72,6 +72,15 @@ struct gsofa_plan {
     unsigned long long* d_mat_te = nullptr;
     unsigned long long* d_mat_reach = nullptr;
     std::vector<unsigned long long> h_mat_te, h_mat_reach;  // last fetch (batches)
+    // reach mode: classes of vertex ranges, rebuilt by every execute
+    // (gsofa_quot.hip); levels 0: none
+    QuotParams quot{};
+    struct QuotCaps {  // entries allocated: range table, levels * n, n, edge list
+        size_t tab = 0, ln = 0, n = 0, eb = 0;
+    } qcap;
+    uint2* d_qtab = nullptr;
+    std::vector<uint2> h_qtab;
+    std::vector<uint32_t> h_qoff;
     uint32_t Q = 0;
     uint32_t nblocks = 0;
     int coop = 1;
@@ -483,6 +492,92 @@ void advance_state(gsofa_plan* P, int32_t gid) {
     advance_groups(P, gid, P->C, 0, (cnt + P->C - 1) / P->C);
 }
 
+void release_quot(gsofa_plan* P) {
+    QuotParams& q = P->quot;
+    dfree(P->d_qtab);
+    dfree(q.comp);
+    dfree(q.info);
+    dfree(q.infoT);
+    dfree(q.nodes);
+    dfree(q.ncnt);
+    dfree(q.nmap);
+    dfree(q.nidx);
+    dfree(q.eb);
+    dfree(q.ctl);
+    q = QuotParams{};
+    P->qcap = gsofa_plan::QuotCaps{};
+}
+
+// Levels of classes for a reach-mode run within `room` bytes: all that the
+// largest matrix has, or none where their arrays would take over an eighth of
+// the room or class rows would pass 32-bit entry numbers.
+uint32_t quot_wanted(int64_t n, int64_t nnz, uint32_t W, int64_t room) {
+    const uint32_t L = quot_levels(W);
+    if (L == 0 || nnz + (int64_t)quot_ext((uint64_t)nnz, L) >= (int64_t)UINT32_MAX) return 0;
+    return quot_bytes(n, nnz, W) <= room / 8 ? L : 0;
+}
+
+// The range table and device arrays of `levels` levels for the plan's matrices
+// (P->h_mat_base, n, nnz); d_ci and d_ciT hold quot_ext entries more.  Arrays
+// that are large enough stay (arenas).  The table's upload is queued.
+int setup_quot(gsofa_plan* P, uint32_t levels) {
+    QuotParams& q = P->quot;
+    q.levels = levels;
+    if (levels == 0) return GSOFA_OK;
+    const size_t n = (size_t)P->n, ln = (size_t)levels * n, ne = (size_t)P->nnz;
+    q.n = (uint32_t)n;
+    q.ext0 = (uint32_t)P->nnz;
+    quot_table(P->h_mat_base, levels, P->h_qtab, P->h_qoff);
+    q.total0 = P->h_qoff[1] << kQuotShift;
+    gsofa_plan::QuotCaps& c = P->qcap;
+    int e = 0;
+    if (c.tab < P->h_qtab.size()) {
+        dfree(P->d_qtab);
+        dfree(q.ncnt);
+        e |= dalloc(&P->d_qtab, P->h_qtab.size());
+        e |= dalloc(&q.ncnt, P->h_qtab.size());
+        c.tab = P->h_qtab.size();
+    }
+    if (c.ln < ln) {
+        dfree(q.comp);
+        dfree(q.info);
+        dfree(q.infoT);
+        e |= dalloc(&q.comp, ln);
+        e |= dalloc(&q.info, ln);
+        e |= dalloc(&q.infoT, ln);
+        c.ln = ln;
+    }
+    if (c.n < n) {
+        dfree(q.nodes);
+        dfree(q.nmap);
+        dfree(q.nidx);
+        e |= dalloc(&q.nodes, 2 * n);
+        e |= dalloc(&q.nmap, n);
+        e |= dalloc(&q.nidx, n);
+        c.n = n;
+    }
+    if (c.eb < ne) {
+        dfree(q.eb);
+        e |= dalloc(&q.eb, ne);
+        c.eb = ne;
+    }
+    if (!q.ctl) e |= dalloc(&q.ctl, 1);
+    if (e) return GSOFA_ERR_ALLOC;
+    q.tab = P->d_qtab;
+    if (hipMemcpyAsync(P->d_qtab, P->h_qtab.data(), sizeof(uint2) * P->h_qtab.size(), hipMemcpyHostToDevice,
+                       P->stream) != hipSuccess) {
+        (void)hipGetLastError();
+        return GSOFA_ERR_HIP;
+    }
+    return GSOFA_OK;
+}
+
+// Bytes of setup_quot's arrays at their capacities (the class rows in d_ci and
+// d_ciT apart).
+int64_t quot_held(const gsofa_plan::QuotCaps& c) {
+    return (int64_t)(12 * c.tab + 36 * c.ln + 16 * c.n + 4 * c.eb + sizeof(QuotCtl));
+}
+
 void release_device(gsofa_plan* P) {
     dfree(P->d_rp);
     dfree(P->d_ci);
@@ -526,6 +621,7 @@ void release_device(gsofa_plan* P) {
     dfree(P->d_rmask);
     dfree(P->d_mat_te);
     dfree(P->d_mat_reach);
+    release_quot(P);
 }
 
 int ensure_cols(gsofa_plan* P, int64_t nl, int64_t nu) {
@@ -1014,7 +1110,10 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         output_need(w, A->n, rp.data(), ci.data(), &nf, &nl, &nu);
         uint32_t nb = 0;
         if (reach_grid(o, bits, nchunks, (uint32_t)A->n, INT64_MAX / 4, &nb) != GSOFA_OK) return -1;
+        const uint32_t ql = quot_wanted(A->n, (int64_t)ci.size(), (uint32_t)A->n,
+                                        o.mem_budget_bytes > 0 ? o.mem_budget_bytes : INT64_MAX / 4);
         return reach_bytes(nb, (uint32_t)A->n, bits) +
+               (ql ? quot_bytes(A->n, (int64_t)ci.size(), (uint32_t)A->n) : 0) +
                block_fixed_bytes(A->n, (int64_t)ci.size(), 1, nchunks, rch_fill_room(nf), (int64_t)(nl + nu)) +
                4 * (int64_t)(A->n + 1) + 4 * (int64_t)ci.size();
     }
@@ -1165,6 +1264,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         return GSOFA_ERR_HIP;
     }
     int e = 0;
+    uint32_t qlev = 0;  // levels of classes (reach mode)
     std::vector<int32_t> rpT, ciT;
     if (P->mode == GSOFA_MODE_REACH) {
         int bits = 0;
@@ -1189,8 +1289,12 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             P->share_chunk_off[1] = (uint32_t)P->h_chunks.size();
             transpose_rows(n, P->h_rp.data(), ci.data(), rpT, ciT);
             const int64_t tbytes = 4 * (int64_t)(n + 1) + 4 * P->nnz + 16 * (int64_t)n_mats;
-            rc = reach_grid(P->opt, bits, std::max<uint64_t>(P->h_chunks.size(), 1), P->W,
-                            std::max<int64_t>(avail - tbytes, 1 << 20), &P->nblocks);
+            const int64_t room = std::max<int64_t>(avail - tbytes, 1 << 20);
+            gsofa_options go = P->opt;
+            qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room);
+            const int64_t qb = qlev ? quot_bytes(n, P->nnz, P->W) : 0;
+            if (go.mem_budget_bytes > 0) go.mem_budget_bytes -= qb;
+            rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), P->W, room - qb, &P->nblocks);
         }
         if (rc) {
             (void)hipStreamDestroy(P->stream);
@@ -1209,7 +1313,8 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         e |= dalloc(&P->d_mat_te, (size_t)n_mats);
         e |= dalloc(&P->d_mat_reach, (size_t)n_mats);
         e |= dalloc(&P->d_rpT, (size_t)n + 1);
-        e |= dalloc(&P->d_ciT, (size_t)P->nnz);
+        e |= dalloc(&P->d_ciT, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
+        e |= setup_quot(P, qlev);
     } else if (P->mode == GSOFA_MODE_BLOCK) {
         int S = 0;
         const uint64_t nsrc = P->hybrid ? P->s_top : share_count(n, P->opt.n_virtual_gpu, 0);
@@ -1271,7 +1376,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         e |= dalloc(&P->d_Utmp, (size_t)need_U);
     }
     e |= dalloc(&P->d_rp, (size_t)n + 1);
-    e |= dalloc(&P->d_ci, (size_t)P->nnz);
+    e |= dalloc(&P->d_ci, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
     e |= dalloc(&P->d_fills, (size_t)P->fill_cap);
     e |= dalloc(&P->d_ctrl, 1);
     e |= dalloc(&P->d_cntL, (size_t)n);
@@ -1503,6 +1608,14 @@ static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
         if (P->structure)  // reserved entries left unused must read as ~0
             HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_fills), 2 * P->fill_cap, 0xFFFFFFFFu, P->stream));
         if (!P->capturing) HIPCHK(hipEventRecord(P->ev[2 + 2 * si], P->stream));
+        if (P->quot.levels) {
+            P->quot.rp = P->d_rp;
+            P->quot.rpT = P->d_rpT;
+            P->quot.ci = P->d_ci;
+            P->quot.ciT = P->d_ciT;
+            HIPCHK(launch_quot(P->quot, P->h_qoff, P->stream));
+        }
+        rp.quot = P->quot;
         if (rp.n_chunks > 0) HIPCHK(launch_reach(rp, P->rbits, P->rthreads, P->stream));
         if (!P->capturing) HIPCHK(hipEventRecord(P->ev[3 + 2 * si], P->stream));
         return GSOFA_OK;
@@ -2451,17 +2564,22 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     o.mode = GSOFA_MODE_AUTO;  // the tuned grid for this batch's signature (slots stay 64)
     if (!apply_tuned(&o, W, nnz, n, count) || resolve_mode(o) != GSOFA_MODE_REACH) o = P->opt;
     o.mem_budget_bytes = 0;
-    int rc = reach_grid(o, bits, nchunks, W, budget - fixed, &nb);
+    const uint32_t qlev = quot_wanted(n, nnz, W, budget - fixed);
+    const int64_t qb = qlev ? quot_bytes(n, nnz, W) : 0;
+    int rc = reach_grid(o, bits, nchunks, W, budget - fixed - qb, &nb);
     if (rc) return rc;
     P->rthreads = reach_threads(o);
     gsofa_plan::Caps& c = P->cap;
     const size_t rows = (size_t)n + 1;
+    const size_t ne = (size_t)std::max<int64_t>(nnz + (int64_t)quot_ext((uint64_t)nnz, qlev), 1);
     // The arena keeps each buffer at the largest size seen.  If keeping them
     // and growing the rest would exceed the budget, it starts over with
     // exactly this batch's sizes (the only path that frees device memory).
     {
         auto mx = [](size_t a, uint64_t b) { return (int64_t)std::max<uint64_t>(a, std::max<uint64_t>(b, 1)); };
-        const int64_t keep = 40 * mx(c.rp, rows) + 8 * mx(c.ci, (uint64_t)nnz) + 8 * mx(c.fills, rch_fill_room(nf)) +
+        gsofa_plan::QuotCaps qc = P->qcap;
+        qc.ln = std::max(qc.ln, (size_t)qlev * (size_t)n);
+        const int64_t keep = quot_held(qc) + 40 * mx(c.rp, rows) + 8 * mx(c.ci, (uint64_t)ne) + 8 * mx(c.fills, rch_fill_room(nf)) +
                              8 * mx(c.L, nl) + 8 * mx(c.U, nu) + 8 * mx(c.scan, scan_tmp_words(n) + 2 * (size_t)n + 8) +
                              reach_bytes((uint32_t)std::max<size_t>(c.nb, nb), (uint32_t)std::max<size_t>(c.wg, W), 64);
         if (keep > budget && P->held > 0) {
@@ -2492,7 +2610,6 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         e |= dalloc(&P->d_row_fk, rows);
         c.rp = rows;
     }
-    const size_t ne = (size_t)std::max<int64_t>(nnz, 1);
     if (c.ci < ne) {
         dfree(P->d_ci);
         dfree(P->d_ciT);
@@ -2542,6 +2659,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         c.chunks = nchunks;
     }
     if (!P->d_ctrl) e |= dalloc(&P->d_ctrl, 1);
+    e |= setup_quot(P, qlev);
     if (e) return GSOFA_ERR_ALLOC;
     // per-workgroup arrays: one stride (their capacity) for every batch,
     // cleared when they grow
@@ -2552,7 +2670,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         dfree(P->d_bstate);
         c.wg = std::max<size_t>(W, c.wg);
         c.nb = std::max<size_t>(nb, c.nb);
-        if (reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64) > budget - fixed) {  // exactly this batch's
+        if (reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64) > budget - fixed - qb) {  // exactly this batch's
             c.wg = W;
             c.nb = nb;
         }
@@ -2568,7 +2686,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     }
     P->held = (int64_t)(c.rp * (4 + 4 + 4 + 4 + 8 + 8 + 8 + 8) + c.ci * 8 + c.fills * 8 + c.L * 8 + c.U * 8 +
                         c.scan * 8 + c.mats * 20 + c.chunks * sizeof(BlkChunk) + sizeof(Ctrl)) +
-              reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64);
+              quot_held(P->qcap) + reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64);
     P->W = (uint32_t)c.wg;  // the kernels' per-workgroup stride
     P->nblocks = nb;
     P->C = (int32_t)(nb * P->S);

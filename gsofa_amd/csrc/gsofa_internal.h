@@ -109,6 +109,49 @@ int resident_blocks(int slots, int device, uint32_t* out);
 const void* blk_kernel_ptr(int slots);
 hipError_t launch_traverse_blk(const BlkParams& p, int slots, size_t lds_bytes, hipStream_t s);
 
+// Classes of vertex ranges (gsofa_quot.hip), built on the device at the start
+// of every reach-mode execute.
+constexpr uint32_t kQuotLevels = 26;  // kMaxN < 2^25
+// log2 of a block's vertices.  A source walks up to a block of single
+// vertices; each halving of the block adds a level of ranges to build.
+// Traversal ms at blocks of 128 / 256 / 512 / 1,024: 48^3 grid 3.29 / 3.27 /
+// 3.45 / 3.65, band n=659,033 6.34 / 5.71 / 5.77 / 6.53, 128 2D grids 31.7 /
+// 33.5 / 36.7 / 42.0, 64^2 natural order 0.405 / 0.398 / 0.456 / 0.598.
+constexpr uint32_t kQuotShift = 8;
+struct QuotCtl {
+    unsigned long long ext, extT;      // class-row entries handed out, over A and A^T
+    unsigned long long nodes0;         // classes of all level-0 ranges
+    unsigned long long eb[kQuotLevels];  // edge-list entries handed out, per level
+};
+struct QuotParams {
+    const int32_t* rp;
+    const int32_t* rpT;
+    int32_t* ci;         // the matrix's columns, then the class rows from ext0 on
+    int32_t* ciT;
+    uint32_t n;          // all vertices (stride of the per-level arrays)
+    uint32_t ext0;
+    uint32_t levels;
+    uint32_t total0;     // vertices of the level-0 ranges
+    const uint2* tab;
+    int32_t* comp;       // levels * n: a vertex's class (a member vertex names it)
+    uint4* info;         // levels * n: of a class: row begin, row end, vertices, their row lengths
+    uint4* infoT;        // the same over A^T
+    int32_t* nodes;      // 2 * n: the ranges' class lists, by level parity
+    uint32_t* ncnt;      // per range of every level: its classes
+    int32_t* nmap;       // n
+    int32_t* nidx;       // n
+    uint32_t* eb;        // nnz
+    QuotCtl* ctl;
+};
+// Contraction does not pay where the level-0 ranges keep over half of their
+// vertices as classes: the traversal then walks plain vertices.
+__device__ __forceinline__ bool quot_off(const QuotParams& p) { return 2ull * p.ctl->nodes0 > (unsigned long long)p.total0; }
+uint32_t quot_levels(uint32_t W);
+uint64_t quot_ext(uint64_t nnz, uint32_t levels);
+int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W);
+void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vector<uint2>& tab, std::vector<uint32_t>& off);
+hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hipStream_t s);
+
 // Reach mode (gsofa_reach.hip): one launch over a work table whose chunks
 // run over A (U rows, TE, |R|) or, with rch_pass_bit() set in their stride,
 // over A^T (L columns, written as (row, column) fills).
@@ -134,6 +177,7 @@ struct RchParams {
     unsigned long long* mat_te;     // per matrix TE and |R| of the A pass (zeroed first), or null
     unsigned long long* mat_reach;
     uint32_t loops;        // stamps per workgroup before its visited words are cleared
+    QuotParams quot;       // levels == 0: no classes, every vertex is walked
 };
 bool rch_threads_valid(int threads);  // threads per reach workgroup: 1024 or 512
 bool rch_bits_valid(int bits);

@@ -50,6 +50,14 @@
 //   whole grid do not queue on one counter.  The round's counters
 //   alternate by parity and the level's by level parity, so a round costs two
 //   barriers and a level no more.
+// * Vertices below the block of the mini-group's lowest source are not walked
+//   one by one: strongly connected classes of block ranges stand for them
+//   (gsofa_quot.hip).  Combine maps each target below that block to its
+//   class, relax takes a class's row, vertex count and row-length sum from
+//   the class table.  |R| and TE add those weights, so they count vertices.
+// * A class's row can hold thousands of targets, which one lane group would
+//   take alone while the workgroup waits: rows over SPLIT_ROW are expanded in
+//   SPLIT_PARTS parts by as many groups.
 // * Sources of a mini-group form an arithmetic sequence first, first-stride,
 //   ... (the cyclic source map of symbfact.cuh:1084-1099 within a share), so
 //   "source j lies above m" is the prefix of slots j < ceil((first-m)/stride).
@@ -279,6 +287,12 @@ constexpr int tab_slots(int threads) {
                              : (threads == NT_WIDE ? NH_WIDE : NH_PAIR);
 }
 
+// Rows longer than SPLIT_ROW are expanded by SPLIT_PARTS lane groups instead of
+// one: the vertex goes to a short LDS list rather than the queue, and the
+// level's pops past the queue's end take one part each.  At most SPLIT_MAX
+// such vertices per level (any more are queued whole).
+constexpr uint32_t SPLIT_ROW = 192, SPLIT_PARTS = 32, SPLIT_MAX = 32;
+
 template <class M, int H>
 struct RLds {
     uint32_t hkey[H];                    // target + 1 (window-local); 0 = empty
@@ -294,6 +308,8 @@ struct RLds {
     uint32_t held[2];                    // some group holds unfolded edges, by round parity
     uint32_t chunk;
     uint32_t fcur;                       // entries handed out of the current fill block
+    uint32_t spn[2];                     // split vertices, by level parity
+    uint4 sp[2][SPLIT_MAX];              // (vertex, row begin, row end, weight)
     unsigned long long fbase;            // the block's first entry in the fill stream
 };
 
@@ -363,6 +379,21 @@ struct RCur {
     const int32_t* ci;
     uint32_t first, count, stride, mat, wb;
     bool tpass;
+    // classes of the vertices below block jb (local vertex below): the group's
+    // sources all lie at or above it
+    const int32_t* comp;
+    const uint4* info;
+    uint32_t jb, below, top;
+    uint64_t cn;  // stride of the per-level arrays
+
+    __device__ __forceinline__ uint32_t level_of(uint32_t m) const {
+        const uint32_t h = 31u - (uint32_t)__builtin_clz((m >> kQuotShift) ^ jb);
+        return h < top ? h : top;
+    }
+    // the node (local) that stands for local vertex m
+    __device__ __forceinline__ uint32_t node(uint32_t m) const {
+        return m < below ? (uint32_t)comp[(uint64_t)level_of(m) * cn + wb + m] - wb : m;
+    }
 };
 
 // Phase A: lane groups of G lanes pop frontier vertices one at a time; a
@@ -372,8 +403,8 @@ struct RCur {
 // vertex's mask folded into it, until the queue is exhausted or the table is
 // full.  Wave-uniform control flow; the groups hold independent vertices.
 template <int H, int G, int E, class M>
-__device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, const uint4* qc, uint32_t size,
-                         uint32_t* cursor, uint32_t rb, RTally& t) {
+__device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, const uint4* qc, uint32_t qsize,
+                         uint32_t size, const uint4* sp, uint32_t* cursor, uint32_t rb, RTally& t) {
     using O = MaskOps<M>;
     constexpr int T = H / 2;
     const uint32_t lane = __lane_id();
@@ -393,7 +424,21 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
             if (idx >= size) {
                 hv.done = true;
             } else {
-                const uint4 e = qc[idx];
+                uint4 e;
+                const bool whole = idx < qsize;
+                if (whole) {
+                    e = qc[idx];
+                } else {  // one part of a split row; the first carries the weight
+                    const uint32_t part = (idx - qsize) % SPLIT_PARTS;
+                    e = sp[(idx - qsize) / SPLIT_PARTS];
+                    const uint32_t len = e.z - e.y;
+                    const uint32_t per = ((len + SPLIT_PARTS - 1u) / SPLIT_PARTS + (uint32_t)(G * E) - 1u) /
+                                         (uint32_t)(G * E) * (uint32_t)(G * E);
+                    const uint32_t o = part * per < len ? part * per : len;
+                    e.z = len - o > per ? e.y + o + per : e.z;
+                    e.y += o;
+                    if (part != 0u) e.w = 0u;
+                }
                 // the mask and the first step's edges load together
                 const M mk = maskc[(merges<M>() ? 2u : 1u) * e.x];
 #pragma unroll
@@ -401,6 +446,9 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
                     const uint32_t ek = e.y + j + (uint32_t)(G * k);
                     m[k] = ek < e.z ? (uint32_t)c.ci[ek] - c.wb : FULLI;
                 }
+#pragma unroll
+                for (int k = 0; k < E; k++)
+                    if (m[k] != FULLI) m[k] = c.node(m[k]);
                 fresh = true;
                 hv.pos = e.y;
                 hv.end = e.z;
@@ -408,8 +456,8 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
                 hv.vm = mk;
                 hv.held = e.y < e.z;
                 if (j == 0u) {
-                    maskc[(merges<M>() ? 2u : 1u) * e.x] = (M)0;  // consumed; refilled two levels later
-                    t.checks += (unsigned long long)(e.z - e.y) * O::popc(mk);
+                    if (whole) maskc[(merges<M>() ? 2u : 1u) * e.x] = (M)0;  // consumed; refilled two levels later
+                    t.checks += (unsigned long long)e.w * O::popc(mk);
                     t.expansions++;
                 }
             }
@@ -428,6 +476,9 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
                     m[k] = FULLI;
                     if (((hv.pend >> k) & 1u) && e < hv.end) m[k] = (uint32_t)c.ci[e] - c.wb;
                 }
+#pragma unroll
+                for (int k = 0; k < E; k++)
+                    if (m[k] != FULLI) m[k] = c.node(m[k]);
             }
             uint32_t left = 0;
 #pragma unroll
@@ -480,8 +531,10 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
         S.tcnt[0] = S.tcnt[1] = S.held[0] = S.held[1] = 0;
         S.fcur = fblk;  // no block yet
         S.fbase = 0;
+        S.spn[0] = S.spn[1] = 0;
     }
     uint32_t rb = 0;  // round parity
+    const bool classes = p.quot.levels != 0u && !quot_off(p.quot);
     for (;;) {
         if (tid == 0) {
             S.chunk = atomicAdd(&p.ctrl->src_next, 1u);
@@ -502,6 +555,12 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
         c.stride = C.stride & ~PASS_T;
         c.mat = C.mat;
         c.wb = p.mat_base[C.mat];
+        c.comp = p.quot.comp;
+        c.info = c.tpass ? p.quot.infoT : p.quot.info;
+        c.cn = p.quot.n;
+        c.top = p.quot.levels - 1u;
+        c.jb = classes ? (c.first - (c.count - 1u) * c.stride - c.wb) >> kQuotShift : 0u;
+        c.below = c.jb << kQuotShift;
         if (epoch >= p.loops) {  // stamps exhausted: clear this workgroup's visited words
             for (uint32_t i = tid; i < W; i += RB) vis[i] = O::make((M)0, 0u);
             epoch = 0;
@@ -517,7 +576,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             vis[s] = O::make(bit, stamp);
             nmask0[(merges<M>() ? 2u : 1u) * s] = bit;  // level 0 uses the first mask
             const uint32_t r0 = (uint32_t)c.rp[sg], r1 = (uint32_t)c.rp[sg + 1];
-            q0[tid] = make_uint4(s, r0, r1, 0u);
+            q0[tid] = make_uint4(s, r0, r1, r1 - r0);
             t.te += r1 - r0;
         }
         if (tid == 0) S.qcnt[0] = c.count;
@@ -526,9 +585,20 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
         uint32_t cur = 0;
         for (uint32_t lev = 0;; lev++) {
             // final since the last barrier; reset during this level's relax
-            const uint32_t size = S.qcnt[cur];
-            if (size == 0) break;
             const uint32_t nxt = cur ^ 1u;
+            const uint32_t qsize = S.qcnt[cur];
+            const uint32_t nsp = S.spn[cur] < SPLIT_MAX ? S.spn[cur] : SPLIT_MAX;
+            const uint32_t size = qsize + SPLIT_PARTS * nsp;
+            // the previous level's split vertices: no part is left, so their
+            // masks are cleared here, before this level's relax fills that array
+            if (w == 0) {
+                const uint32_t done = S.spn[nxt] < SPLIT_MAX ? S.spn[nxt] : SPLIT_MAX;
+                if (tid < done)
+                    nmask0[merges<M>() ? 2ull * S.sp[nxt][tid].x + nxt : (uint64_t)nxt * W + S.sp[nxt][tid].x] = (M)0;
+                wave_sync();
+                if (tid == 0) S.spn[nxt] = 0;
+            }
+            if (size == 0) break;
             // this level's and the next level's masks: side by side per vertex
             // (merging widths, index 2v) or two arrays (index v)
             constexpr uint32_t MS = merges<M>() ? 2u : 1u;
@@ -550,7 +620,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                     S.fbase = aadd64(&p.ctrl->fill_pos, fblk);
                     S.fcur = 0;
                 }
-                rcombine<H, G, E, M>(S, hv, c, maskc, qc, size, cursor, rb, t);
+                rcombine<H, G, E, M>(S, hv, c, maskc, qc, qsize, size, S.sp[cur], cursor, rb, t);
                 if (hv.held && (lane % G) == 0u) atomicOr(&S.held[rb], 1u);
                 __syncthreads();
                 // final for this round: the cursor moves only in phase A
@@ -572,14 +642,24 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                     }
                     const uint32_t mg = m + c.wb;
                     M up = (M)0;
-                    uint32_t r0 = 0, r1 = 0;
+                    uint32_t r0 = 0, r1 = 0, wt = 0;
                     bool enq = false;
                     if (ok) {
                         const VW vw = vis[m];
                         const M mc = merges<M>() ? maskc[MS * m] : (M)0;
                         const M mn = maskn[MS * m];
-                        r0 = (uint32_t)c.rp[mg];
-                        r1 = (uint32_t)c.rp[mg + 1];
+                        uint32_t vc = 1;  // vertices of the node
+                        if (m < c.below) {
+                            const uint4 in = c.info[(uint64_t)c.level_of(m) * c.cn + mg];
+                            r0 = in.x;
+                            r1 = in.y;
+                            vc = in.z;
+                            wt = in.w;
+                        } else {
+                            r0 = (uint32_t)c.rp[mg];
+                            r1 = (uint32_t)c.rp[mg + 1];
+                            wt = r1 - r0;
+                        }
                         const M vv = O::get(vw, stamp);
                         const M nw = mk & ~vv;
                         if (nw) {
@@ -587,7 +667,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                             const M bl = nw & above_mask<M>(mg, c.first, c.stride, c.count);
                             up = lev ? (nw & ~bl) : (M)0;  // level 0: A's own entries
                             if (bl) {
-                                if (merges<M>() && lev != 0u && mc) {
+                                if (merges<M>() && lev != 0u && mc && r1 - r0 <= SPLIT_ROW) {
                                     // still queued for this level and not yet
                                     // popped: it expands these bits too, one
                                     // expansion fewer (not at level 0, whose
@@ -598,8 +678,15 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                                     enq = mn == (M)0;
                                 }
                                 const uint32_t nb = O::popc(bl);
-                                t.reach += nb;
-                                t.te += (unsigned long long)nb * (r1 - r0);
+                                t.reach += (unsigned long long)nb * vc;
+                                t.te += (unsigned long long)nb * wt;
+                                if (enq && r1 - r0 > SPLIT_ROW) {
+                                    const uint32_t k = atomicAdd(&S.spn[nxt], 1u);
+                                    if (k < SPLIT_MAX) {
+                                        S.sp[nxt][k] = make_uint4(m, r0, r1, wt);
+                                        enq = false;
+                                    }
+                                }
                             }
                         }
                     }
@@ -608,7 +695,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                         uint32_t qb = 0;
                         if (lane == 0) qb = atomicAdd(&S.qcnt[nxt], (uint32_t)__popcll(em));
                         qb = bcast0(qb);
-                        if (enq) qn[qb + rank_in(em)] = make_uint4(m, r0, r1, 0u);
+                        if (enq) qn[qb + rank_in(em)] = make_uint4(m, r0, r1, wt);
                     }
                     const uint32_t nf = O::popc(up);
                     t.fills += nf;

@@ -1,0 +1,108 @@
+"""GPU parity of reach mode over vertex classes (strongly connected classes of
+block ranges stand for their vertices) against the CPU oracle: block and range
+edges, patterns without classes, patterns that keep too many nodes to merge,
+rows long enough to be split over lane groups, batches and replays."""
+import numpy as np
+import pytest
+
+from gpu_util import assert_same_structure
+
+pytestmark = pytest.mark.gpu
+
+BLOCK = 256
+
+
+def _oracle(A):
+    from oracle import oracle
+    return oracle.symbfact(A.colbeg, A.colend, A.csr, A.n)
+
+
+def _from_edges(n, rows, cols):
+    import gsofa_amd as g
+    d = np.arange(n, dtype=np.int64)
+    key = np.unique(np.concatenate([np.asarray(rows, np.int64) * n + cols, d * n + d]))
+    end = np.cumsum(np.bincount(key // n, minlength=n))
+    return g.CsrMatrix(n, np.concatenate([[0], end[:-1]]), end, key % n)
+
+
+def _check(A, **kw):
+    import gsofa_amd as g
+    print("case: n", A.n, "nnz", A.nnz, kw, flush=True)
+    r = g.symbfact(A, mode="reach", **kw)
+    assert r.edge_checks >= r.te_alg
+    assert_same_structure(r, _oracle(A))
+
+
+@pytest.mark.parametrize("bits", [32, 64, 128, 256])
+@pytest.mark.parametrize("n", [BLOCK, BLOCK + 1, 2 * BLOCK, 2 * BLOCK + 1, 3 * BLOCK - 1, 4 * BLOCK + 1, 9 * BLOCK + 77])
+def test_range_edges(n, bits):
+    import gsofa_amd as g
+    _check(g.gen_band(n, 30, 4.0, n + bits), block_slots=bits)
+
+
+@pytest.mark.parametrize("threads", [512, 1024])
+@pytest.mark.parametrize("lam", [1.2, 2.0, 3.0])
+def test_few_classes(lam, threads):
+    """Sparse one-directional bands: most vertices stay classes of their own,
+    at the lowest density so many that classes are not used at all."""
+    import gsofa_amd as g
+    _check(g.gen_band(20011, 200, lam, 7), block_slots=64, workgroup_threads=threads)
+
+
+def test_too_many_nodes():
+    """Ranges of over 4,096 nodes keep their halves' classes: pairs (2i, 2i+1)
+    are strongly connected, the pairs form an acyclic chain of chains."""
+    n = 12001
+    i = np.arange(0, n - 1, 2)
+    rows = np.concatenate([i, i + 1, i[:-9]])
+    cols = np.concatenate([i + 1, i, i[:-9] + 18])
+    _check(_from_edges(n, rows, cols), block_slots=32)
+    _check(_from_edges(n, cols, rows), block_slots=32)
+
+
+def test_acyclic():
+    n = 1500
+    rng = np.random.default_rng(3)
+    i, j = rng.integers(0, n, 6000), rng.integers(0, n, 6000)
+    lo, hi = np.minimum(i, j), np.maximum(i, j)
+    _check(_from_edges(n, lo, hi))
+    _check(_from_edges(n, hi, lo))
+
+
+@pytest.mark.parametrize("bits", [32, 64, 256])
+@pytest.mark.parametrize("hubs,length", [(1, 193), (3, 2900), (60, 250)])
+def test_long_rows(hubs, length, bits):
+    """Hub rows and columns longer than the split length, more of them than
+    the split list holds, below, among and above the other vertices."""
+    n = 3001
+    rng = np.random.default_rng(hubs)
+    rows, cols = [], []
+    for h in rng.choice(n, hubs, replace=False):
+        t = rng.choice(n, length, replace=False)
+        rows += [np.full(length, h), t]
+        cols += [t, np.full(length, h)]
+    i = np.arange(n - 1)
+    rows += [i, i[::3] + 1]
+    cols += [i + 1, i[::3]]
+    _check(_from_edges(n, np.concatenate(rows), np.concatenate(cols)), block_slots=bits)
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(graph=True), dict(counts_only=True)])
+def test_batch_of_sizes(kw):
+    """Matrices below, at and above a block in one plan, executed three times."""
+    import gsofa_amd as g
+    import gsofa_amd.configs as cf
+    mats = [cf.batch_matrix(s, s) for s in (1, 15, 16, 17, 40, 70)] + [g.gen_band(2 * BLOCK + 1, 20, 3.0, 1),
+                                                                      cf.grid64_natural()]
+    orc = [_oracle(A) for A in mats]
+    print("case: batch", kw, flush=True)
+    with g.Plan(mats, mode="reach", **kw) as p:
+        for _ in range(3):
+            p.execute()
+            for b, o in enumerate(orc):
+                r = p.fetch_matrix(b)
+                if kw.get("counts_only"):
+                    assert r.fill_count == o.fill_count and r.te_alg == o.te_alg and r.reach == o.reach
+                    np.testing.assert_array_equal(r.row_fill, o.row_fill)
+                else:
+                    assert_same_structure(r, o)
