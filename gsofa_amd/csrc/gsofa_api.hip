@@ -93,7 +93,15 @@ struct gsofa_plan {
     uint64_t* d_q1 = nullptr;
     uint64_t* d_fills = nullptr;
     uint64_t fill_cap = 0;
-    uint64_t fill_need = 0;  // bounded plans: the fills the row bounds allow
+    // reach mode: records of (vertex, first source, mask) in place of the fill
+    // stream (fill_cap of them), where each chunk's lie, L counts with record
+    // counts, and the rows' record lists with their offsets
+    uint4* d_rec = nullptr;
+    uint4* d_grp = nullptr;
+    unsigned long long* d_cnt64 = nullptr;
+    uint4* d_list = nullptr;
+    int64_t* d_rptr = nullptr;
+    uint64_t list_cap = 0;
     Ctrl* d_ctrl = nullptr;
     // Output sized from the row bounds of gsofa_fill_bound: the fill stream
     // cannot overflow and the L/U columns exist before the traversal, so an
@@ -312,11 +320,15 @@ uint64_t label_words(int32_t n, int32_t N, int32_t C, int32_t gid_lo, int32_t gi
 
 // Output one execute needs at most, from the row bounds of lu_row_bounds:
 // fills, L and U entries of the rows it processes (every share, one share, or
-// for a spilled run the largest share).  rp/ci: packed rows.
+// for a spilled run the largest share).  rp/ci: packed rows.  bits > 0 (reach
+// mode): also the records of one pass, for groups of so many sources.
 void output_need(const gsofa_options& o, int32_t n, const int32_t* rp, const int32_t* ci, uint64_t* need_fill,
-                 uint64_t* need_L, uint64_t* need_U) {
+                 uint64_t* need_L, uint64_t* need_U, int bits = 0, const std::vector<uint32_t>* mat_base = nullptr,
+                 uint64_t* need_rec = nullptr) {
     std::vector<int64_t> Lb, Ub;
-    lu_row_bounds(n, rp, ci, Lb, Ub);
+    std::vector<int32_t> parent;
+    lu_row_bounds(n, rp, ci, Lb, Ub, bits ? &parent : nullptr);
+    if (bits) *need_rec = reach_record_bound(*mat_base, parent, Ub, bits);
     const int32_t N = std::max(1, o.n_virtual_gpu);
     std::vector<uint64_t> fs((size_t)N, 0), ls((size_t)N, 0), us((size_t)N, 0);
     for (int32_t i = 0; i < n; i++) {
@@ -492,6 +504,20 @@ void advance_state(gsofa_plan* P, int32_t gid) {
     advance_groups(P, gid, P->C, 0, (cnt + P->C - 1) / P->C);
 }
 
+// The fill stream, or reach mode's records and record lists, of P->fill_cap
+// entries (list: records of the A^T pass, at most).
+int alloc_stream(gsofa_plan* P, uint64_t list) {
+    if (P->mode != GSOFA_MODE_REACH) {
+        dfree(P->d_fills);
+        return dalloc(&P->d_fills, (size_t)P->fill_cap);
+    }
+    dfree(P->d_rec);
+    dfree(P->d_list);
+    P->list_cap = std::max<uint64_t>(list, 1);
+    if (dalloc(&P->d_rec, (size_t)P->fill_cap) || dalloc(&P->d_list, (size_t)P->list_cap)) return GSOFA_ERR_ALLOC;
+    return GSOFA_OK;
+}
+
 void release_quot(gsofa_plan* P) {
     QuotParams& q = P->quot;
     dfree(P->d_qtab);
@@ -587,6 +613,11 @@ void release_device(gsofa_plan* P) {
     dfree(P->d_q0);
     dfree(P->d_q1);
     dfree(P->d_fills);
+    dfree(P->d_rec);
+    dfree(P->d_grp);
+    dfree(P->d_cnt64);
+    dfree(P->d_list);
+    dfree(P->d_rptr);
     dfree(P->d_ctrl);
     dfree(P->d_cntL);
     dfree(P->d_cntU);
@@ -625,18 +656,19 @@ void release_device(gsofa_plan* P) {
 }
 
 int ensure_cols(gsofa_plan* P, int64_t nl, int64_t nu) {
+    const bool staged = P->mode != GSOFA_MODE_REACH;  // columns sorted from a staging copy
     if (nl > P->Lcap) {
         dfree(P->d_Lcol);
         dfree(P->d_Ltmp);
         int64_t cap = nl + nl / 8 + 1024;
-        if (dalloc(&P->d_Lcol, (size_t)cap) || dalloc(&P->d_Ltmp, (size_t)cap)) return GSOFA_ERR_ALLOC;
+        if (dalloc(&P->d_Lcol, (size_t)cap) || (staged && dalloc(&P->d_Ltmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Lcap = cap;
     }
     if (nu > P->Ucap) {
         dfree(P->d_Ucol);
         dfree(P->d_Utmp);
         int64_t cap = nu + nu / 8 + 1024;
-        if (dalloc(&P->d_Ucol, (size_t)cap) || dalloc(&P->d_Utmp, (size_t)cap)) return GSOFA_ERR_ALLOC;
+        if (dalloc(&P->d_Ucol, (size_t)cap) || (staged && dalloc(&P->d_Utmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Ucap = cap;
     }
     return GSOFA_OK;
@@ -1107,7 +1139,10 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         gsofa_options w = o;
         w.n_virtual_gpu = 1;
         w.virtual_gpu_id = -1;
-        output_need(w, A->n, rp.data(), ci.data(), &nf, &nl, &nu);
+        const std::vector<uint32_t> mb{0u, (uint32_t)A->n};
+        uint64_t nr = 0;
+        output_need(w, A->n, rp.data(), ci.data(), &nf, &nl, &nu, bits, &mb, &nr);
+        nf = reach_reserve(nf, nl + nu, nr);
         uint32_t nb = 0;
         if (reach_grid(o, bits, nchunks, (uint32_t)A->n, INT64_MAX / 4, &nb) != GSOFA_OK) return -1;
         const uint32_t ql = quot_wanted(A->n, (int64_t)ci.size(), (uint32_t)A->n,
@@ -1216,9 +1251,21 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     // Output reserve from the row bounds: the fills, L and U entries of the
     // rows one execute processes (every share, one share, or for a spilled
     // run the largest share).
-    uint64_t need_fill = 0, need_L = 0, need_U = 0;
+    uint64_t need_fill = 0, need_L = 0, need_U = 0, need_rec = 0;
+    if (reach) {
+        int bits = 0;
+        rc = choose_bits(P->opt, n_mats, (uint64_t)n, &bits);
+        if (rc) {
+            (void)hipStreamDestroy(P->stream);
+            delete P;
+            return rc;
+        }
+        P->rbits = bits;
+    }
     if (P->opt.output_capacity <= 0 && n > 0) {
-        output_need(P->opt, n, P->h_rp.data(), ci.data(), &need_fill, &need_L, &need_U);
+        output_need(P->opt, n, P->h_rp.data(), ci.data(), &need_fill, &need_L, &need_U, P->rbits, &P->h_mat_base,
+                    &need_rec);
+        if (reach) need_fill = reach_reserve(need_fill, need_L + need_U, need_rec);
         const int64_t out_bytes = output_bytes(reach ? rch_fill_room(need_fill) : need_fill, need_L, need_U);
         if (out_bytes <= avail / 2) {
             P->bounded = true;
@@ -1267,12 +1314,10 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     uint32_t qlev = 0;  // levels of classes (reach mode)
     std::vector<int32_t> rpT, ciT;
     if (P->mode == GSOFA_MODE_REACH) {
-        int bits = 0;
-        rc = choose_bits(P->opt, n_mats, (uint64_t)n, &bits);
+        const int bits = P->rbits;
         P->S = (uint32_t)bits;
-        P->rbits = bits;
         P->rthreads = reach_threads(P->opt);
-        if (!rc) {
+        {
             // the A pass's chunks, deepest first, each followed by the same
             // sources' chunk of the A^T pass: one launch runs both
             build_chunks(P);
@@ -1309,7 +1354,9 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         e |= dalloc(&P->d_bstate, (size_t)P->nblocks);
         e |= dalloc(&P->d_mat_base, (size_t)n_mats + 1);
         e |= dalloc(&P->d_chunks, std::max<size_t>(P->h_chunks.size(), 1));
-        e |= dalloc(&P->d_row_fk, (size_t)n);
+        e |= dalloc(&P->d_grp, std::max<size_t>(P->h_chunks.size(), 1));
+        e |= dalloc(&P->d_cnt64, (size_t)n);
+        e |= dalloc(&P->d_rptr, (size_t)n + 1);
         e |= dalloc(&P->d_mat_te, (size_t)n_mats);
         e |= dalloc(&P->d_mat_reach, (size_t)n_mats);
         e |= dalloc(&P->d_rpT, (size_t)n + 1);
@@ -1366,18 +1413,19 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     if ((P->opt.flags & GSOFA_FLAG_SPILL) && P->opt.output_capacity <= 0)  // one share's fills at a time
         P->fill_cap = std::max<uint64_t>(P->fill_cap / (uint64_t)std::max(1, P->opt.n_virtual_gpu), 1u << 20);
     if (P->bounded) {
-        P->fill_cap = P->mode == GSOFA_MODE_REACH ? rch_fill_room(need_fill) : std::max<uint64_t>(need_fill, 1);
-        P->fill_need = need_fill;
+        P->fill_cap = P->mode == GSOFA_MODE_REACH ? 2 * need_rec : std::max<uint64_t>(need_fill, 1);
         P->Lcap = (int64_t)need_L;
         P->Ucap = (int64_t)need_U;
         e |= dalloc(&P->d_Lcol, (size_t)need_L);
-        e |= dalloc(&P->d_Ltmp, (size_t)need_L);
         e |= dalloc(&P->d_Ucol, (size_t)need_U);
-        e |= dalloc(&P->d_Utmp, (size_t)need_U);
+        if (!reach) {
+            e |= dalloc(&P->d_Ltmp, (size_t)need_L);
+            e |= dalloc(&P->d_Utmp, (size_t)need_U);
+        }
     }
     e |= dalloc(&P->d_rp, (size_t)n + 1);
     e |= dalloc(&P->d_ci, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
-    e |= dalloc(&P->d_fills, (size_t)P->fill_cap);
+    if (!(P->opt.flags & GSOFA_FLAG_COUNTS_ONLY) || !reach) e |= alloc_stream(P, P->bounded ? need_rec : P->fill_cap);
     e |= dalloc(&P->d_ctrl, 1);
     e |= dalloc(&P->d_cntL, (size_t)n);
     e |= dalloc(&P->d_cntU, (size_t)n);
@@ -1562,6 +1610,33 @@ static TravParams grid_params(const gsofa_plan* P, int32_t gid) {
     return tp;
 }
 
+static RowParams row_params(const gsofa_plan* P) {
+    RowParams r{};
+    r.n = P->n;
+    r.rp = P->d_rp;
+    r.ci = P->d_ci;
+    r.chunks = P->d_chunks;
+    r.n_chunks = (uint32_t)P->h_chunks.size();
+    r.slots = (uint32_t)std::min(P->rbits, 64);
+    r.words = (uint32_t)std::max(P->rbits / 64, 1);
+    r.rec = P->d_rec;
+    r.grp = P->d_grp;
+    r.cntU = P->d_cntU;
+    r.cntL = P->d_cnt64;
+    r.row_fill = P->d_rowfill;
+    r.sums = P->d_scan;
+    r.L_rowptr = P->d_Lrp;
+    r.U_rowptr = P->d_Urp;
+    r.R_ptr = P->d_rptr;
+    r.list = P->d_list;
+    r.list_cap = (int64_t)P->list_cap;
+    r.L_col = P->d_Lcol;
+    r.U_col = P->d_Ucol;
+    r.L_cap = P->Lcap;
+    r.U_cap = P->Ucap;
+    return r;
+}
+
 // One share's traversal, bracketed by events 2+2si / 3+2si.
 static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
     const int32_t n = P->n;
@@ -1591,22 +1666,20 @@ static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
         rp.vis = P->d_vis;
         rp.nmask = P->d_rmask;
         rp.q = P->d_qgv;
-        rp.fills = P->d_fills;
-        rp.fill_cap = P->structure ? P->fill_cap : 0;  // counts only: per-row tallies, no fill stream
-        rp.fill_blk = rch_fill_block(P->fill_need ? P->fill_need : P->fill_cap, P->nblocks);
+        rp.rec = P->d_rec;
+        rp.rec_cap = P->structure ? P->fill_cap : 0;
+        rp.grp = P->d_grp;
         rp.ctrl = P->d_ctrl;
         rp.bstate = P->d_bstate;
-        rp.row_fills = P->d_row_fk;
+        rp.cntU = P->d_cntU;
+        rp.cntL = P->d_cnt64;
         rp.mat_te = P->d_mat_te;
         rp.mat_reach = P->d_mat_reach;
         rp.loops = std::min(0xFFFFFFFFu, P->span_cap);
         HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_mat_te), 2 * (uint64_t)P->n_mats, 0u, P->stream));
         HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_mat_reach), 2 * (uint64_t)P->n_mats, 0u, P->stream));
-        if (!P->structure)  // both passes add their fills per row
-            HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_row_fk), 2 * (uint64_t)n, 0u, P->stream));
+        HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_cnt64), 2 * (uint64_t)n, 0u, P->stream));
         HIPCHK(launch_fill(&P->d_ctrl->src_next, 1, 0u, P->stream));
-        if (P->structure)  // reserved entries left unused must read as ~0
-            HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_fills), 2 * P->fill_cap, 0xFFFFFFFFu, P->stream));
         if (!P->capturing) HIPCHK(hipEventRecord(P->ev[2 + 2 * si], P->stream));
         if (P->quot.levels) {
             P->quot.rp = P->d_rp;
@@ -1618,6 +1691,7 @@ static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
         rp.quot = P->quot;
         if (rp.n_chunks > 0) HIPCHK(launch_reach(rp, P->rbits, P->rthreads, P->stream));
         if (!P->capturing) HIPCHK(hipEventRecord(P->ev[3 + 2 * si], P->stream));
+        if (!P->structure) HIPCHK(launch_row_fills(row_params(P), P->stream));
         return GSOFA_OK;
     }
     if (P->mode == GSOFA_MODE_BLOCK) {
@@ -1674,6 +1748,7 @@ static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
 // totals are read when needed, read_totals).
 static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t gpu_id, bool on_device = false) {
     const int32_t n = P->n;
+    const bool reach = P->mode == GSOFA_MODE_REACH;
     FinalParams f{};
     f.n = n;
     f.rp = P->d_rp;
@@ -1689,9 +1764,13 @@ static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t g
     f.cntL = P->d_cntL;
     f.cntU = P->d_cntU;
     f.scan_tmp = P->d_scan;
-    HIPCHK(launch_count(f, P->stream));
-    HIPCHK(exclusive_scan_u32_to_i64(P->d_cntL, P->d_Lrp, n, P->d_scan, P->stream));
-    HIPCHK(exclusive_scan_u32_to_i64(P->d_cntU, P->d_Urp, n, P->d_scan, P->stream));
+    if (reach) {
+        HIPCHK(launch_row_ptrs(row_params(P), P->stream));
+    } else {
+        HIPCHK(launch_count(f, P->stream));
+        HIPCHK(exclusive_scan_u32_to_i64(P->d_cntL, P->d_Lrp, n, P->d_scan, P->stream));
+        HIPCHK(exclusive_scan_u32_to_i64(P->d_cntU, P->d_Urp, n, P->d_scan, P->stream));
+    }
     if (on_device) {
         P->totals_known = false;
     } else {
@@ -1704,6 +1783,10 @@ static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t g
         P->totals_known = true;
         int rc = ensure_cols(P, P->nnzL, P->nnzU);
         if (rc) return rc;
+    }
+    if (reach) {
+        HIPCHK(launch_rows(row_params(P), P->stream));
+        return GSOFA_OK;
     }
     f.L_col = P->d_Ltmp;
     f.U_col = P->d_Utmp;
@@ -2036,10 +2119,9 @@ int gsofa_plan_execute(gsofa_plan* P) {
         HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
         if (P->stats.abort) return GSOFA_ERR_DEVICE_TIMEOUT;
         if (!P->structure || P->stats.fill_pos <= P->fill_cap) break;
-        // fill stream outgrew its reserve: grow to the exact size and rerun
-        dfree(P->d_fills);
+        // the stream outgrew its reserve: grow to the exact size and rerun
         P->fill_cap = P->stats.fill_pos + P->stats.fill_pos / 16 + 1024;
-        if (dalloc(&P->d_fills, (size_t)P->fill_cap)) return GSOFA_ERR_ALLOC;
+        if (alloc_stream(P, P->fill_cap)) return GSOFA_ERR_ALLOC;
     }
     if (P->structure && P->stats.fill_pos > P->fill_cap) return GSOFA_ERR_ALLOC;
 
@@ -2101,7 +2183,7 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
         if (P->mode == GSOFA_MODE_REACH) {
             r->row_fill = (int64_t*)malloc(sizeof(int64_t) * (size_t)n);
             if (!r->row_fill) return GSOFA_ERR_ALLOC;
-            HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_row_fk, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
+            HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
                                       P->stream), P->stream);
             HIPCHK_OUT(fetch_mat_totals(P), P->stream);
             HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
@@ -2349,9 +2431,11 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
         T.get(&d_lrow, (size_t)P->nnzL) || T.get(&d_urow, (size_t)P->nnzU))
         return GSOFA_ERR_ALLOC;
     // L and U by columns; the staging arrays of the structure pass are free now
-    HIPCHK_OUT(transpose_structure(P->d_Lrp, P->d_Lcol, P->nnzL, n, P->d_cntL, d_xl, P->d_scan, P->d_Ltmp, d_lrow,
+    int32_t *t_l = P->d_Ltmp, *t_u = P->d_Utmp;
+    if ((!t_l && T.get(&t_l, (size_t)P->nnzL)) || (!t_u && T.get(&t_u, (size_t)P->nnzU))) return GSOFA_ERR_ALLOC;
+    HIPCHK_OUT(transpose_structure(P->d_Lrp, P->d_Lcol, P->nnzL, n, P->d_cntL, d_xl, P->d_scan, t_l, d_lrow,
                                    P->stream), P->stream);
-    HIPCHK_OUT(transpose_structure(P->d_Urp, P->d_Ucol, P->nnzU, n, P->d_cntU, d_xu, P->d_scan, P->d_Utmp, d_urow,
+    HIPCHK_OUT(transpose_structure(P->d_Urp, P->d_Ucol, P->nnzU, n, P->d_cntU, d_xu, P->d_scan, t_u, d_urow,
                                    P->stream), P->stream);
     // supernode subscripts
     int64_t nsub = 0;
@@ -2452,6 +2536,8 @@ int gsofa_symbfact(const gsofa_matrix* A, const gsofa_options* opt, gsofa_result
 
 namespace gsofa {
 
+constexpr int kArenaBits = 64;
+
 int pack_matrix(const gsofa_matrix* A, PackedMatrix* M) {
     const int rc = validate(A);
     if (rc) return rc;
@@ -2462,8 +2548,19 @@ int pack_matrix(const gsofa_matrix* A, PackedMatrix* M) {
     transpose_rows(M->n, M->rp.data(), M->ci.data(), M->rpT, M->ciT);
     gsofa_options o;
     gsofa_options_default(&o);
-    output_need(o, M->n, M->rp.data(), M->ci.data(), &M->need_fill, &M->need_L, &M->need_U);
+    const std::vector<uint32_t> mb{0u, (uint32_t)M->n};
+    output_need(o, M->n, M->rp.data(), M->ci.data(), &M->need_fill, &M->need_L, &M->need_U, kArenaBits, &mb,
+                &M->need_rec);
+    M->need_fill = reach_reserve(M->need_fill, M->need_L + M->need_U, M->need_rec);
     return GSOFA_OK;
+}
+
+uint64_t rch_fill_room(uint64_t need) { return need + need / 15 + need / 8 + (1ull << 20) + 1; }
+
+uint64_t reach_reserve(uint64_t fills, uint64_t lu, uint64_t records) {
+    // 16 B per record of either pass and per list entry; columns 4 B each,
+    // accounted with 8
+    return 48 * records > 8 * rch_fill_room(fills) + 4 * lu ? std::max(fills, 6 * records) : fills;
 }
 
 int64_t reach_fixed_bytes(int64_t n, int64_t nnz, int32_t n_mats, uint64_t nchunks, uint64_t fills, uint64_t lu) {
@@ -2500,8 +2597,9 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     HIPCHK(hipSetDevice(P->device));
     int64_t n = 0, nnz = 0;
     uint32_t W = 1;
-    uint64_t nf = 0, nl = 0, nu = 0;
+    uint64_t nf = 0, nl = 0, nu = 0, nr = 0;
     for (int32_t b = 0; b < count; b++) {
+        nr += mats[b]->need_rec;
         n += mats[b]->n;
         nnz += mats[b]->nnz;
         W = std::max<uint32_t>(W, (uint32_t)mats[b]->n);
@@ -2539,7 +2637,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     // chunks: every matrix's, deepest first, each followed by its A^T twin.
     // Arenas keep 64 sources per workgroup, so the visited words keep one
     // layout from batch to batch.
-    const int bits = 64;
+    const int bits = kArenaBits;
     P->S = (uint32_t)bits;
     P->rbits = bits;
     P->W = W;
@@ -2579,8 +2677,8 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         auto mx = [](size_t a, uint64_t b) { return (int64_t)std::max<uint64_t>(a, std::max<uint64_t>(b, 1)); };
         gsofa_plan::QuotCaps qc = P->qcap;
         qc.ln = std::max(qc.ln, (size_t)qlev * (size_t)n);
-        const int64_t keep = quot_held(qc) + 40 * mx(c.rp, rows) + 8 * mx(c.ci, (uint64_t)ne) + 8 * mx(c.fills, rch_fill_room(nf)) +
-                             8 * mx(c.L, nl) + 8 * mx(c.U, nu) + 8 * mx(c.scan, scan_tmp_words(n) + 2 * (size_t)n + 8) +
+        const int64_t keep = quot_held(qc) + 48 * mx(c.rp, rows) + 8 * mx(c.ci, (uint64_t)ne) + 24 * mx(c.fills, 2 * nr) +
+                             4 * mx(c.L, nl) + 4 * mx(c.U, nu) + 8 * mx(c.scan, scan_tmp_words(n) + 2 * (size_t)n + 8) +
                              reach_bytes((uint32_t)std::max<size_t>(c.nb, nb), (uint32_t)std::max<size_t>(c.wg, W), 64);
         if (keep > budget && P->held > 0) {
             HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
@@ -2599,7 +2697,8 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         dfree(P->d_Lrp);
         dfree(P->d_Urp);
         dfree(P->d_rowfill);
-        dfree(P->d_row_fk);
+        dfree(P->d_cnt64);
+        dfree(P->d_rptr);
         e |= dalloc(&P->d_rp, rows);
         e |= dalloc(&P->d_rpT, rows);
         e |= dalloc(&P->d_cntL, rows);
@@ -2607,7 +2706,8 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         e |= dalloc(&P->d_Lrp, rows);
         e |= dalloc(&P->d_Urp, rows);
         e |= dalloc(&P->d_rowfill, rows);
-        e |= dalloc(&P->d_row_fk, rows);
+        e |= dalloc(&P->d_cnt64, rows);
+        e |= dalloc(&P->d_rptr, rows);
         c.rp = rows;
     }
     if (c.ci < ne) {
@@ -2617,25 +2717,21 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         e |= dalloc(&P->d_ciT, ne);
         c.ci = ne;
     }
-    const size_t nfe = (size_t)rch_fill_room(nf);
+    const size_t nfe = (size_t)(2 * nr);
     if (c.fills < nfe) {
-        dfree(P->d_fills);
-        e |= dalloc(&P->d_fills, nfe);
+        P->fill_cap = nfe;
+        e |= alloc_stream(P, nr);
         c.fills = nfe;
     }
     const size_t nle = (size_t)std::max<uint64_t>(nl, 1), nue = (size_t)std::max<uint64_t>(nu, 1);
     if (c.L < nle) {
         dfree(P->d_Lcol);
-        dfree(P->d_Ltmp);
         e |= dalloc(&P->d_Lcol, nle);
-        e |= dalloc(&P->d_Ltmp, nle);
         c.L = nle;
     }
     if (c.U < nue) {
         dfree(P->d_Ucol);
-        dfree(P->d_Utmp);
         e |= dalloc(&P->d_Ucol, nue);
-        e |= dalloc(&P->d_Utmp, nue);
         c.U = nue;
     }
     P->scan_words = scan_tmp_words(n) + 2 * (size_t)n + 8;
@@ -2655,6 +2751,8 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     }
     if (c.chunks < nchunks) {
         dfree(P->d_chunks);
+        dfree(P->d_grp);
+        e |= dalloc(&P->d_grp, (size_t)nchunks);
         e |= dalloc(&P->d_chunks, (size_t)nchunks);
         c.chunks = nchunks;
     }
@@ -2684,14 +2782,13 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         HIPCHK(hipMemsetAsync(P->d_rmask, 0, 16 * nbw, P->stream));
         HIPCHK(hipMemsetAsync(P->d_bstate, 0, sizeof(uint32_t) * c.nb, P->stream));
     }
-    P->held = (int64_t)(c.rp * (4 + 4 + 4 + 4 + 8 + 8 + 8 + 8) + c.ci * 8 + c.fills * 8 + c.L * 8 + c.U * 8 +
-                        c.scan * 8 + c.mats * 20 + c.chunks * sizeof(BlkChunk) + sizeof(Ctrl)) +
+    P->held = (int64_t)(c.rp * (4 + 4 + 4 + 4 + 8 + 8 + 8 + 8 + 8) + c.ci * 8 + c.fills * 24 + c.L * 4 + c.U * 4 +
+                        c.scan * 8 + c.mats * 20 + c.chunks * (sizeof(BlkChunk) + 16) + sizeof(Ctrl)) +
               quot_held(P->qcap) + reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64);
     P->W = (uint32_t)c.wg;  // the kernels' per-workgroup stride
     P->nblocks = nb;
     P->C = (int32_t)(nb * P->S);
-    P->fill_cap = nfe;
-    P->fill_need = nf;
+    P->fill_cap = c.fills;
     P->Lcap = (int64_t)c.L;
     P->Ucap = (int64_t)c.U;
     P->bounded = true;
@@ -2748,7 +2845,7 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
     r->row_fill = (int64_t*)malloc(sizeof(int64_t) * (size_t)std::max(nb, 1));
     if (!r->row_fill) return GSOFA_ERR_ALLOC;
     if (!P->structure) {  // counts only: the kernels' per-row tallies
-        HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_row_fk + b0, sizeof(int64_t) * (size_t)nb, hipMemcpyDeviceToHost,
+        HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill + b0, sizeof(int64_t) * (size_t)nb, hipMemcpyDeviceToHost,
                                   P->stream), P->stream);
         HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
         r->te_alg = te;

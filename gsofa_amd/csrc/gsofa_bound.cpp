@@ -53,11 +53,13 @@ int32_t find_root(std::vector<int32_t>& anc, int32_t x) {
 }  // namespace
 
 // rp/ci: packed rows (sorted, duplicate-free), n rows.  On return
-// Lb[i] >= |L_i|, Ub[i] >= |U_i| (both strict, A's own entries included).
+// Lb[i] >= |L_i|, Ub[i] >= |U_i| (both strict, A's own entries included); the
+// elimination tree of A + A^T goes to *parent_out if given.
 void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int64_t>& Lb,
-                   std::vector<int64_t>& Ub) {
+                   std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out) {
     Lb.assign((size_t)n, 0);
     Ub.assign((size_t)n, 0);
+    if (parent_out) parent_out->clear();
     if (n <= 0) return;
     // S's strictly lower entries as (hi, lo) pairs, in two layouts:
     // by hi (row hi's lower neighbours) and by lo (column lo's rows below)
@@ -162,6 +164,28 @@ void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<
     for (int32_t j = 0; j < n; j++)  // subtree sums: children precede parents
         if (parent[(size_t)j] >= 0) w[(size_t)parent[(size_t)j]] += w[(size_t)j];
     for (int32_t j = 0; j < n; j++) Ub[(size_t)j] = w[(size_t)j];
+    if (parent_out) parent_out->swap(parent);
+}
+
+// Records of one reach-mode pass at most (per mask word of 64 or 32 sources, a
+// record for every vertex that a group of `bits` sources reaches at or above
+// itself; groups are cut from each matrix's last vertex down).  A source's
+// vertices above it lie in its column of C, and a column's entries but the
+// parent lie in the parent's column, so a group reaches its own vertices and
+// the columns of those whose parent is outside the group.
+uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
+                            const std::vector<int64_t>& Ub, int bits) {
+    uint64_t sum = 0;
+    for (size_t b = 0; b + 1 < mat_base.size(); b++) {
+        for (int64_t hi = (int64_t)mat_base[b + 1]; hi > (int64_t)mat_base[b]; hi -= bits) {
+            const int64_t lo = std::max<int64_t>(hi - bits, (int64_t)mat_base[b]);
+            uint64_t items = (uint64_t)(hi - lo);
+            for (int64_t j = lo; j < hi; j++)
+                if (parent[(size_t)j] < 0 || parent[(size_t)j] >= hi) items += (uint64_t)Ub[(size_t)j];
+            sum += items;
+        }
+    }
+    return sum * (uint64_t)(bits > 64 ? bits / 64 : 1);
 }
 
 }  // namespace gsofa

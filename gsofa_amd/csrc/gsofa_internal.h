@@ -56,7 +56,9 @@ int validate_matrix(const gsofa_matrix* A);
 // from the elimination tree of A + A^T (gsofa_bound.cpp).  rp/ci are packed
 // rows, sorted and duplicate-free.
 void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int64_t>& Lb,
-                   std::vector<int64_t>& Ub);
+                   std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out = nullptr);
+uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
+                            const std::vector<int64_t>& Ub, int bits);
 
 constexpr int kBlockSlots = 32;      // largest source-slot count per workgroup in block mode
 constexpr int kBatchSlots = 16;      // slots per workgroup for batches of matrices by default
@@ -168,12 +170,13 @@ struct RchParams {
     void* vis;             // nblocks * W visited words (8 B at 32 slots, 16 B at 64)
     void* nmask;           // nblocks * 2 * W slot masks, this level's and the next's (slots/8 B each)
     uint4* q;              // nblocks * 2 * W frontier entries (v, row begin, row end, -)
-    uint64_t* fills;       // entries a workgroup reserved but did not use hold ~0 (set before launch)
-    uint64_t fill_cap;     // 0: count fills per row without writing the fill stream
-    uint32_t fill_blk;     // fill-stream entries a workgroup reserves at once (rch_fill_block)
-    Ctrl* ctrl;
+    uint4* rec;            // records (vertex, first source, mask of 64 or 32 sources), see gsofa_rows.hip
+    uint64_t rec_cap;      // 0: counts only, no records
+    uint4* grp;            // per chunk: its records' start (two words) and their count per mask word
+    Ctrl* ctrl;            // fill_pos: records reserved
     uint32_t* bstate;      // per workgroup: stamp of its last mini-group
-    unsigned long long* row_fills;  // counts only: fills per row, added by both passes (zeroed first)
+    uint32_t* cntU;        // n: U entries of each row
+    unsigned long long* cntL;  // n: L entries of each row, its L records in the high half (zeroed first)
     unsigned long long* mat_te;     // per matrix TE and |R| of the A pass (zeroed first), or null
     unsigned long long* mat_reach;
     uint32_t loops;        // stamps per workgroup before its visited words are cleared
@@ -184,14 +187,11 @@ bool rch_bits_valid(int bits);
 const void* rch_kernel_ptr(int bits, int threads);
 int64_t reach_bytes(uint32_t nb, uint32_t W, int bits);
 uint32_t rch_pass_bit();
-// Fill-stream room of a reach-mode run whose fills are at most `need`: its
-// workgroups reserve the stream in blocks and may leave part of each unused
-// (at most a sixteenth of a block, and the last block of each workgroup).
-// rch_fill_room holds for any grid of up to 1024 workgroups whose block size
-// comes from rch_fill_block(need, nblocks).
+// Output reserve, in 8-byte entries, that a reach-mode run with these fills is
+// accounted with: never below what its records take (reach_reserve).
 uint64_t rch_fill_room(uint64_t need);
+uint64_t reach_reserve(uint64_t fills, uint64_t lu, uint64_t records);
 int64_t rch_visit_bytes(int bits);  // visited word of a reach workgroup: 8, 16 or 32 B
-uint32_t rch_fill_block(uint64_t need, uint32_t nblocks);
 hipError_t launch_reach(const RchParams& p, int bits, int threads, hipStream_t s);
 int reach_resident(int device, int threads, uint32_t* out);
 int reach_threads(const gsofa_options& o);  // 0 -> 1024
@@ -252,6 +252,7 @@ struct PackedMatrix {
     int64_t nnz = 0;
     std::vector<int32_t> rp, ci, rpT, ciT;
     uint64_t need_fill = 0, need_L = 0, need_U = 0;
+    uint64_t need_rec = 0;  // records of one pass
 };
 int pack_matrix(const gsofa_matrix* A, PackedMatrix* M);
 // Arena: a reach-mode plan that takes one batch after another in its own
@@ -266,6 +267,35 @@ int64_t arena_held_bytes(const gsofa_plan* P);
 // workgroups, and per traversal workgroup.
 int64_t reach_fixed_bytes(int64_t n, int64_t nnz, int32_t n_mats, uint64_t nchunks, uint64_t fills,
                           uint64_t lu);
+// Rows from a reach-mode run's records (gsofa_rows.hip).
+struct RowParams {
+    int32_t n;
+    const int32_t* rp;
+    const int32_t* ci;
+    const BlkChunk* chunks;
+    uint32_t n_chunks;     // A-pass chunks at even places, their A^T twins behind them
+    uint32_t slots;        // sources of a mask word: 64 or 32
+    uint32_t words;        // mask words of a mini-group
+    const uint4* rec;
+    const uint4* grp;
+    const uint32_t* cntU;
+    unsigned long long* cntL;
+    int64_t* row_fill;
+    int64_t* sums;         // row_sum_words(n) (null: counts only)
+    int64_t* L_rowptr;
+    int64_t* U_rowptr;
+    int64_t* R_ptr;        // n + 1: offsets of the rows' record lists
+    uint4* list;           // the lists
+    int64_t list_cap;
+    int32_t* L_col;
+    int32_t* U_col;
+    int64_t L_cap, U_cap;  // entries allocated: no write beyond
+};
+size_t row_sum_words(int64_t n);
+hipError_t launch_row_fills(const RowParams& p, hipStream_t s);
+hipError_t launch_row_ptrs(const RowParams& p, hipStream_t s);
+hipError_t launch_rows(const RowParams& p, hipStream_t s);
+
 struct FinalParams {
     int32_t n;
     const int32_t* rp;

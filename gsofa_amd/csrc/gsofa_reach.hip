@@ -43,13 +43,16 @@
 //        from level 1 on: level 0 expands the sources themselves, whose
 //        neighbours are A's own entries).
 //   Targets are unique within a round, so the visited word, the next-level
-//   mask and the queue append need no global atomics.  Fills go to the
-//   fill stream through blocks that a workgroup reserves with one global
-//   atomic and hands out to its waves from LDS (the reserved entries it
-//   leaves unused hold ~0, which the structure pass skips), so waves of the
-//   whole grid do not queue on one counter.  The round's counters
+//   mask and the queue append need no global atomics.  The round's counters
 //   alternate by parity and the level's by level parity, so a round costs two
 //   barriers and a level no more.
+// * Nothing is written per entry during the search.  A vertex above the group
+//   goes to a list when it is first reached; at the group's end the final
+//   visited word of each, and of the group's own vertices, is all entries of
+//   that vertex for the group.  The words become records (vertex, first
+//   source, mask of 64 sources), sorted by vertex with an LDS bitmap, from
+//   which gsofa_rows.hip writes the rows; the A pass also counts its rows' U
+//   entries, the A^T pass adds to its targets' L counts.
 // * Vertices below the block of the mini-group's lowest source are not walked
 //   one by one: strongly connected classes of block ranges stand for them
 //   (gsofa_quot.hip).  Combine maps each target below that block to its
@@ -251,6 +254,12 @@ struct MaskOps<M256> {
     }
 };
 
+// 64-bit word k of a mask.
+__device__ __forceinline__ uint64_t mask_word(uint32_t m, int) { return m; }
+__device__ __forceinline__ uint64_t mask_word(uint64_t m, int) { return m; }
+__device__ __forceinline__ uint64_t mask_word(u128 m, int k) { return (uint64_t)(k ? m >> 64 : m); }
+__device__ __forceinline__ uint64_t mask_word(const M256& m, int k) { return m.w[k]; }
+
 // OR into an LDS mask (128 and 256 slots: per 64-bit word that has bits).
 __device__ __forceinline__ void mask_or(uint32_t* p, uint32_t v) { atomicOr(p, v); }
 __device__ __forceinline__ void mask_or(uint64_t* p, uint64_t v) {
@@ -298,7 +307,9 @@ struct RLds {
     uint32_t hkey[H];                    // target + 1 (window-local); 0 = empty
     M hmask[H];                          // OR of the masks folded into the target this round
     uint16_t ent[H];                     // occupied hash slots in insertion order
-    unsigned long long s_fill[MaskOps<M>::BITS];  // counts only: U fills per slot (A pass)
+    uint32_t s_cnt[MaskOps<M>::BITS];    // A pass: U entries per slot
+    uint32_t wsum[16];                   // per-wave sums of a block scan
+    uint32_t nup, tmax;                  // vertices above the group reached so far; the largest
     unsigned long long acc[8];           // workgroup totals: fills, checks, -, expansions,
                                          // TE and |R| of the A pass, of the A^T pass
     unsigned long long cte, creach;      // the current mini-group's TE and |R|
@@ -307,10 +318,9 @@ struct RLds {
     uint32_t tcnt[2];                    // inserts of this round, by round parity
     uint32_t held[2];                    // some group holds unfolded edges, by round parity
     uint32_t chunk;
-    uint32_t fcur;                       // entries handed out of the current fill block
     uint32_t spn[2];                     // split vertices, by level parity
     uint4 sp[2][SPLIT_MAX];              // (vertex, row begin, row end, weight)
-    unsigned long long fbase;            // the block's first entry in the fill stream
+    unsigned long long rbase;            // the group's first record
 };
 
 // Hash slot of window-local target m, inserting it if new; FULLI when it is
@@ -525,12 +535,9 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
         S.hmask[i] = (M)0;
     }
     if (tid < 8) S.acc[tid] = 0;
-    const uint32_t fblk = p.fill_blk, fmax = p.fill_blk >> 4;  // block; largest batch served from it
     if (tid == 0) {
         S.qcnt[0] = S.qcnt[1] = 0;
         S.tcnt[0] = S.tcnt[1] = S.held[0] = S.held[1] = 0;
-        S.fcur = fblk;  // no block yet
-        S.fbase = 0;
         S.spn[0] = S.spn[1] = 0;
     }
     uint32_t rb = 0;  // round parity
@@ -540,8 +547,9 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             S.chunk = atomicAdd(&p.ctrl->src_next, 1u);
             S.cte = S.creach = 0;
             S.cursor[0] = S.cursor[1] = 0;
+            S.nup = S.tmax = 0;
         }
-        if (tid < (uint32_t)O::BITS) S.s_fill[tid] = 0;
+        if (tid < (uint32_t)O::BITS) S.s_cnt[tid] = 0;
         __syncthreads();
         const uint32_t ck = S.chunk;
         if (ck >= p.n_chunks) break;
@@ -580,6 +588,12 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             t.te += r1 - r0;
         }
         if (tid == 0) S.qcnt[0] = c.count;
+        // No vertex above the group is ever queued, so the queue arrays' entries
+        // past the group's largest source hold the list of those reached (in
+        // the first array) and its sorted copy (in the second).
+        const uint32_t fl = c.first - c.wb;
+        uint32_t* const ulist = reinterpret_cast<uint32_t*>(q0 + fl + 1u);
+        uint32_t* const slist = reinterpret_cast<uint32_t*>(q0 + W + fl + 1u);
         __syncthreads();
 
         uint32_t cur = 0;
@@ -614,12 +628,6 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             hv.pos = hv.end = 0u;
             hv.vm = (M)0;
             for (;;) {  // rounds, two barriers each
-                // a fresh fill block once the current one may not hold a
-                // batch; relax reads fbase and fcur only after the next barrier
-                if (tid == 0 && p.fill_cap != 0ull && S.fcur + fmax > fblk) {
-                    S.fbase = aadd64(&p.ctrl->fill_pos, fblk);
-                    S.fcur = 0;
-                }
                 rcombine<H, G, E, M>(S, hv, c, maskc, qc, qsize, size, S.sp[cur], cursor, rb, t);
                 if (hv.held && (lane % G) == 0u) atomicOr(&S.held[rb], 1u);
                 __syncthreads();
@@ -643,7 +651,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                     const uint32_t mg = m + c.wb;
                     M up = (M)0;
                     uint32_t r0 = 0, r1 = 0, wt = 0;
-                    bool enq = false;
+                    bool enq = false, above = false;
                     if (ok) {
                         const VW vw = vis[m];
                         const M mc = merges<M>() ? maskc[MS * m] : (M)0;
@@ -666,6 +674,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                             vis[m] = O::make(vv | nw, stamp);
                             const M bl = nw & above_mask<M>(mg, c.first, c.stride, c.count);
                             up = lev ? (nw & ~bl) : (M)0;  // level 0: A's own entries
+                            above = m > fl && !vv;
                             if (bl) {
                                 if (merges<M>() && lev != 0u && mc && r1 - r0 <= SPLIT_ROW) {
                                     // still queued for this level and not yet
@@ -697,36 +706,15 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                         qb = bcast0(qb);
                         if (enq) qn[qb + rank_in(em)] = make_uint4(m, r0, r1, wt);
                     }
-                    const uint32_t nf = O::popc(up);
-                    t.fills += nf;
-                    if (__ballot(nf != 0u)) {
-                        if (p.fill_cap != 0ull) {
-                            // (row << 32) | column, one reservation per wave:
-                            // from the workgroup's block, or (a batch larger
-                            // than a sixteenth of a block, or one that no
-                            // longer fits it) straight from the stream
-                            const uint32_t incl = wave_incl_scan(nf);
-                            const uint32_t total = __shfl(incl, WAVE - 1, WAVE);
-                            uint64_t fp = 0;
-                            if (lane == 0) {
-                                const uint32_t old = total <= fmax ? atomicAdd(&S.fcur, total) : FULLI;
-                                fp = (old != FULLI && old + total <= fblk) ? S.fbase + old
-                                                                           : aadd64(&p.ctrl->fill_pos, total);
-                            }
-                            fp = bcast0_64(fp) + (incl - nf);
-                            O::for_each_bit(up, [&](uint32_t j) {
-                                const uint32_t src = c.first - j * c.stride;
-                                const uint64_t pr = c.tpass ? (((uint64_t)mg << 32) | src)
-                                                            : (((uint64_t)src << 32) | mg);
-                                if (fp < p.fill_cap) p.fills[fp] = pr;
-                                fp++;
-                            });
-                        } else if (nf) {  // counts only: fills per row
-                            if (c.tpass) {
-                                aadd64(&p.row_fills[mg], nf);
-                            } else {
-                                O::for_each_bit(up, [&](uint32_t j) { atomicAdd(&S.s_fill[j], 1ull); });
-                            }
+                    t.fills += O::popc(up);
+                    const uint64_t um = __ballot(above);
+                    if (um) {
+                        uint32_t ub = 0;
+                        if (lane == 0) ub = atomicAdd(&S.nup, (uint32_t)__popcll(um));
+                        ub = bcast0(ub);
+                        if (above) {
+                            ulist[ub + rank_in(um)] = m;
+                            atomicMax(&S.tmax, m);
                         }
                     }
                 }
@@ -763,8 +751,90 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
                 aadd64(&p.mat_reach[c.mat], S.creach);
             }
         }
-        if (p.fill_cap == 0ull && !c.tpass && tid < c.count && S.s_fill[tid])
-            aadd64(&p.row_fills[c.first - tid * c.stride], S.s_fill[tid]);
+        // ---- the group's entries, from the final visited words: items are the
+        // group's own vertices in increasing order, then those above it
+        constexpr int NW = O::BITS > 64 ? O::BITS / 64 : 1;
+        const uint32_t nup = S.nup, items = c.count + nup;
+        const bool rec = p.rec_cap != 0ull;
+        if (rec) {
+            // sorted by LDS bitmap windows over the vertices from fl + 1 on
+            // (the target table's masks, all zero between rounds)
+            uint32_t* bm = reinterpret_cast<uint32_t*>(S.hmask);
+            constexpr uint32_t BW = (uint32_t)(H * sizeof(M) / 4);
+            const uint32_t all = nup ? ((S.tmax - fl - 1u) >> 5) + 1u : 0u;
+            uint32_t sorted = 0;
+            for (uint32_t w0 = 0; w0 < all; w0 += BW) {
+                const uint32_t nw = all - w0 < BW ? all - w0 : BW;
+                for (uint32_t i = tid; i < nup; i += RB) {
+                    const uint32_t o = ulist[i] - fl - 1u;
+                    if ((o >> 5) - w0 < nw) atomicOr(&bm[(o >> 5) - w0], 1u << (o & 31u));
+                }
+                __syncthreads();
+                const uint32_t per = (nw + RB - 1u) / RB;
+                const uint32_t b0 = tid * per < nw ? tid * per : nw;
+                const uint32_t b1 = b0 + per < nw ? b0 + per : nw;
+                uint32_t cnt = 0;
+                for (uint32_t b = b0; b < b1; b++) cnt += (uint32_t)__popc(bm[b]);
+                const uint32_t incl = wave_incl_scan(cnt);
+                if (lane == WAVE - 1) S.wsum[w] = incl;
+                __syncthreads();
+                uint32_t pos = sorted + incl - cnt;
+                for (uint32_t k = 0; k < (uint32_t)(RB / WAVE); k++) {
+                    if (k < w) pos += S.wsum[k];
+                    sorted += S.wsum[k];
+                }
+                for (uint32_t b = b0; b < b1; b++) {
+                    for (uint32_t x = bm[b]; x; x &= x - 1u)
+                        slist[pos++] = fl + 1u + ((w0 + b) << 5) + (uint32_t)__builtin_ctz(x);
+                    bm[b] = 0u;
+                }
+                __syncthreads();
+            }
+            if (tid == 0) {
+                const unsigned long long o = aadd64(&p.ctrl->fill_pos, (unsigned long long)NW * items);
+                const bool fits = o + (unsigned long long)NW * items <= p.rec_cap;
+                S.rbase = fits ? o : ~0ull;
+                p.grp[ck] = make_uint4((uint32_t)o, (uint32_t)(o >> 32), fits ? items : 0u, 0u);
+            }
+            __syncthreads();
+        }
+        const uint64_t r0 = rec ? S.rbase : ~0ull;
+        const uint32_t* up_list = rec ? slist : ulist;
+        uint32_t acc[NW] = {};
+        for (uint32_t i0 = w * WAVE; i0 < items; i0 += RB) {
+            const uint32_t i = i0 + lane;
+            uint32_t m = 0;
+            M mk = (M)0;
+            if (i < items) {
+                m = i < c.count ? fl - (c.count - 1u - i) : up_list[i - c.count];
+                mk = O::get(vis[m], stamp);
+                if (i < c.count) mk = mk & ~O::prefix(c.count - i);  // sources below the vertex
+            }
+#pragma unroll
+            for (int k = 0; k < NW; k++) {
+                const uint64_t wd = mask_word(mk, k);
+                if (i < items) {
+                    if (r0 != ~0ull)
+                        p.rec[r0 + (uint64_t)k * items + i] =
+                            make_uint4(c.wb + m, c.first - 64u * (uint32_t)k, (uint32_t)wd, (uint32_t)(wd >> 32));
+                    if (c.tpass && wd) aadd64(&p.cntL[c.wb + m], (1ull << 32) | (unsigned long long)__popcll(wd));
+                }
+                if (!c.tpass) {
+#pragma unroll
+                    for (int j = 0; j < (O::BITS < 64 ? O::BITS : 64); j++) {
+                        const uint32_t n = (uint32_t)__popcll(__ballot((wd >> j) & 1ull));
+                        if (lane == (uint32_t)j) acc[k] += n;
+                    }
+                }
+            }
+        }
+        if (!c.tpass) {
+#pragma unroll
+            for (int k = 0; k < NW; k++)
+                if (acc[k]) atomicAdd(&S.s_cnt[64 * k + (int)lane], acc[k]);
+            __syncthreads();
+            if (tid < c.count) p.cntU[c.first - tid * c.stride] = S.s_cnt[tid];
+        }
         __syncthreads();
     }
     if (t.fills) atomicAdd(&S.acc[0], t.fills);
@@ -828,21 +898,7 @@ int64_t reach_bytes(uint32_t nb, uint32_t W, int bits) {
     return (int64_t)nb * ((vw + 2 * mw + 32) * (int64_t)W + 8);
 }
 
-// Every block a workgroup gives up held more than 15/16 of a block of fills:
-// a batch is served from a block only if it is at most a sixteenth of it,
-// and the block is given up once the rest may not hold such a batch.  With
-// its last block, a workgroup's fill-stream span is below 16/15 of its fills
-// plus one block; over the grid, below 16/15 need + nblocks * block.  The
-// block size keeps nblocks * block within need/8 + 2^20, which
-// rch_fill_room covers (the 64-entry floor keeps that for nblocks <= 16384).
-uint32_t rch_fill_block(uint64_t need, uint32_t nblocks) {
-    const uint64_t nb = std::max<uint32_t>(nblocks, 1u);
-    uint32_t blk = 1u << 16;
-    while (blk > 64u && nb * blk > need / 8 + (1ull << 20)) blk >>= 1;
-    return blk;
-}
 int64_t rch_visit_bytes(int bits) { return bits == 256 ? 48 : bits == 128 ? 32 : bits == 64 ? 16 : 8; }
-uint64_t rch_fill_room(uint64_t need) { return need + need / 15 + need / 8 + (1ull << 20) + 1; }
 
 hipError_t launch_reach(const RchParams& p, int bits, int threads, hipStream_t s) {
     if (!rch_bits_valid(bits) || !rch_threads_valid(threads)) return hipErrorInvalidValue;
