@@ -1034,17 +1034,15 @@ int choose_bits(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* bits
         return GSOFA_OK;
     }
     uint32_t nb = 0;
-    int rc = reach_resident(o.device, reach_threads(o), &nb);
+    int rc = reach_resident(o.device, o.workgroup_threads != 0 ? o.workgroup_threads : 1024, &nb);
     if (rc) return rc;
     *bits = (nsrc + 63) / 64 >= nb ? 64 : 32;
     return GSOFA_OK;
 }
 
-int reach_threads(const gsofa_options& o) { return o.workgroup_threads != 0 ? o.workgroup_threads : 1024; }
-
 int reach_resident(int device, int threads, uint32_t* out) {
     int occ = 0, cus = 0;
-    if (!rch_threads_valid(threads)) return GSOFA_ERR_INVALID;
+    if (!rch_shape_valid(threads)) return GSOFA_ERR_INVALID;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, rch_kernel_ptr(64, threads), threads, 0) != hipSuccess ||
         occ <= 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         (void)hipGetLastError();
@@ -1054,11 +1052,25 @@ int reach_resident(int device, int threads, uint32_t* out) {
     return GSOFA_OK;
 }
 
-// As block_grid, for the reach kernel's per-workgroup arrays.
-int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint32_t W, int64_t avail, uint32_t* nb_out) {
+// As block_grid, for the reach kernel's per-workgroup arrays; also the
+// workgroup shape.  records: of one pass, at most (0: unknown).
+int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint32_t W, int64_t avail,
+               uint32_t* nb_out, int* threads_out) {
+    if (o.workgroup_threads != 0 && !rch_threads_valid(o.workgroup_threads)) return GSOFA_ERR_INVALID;
     if (o.mem_budget_bytes > 0) avail = std::min<int64_t>(avail, o.mem_budget_bytes);
+    int threads = o.workgroup_threads;
+    if (threads == 0) {
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess) {
+            (void)hipGetLastError();
+            return GSOFA_ERR_HIP;
+        }
+        const uint64_t groups = std::max<uint64_t>(nchunks / 2, 1) * (uint64_t)std::max(bits / 64, 1);
+        threads = reach_shape(nchunks, records ? records / groups : UINT64_MAX, W, bits, (uint32_t)cus, avail);
+    }
+    *threads_out = threads;
     uint32_t nb = 0;
-    const int rc = reach_resident(o.device, reach_threads(o), &nb);
+    const int rc = reach_resident(o.device, threads, &nb);
     if (rc) return rc;
     if (o.grid_blocks > 0) nb = std::min<uint32_t>(nb, (uint32_t)o.grid_blocks);
     if (o.chunk > 0) nb = std::min<uint32_t>(nb, (uint32_t)std::max(1, o.chunk / bits));
@@ -1144,7 +1156,8 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         output_need(w, A->n, rp.data(), ci.data(), &nf, &nl, &nu, bits, &mb, &nr);
         nf = reach_reserve(nf, nl + nu, nr);
         uint32_t nb = 0;
-        if (reach_grid(o, bits, nchunks, (uint32_t)A->n, INT64_MAX / 4, &nb) != GSOFA_OK) return -1;
+        int threads = 0;
+        if (reach_grid(o, bits, 2 * nchunks, nr, (uint32_t)A->n, INT64_MAX / 4, &nb, &threads) != GSOFA_OK) return -1;
         const uint32_t ql = quot_wanted(A->n, (int64_t)ci.size(), (uint32_t)A->n,
                                         o.mem_budget_bytes > 0 ? o.mem_budget_bytes : INT64_MAX / 4);
         return reach_bytes(nb, (uint32_t)A->n, bits) +
@@ -1316,7 +1329,6 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     if (P->mode == GSOFA_MODE_REACH) {
         const int bits = P->rbits;
         P->S = (uint32_t)bits;
-        P->rthreads = reach_threads(P->opt);
         {
             // the A pass's chunks, deepest first, each followed by the same
             // sources' chunk of the A^T pass: one launch runs both
@@ -1339,7 +1351,8 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room);
             const int64_t qb = qlev ? quot_bytes(n, P->nnz, P->W) : 0;
             if (go.mem_budget_bytes > 0) go.mem_budget_bytes -= qb;
-            rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), P->W, room - qb, &P->nblocks);
+            rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), need_rec, P->W, room - qb, &P->nblocks,
+                            &P->rthreads);
         }
         if (rc) {
             (void)hipStreamDestroy(P->stream);
@@ -2664,9 +2677,8 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     o.mem_budget_bytes = 0;
     const uint32_t qlev = quot_wanted(n, nnz, W, budget - fixed);
     const int64_t qb = qlev ? quot_bytes(n, nnz, W) : 0;
-    int rc = reach_grid(o, bits, nchunks, W, budget - fixed - qb, &nb);
+    int rc = reach_grid(o, bits, nchunks, nr, W, budget - fixed - qb, &nb, &P->rthreads);
     if (rc) return rc;
-    P->rthreads = reach_threads(o);
     gsofa_plan::Caps& c = P->cap;
     const size_t rows = (size_t)n + 1;
     const size_t ne = (size_t)std::max<int64_t>(nnz + (int64_t)quot_ext((uint64_t)nnz, qlev), 1);

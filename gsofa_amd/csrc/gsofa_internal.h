@@ -182,7 +182,9 @@ struct RchParams {
     uint32_t loops;        // stamps per workgroup before its visited words are cleared
     QuotParams quot;       // levels == 0: no classes, every vertex is walked
 };
-bool rch_threads_valid(int threads);  // threads per reach workgroup: 1024 or 512
+bool rch_threads_valid(int threads);  // a caller's choice of threads per reach workgroup: 1024 or 512
+bool rch_shape_valid(int threads);    // any shape there is: 256 too
+int reach_shape(uint64_t chunks, uint64_t reach, uint32_t W, int bits, uint32_t cus, int64_t room);
 bool rch_bits_valid(int bits);
 const void* rch_kernel_ptr(int bits, int threads);
 int64_t reach_bytes(uint32_t nb, uint32_t W, int bits);
@@ -194,14 +196,14 @@ uint64_t reach_reserve(uint64_t fills, uint64_t lu, uint64_t records);
 int64_t rch_visit_bytes(int bits);  // visited word of a reach workgroup: 8, 16 or 32 B
 hipError_t launch_reach(const RchParams& p, int bits, int threads, hipStream_t s);
 int reach_resident(int device, int threads, uint32_t* out);
-int reach_threads(const gsofa_options& o);  // 0 -> 1024
 int resolve_mode(const gsofa_options& o);
 // Tuned knobs (gsofa_amd/tune.py's table) for a workload: its signature, and
 // the entry applied to options left at their defaults (true if one applied).
 std::string tune_signature(int64_t n_max, int64_t nnz, int64_t n_total, int32_t n_mats);
 bool apply_tuned(gsofa_options* o, int64_t n_max, int64_t nnz, int64_t n_total, int32_t n_mats);
 int choose_bits(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* bits);
-int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint32_t W, int64_t avail, uint32_t* nb_out);
+int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint32_t W, int64_t avail,
+               uint32_t* nb_out, int* threads_out);
 void transpose_rows(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int32_t>& rpT,
                     std::vector<int32_t>& ciT);
 

@@ -77,29 +77,30 @@ using namespace dev;
 
 // Workgroup shapes (threads, hash slots of the target table; a round takes
 // at most half the slots in new targets, so the load stays below 1/2 +
-// threads/slots):
+// threads/slots).  16 waves share a CU in each:
 //   wide: one 1024-thread workgroup per CU and the largest table that fits
 //         the CU's 160 KB of LDS at 64 slots: fewest rounds per level;
 //   pair: two 512-thread workgroups per CU with half the table each: one
-//         workgroup runs while the other waits at a barrier.
+//         workgroup runs while the other waits at a barrier;
+//   quad: four 256-thread workgroups per CU with a quarter of it, where a
+//         level's frontier is a few hundred targets and barriers are most of
+//         its time.
+// reach_shape picks one.
 constexpr int NT_WIDE = 1024, NH_WIDE = 11264;
 constexpr int NT_PAIR = 512, NH_PAIR = 5632;
+constexpr int NT_QUAD = 256, NH_QUAD = 2656;
 constexpr uint32_t FULLI = 0xFFFFFFFFu;
 constexpr uint32_t PASS_T = 0x80000000u;  // chunk stride bit: the A^T pass
-// Lane groups: 256 per workgroup, each taking 12 edges of its vertex per
-// step: 4 lanes x 3 edges at 1024 threads, 2 lanes x 6 edges at 512 (256
-// groups measured faster than 128 or 512 at either size).  GSOFA_RG and
-// GSOFA_RE, when defined at build time, set one shape for both.
-#ifndef GSOFA_RG
-#define GSOFA_RG 0
-#endif
-#ifndef GSOFA_RE
-#define GSOFA_RE 0
-#endif
+// Lane groups: lanes per vertex and edges per lane and step.  Execute ms with
+// (48^3 grid, 128 2D grids, band n = 659,033, 64 slots) at pair 2 x 6: 3.82,
+// 25.0, 7.6; 4 x 3: 3.22, 19.7, 6.6; 8 x 2: 2.89, 17.1, 6.4; 16 x 1: 2.92,
+// 18.7, 7.2.  At quad 2 x 6: 4.23, 16.0, 6.1; 4 x 3: 3.69, 13.6, 5.7; 8 x 2:
+// 3.53, 12.9, 6.0; 16 x 1: 3.58, 15.2, 7.0.  At wide, which runs the few
+// groups of small matrices, 4 x 3 takes 0.50 ms on a 64^2 grid, 16 x 1 0.55.
 template <int NT>
-constexpr int lanes_per_vertex() { return GSOFA_RG > 0 ? GSOFA_RG : NT / 256; }
+constexpr int lanes_per_vertex() { return NT == NT_PAIR ? 8 : 4; }
 template <int NT>
-constexpr int edges_per_lane() { return GSOFA_RE > 0 ? GSOFA_RE : 12 / lanes_per_vertex<NT>(); }
+constexpr int edges_per_lane() { return NT == NT_PAIR ? 2 : 3; }
 
 template <class M>
 struct MaskOps;
@@ -291,9 +292,11 @@ constexpr bool merges() { return sizeof(M) <= 8; }
 // table that fits the CU's LDS (4 B key, the mask, 2 B entry per slot).
 template <class M>
 constexpr int tab_slots(int threads) {
-    return sizeof(M) == 32   ? (threads == NT_WIDE ? 4224 : 2048)
-           : sizeof(M) == 16 ? (threads == NT_WIDE ? 7168 : 3584)
-                             : (threads == NT_WIDE ? NH_WIDE : NH_PAIR);
+    return sizeof(M) == 32   ? (threads == NT_WIDE ? 4224 : threads == NT_PAIR ? 2048 : 960)
+           : sizeof(M) == 16 ? (threads == NT_WIDE ? 7168 : threads == NT_PAIR ? 3584 : 1696)
+           : threads == NT_WIDE ? NH_WIDE
+           : threads == NT_PAIR ? NH_PAIR
+                                : NH_QUAD;
 }
 
 // Rows longer than SPLIT_ROW are expanded by SPLIT_PARTS lane groups instead of
@@ -860,6 +863,30 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
 bool rch_bits_valid(int bits) { return bits == 32 || bits == 64 || bits == 128 || bits == 256; }
 bool rch_threads_valid(int threads) { return threads == NT_WIDE || threads == NT_PAIR; }
 
+bool rch_shape_valid(int threads) { return rch_threads_valid(threads) || threads == NT_QUAD; }
+
+// The shape for `chunks` mini-groups (both passes) of matrices of up to W
+// vertices, whose groups reach `reach` vertices at or above themselves on
+// average (from the record bound), on `cus` CUs:
+//   wide  while every mini-group has a CU of its own;
+//   quad  where several mini-groups queue per CU and they are narrow;
+//   pair  otherwise.
+// More workgroups hold more per-vertex arrays, so a shape is taken only while
+// those stay within `room` bytes (quad 8 GiB, pair half the room and 32 GiB);
+// pair's 256-slot kernel has registers for one workgroup per CU.  Execute ms at wide /
+// pair / quad: 64^2 grid (256 mini-groups) 0.50 / 0.56 / 0.68; 181^2 grid
+// (1,024) 1.10 / 0.83 / 0.90; 33^3 (1,124) 1.70 / 1.42 / 1.85; 48^3 (3,456 of
+// about 1,600 vertices) 3.69 / 2.89 / 3.53; band n = 100,003 (3,126 of about
+// 400) 1.54 / 1.23 / 1.18; 128 2D grids (64,800 of about 250) 32.9 / 17.1 /
+// 13.6.
+int reach_shape(uint64_t chunks, uint64_t reach, uint32_t W, int bits, uint32_t cus, int64_t room) {
+    if (chunks <= cus) return NT_WIDE;
+    const int64_t quad = reach_bytes((uint32_t)std::min<uint64_t>(4ull * cus, chunks), W, bits);
+    if (chunks >= 8ull * cus && reach <= 512 && quad <= std::min<int64_t>(room, 8ll << 30)) return NT_QUAD;
+    const int64_t pair = reach_bytes((uint32_t)std::min<uint64_t>(2ull * cus, chunks), W, bits);
+    return bits < 256 && pair <= std::min<int64_t>(room / 2, 32ll << 30) ? NT_PAIR : NT_WIDE;
+}
+
 namespace {
 template <int NT, class M>
 const void* kptr() {
@@ -888,7 +915,7 @@ void klaunch_bits(const RchParams& p, int bits, hipStream_t s) {
 }  // namespace
 
 const void* rch_kernel_ptr(int bits, int threads) {
-    return threads == NT_PAIR ? kptr_bits<NT_PAIR>(bits) : kptr_bits<NT_WIDE>(bits);
+    return threads == NT_QUAD ? kptr_bits<NT_QUAD>(bits) : threads == NT_PAIR ? kptr_bits<NT_PAIR>(bits) : kptr_bits<NT_WIDE>(bits);
 }
 uint32_t rch_pass_bit() { return PASS_T; }
 // Per workgroup: visited words (8, 16 or 32 B), two next-level masks, two
@@ -901,8 +928,9 @@ int64_t reach_bytes(uint32_t nb, uint32_t W, int bits) {
 int64_t rch_visit_bytes(int bits) { return bits == 256 ? 48 : bits == 128 ? 32 : bits == 64 ? 16 : 8; }
 
 hipError_t launch_reach(const RchParams& p, int bits, int threads, hipStream_t s) {
-    if (!rch_bits_valid(bits) || !rch_threads_valid(threads)) return hipErrorInvalidValue;
-    if (threads == NT_PAIR) klaunch_bits<NT_PAIR>(p, bits, s);
+    if (!rch_bits_valid(bits) || !rch_shape_valid(threads)) return hipErrorInvalidValue;
+    if (threads == NT_QUAD) klaunch_bits<NT_QUAD>(p, bits, s);
+    else if (threads == NT_PAIR) klaunch_bits<NT_PAIR>(p, bits, s);
     else klaunch_bits<NT_WIDE>(p, bits, s);
     return hipGetLastError();
 }

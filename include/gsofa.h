@@ -106,7 +106,8 @@ typedef struct gsofa_options {
                                   /* 0 = 64, or 32 when fewer chunks than workgroups        */
     int32_t workgroup_threads;    /* reach mode: threads per workgroup, 1024 (one per CU,   */
                                   /* the largest target table) or 512 (two per CU, half    */
-                                  /* the table each); 0 = 1024                              */
+                                  /* the table each); 0 = chosen by the number and width   */
+                                  /* of the source groups (also 256, four per CU)           */
 } gsofa_options;
 
 /* Execution modes of the traversal (identical results):

@@ -106,3 +106,21 @@ def test_batch_of_sizes(kw):
                     np.testing.assert_array_equal(r.row_fill, o.row_fill)
                 else:
                     assert_same_structure(r, o)
+
+
+@pytest.mark.parametrize("bits", [32, 64, 128, 256])
+def test_narrow_groups(bits):
+    """Thousands of narrow mini-groups take four workgroups per CU."""
+    import gsofa_amd as g
+    if bits == 256:
+        mats = [g.gen_band(14001, 12, 3.0, s) for s in range(5)] * 4
+    else:
+        mats = [g.gen_grid(s, s, 1, nd_leaf=64, extra_prob=0.05, extra_dist=3, seed=s) for s in (3, 150, 171, 256)]
+        mats.append(g.gen_grid(257, 255, 1, nd_leaf=64, seed=9))
+    print("case: narrow groups, bits", bits, flush=True)
+    with g.Plan(mats, mode="reach", block_slots=bits) as p:
+        p.execute()
+        for b, A in enumerate(mats[:5]):
+            r = p.fetch_matrix(b)
+            assert r.grid_blocks > 512
+            assert_same_structure(r, _oracle(A))
