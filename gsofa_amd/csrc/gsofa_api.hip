@@ -75,7 +75,7 @@ struct gsofa_plan {
     // reach mode: classes of vertex ranges, rebuilt by every execute
     // (gsofa_quot.hip); levels 0: none
     QuotParams quot{};
-    struct QuotCaps {  // entries allocated: range table, levels * n, n, edge list
+    struct QuotCaps {  // entries allocated: range table, levels * n, n, edge lists
         size_t tab = 0, ln = 0, n = 0, eb = 0;
     } qcap;
     uint2* d_qtab = nullptr;
@@ -524,10 +524,9 @@ void release_quot(gsofa_plan* P) {
     dfree(q.comp);
     dfree(q.info);
     dfree(q.infoT);
-    dfree(q.nodes);
     dfree(q.ncnt);
+    dfree(q.blist);
     dfree(q.nmap);
-    dfree(q.nidx);
     dfree(q.eb);
     dfree(q.ctl);
     q = QuotParams{};
@@ -550,18 +549,21 @@ int setup_quot(gsofa_plan* P, uint32_t levels) {
     QuotParams& q = P->quot;
     q.levels = levels;
     if (levels == 0) return GSOFA_OK;
-    const size_t n = (size_t)P->n, ln = (size_t)levels * n, ne = (size_t)P->nnz;
+    const size_t n = (size_t)P->n, ln = (size_t)levels * n;
     q.n = (uint32_t)n;
     q.ext0 = (uint32_t)P->nnz;
     quot_table(P->h_mat_base, levels, P->h_qtab, P->h_qoff);
-    q.total0 = P->h_qoff[1] << kQuotShift;
+    q.judge = std::min(kQuotJudge, levels - 1u);
+    q.judged = (P->h_qoff[q.judge + 1] - P->h_qoff[q.judge]) << (kQuotShift + q.judge);
     gsofa_plan::QuotCaps& c = P->qcap;
     int e = 0;
     if (c.tab < P->h_qtab.size()) {
         dfree(P->d_qtab);
         dfree(q.ncnt);
         e |= dalloc(&P->d_qtab, P->h_qtab.size());
+        dfree(q.blist);
         e |= dalloc(&q.ncnt, P->h_qtab.size());
+        e |= dalloc(&q.blist, P->h_qtab.size());
         c.tab = P->h_qtab.size();
     }
     if (c.ln < ln) {
@@ -574,18 +576,14 @@ int setup_quot(gsofa_plan* P, uint32_t levels) {
         c.ln = ln;
     }
     if (c.n < n) {
-        dfree(q.nodes);
         dfree(q.nmap);
-        dfree(q.nidx);
-        e |= dalloc(&q.nodes, 2 * n);
-        e |= dalloc(&q.nmap, n);
-        e |= dalloc(&q.nidx, n);
+        e |= dalloc(&q.nmap, 2 * n);
         c.n = n;
     }
-    if (c.eb < ne) {
+    if (c.eb < (size_t)P->nnz) {
         dfree(q.eb);
-        e |= dalloc(&q.eb, ne);
-        c.eb = ne;
+        e |= dalloc(&q.eb, (size_t)P->nnz);
+        c.eb = (size_t)P->nnz;
     }
     if (!q.ctl) e |= dalloc(&q.ctl, 1);
     if (e) return GSOFA_ERR_ALLOC;
@@ -601,7 +599,7 @@ int setup_quot(gsofa_plan* P, uint32_t levels) {
 // Bytes of setup_quot's arrays at their capacities (the class rows in d_ci and
 // d_ciT apart).
 int64_t quot_held(const gsofa_plan::QuotCaps& c) {
-    return (int64_t)(12 * c.tab + 36 * c.ln + 16 * c.n + 4 * c.eb + sizeof(QuotCtl));
+    return (int64_t)(16 * c.tab + 36 * c.ln + 8 * c.n + 4 * c.eb + sizeof(QuotCtl));
 }
 
 void release_device(gsofa_plan* P) {

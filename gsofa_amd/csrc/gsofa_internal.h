@@ -113,41 +113,41 @@ hipError_t launch_traverse_blk(const BlkParams& p, int slots, size_t lds_bytes, 
 
 // Classes of vertex ranges (gsofa_quot.hip), built on the device at the start
 // of every reach-mode execute.
-constexpr uint32_t kQuotLevels = 26;  // kMaxN < 2^25
 // log2 of a block's vertices.  A source walks up to a block of single
 // vertices; each halving of the block adds a level of ranges to build.
-// Traversal ms at blocks of 128 / 256 / 512 / 1,024: 48^3 grid 3.29 / 3.27 /
-// 3.45 / 3.65, band n=659,033 6.34 / 5.71 / 5.77 / 6.53, 128 2D grids 31.7 /
-// 33.5 / 36.7 / 42.0, 64^2 natural order 0.405 / 0.398 / 0.456 / 0.598.
-constexpr uint32_t kQuotShift = 8;
+// Execute ms at blocks of 64 / 128 / 256: 48^3 grid 2.47 / 2.52 / 2.61, 128 2D
+// grids 11.4 / 11.6 / 12.9, 27^3 0.91 / 0.91 / 1.01, n = 11,948 band 0.40 /
+// 0.38 / 0.42, band n = 659,033 - / 4.83 / 4.67.
+constexpr uint32_t kQuotShift = 7;
 struct QuotCtl {
-    unsigned long long ext, extT;      // class-row entries handed out, over A and A^T
-    unsigned long long nodes0;         // classes of all level-0 ranges
-    unsigned long long eb[kQuotLevels];  // edge-list entries handed out, per level
+    unsigned long long nodes;          // classes of the judged level's ranges
+    uint32_t big[8];                   // ranges of a low level left to large workgroups
 };
 struct QuotParams {
     const int32_t* rp;
     const int32_t* rpT;
-    int32_t* ci;         // the matrix's columns, then the class rows from ext0 on
+    int32_t* ci;         // the matrix's columns (ext0 of them), then as many for each level's class rows
     int32_t* ciT;
     uint32_t n;          // all vertices (stride of the per-level arrays)
     uint32_t ext0;
     uint32_t levels;
-    uint32_t total0;     // vertices of the level-0 ranges
+    uint32_t judge;      // the level by whose classes quot_off judges
+    uint32_t judged;     // vertices of its ranges
     const uint2* tab;
-    int32_t* comp;       // levels * n: a vertex's class (a member vertex names it)
+    int32_t* comp;       // levels * n: a vertex's class, numbered from its range's first vertex on
     uint4* info;         // levels * n: of a class: row begin, row end, vertices, their row lengths
     uint4* infoT;        // the same over A^T
-    int32_t* nodes;      // 2 * n: the ranges' class lists, by level parity
     uint32_t* ncnt;      // per range of every level: its classes
-    int32_t* nmap;       // n
-    int32_t* nidx;       // n
-    uint32_t* eb;        // nnz
+    uint32_t* blist;     // ranges of a low level left to large workgroups
+    int32_t* nmap;       // 2 * n: class of a class of the level below, by level parity
+    uint32_t* eb;        // nnz: edge lists of those ranges
     QuotCtl* ctl;
 };
-// Contraction does not pay where the level-0 ranges keep over half of their
-// vertices as classes: the traversal then walks plain vertices.
-__device__ __forceinline__ bool quot_off(const QuotParams& p) { return 2ull * p.ctl->nodes0 > (unsigned long long)p.total0; }
+// Classes do not pay where ranges of 2^(kQuotShift + kQuotJudge) vertices keep
+// over half of them as classes: the traversal then walks plain vertices.
+// (Smaller ranges say little: a banded matrix has few edges within them.)
+constexpr uint32_t kQuotJudge = 3;
+__device__ __forceinline__ bool quot_off(const QuotParams& p) { return 2ull * p.ctl->nodes > (unsigned long long)p.judged; }
 uint32_t quot_levels(uint32_t W);
 uint64_t quot_ext(uint64_t nnz, uint32_t levels);
 int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W);

@@ -21,19 +21,23 @@
 //
 // Classes need not be maximal for the results to be right (any strongly
 // connected set will do), so the search for them is bounded: a range with too
-// many nodes keeps its halves' classes, and the label rounds below stop at a
-// fixed count.
+// many nodes keeps its halves' classes, and label rounds stop at a fixed count.
 //
-// What bounds it: latency.  A level is two launches; a range is a chain of
-// dependent gathers (column, class, node number) and barriers of one
-// workgroup, 20-100 us a level however many ranges it has, until ranges
-// outnumber the CUs.
+// What bounds it: latency.  A level is one launch; a range is a chain of
+// dependent gathers (row, column, class, class of the class) and barriers,
+// 15-20 us of one workgroup whatever its nodes, up to 50 us with rows of
+// thousands of targets.  So a range's nodes are closed as a bit matrix
+// (2.2 us for 64 nodes, 10 us for 128, 35 us for 256), lanes that share a row
+// step its cursor once, rows of a level lie where the matrix's rows lie (no
+// allocation), and the vertices' classes of one level are written behind the
+// ranges of the next.
 //
 // Measured, traversal of one execute walking vertices -> classes (the
-// classes' construction included): band n = 659,033 780 -> 5.8 ms, band
-// n = 100,003 32.3 -> 1.5, 48^3 grid 64.9 -> 3.3, 128 2D grids 278 -> 33.5,
-// 181^2 grid 16.4 -> 1.0, n = 11,948 1.13 -> 0.37.  At 48^3 the construction
-// takes 0.73 ms of the 3.3, at the 128 grids 1.8 of 33.5.
+// classes' construction included): band n = 659,033 780 -> 4.0 ms, band
+// n = 100,003 32.3 -> 0.71, 48^3 grid 64.9 -> 1.57, 128 2D grids 278 -> 10.0,
+// 181^2 grid 16.4 -> 0.68, n = 11,948 1.13 -> 0.24.  The construction with
+// label rounds for every range and two launches a level took 0.73 ms at 48^3,
+// now 0.36; at the 128 grids 1.8, now 0.8; at the band 1.45, now 0.45.
 #include <algorithm>
 
 #include "gsofa_device.h"
@@ -45,168 +49,174 @@ namespace {
 
 using dev::WAVE;
 
-constexpr uint16_t NOROOT = 0xFFFFu;
 constexpr uint32_t NOIDX = 0xFFFFFFFFu;
-constexpr int ROUNDS = 4;       // label rounds per range
-constexpr int ITERS = 96;       // label iterations per round, at most
+constexpr uint16_t INERT = 0xFFFFu;
 constexpr uint32_t SHORT_ROW = 64;   // rows up to here: 8 lanes each
-constexpr uint32_t MID_ROW = 2048;   // rows up to here: one wave each; longer ones: the workgroup
-constexpr int QBASE_CAP = 1 << kQuotShift;  // vertices of a level-0 range
-constexpr int QCAP = 4096;           // nodes of a higher range whose classes are merged
-constexpr int QBASE_NT = 256, QNT = 1024;
+constexpr uint32_t MID_ROW = 256;    // rows up to here: one wave each; longer ones: the workgroup
+constexpr int QN = 256;              // live nodes whose reachability is closed as a bit matrix
+constexpr int QM = 4096;             // nodes of a range, at most, if its halves' classes are to be merged
+// Ranges with more live nodes are rare where classes pay at all: sparse bands
+// near the bottom, before their main class forms.  At levels up to QBIG_LEVEL
+// they go to a few large workgroups that take up to QCAP by label rounds.
+constexpr int QCAP = 2048;
+constexpr uint32_t QBIG_LEVEL = 4, QBIG_GRID = 256;
+constexpr int ROUNDS = 4, ITERS = 96;  // label rounds of a range and iterations of a round, at most
+constexpr int QB = 1 << kQuotShift;  // vertices of a block
+constexpr int QNT = QB, QNT_LEVEL = 512, QNT_BIG = 1024;
+static_assert(QB <= QN && QB % WAVE == 0, "a block's vertices are the nodes of one bit matrix");
 
-template <int CAP>
+template <int N>
 struct QLds {
-    int32_t node[CAP];
-    uint32_t rb[CAP], re[CAP];      // the node's row
-    uint32_t fw[CAP], bw[CAP];      // labels; then the class's first member and size
-    uint32_t a0[CAP], a1[CAP], a2[CAP];  // class sums and row cursor
-    uint16_t root[CAP];
-    unsigned long long ebase;
-    uint32_t total, ne, left, got, nnew;
+    uint32_t rb[2 * N], re[2 * N];       // the live nodes' rows over A, then over A^T
+    uint32_t cnt[N], deg[2 * N];         // their vertices, their vertices' row lengths
+    uint16_t node[N];                    // live node k's number in the range
+    uint16_t root[N];                    // class of a live node, named by one of its nodes
+    union {
+        struct {                         // classes by closure
+            uint64_t adj[QN][QN / 64];   // reachability
+            uint64_t tr[QN][QN / 64];    // its transpose
+        } c;
+        struct {                         // classes by label rounds
+            uint32_t fw[N], bw[N];
+        } l;
+        struct {                         // then, of class c:
+            uint32_t id[N], size[N];         // its number, its members
+            uint32_t sumA[N], sumT[N];       // their row lengths (later row cursors)
+            uint32_t vcnt[N], degA[N], degT[N];
+        } s;
+    } u;
+    uint32_t ne, nlive, nnew, offA, offT, left, got;
     uint32_t chg[3];
+    uint16_t live[QM];                   // more than QN nodes: place among the live ones, or INERT
 };
 
-// f(i, k, end, step) covers edges k, k + step, .. k + 3 step (below end) of
-// node i; every edge of every row is covered once by the workgroup.
-template <int NT, class F>
-__device__ __forceinline__ void each_row(const uint32_t* rb, const uint32_t* re, uint32_t m, F f) {
+// f(i, k, end, step, W) covers edges k, k + step, .. k + 3 step (below end) of
+// row i = [rb(i), re(i)); every edge of every row is covered once by the
+// workgroup.  W lanes of a wave (8 or 64) work on the row together and call f
+// together.
+template <int NT, class Row, class F>
+__device__ __forceinline__ void each_row(uint32_t m, Row row, F f) {
     const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / WAVE;
     for (uint32_t i = tid / 8u; i < m; i += NT / 8) {
-        const uint32_t b = rb[i], e = re[i];
-        if (e - b > SHORT_ROW) continue;
-        for (uint32_t k = b + (tid & 7u); k < e; k += 32u) f(i, k, e, 8u);
+        const uint2 r = row(i);
+        if (r.y - r.x > SHORT_ROW) continue;
+        for (uint32_t k = r.x; k < r.y; k += 32u) f(i, k + (tid & 7u), r.y, 8u, 8);
     }
     uint32_t turn = 0;
     for (uint32_t t0 = 0; t0 < m; t0 += WAVE) {
         const uint32_t i0 = t0 + lane;
-        const uint32_t len = i0 < m ? re[i0] - rb[i0] : 0u;
+        const uint2 r0 = i0 < m ? row(i0) : make_uint2(0u, 0u);
+        const uint32_t len = r0.y - r0.x;
         for (uint64_t b = __ballot(len > SHORT_ROW && len <= MID_ROW); b; b &= b - 1ull) {
             if (turn++ % (uint32_t)(NT / WAVE) != w) continue;
             const uint32_t i = t0 + (uint32_t)__builtin_ctzll(b);
-            for (uint32_t k = rb[i] + lane; k < re[i]; k += 4u * WAVE) f(i, k, re[i], (uint32_t)WAVE);
+            const uint2 r = row(i);
+            for (uint32_t k = r.x; k < r.y; k += 4u * WAVE) f(i, k + lane, r.y, (uint32_t)WAVE, WAVE);
         }
         for (uint64_t b = __ballot(len > MID_ROW); b; b &= b - 1ull) {
             const uint32_t i = t0 + (uint32_t)__builtin_ctzll(b);
-            for (uint32_t k = rb[i] + tid; k < re[i]; k += 4u * NT) f(i, k, re[i], (uint32_t)NT);
+            const uint2 r = row(i);
+            for (uint32_t k = r.x + w * WAVE; k < r.y; k += 4u * NT) f(i, k + lane, r.y, (uint32_t)NT, WAVE);
         }
     }
 }
 
-// One workgroup per range.  Nodes are the halves' classes (BASE: vertices).
-//  1. The edges among the range's nodes go to a list (node pairs).
-//  2. Classes by label rounds: every node carries the largest label that
-//     reaches it and the largest that it reaches; where both are the same
-//     node c, the node is strongly connected with c.  Labels of heavy nodes
-//     are larger, so the range's main class is found in the first round and
-//     is not hidden behind single vertices that only lead into or out of it.
-//     Assigned nodes leave the graph; the next round looks at the rest.
-//  3. Each class of two or more nodes gets a row: its members' targets
-//     outside the class, over A and over A^T.  Other nodes keep theirs.
-template <int CAP, int NT, bool BASE>
-__global__ __launch_bounds__(NT) void k_quot_classes(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ctab0) {
-    __shared__ QLds<CAP> S;
-    if (!BASE && quot_off(p)) return;
+// Strongly connected classes of m <= 64 NW nodes from their adjacency bits
+// S.u.c.adj (rows of nodes at or above m empty): Warshall's closure, 64 pivots
+// at a time.  Thread i of the first 64 NW holds row i as dwords; the wave of
+// the pivots closes its own rows by lane broadcasts (one and-or per dword and
+// pivot), publishes them, and the other rows take them from LDS.  root[i]: the
+// smallest node that i reaches and that reaches i.  Called by the whole
+// workgroup.
+template <int NW, int N>
+__device__ __forceinline__ void closure_classes(QLds<N>& S, uint32_t m) {
+    constexpr int ND = 2 * NW, QD = QN / 32;
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / WAVE;
+    const bool row = tid < (uint32_t)(64 * NW);
+    uint32_t(*adj)[QD] = reinterpret_cast<uint32_t(*)[QD]>(S.u.c.adj);
+    uint32_t r[ND];
+#pragma unroll
+    for (int q = 0; q < ND; q++) r[q] = row ? adj[tid][q] : 0u;
+#pragma unroll
+    for (int b = 0; b < NW; b++) {
+        if (w == (uint32_t)b) {
+#pragma unroll
+            for (int k = 0; k < 64; k++) {
+                const uint32_t has = 0u - ((r[2 * b + (k >> 5)] >> (k & 31)) & 1u);
+#pragma unroll
+                for (int q = 0; q < ND; q++) r[q] |= (uint32_t)__builtin_amdgcn_readlane((int)r[q], k) & has;
+            }
+            if (NW > 1) {
+#pragma unroll
+                for (int q = 0; q < ND; q++) adj[tid][q] = r[q];
+            }
+        }
+        if (NW > 1) {
+            __syncthreads();
+            if (row && w != (uint32_t)b) {
+#pragma unroll 8
+                for (int k = 0; k < 64; k++) {
+                    const uint32_t has = 0u - ((r[2 * b + (k >> 5)] >> (k & 31)) & 1u);
+#pragma unroll
+                    for (int q = 0; q < ND; q++) r[q] |= adj[64 * b + k][q] & has;
+                }
+            }
+            // the next block's pivots write their own rows of adj only
+        }
+    }
+    // transpose: the ballot of bit 64 q + k over wave w is word w of row 64 q + k
+    if (row) {
+#pragma unroll
+        for (int q = 0; q < NW; q++) {
+            uint64_t mine = 0;
+#pragma unroll
+            for (int k = 0; k < 64; k++) {
+                const uint64_t bal = __ballot((r[2 * q + (k >> 5)] >> (k & 31)) & 1u);
+                if (lane == (uint32_t)k) mine = bal;
+            }
+            S.u.c.tr[64 * q + (int)lane][w] = mine;
+        }
+    }
+    __syncthreads();
+    if (tid < m) {
+        uint32_t c = tid;
+#pragma unroll
+        for (int q = NW - 1; q >= 0; q--) {
+            const uint64_t both = (((uint64_t)r[2 * q + 1] << 32) | r[2 * q]) & S.u.c.tr[tid][q];
+            if (both) {
+                const uint32_t j = 64u * (uint32_t)q + (uint32_t)__builtin_ctzll(both);
+                c = j < c ? j : c;
+            }
+        }
+        S.root[tid] = (uint16_t)c;
+    }
+}
+
+// Classes of m <= N nodes by label rounds over the edge list eb (node pairs):
+// every node carries the largest label that reaches it and the largest that it
+// reaches; where both are the same node c, the node is strongly connected with
+// c.  Labels of heavy nodes are larger, so the range's main class is found in
+// the first round and is not hidden behind single vertices that only lead into
+// or out of it.  Assigned nodes leave the graph; the next round looks at the
+// rest.  Nodes left after ROUNDS stay classes of their own.
+template <int N, int NT>
+__device__ __forceinline__ void label_classes(QLds<N>& S, uint32_t m, uint32_t ne, const uint32_t* eb) {
     const uint32_t tid = threadIdx.x;
-    const uint2 R = p.tab[tab0 + blockIdx.x];
-    const uint32_t size = 1u << (kQuotShift + lev);
-    const uint32_t x = R.x;
-    const int32_t* comp_prev = BASE ? nullptr : p.comp + (uint64_t)(lev - 1u) * p.n;
-    const uint4* info_prev = BASE ? nullptr : p.info + (uint64_t)(lev - 1u) * p.n;
-    const uint4* infoT_prev = BASE ? nullptr : p.infoT + (uint64_t)(lev - 1u) * p.n;
-    uint4* info_cur = p.info + (uint64_t)lev * p.n;
-    uint4* infoT_cur = p.infoT + (uint64_t)lev * p.n;
-    const int32_t* nodes_prev = p.nodes + (uint64_t)((lev + 1u) & 1u) * p.n;
-    int32_t* nodes_cur = p.nodes + (uint64_t)(lev & 1u) * p.n;
-    uint32_t m0 = size, m = size;
-    if (!BASE) {
-        m0 = p.ncnt[ctab0 + R.y];
-        m = m0 + p.ncnt[ctab0 + R.y + 1u];
-    }
-    const uint32_t xr = x + size / 2u;
-    auto node_at = [&](uint32_t i) {
-        return BASE ? (int32_t)(x + i) : i < m0 ? nodes_prev[x + i] : nodes_prev[xr + i - m0];
-    };
-    if (m > (uint32_t)CAP) {  // too many nodes: the halves' classes stand
-        for (uint32_t i = tid; i < m; i += NT) {
-            const int32_t v = node_at(i);
-            p.nmap[v] = v;
-            nodes_cur[x + i] = v;
-            info_cur[v] = info_prev[v];
-            infoT_cur[v] = infoT_prev[v];
-        }
-        if (tid == 0) p.ncnt[tab0 + blockIdx.x] = m;
-        return;
-    }
-    auto row_of = [&](int32_t v, bool t) {
-        if (!BASE) return t ? infoT_prev[v] : info_prev[v];
-        const int32_t* rp = t ? p.rpT : p.rp;
-        const uint32_t b = (uint32_t)rp[v], e = (uint32_t)rp[v + 1];
-        return make_uint4(b, e, 1u, e - b);
-    };
-    if (tid == 0) {
-        S.total = S.ne = S.nnew = 0;
-        S.chg[0] = S.chg[1] = S.chg[2] = 0;
-    }
-    __syncthreads();
-    {
-        uint32_t len = 0;
-        for (uint32_t i = tid; i < m; i += NT) {
-            const int32_t v = node_at(i);
-            const uint4 r = row_of(v, false);
-            S.node[i] = v;
-            S.rb[i] = r.x;
-            S.re[i] = r.y;
-            S.a2[i] = r.z;
-            S.root[i] = NOROOT;
-            if (!BASE) p.nidx[v] = (int32_t)i;
-            len += r.y - r.x;
-        }
-        if (len) atomicAdd(&S.total, len);
-    }
-    __syncthreads();  // also: this workgroup's nidx writes are done
-    if (tid == 0) S.ebase = atomicAdd(&p.ctl->eb[lev], (unsigned long long)S.total);
-    __syncthreads();
-    uint32_t* eb = p.eb + S.ebase;
-    // local node of target v, NOIDX outside the range
-    auto local = [&](int32_t v) {
-        const uint32_t o = (uint32_t)v - x;
-        if (o >= size) return NOIDX;
-        return BASE ? o : (uint32_t)p.nidx[comp_prev[v]];
-    };
-    // ---- 1. edges among the nodes
-    each_row<NT>(S.rb, S.re, m, [&](uint32_t i, uint32_t k, uint32_t e, uint32_t st) {
-        int32_t v[4];
-        uint32_t t[4];
-        uint32_t cnt = 0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = k + q * st < e ? p.ci[k + q * st] : -1;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            t[q] = v[q] >= 0 ? local(v[q]) : NOIDX;
-            if (t[q] == i) t[q] = NOIDX;
-            cnt += t[q] != NOIDX;
-        }
-        if (!cnt) return;
-        uint32_t o = atomicAdd(&S.ne, cnt);
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (t[q] != NOIDX) eb[o++] = (i << 16) | t[q];
-    });
-    __syncthreads();
-    const uint32_t ne = S.ne;
-    // ---- 2. classes
-    // label: weight class, then a permuted node number (its inverse names the node)
-    constexpr uint32_t PM = 2531u;  // odd: a bijection modulo CAP
+    constexpr uint32_t PM = 2531u;  // odd: a bijection modulo N
     uint32_t inv = PM;              // PM * inv = 1 modulo 2^32, by Newton's iteration
     for (int k = 0; k < 4; k++) inv *= 2u - PM * inv;
+    uint32_t* fw = S.u.l.fw;
+    uint32_t* bw = S.u.l.bw;
     auto label = [&](uint32_t i) {
-        return ((31u - (uint32_t)__builtin_clz(S.a2[i] | 1u)) << 16) | ((i * PM) & (uint32_t)(CAP - 1));
+        return ((31u - (uint32_t)__builtin_clz(S.cnt[i] | 1u)) << 16) | ((i * PM) & (uint32_t)(N - 1));
     };
-    auto named = [&](uint32_t l) { return (l * inv) & (uint32_t)(CAP - 1); };
+    auto named = [&](uint32_t l) { return (l * inv) & (uint32_t)(N - 1); };
+    for (uint32_t i = tid; i < m; i += NT) S.root[i] = INERT;
+    if (tid < 3) S.chg[tid] = 0;
     for (int rd = 0; rd < ROUNDS; rd++) {
+        __syncthreads();
         for (uint32_t i = tid; i < m; i += NT)
-            if (S.root[i] == NOROOT) S.fw[i] = S.bw[i] = label(i);
+            if (S.root[i] == INERT) fw[i] = bw[i] = label(i);
         if (tid == 0) S.left = S.got = 0;
         __syncthreads();
         for (int it = 0; it < ITERS; it++) {
@@ -219,29 +229,29 @@ __global__ __launch_bounds__(NT) void k_quot_classes(QuotParams p, uint32_t lev,
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
                     const uint32_t a = ed[q] >> 16, b = ed[q] & 0xFFFFu;
-                    if (a == b || S.root[a] != NOROOT || S.root[b] != NOROOT) continue;
-                    const uint32_t fa = S.fw[a], ba = S.bw[a], fb = S.fw[b], bb = S.bw[b];
+                    if (a == b || S.root[a] != INERT || S.root[b] != INERT) continue;
+                    const uint32_t fa = fw[a], ba = bw[a], fb = fw[b], bb = bw[b];
                     if (fa > fb) {
-                        atomicMax(&S.fw[b], fa);
+                        atomicMax(&fw[b], fa);
                         ch = true;
                     }
                     if (bb > ba) {
-                        atomicMax(&S.bw[a], bb);
+                        atomicMax(&bw[a], bb);
                         ch = true;
                     }
                 }
             }
             // what reaches (is reached by) a node's label reaches (is reached by) the node
             for (uint32_t i = tid; i < m; i += NT) {
-                if (S.root[i] != NOROOT) continue;
-                const uint32_t f = S.fw[i], b = S.bw[i];
-                const uint32_t f2 = S.fw[named(f)], b2 = S.bw[named(b)];
+                if (S.root[i] != INERT) continue;
+                const uint32_t f = fw[i], b = bw[i];
+                const uint32_t f2 = fw[named(f)], b2 = bw[named(b)];
                 if (f2 > f) {
-                    atomicMax(&S.fw[i], f2);
+                    atomicMax(&fw[i], f2);
                     ch = true;
                 }
                 if (b2 > b) {
-                    atomicMax(&S.bw[i], b2);
+                    atomicMax(&bw[i], b2);
                     ch = true;
                 }
             }
@@ -253,9 +263,9 @@ __global__ __launch_bounds__(NT) void k_quot_classes(QuotParams p, uint32_t lev,
         if (tid < 3) S.chg[tid] = 0;
         uint32_t left = 0, got = 0;
         for (uint32_t i = tid; i < m; i += NT) {
-            if (S.root[i] != NOROOT) continue;
-            if (S.fw[i] == S.bw[i]) {
-                const uint32_t c = named(S.fw[i]);
+            if (S.root[i] != INERT) continue;
+            if (fw[i] == bw[i]) {
+                const uint32_t c = named(fw[i]);
                 S.root[i] = (uint16_t)c;
                 got += c != i;
             } else {
@@ -265,111 +275,345 @@ __global__ __launch_bounds__(NT) void k_quot_classes(QuotParams p, uint32_t lev,
         if (left) atomicAdd(&S.left, left);
         if (got) atomicAdd(&S.got, got);
         __syncthreads();
-        const bool stop = S.left == 0 || (S.got == 0 && rd > 0);
-        __syncthreads();
-        if (stop) break;
-    }
-    // class c: the members with root c; fw: its first member, bw: its size
-    for (uint32_t i = tid; i < m; i += NT) {
-        S.fw[i] = NOIDX;
-        S.bw[i] = 0;
-        if (S.root[i] == NOROOT) S.root[i] = (uint16_t)i;
+        if (S.left == 0 || (S.got == 0 && rd > 0)) break;
     }
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += NT) {
-        atomicMin(&S.fw[S.root[i]], i);
-        atomicAdd(&S.bw[S.root[i]], 1u);
-    }
+    for (uint32_t i = tid; i < m; i += NT)
+        if (S.root[i] == INERT) S.root[i] = (uint16_t)i;
     __syncthreads();
-    for (uint32_t i = tid; i < m; i += NT) {
-        const uint32_t c = S.root[i], f = S.fw[c];
-        const int32_t v = S.node[i], nv = S.node[f];
-        if (BASE) p.comp[v] = nv;
-        else p.nmap[v] = nv;
-        if (f == i) {
-            nodes_cur[x + atomicAdd(&S.nnew, 1u)] = v;
-            if (S.bw[c] == 1u) {  // not merged: keeps its rows
-                info_cur[v] = row_of(v, false);
-                infoT_cur[v] = row_of(v, true);
-            }
-        }
-    }
-    // ---- 3. rows of merged classes, over A then over A^T
-    for (int side = 0; side < 2; side++) {
-        const bool t = side == 1;
-        __syncthreads();
-        for (uint32_t i = tid; i < m; i += NT) {
-            S.a0[i] = S.a1[i] = 0;
-            if (!t) S.a2[i] = 0;
-        }
-        __syncthreads();
-        for (uint32_t i = tid; i < m; i += NT) {
-            const uint32_t c = S.root[i];
-            const bool merged = S.bw[c] > 1u;
-            const uint4 r = merged ? row_of(S.node[i], t) : make_uint4(0u, 0u, 0u, 0u);
-            S.rb[i] = r.x;  // unmerged nodes: an empty row
-            S.re[i] = r.y;
-            if (!merged) continue;
-            atomicAdd(&S.a0[c], r.y - r.x);
-            atomicAdd(&S.a1[c], r.w);
-            if (!t) atomicAdd(&S.a2[c], r.z);
-        }
-        __syncthreads();
-        uint4* info = t ? infoT_cur : info_cur;
-        int32_t* cols = t ? p.ciT : p.ci;
-        for (uint32_t i = tid; i < m; i += NT) {
-            const uint32_t c = S.root[i];
-            if (S.fw[c] != i || S.bw[c] == 1u) continue;
-            // room for every member's row; the levels' rows never exceed the
-            // matrix's entries, so the reserve of one matrix per level holds
-            const uint32_t b = p.ext0 + (uint32_t)atomicAdd(t ? &p.ctl->extT : &p.ctl->ext, (unsigned long long)S.a0[c]);
-            info[S.node[i]] = make_uint4(b, b, S.a2[c], S.a1[c]);
-            S.a0[c] = b;
-        }
-        __syncthreads();
-        each_row<NT>(S.rb, S.re, m, [&](uint32_t i, uint32_t k, uint32_t e, uint32_t st) {
-            int32_t v[4];
-            uint32_t cnt = 0;
-            const uint32_t c = S.root[i];
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = k + q * st < e ? cols[k + q * st] : -1;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                if (v[q] < 0) continue;
-                const uint32_t l = local(v[q]);
-                if (l != NOIDX && S.root[l] == c) v[q] = -1;
-                else cnt++;
-            }
-            if (!cnt) return;
-            uint32_t o = atomicAdd(&S.a0[c], cnt);
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-                if (v[q] >= 0) cols[o++] = v[q];
-        });
-        __syncthreads();
-        for (uint32_t i = tid; i < m; i += NT) {
-            const uint32_t c = S.root[i];
-            if (S.fw[c] == i && S.bw[c] > 1u) info[S.node[i]].y = S.a0[c];
-        }
-    }
-    if (tid == 0) {
-        p.ncnt[tab0 + blockIdx.x] = S.nnew;
-        if (BASE) atomicAdd(&p.ctl->nodes0, (unsigned long long)S.nnew);
-    }
+    // a class may be named by a node that is not in it (a round cut short):
+    // name it by its smallest member
+    for (uint32_t i = tid; i < m; i += NT) fw[i] = NOIDX;
+    __syncthreads();
+    for (uint32_t i = tid; i < m; i += NT) atomicMin(&fw[S.root[i]], i);
+    __syncthreads();
+    for (uint32_t i = tid; i < m; i += NT) bw[i] = fw[S.root[i]];
+    __syncthreads();
+    for (uint32_t i = tid; i < m; i += NT) S.root[i] = (uint16_t)bw[i];
 }
 
-// Classes of every vertex of the level's ranges, from the level below.
-__global__ __launch_bounds__(256) void k_quot_map(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ranges) {
-    if (quot_off(p)) return;
+// One range, by the whole workgroup.  Nodes are the halves' classes (BASE:
+// vertices); class k of a range is numbered x + k, x its first vertex.
+//  1. Live nodes: all of them up to QN; of more, those with an edge from and
+//     an edge to another node of the range (the others are in no cycle).
+//  2. The live nodes' edges as bits, and their classes by closure.
+//  3. Each class of two or more nodes gets a row: its members' targets outside
+//     the class, over A and over A^T.  Other nodes keep theirs.
+// A range of more than QM nodes, or N live ones, keeps its halves' classes;
+// with `defer`, one of more than N live ones is left to a larger N: returns
+// false, having written nothing.
+template <int N, int NT, bool BASE>
+__device__ bool range_classes(QLds<N>& S, const QuotParams& p, uint32_t lev, uint32_t tab0, uint32_t ctab0,
+                              uint32_t range, bool defer) {
+    const uint32_t tid = threadIdx.x, lane = __lane_id();
+    const uint64_t ln = p.n;
+    const uint2 R = p.tab[tab0 + range];
+    const uint32_t size = 1u << (kQuotShift + lev), x = R.x, xr = x + size / 2u;
+    const uint4* info_prev = BASE ? nullptr : p.info + (lev - 1u) * ln;
+    const uint4* infoT_prev = BASE ? nullptr : p.infoT + (lev - 1u) * ln;
+    uint4* info_cur = p.info + lev * ln;
+    uint4* infoT_cur = p.infoT + lev * ln;
+    int32_t* map_cur = p.nmap + (lev & 1u) * ln;
+    const int32_t* map_prev = p.nmap + ((lev + 1u) & 1u) * ln;
+    uint32_t m0 = size, m = size;
+    if (!BASE) {
+        m0 = p.ncnt[ctab0 + R.y];
+        m = m0 + p.ncnt[ctab0 + R.y + 1u];
+    }
+    auto node_at = [&](uint32_t i) { return BASE || i < m0 ? x + i : xr + (i - m0); };
+    auto row_of = [&](uint32_t v, bool t) {
+        if (!BASE) return t ? infoT_prev[v] : info_prev[v];
+        const int32_t* rp = t ? p.rpT : p.rp;
+        const uint32_t b = (uint32_t)rp[v], e = (uint32_t)rp[v + 1];
+        return make_uint4(b, e, 1u, e - b);
+    };
+    // node number of target v, NOIDX outside the range
+    auto local = [&](int32_t v) {
+        const uint32_t o = (uint32_t)v - x;
+        if (o >= size) return NOIDX;
+        if (BASE) return o;
+        uint32_t c;
+        if (lev == 1u) c = (uint32_t)p.comp[v];
+        else c = (uint32_t)map_prev[p.comp[(lev - 2u) * ln + (uint32_t)v]];
+        return c < xr ? c - x : m0 + (c - xr);
+    };
+    if (tid == 0) S.nlive = S.nnew = S.offA = S.offT = S.ne = 0;
+    const bool sparse = !BASE && m > (uint32_t)QN;  // nodes to be sifted first
+    bool merge = m <= (uint32_t)QM;
+    if (sparse && merge) {
+        for (uint32_t i = tid; i < m; i += NT) S.live[i] = 0;
+        __syncthreads();
+        // bit 0: an edge to another node, bit 1: from another node (words of
+        // two nodes, so that the bits can be set with 32-bit atomics)
+        uint32_t* flag = reinterpret_cast<uint32_t*>(S.live);
+        each_row<NT>(
+            m,
+            [&](uint32_t i) {
+                const uint4 r = info_prev[node_at(i)];
+                return make_uint2(r.x, r.y);
+            },
+            [&](uint32_t i, uint32_t k, uint32_t e, uint32_t st, int) {
+                int32_t v[4];
+                uint32_t l[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = k + q * st < e ? p.ci[k + q * st] : -1;
+#pragma unroll
+                for (int q = 0; q < 4; q++) l[q] = v[q] >= 0 ? local(v[q]) : NOIDX;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    if (l[q] == NOIDX || l[q] == i) continue;
+                    atomicOr(&flag[i >> 1], 1u << (16u * (i & 1u)));
+                    atomicOr(&flag[l[q] >> 1], 2u << (16u * (l[q] & 1u)));
+                }
+            });
+        __syncthreads();
+        for (uint32_t i = tid; i < m; i += NT) {
+            uint32_t k = INERT;
+            if (S.live[i] == 3u) {
+                k = atomicAdd(&S.nlive, 1u);
+                if (k < (uint32_t)N) S.node[k] = (uint16_t)i;
+            }
+            S.live[i] = (uint16_t)(k < (uint32_t)N ? k : INERT);
+        }
+        __syncthreads();
+        merge = S.nlive <= (uint32_t)N;
+        if (!merge && defer) return false;
+    }
+    if (!merge) {  // the halves' classes stand
+        for (uint32_t i = tid; i < m; i += NT) {
+            const uint32_t v = node_at(i);
+            map_cur[v] = (int32_t)(x + i);
+            info_cur[x + i] = info_prev[v];
+            infoT_cur[x + i] = infoT_prev[v];
+        }
+        if (tid == 0) {
+            p.ncnt[tab0 + range] = m;
+            if (lev == p.judge) atomicAdd(&p.ctl->nodes, (unsigned long long)m);
+        }
+        return true;
+    }
+    const uint32_t nl = sparse ? S.nlive : m;
+    auto node_of = [&](uint32_t k) { return node_at(sparse ? S.node[k] : k); };
+    // live node of target v, NOIDX for other nodes and outside the range
+    auto live = [&](int32_t v) {
+        const uint32_t l = local(v);
+        if (!sparse || l == NOIDX) return l;
+        return S.live[l] == INERT ? NOIDX : (uint32_t)S.live[l];
+    };
+    for (uint32_t k = tid; k < nl; k += NT) {
+        const uint32_t v = node_of(k);
+        const uint4 a = row_of(v, false), t = row_of(v, true);
+        S.rb[k] = a.x;
+        S.re[k] = a.y;
+        S.rb[nl + k] = t.x;
+        S.re[nl + k] = t.y;
+        S.cnt[k] = a.z;
+        S.deg[k] = a.w;
+        S.deg[N + k] = t.w;
+    }
+    const bool bits = N == QN || nl <= (uint32_t)QN;
+    uint32_t* eb = p.eb + p.rp[x];  // the range's rows leave room for its edges
+    if (bits && tid < (uint32_t)(BASE ? QB : QN)) {
+#pragma unroll
+        for (int q = 0; q < QN / 64; q++) S.u.c.adj[tid][q] = 0ull;
+    }
+    __syncthreads();
+    auto lds_row = [&](uint32_t i) { return make_uint2(S.rb[i], S.re[i]); };
+    each_row<NT>(nl, lds_row, [&](uint32_t i, uint32_t k, uint32_t e, uint32_t st, int) {
+        int32_t v[4];
+        uint32_t l[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = k + q * st < e ? p.ci[k + q * st] : -1;
+#pragma unroll
+        for (int q = 0; q < 4; q++) l[q] = v[q] >= 0 ? live(v[q]) : NOIDX;
+        if (bits) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (l[q] != NOIDX)
+                    atomicOr(reinterpret_cast<unsigned long long*>(&S.u.c.adj[i][l[q] >> 6]), 1ull << (l[q] & 63u));
+            return;
+        }
+        uint32_t cnt = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) cnt += l[q] != NOIDX && l[q] != i;
+        if (!cnt) return;
+        uint32_t o = atomicAdd(&S.ne, cnt);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (l[q] != NOIDX && l[q] != i) eb[o++] = (i << 16) | l[q];
+    });
+    __syncthreads();
+    if constexpr (BASE) {
+        closure_classes<QB / 64>(S, nl);
+    } else {
+        if (N > QN && !bits) label_classes<N, NT>(S, nl, S.ne, eb);
+        else if (nl <= 64u) closure_classes<1>(S, nl);
+        else if (nl <= 128u) closure_classes<2>(S, nl);
+        else closure_classes<QN / 64>(S, nl);
+    }
+    __syncthreads();
+    for (uint32_t c = tid; c < nl; c += NT) {
+        S.u.s.size[c] = 0;
+        S.u.s.sumA[c] = S.u.s.sumT[c] = S.u.s.vcnt[c] = S.u.s.degA[c] = S.u.s.degT[c] = 0;
+    }
+    __syncthreads();
+    // sums per class: the first lane's class of each wave by wave sums (a range
+    // mostly has one large class), the others by atomics
+    for (uint32_t k0 = tid - lane; k0 < nl; k0 += NT) {
+        const uint32_t k = k0 + lane;
+        const bool in = k < nl;
+        const uint32_t c = in ? S.root[k] : NOIDX;
+        const uint32_t la = in ? S.re[k] - S.rb[k] : 0u, lt = in ? S.re[nl + k] - S.rb[nl + k] : 0u;
+        const uint32_t vc = in ? S.cnt[k] : 0u, da = in ? S.deg[k] : 0u, dt = in ? S.deg[N + k] : 0u;
+        const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+        const bool same = c == c0;
+        const uint32_t members = (uint32_t)__popcll(__ballot(same));
+        unsigned long long x0 = same ? ((unsigned long long)la << 32) | lt : 0ull;
+        unsigned long long x1 = same ? ((unsigned long long)da << 32) | dt : 0ull;
+        unsigned long long x2 = same ? vc : 0u;
+        x0 = dev::wave_sum64(x0);  // each half stays below 2^32: row lengths of one matrix
+        x1 = dev::wave_sum64(x1);
+        x2 = dev::wave_sum64(x2);
+        if (in && (!same || lane == 0)) {
+            atomicAdd(&S.u.s.size[c], same ? members : 1u);
+            atomicAdd(&S.u.s.sumA[c], same ? (uint32_t)(x0 >> 32) : la);
+            atomicAdd(&S.u.s.sumT[c], same ? (uint32_t)x0 : lt);
+            atomicAdd(&S.u.s.degA[c], same ? (uint32_t)(x1 >> 32) : da);
+            atomicAdd(&S.u.s.degT[c], same ? (uint32_t)x1 : dt);
+            atomicAdd(&S.u.s.vcnt[c], same ? (uint32_t)x2 : vc);
+        }
+    }
+    __syncthreads();
+    // class numbers; a merged class's rows get room for all its members': a
+    // range's rows never exceed the matrix's entries in the range's rows, so
+    // each level has one matrix's worth of room, divided like the matrix
+    const uint32_t baseA = p.ext0 * (1u + lev) + (uint32_t)p.rp[x];
+    const uint32_t baseT = p.ext0 * (1u + lev) + (uint32_t)p.rpT[x];
+    for (uint32_t c = tid; c < nl; c += NT) {
+        const uint32_t n = S.u.s.size[c];
+        if (n == 0u) continue;
+        const uint32_t id = x + atomicAdd(&S.nnew, 1u);
+        uint4 a = make_uint4(S.rb[c], S.re[c], S.u.s.vcnt[c], S.u.s.degA[c]);  // one member: c itself
+        uint4 t = make_uint4(S.rb[nl + c], S.re[nl + c], S.u.s.vcnt[c], S.u.s.degT[c]);
+        if (n > 1u) {
+            a.x = a.y = baseA + atomicAdd(&S.offA, S.u.s.sumA[c]);
+            t.x = t.y = baseT + atomicAdd(&S.offT, S.u.s.sumT[c]);
+            S.u.s.sumA[c] = a.x;
+            S.u.s.sumT[c] = t.x;
+        }
+        info_cur[id] = a;  // a merged class's row end follows
+        infoT_cur[id] = t;
+        S.u.s.id[c] = id;
+    }
+    __syncthreads();
+    for (uint32_t k = tid; k < nl; k += NT) {
+        const uint32_t c = S.root[k], v = node_of(k);
+        if (BASE) p.comp[v] = (int32_t)S.u.s.id[c];
+        else map_cur[v] = (int32_t)S.u.s.id[c];
+        if (S.u.s.size[c] == 1u) S.rb[k] = S.re[k] = S.rb[nl + k] = S.re[nl + k] = 0u;  // no row to build
+    }
+    if (sparse) {  // the other nodes stay as they are
+        for (uint32_t i = tid; i < m; i += NT) {
+            if (S.live[i] != INERT) continue;
+            const uint32_t v = node_at(i), id = x + atomicAdd(&S.nnew, 1u);
+            map_cur[v] = (int32_t)id;
+            info_cur[id] = info_prev[v];
+            infoT_cur[id] = infoT_prev[v];
+        }
+    }
+    __syncthreads();
+    each_row<NT>(2u * nl, lds_row, [&](uint32_t i, uint32_t k, uint32_t e, uint32_t st, int W) {
+        const bool t = i >= nl;
+        int32_t* cols = t ? p.ciT : p.ci;
+        int32_t v[4];
+        uint32_t l[4], cnt = 0;
+        const uint32_t c = S.root[t ? i - nl : i];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = k + q * st < e ? cols[k + q * st] : -1;
+#pragma unroll
+        for (int q = 0; q < 4; q++) l[q] = v[q] >= 0 ? live(v[q]) : NOIDX;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (l[q] != NOIDX && S.root[l[q]] == c) v[q] = -1;
+            cnt += v[q] >= 0;
+        }
+        // one cursor step for the lanes that share the row
+        uint32_t incl = cnt;
+        for (int d = 1; d < W; d <<= 1) {
+            const uint32_t y = __shfl_up(incl, d, W);
+            if ((lane & (uint32_t)(W - 1)) >= (uint32_t)d) incl += y;
+        }
+        const uint32_t all = __shfl(incl, W - 1, W);
+        if (all == 0u) return;
+        uint32_t o = 0;
+        if ((lane & (uint32_t)(W - 1)) == 0u) o = atomicAdd(t ? &S.u.s.sumT[c] : &S.u.s.sumA[c], all);
+        o = __shfl(o, 0, W) + incl - cnt;
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (v[q] >= 0) cols[o++] = v[q];
+    });
+    __syncthreads();
+    for (uint32_t c = tid; c < nl; c += NT) {
+        if (S.u.s.size[c] <= 1u) continue;
+        info_cur[S.u.s.id[c]].y = S.u.s.sumA[c];
+        infoT_cur[S.u.s.id[c]].y = S.u.s.sumT[c];
+    }
+    if (tid == 0) {
+        p.ncnt[tab0 + range] = S.nnew;
+        if (lev == p.judge) atomicAdd(&p.ctl->nodes, (unsigned long long)S.nnew);
+    }
+    return true;
+}
+
+__global__ __launch_bounds__(QNT) void k_quot_base(QuotParams p) {
+    __shared__ QLds<QN> S;
+    (void)range_classes<QN, QNT, true>(S, p, 0u, 0u, 0u, blockIdx.x, false);
+}
+
+// Classes of every vertex of level `lev`'s ranges, from the level below:
+// `blocks` blocks from `block` on share the work.
+__device__ __forceinline__ void map_level(const QuotParams& p, uint32_t lev, uint32_t tab0, uint32_t ranges,
+                                          uint32_t block, uint32_t blocks) {
     const uint32_t sh = kQuotShift + lev;
     const uint64_t total = (uint64_t)ranges << sh;
     const int32_t* prev = p.comp + (uint64_t)(lev - 1u) * p.n;
+    const int32_t* map = p.nmap + (uint64_t)(lev & 1u) * p.n;
     int32_t* cur = p.comp + (uint64_t)lev * p.n;
-    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < total;
-         k += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t k = (uint64_t)block * blockDim.x + threadIdx.x; k < total; k += (uint64_t)blocks * blockDim.x) {
         const uint32_t v = p.tab[tab0 + (uint32_t)(k >> sh)].x + ((uint32_t)k & ((1u << sh) - 1u));
-        cur[v] = p.nmap[prev[v]];
+        cur[v] = map[prev[v]];
     }
+}
+
+// The ranges of a level, one workgroup each.  The blocks behind them write the
+// classes of the level below (lev >= 2), which this level's own look-ups take
+// in two steps instead.
+__global__ __launch_bounds__(QNT_LEVEL) void k_quot_level(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ctab0,
+                                                          uint32_t ranges, uint32_t cranges) {
+    __shared__ QLds<QN> S;
+    if (lev > p.judge && quot_off(p)) return;
+    if (blockIdx.x >= ranges) {
+        map_level(p, lev - 1u, ctab0, cranges, blockIdx.x - ranges, gridDim.x - ranges);
+        return;
+    }
+    if (!range_classes<QN, QNT_LEVEL, false>(S, p, lev, tab0, ctab0, blockIdx.x, lev <= QBIG_LEVEL) &&
+        threadIdx.x == 0)
+        p.blist[atomicAdd(&p.ctl->big[lev], 1u)] = blockIdx.x;
+}
+
+// The ranges that k_quot_level left.
+__global__ __launch_bounds__(QNT_BIG) void k_quot_big(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ctab0) {
+    __shared__ QLds<QCAP> S;
+    const uint32_t cnt = p.ctl->big[lev];
+    for (uint32_t i = blockIdx.x; i < cnt; i += gridDim.x) {
+        (void)range_classes<QCAP, QNT_BIG, false>(S, p, lev, tab0, ctab0, p.blist[i], false);
+        __syncthreads();  // S is read before the next range resets it
+    }
+}
+
+__global__ __launch_bounds__(QNT_LEVEL) void k_quot_map(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ranges) {
+    if (quot_off(p)) return;
+    map_level(p, lev, tab0, ranges, blockIdx.x, gridDim.x);
 }
 
 }  // namespace
@@ -388,8 +632,8 @@ uint64_t quot_ext(uint64_t nnz, uint32_t levels) { return nnz * levels; }
 int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W) {
     const int64_t L = quot_levels(W);
     if (L == 0) return 0;
-    return L * n * (4 + 32) + 16 * n + 4 * nnz + 8 * (int64_t)quot_ext((uint64_t)nnz, (uint32_t)L) +
-           12 * ((n >> kQuotShift) * 2 + L + 1) + (int64_t)sizeof(QuotCtl) + 4096;
+    return L * n * (4 + 32) + 8 * n + 4 * nnz + 8 * (int64_t)quot_ext((uint64_t)nnz, (uint32_t)L) +
+           16 * ((n >> kQuotShift) * 2 + L + 1) + (int64_t)sizeof(QuotCtl) + 4096;
 }
 
 // Ranges of every level: tab[off[h] ..] = (first vertex, entry of the first
@@ -415,19 +659,24 @@ void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vec
 hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hipStream_t s) {
     hipError_t e = launch_fill(reinterpret_cast<uint32_t*>(p.ctl), sizeof(QuotCtl) / 4, 0u, s);
     if (e != hipSuccess) return e;
-    for (uint32_t h = 0; h < p.levels; h++) {
-        const uint32_t ranges = off[h + 1] - off[h];
-        if (ranges == 0) break;
-        if (h == 0) {
-            hipLaunchKernelGGL((k_quot_classes<QBASE_CAP, QBASE_NT, true>), dim3(ranges), dim3(QBASE_NT), 0, s, p, h,
-                               off[h], 0u);
-        } else {
-            hipLaunchKernelGGL((k_quot_classes<QCAP, QNT, false>), dim3(ranges), dim3(QNT), 0, s, p, h, off[h],
+    auto map_blocks = [](uint64_t vertices) {
+        return (uint32_t)std::min<uint64_t>((vertices + QNT_LEVEL - 1) / QNT_LEVEL, 1024);
+    };
+    hipLaunchKernelGGL(k_quot_base, dim3(off[1]), dim3(QNT), 0, s, p);
+    uint32_t h = 1;
+    for (; h < p.levels && off[h + 1] > off[h]; h++) {
+        const uint32_t ranges = off[h + 1] - off[h], below = off[h] - off[h - 1];
+        const uint32_t mb = h >= 2 ? map_blocks((uint64_t)below << (kQuotShift + h - 1)) : 0u;
+        hipLaunchKernelGGL(k_quot_level, dim3(ranges + mb), dim3(QNT_LEVEL), 0, s, p, h, off[h], off[h - 1], ranges,
+                           below);
+        if (h <= QBIG_LEVEL)
+            hipLaunchKernelGGL(k_quot_big, dim3(std::min(ranges, QBIG_GRID)), dim3(QNT_BIG), 0, s, p, h, off[h],
                                off[h - 1]);
-            const uint64_t total = (uint64_t)ranges << (kQuotShift + h);
-            hipLaunchKernelGGL(k_quot_map, dim3((uint32_t)std::min<uint64_t>((total + 255) / 256, 2048)), dim3(256),
-                               0, s, p, h, off[h], ranges);
-        }
+    }
+    if (h >= 2) {
+        const uint32_t ranges = off[h] - off[h - 1];
+        hipLaunchKernelGGL(k_quot_map, dim3(map_blocks((uint64_t)ranges << (kQuotShift + h - 1))), dim3(QNT_LEVEL), 0,
+                           s, p, h - 1u, off[h - 1], ranges);
     }
     return hipGetLastError();
 }

@@ -50,7 +50,7 @@ def test_few_classes(lam, threads):
 
 
 def test_too_many_nodes():
-    """Ranges of over 4,096 nodes keep their halves' classes: pairs (2i, 2i+1)
+    """Ranges of over 256 live nodes keep their halves' classes: pairs (2i, 2i+1)
     are strongly connected, the pairs form an acyclic chain of chains."""
     n = 12001
     i = np.arange(0, n - 1, 2)
