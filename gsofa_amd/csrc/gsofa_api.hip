@@ -1641,6 +1641,8 @@ static RowParams row_params(const gsofa_plan* P) {
     r.R_ptr = P->d_rptr;
     r.list = P->d_list;
     r.list_cap = (int64_t)P->list_cap;
+    r.long_rows = P->d_cntL;  // unused otherwise in reach mode
+    r.long_count = &P->d_ctrl->cursor[0];
     r.L_col = P->d_Lcol;
     r.U_col = P->d_Ucol;
     r.L_cap = P->Lcap;
@@ -1687,10 +1689,13 @@ static int run_share(gsofa_plan* P, int32_t gid, size_t si) {
         rp.mat_te = P->d_mat_te;
         rp.mat_reach = P->d_mat_reach;
         rp.loops = std::min(0xFFFFFFFFu, P->span_cap);
-        HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_mat_te), 2 * (uint64_t)P->n_mats, 0u, P->stream));
-        HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_mat_reach), 2 * (uint64_t)P->n_mats, 0u, P->stream));
-        HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_cnt64), 2 * (uint64_t)n, 0u, P->stream));
-        HIPCHK(launch_fill(&P->d_ctrl->src_next, 1, 0u, P->stream));
+        ZeroSpans z{};  // the counters too: reach mode has one share
+        z.add(P->d_ctrl, sizeof(Ctrl));
+        z.add(P->d_mat_te, sizeof(unsigned long long) * (uint64_t)P->n_mats);
+        z.add(P->d_mat_reach, sizeof(unsigned long long) * (uint64_t)P->n_mats);
+        z.add(P->d_cnt64, sizeof(unsigned long long) * (uint64_t)n);
+        if (P->quot.levels) z.add(P->quot.ctl, sizeof(QuotCtl));
+        HIPCHK(launch_zero(z, P->stream));
         if (!P->capturing) HIPCHK(hipEventRecord(P->ev[2 + 2 * si], P->stream));
         if (P->quot.levels) {
             P->quot.rp = P->d_rp;
@@ -1993,7 +1998,8 @@ static void finish_timing(gsofa_plan* P, size_t nshares) {
 // sequence can be captured in a graph.
 static int queue_bounded(gsofa_plan* P, const std::vector<int32_t>& shares, int32_t N, bool all_rows,
                          Ctrl* stats) {
-    HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_ctrl), sizeof(Ctrl) / 4, 0u, P->stream));
+    if (P->mode != GSOFA_MODE_REACH)  // reach mode clears it with its other counters
+        HIPCHK(launch_fill(reinterpret_cast<uint32_t*>(P->d_ctrl), sizeof(Ctrl) / 4, 0u, P->stream));
     if (!P->capturing) HIPCHK(hipEventRecord(P->ev[0], P->stream));
     for (size_t si = 0; si < shares.size(); si++) {
         int rc = run_share(P, shares[si], si);

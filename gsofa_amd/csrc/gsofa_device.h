@@ -26,6 +26,11 @@ __device__ __forceinline__ uint64_t bcast0_64(uint64_t v) {
     uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return ((uint64_t)hi << 32) | lo;
 }
+// Lane `src`'s value (wave-uniform src).
+__device__ __forceinline__ uint64_t bcast_64(uint64_t v, int src) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), src) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, src);
+}
 
 template <class T>
 __device__ __forceinline__ T ld_agent(T* p) {

@@ -22,7 +22,7 @@ struct Ctrl {
     uint32_t pad0;
     // rotating per-level counters (level L reads slot L%3)
     unsigned long long qcnt[3];   // queue sizes (pairs appended, may exceed capacity)
-    uint32_t cursor[4];           // work-fetch cursors
+    uint32_t cursor[4];           // work-fetch cursors; reach mode: [0] counts the rows of many records
     unsigned long long orphans;   // frontier pairs parked in the overflow bitmap
     unsigned long long fill_pos;  // fill append position
     // statistics, accumulated once per block at kernel end
@@ -244,6 +244,18 @@ const void* traverse_kernel_ptr();
 size_t traverse_lds_bytes();
 
 hipError_t launch_fill(uint32_t* p, uint64_t count, uint32_t value, hipStream_t s);
+// Arrays of 32-bit words to clear together.
+struct ZeroSpans {
+    static constexpr int MAX = 6;
+    uint32_t* p[MAX];
+    uint64_t words[MAX];
+    int count;
+    void add(void* q, uint64_t bytes) {
+        p[count] = static_cast<uint32_t*>(q);
+        words[count++] = bytes / 4;
+    }
+};
+hipError_t launch_zero(const ZeroSpans& z, hipStream_t s);
 hipError_t launch_add(int32_t* p, uint64_t count, int32_t delta, hipStream_t s);  // p[i] += delta
 
 // A matrix prepared on the host for a reach-mode arena (the request server
@@ -289,6 +301,8 @@ struct RowParams {
     int64_t* R_ptr;        // n + 1: offsets of the rows' record lists
     uint4* list;           // the lists
     int64_t list_cap;
+    uint32_t* long_rows;   // n: rows of over 64 records
+    uint32_t* long_count;  // zero on entry
     int32_t* L_col;
     int32_t* U_col;
     int64_t L_cap, U_cap;  // entries allocated: no write beyond
@@ -338,7 +352,7 @@ struct SuperParams {
     int32_t* supno;        // n
     int32_t* super_start;  // n+1
     int32_t* n_super;      // 1
-    int64_t* tmp64;        // scratch: 2n+1 + scan_tmp_words(n)
+    int64_t* tmp64;        // scratch: two words per 2,048 rows
     uint32_t* flag;        // n scratch
     const uint32_t* pass;  // optional, n: row i-1 is in L_i (then L_col is not read)
 };

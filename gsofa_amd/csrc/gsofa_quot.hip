@@ -656,9 +656,8 @@ void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vec
     off[levels] = (uint32_t)tab.size();
 }
 
+// p.ctl is zero on entry.
 hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hipStream_t s) {
-    hipError_t e = launch_fill(reinterpret_cast<uint32_t*>(p.ctl), sizeof(QuotCtl) / 4, 0u, s);
-    if (e != hipSuccess) return e;
     auto map_blocks = [](uint64_t vertices) {
         return (uint32_t)std::min<uint64_t>((vertices + QNT_LEVEL - 1) / QNT_LEVEL, 1024);
     };

@@ -19,8 +19,11 @@
 //
 // Measured against what it replaces, a stream of 8 B per fill that was cleared,
 // counted per row, scattered and sorted (structure pass with supernodes,
-// traversal, in ms, before -> now): 48^3 grid 5.6 -> 0.9, 3.27 -> 2.78; band
-// n = 659,033 5.8 -> 0.8, 5.71 -> 4.72; 128 2D grids 7.0 -> 1.8, 33.5 -> 31.2.
+// traversal, in ms, before -> now): 48^3 grid 5.6 -> 0.73, 3.27 -> 2.78; band
+// n = 659,033 5.8 -> 0.65, 5.71 -> 4.72; 128 2D grids 7.0 -> 1.1, 33.5 -> 31.2.
+// Rows of L with four rows a wave, and those of over 64 records from a list: 0.48
+// -> 0.32 ms at 48^3, 0.90 -> 0.46 at the 128 grids (a workgroup's barriers per
+// long row and a wave for every short one before).
 // 217 M fills of the 48^3 grid are 1.74 GB of stream, its records 0.1 GB.
 #include <algorithm>
 
@@ -37,9 +40,9 @@ using dev::rank_in;
 constexpr int RT = 256;             // threads per block
 constexpr int SITEMS = 8;           // rows per thread of a scan tile
 constexpr int STILE = RT * SITEMS;
-constexpr uint32_t LSLOTS = 4096;   // records of a long row held in LDS at once
-constexpr uint32_t WREC = 64;       // rows of up to so many records: one wave each
-constexpr int LROWS = 16;           // rows scanned per step for longer ones
+constexpr uint32_t LSLOTS = 2048;   // record slots of a wave, for rows of over 64 records
+constexpr uint32_t LGRID = 512;     // workgroups of k_rows_long: two per CU by their slots
+constexpr uint32_t SUB = 16;        // lanes of a row of up to so many records
 
 // Inclusive scan over the block of one value per thread; total in *sum.
 __device__ __forceinline__ int64_t block_scan(int64_t x, int64_t* sh, int64_t* sum) {
@@ -64,34 +67,60 @@ __device__ __forceinline__ int64_t block_scan(int64_t x, int64_t* sh, int64_t* s
 }
 
 // Per row: its fills (the rows' entries less A's own), and per tile of rows the
-// sums of L entries, U entries and L records.
+// sums of L entries, U entries and L records.  Whether A holds a row's diagonal
+// comes from a binary search, all of a thread's rows in step.
 __global__ __launch_bounds__(RT) void k_row_sums(RowParams p) {
-    __shared__ int64_t sh[RT / WAVE];
-    const int64_t base = (int64_t)blockIdx.x * STILE + (int64_t)threadIdx.x * SITEMS;
-    int64_t l = 0, u = 0, r = 0;
+    __shared__ unsigned long long sh[3];
+    if (threadIdx.x < 3) sh[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * STILE + threadIdx.x;
+    int32_t lo[SITEMS], len[SITEMS], end[SITEMS];
 #pragma unroll
     for (int k = 0; k < SITEMS; k++) {
-        const int64_t s = base + k;
-        if (s >= p.n) break;
+        const int64_t s = base + (int64_t)k * RT;
+        lo[k] = s < p.n ? p.rp[s] : 0;
+        end[k] = s < p.n ? p.rp[s + 1] : 0;
+        len[k] = end[k] - lo[k];
+    }
+    for (bool more = true; more;) {
+        more = false;
+#pragma unroll
+        for (int k = 0; k < SITEMS; k++) {
+            if (len[k] <= 0) continue;
+            const int32_t half = len[k] >> 1;
+            if (p.ci[lo[k] + half] < (int32_t)(base + (int64_t)k * RT)) {
+                lo[k] += half + 1;
+                len[k] -= half + 1;
+            } else {
+                len[k] = half;
+            }
+            more |= len[k] > 0;
+        }
+    }
+    unsigned long long l = 0, u = 0, r = 0;
+#pragma unroll
+    for (int k = 0; k < SITEMS; k++) {
+        const int64_t s = base + (int64_t)k * RT;
+        if (s >= p.n) continue;
         const unsigned long long c = p.cntL[s];
         const int64_t cl = (int64_t)(uint32_t)c, cu = p.cntU[s];
-        int64_t own = 0;  // A's entries off the diagonal
-        for (int32_t e = p.rp[s]; e < p.rp[s + 1]; e++) own += p.ci[e] != (int32_t)s;
-        p.row_fill[s] = cl + cu - own;
-        l += cl;
-        u += cu;
-        r += (int64_t)(c >> 32);
+        const int64_t diag = lo[k] < end[k] && p.ci[lo[k]] == (int32_t)s;
+        p.row_fill[s] = cl + cu - ((int64_t)(end[k] - p.rp[s]) - diag);
+        l += (unsigned long long)cl;
+        u += (unsigned long long)cu;
+        r += c >> 32;
     }
     if (!p.sums) return;  // counts only
-    int64_t tl, tu, tr;
-    block_scan(l, sh, &tl);
-    block_scan(u, sh, &tu);
-    block_scan(r, sh, &tr);
-    if (threadIdx.x == 0) {
-        p.sums[3 * blockIdx.x] = tl;
-        p.sums[3 * blockIdx.x + 1] = tu;
-        p.sums[3 * blockIdx.x + 2] = tr;
+    l = dev::wave_sum64(l);
+    u = dev::wave_sum64(u);
+    r = dev::wave_sum64(r);
+    if (__lane_id() == 0) {
+        atomicAdd(&sh[0], l);
+        atomicAdd(&sh[1], u);
+        atomicAdd(&sh[2], r);
     }
+    __syncthreads();
+    if (threadIdx.x < 3) p.sums[3 * blockIdx.x + threadIdx.x] = (int64_t)sh[threadIdx.x];
 }
 
 // Row pointers: each block adds up the tiles before its own.
@@ -221,23 +250,120 @@ __device__ __forceinline__ uint64_t lane_mask(uint32_t lo, uint32_t hi, uint32_t
            (uint32_t)__builtin_amdgcn_readlane((int)lo, (int)i);
 }
 
-// Rows that take records from many groups, up to WREC of them: one wave per
-// row sorts them by first source and stores each.
+// A wave's row of nt <= 64 records, sorted by first source in registers.
+__device__ void row_in_registers(uint32_t S, const uint4* list, int64_t b, uint32_t nt, int32_t* dst, int64_t q0,
+                                 int64_t cap) {
+    const uint32_t lane = __lane_id();
+    const uint4 t = lane < nt ? list[b + lane] : make_uint4(0u, ~0u, 0u, 0u);
+    uint32_t f = t.y, lo = t.z, hi = t.w;  // first sources are distinct in a row; empty lanes last
+    for (uint32_t k = 2; k < 2u * nt; k <<= 1) {
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+            const uint32_t of = __shfl_xor(f, (int)j), ol = __shfl_xor(lo, (int)j), oh = __shfl_xor(hi, (int)j);
+            const bool keep_min = ((lane & j) == 0u) == ((lane & k) == 0u);
+            if (keep_min ? of < f : of > f) {
+                f = of;
+                lo = ol;
+                hi = oh;
+            }
+        }
+    }
+    const uint32_t c = (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
+    const uint32_t before = dev::wave_incl_scan(c) - c;
+    for (uint32_t i = 0; i < nt; i++)
+        store_record(lane_mask(lo, hi, i), (uint32_t)__builtin_amdgcn_readlane((int)f, (int)i), S, lane, dst,
+                     q0 + (uint32_t)__builtin_amdgcn_readlane((int)before, (int)i), cap);
+}
+
+// A wave's row of any number of records: they go to LDS slots by first source
+// (a row's first sources differ by multiples of the word), a window of LSLOTS
+// at a time, and are stored in slot order.
+__device__ void row_by_slots(uint32_t S, const uint4* list, int64_t b, int64_t e, int32_t* dst, int64_t q0,
+                             int64_t cap, uint64_t* slot) {
+    const uint32_t lane = __lane_id();
+    uint32_t lo = ~0u, hi = 0u;
+    for (int64_t i = b + lane; i < e; i += WAVE) {
+        const uint32_t f = list[i].y;
+        lo = f < lo ? f : lo;
+        hi = f > hi ? f : hi;
+    }
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const uint32_t ol = __shfl_xor(lo, d), oh = __shfl_xor(hi, d);
+        lo = ol < lo ? ol : lo;
+        hi = oh > hi ? oh : hi;
+    }
+    const uint32_t all = (hi - lo) / S + 1u;
+    for (uint32_t s0 = 0; s0 < all; s0 += LSLOTS) {
+        const uint32_t ns = all - s0 < LSLOTS ? all - s0 : LSLOTS;
+        const uint32_t tiles = (ns + WAVE - 1u) / WAVE;
+        for (uint32_t k = 0; k < tiles; k++) slot[k * WAVE + lane] = 0ull;
+        dev::wave_sync();
+        for (int64_t i = b + lane; i < e; i += WAVE) {
+            const uint4 x = list[i];
+            const uint32_t k = (x.y - lo) / S - s0;
+            if (k < ns) slot[k] = ((uint64_t)x.w << 32) | x.z;
+        }
+        dev::wave_sync();
+        for (uint32_t k = 0; k < tiles; k++) {
+            const uint64_t x = slot[k * WAVE + lane];
+            const uint32_t c = (uint32_t)__popcll(x);
+            const uint32_t incl = dev::wave_incl_scan(c);
+            for (uint64_t some = __ballot(c != 0u); some; some &= some - 1ull) {
+                const uint32_t i = (uint32_t)__builtin_ctzll(some);
+                store_record(lane_mask((uint32_t)x, (uint32_t)(x >> 32), i), lo + (s0 + k * WAVE + i) * S, S, lane, dst,
+                             q0 + (uint32_t)__builtin_amdgcn_readlane((int)(incl - c), (int)i), cap);
+            }
+            q0 += (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+        }
+        dev::wave_sync();  // slots are read before the next window clears them
+    }
+}
+
+// Rows that take records from many groups.  A wave takes four rows at a time:
+// SUB lanes each while none has over SUB records (most rows of banded and 2D
+// matrices), else one after the other; rows of over 64 records go to the list
+// of k_rows_long, whose LDS slots would leave this kernel few waves.
 __global__ __launch_bounds__(RT) void k_rows_by_target(RowParams p, const int64_t* ptr, const uint4* list,
                                                        const int64_t* rowptr, int32_t* dst, int64_t cap) {
-    const uint32_t lane = __lane_id(), S = p.slots;
+    constexpr uint32_t PER = WAVE / SUB;
+    const uint32_t lane = __lane_id(), S = p.slots, sub = lane / SUB, l = lane % SUB;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t waves = gridDim.x * (RT / WAVE);
-    for (uint32_t r = blockIdx.x * (RT / WAVE) + w; r < (uint32_t)p.n; r += waves) {
-        const int64_t b = ptr[r], e = ptr[r + 1];
-        if (e <= b || e - b > (int64_t)WREC || e > p.list_cap) continue;
-        const uint32_t nt = (uint32_t)(e - b);
-        const uint4 t = lane < nt ? list[b + lane] : make_uint4(0u, ~0u, 0u, 0u);
-        uint32_t f = t.y, lo = t.z, hi = t.w;  // first sources are distinct in a row; empty lanes last
-        for (uint32_t k = 2; k < 2u * nt; k <<= 1) {
+    const uint32_t step = gridDim.x * (RT / WAVE) * PER;
+    for (uint32_t r0 = (blockIdx.x * (RT / WAVE) + w) * PER; r0 < (uint32_t)p.n; r0 += step) {
+        const uint32_t r = r0 + sub;
+        int64_t b = 0, e = 0, q = 0;
+        if (r < (uint32_t)p.n) {
+            b = ptr[r];
+            e = ptr[r + 1];
+            q = rowptr[r];
+        }
+        if (e > p.list_cap) e = b;
+        const uint32_t nt = e - b > 0xFFFF ? 0xFFFFu : (uint32_t)(e - b);
+        uint32_t most = nt;
+#pragma unroll
+        for (uint32_t d = SUB; d < WAVE; d <<= 1) {
+            const uint32_t o = __shfl_xor(most, (int)d);
+            most = o > most ? o : most;
+        }
+        most = __builtin_amdgcn_readfirstlane(most);
+        if (most == 0u) continue;
+        if (most > SUB) {
+            for (uint32_t k = 0; k < PER; k++) {
+                const int src = (int)(k * SUB);
+                const int64_t bk = (int64_t)dev::bcast_64((uint64_t)b, src), ek = (int64_t)dev::bcast_64((uint64_t)e, src);
+                const int64_t qk = (int64_t)dev::bcast_64((uint64_t)q, src);
+                if (ek <= bk) continue;
+                if (ek - bk <= WAVE) row_in_registers(S, list, bk, (uint32_t)(ek - bk), dst, qk, cap);
+                else if (lane == 0) p.long_rows[atomicAdd(p.long_count, 1u)] = r0 + k;
+            }
+            continue;
+        }
+        const uint4 t = l < nt ? list[b + l] : make_uint4(0u, ~0u, 0u, 0u);
+        uint32_t f = t.y, lo = t.z, hi = t.w;
+        for (uint32_t k = 2; k < 2u * most; k <<= 1) {
             for (uint32_t j = k >> 1; j > 0; j >>= 1) {
                 const uint32_t of = __shfl_xor(f, (int)j), ol = __shfl_xor(lo, (int)j), oh = __shfl_xor(hi, (int)j);
-                const bool keep_min = ((lane & j) == 0u) == ((lane & k) == 0u);
+                const bool keep_min = ((l & j) == 0u) == ((l & k) == 0u);
                 if (keep_min ? of < f : of > f) {
                     f = of;
                     lo = ol;
@@ -245,96 +371,42 @@ __global__ __launch_bounds__(RT) void k_rows_by_target(RowParams p, const int64_
                 }
             }
         }
-        const uint32_t c = (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
-        const uint32_t before = dev::wave_incl_scan(c) - c;
-        const int64_t q0 = rowptr[r];
-        for (uint32_t i = 0; i < nt; i++)
-            store_record(lane_mask(lo, hi, i), (uint32_t)__builtin_amdgcn_readlane((int)f, (int)i), S, lane, dst,
-                         q0 + (uint32_t)__builtin_amdgcn_readlane((int)before, (int)i), cap);
+        // a record's columns in increasing order: lane l of the row has its bits
+        // S - 1 - 4 l down to S - 4 - 4 l
+        for (uint32_t i = 0; i < most; i++) {
+            const uint64_t m = ((uint64_t)__shfl(hi, (int)i, SUB) << 32) | __shfl(lo, (int)i, SUB);
+            const uint32_t fi = __shfl(f, (int)i, SUB);
+            const uint32_t top = S - 1u - 4u * l;  // wraps past the word's bits
+            const uint32_t nib = i < nt && top < S ? (uint32_t)(m >> (top - 3u)) & 15u : 0u;
+            const uint32_t c = (uint32_t)__popc(nib);
+            uint32_t incl = c;
+#pragma unroll
+            for (uint32_t d = 1; d < SUB; d <<= 1) {
+                const uint32_t y = __shfl_up(incl, d, SUB);
+                if (l >= d) incl += y;
+            }
+            int64_t at = q + (incl - c);
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; j++) {
+                if ((nib >> (3u - j)) & 1u) {
+                    if (at < cap) dst[at] = (int32_t)(fi - (top - j));
+                    at++;
+                }
+            }
+            q += __shfl(incl, (int)SUB - 1, SUB);
+        }
     }
 }
 
-// Rows of more records: one block per row puts them into LDS slots by first
-// source (a row's first sources differ by multiples of the word), a window of
-// LSLOTS at a time, and stores them in slot order.
-__global__ __launch_bounds__(RT) void k_rows_by_target_long(RowParams p, const int64_t* ptr, const uint4* list,
-                                                            const int64_t* rowptr, int32_t* dst, int64_t cap) {
-    __shared__ uint64_t slot[LSLOTS];
-    __shared__ uint32_t sum[LSLOTS / WAVE];
-    __shared__ uint32_t red[2];
-    __shared__ uint64_t longs;
-    const uint32_t t = threadIdx.x, lane = __lane_id(), S = p.slots;
-    const uint32_t w = __builtin_amdgcn_readfirstlane(t / WAVE);
-    for (uint32_t r0 = blockIdx.x * LROWS; r0 < (uint32_t)p.n; r0 += gridDim.x * LROWS) {
-        if (t < WAVE) {
-            bool lng = false;
-            if (t < LROWS && r0 + t < (uint32_t)p.n) {
-                const int64_t b = ptr[r0 + t], e = ptr[r0 + t + 1];
-                lng = e - b > (int64_t)WREC && e <= p.list_cap;
-            }
-            const uint64_t m = __ballot(lng);
-            if (t == 0) longs = m;
-        }
-        __syncthreads();
-        for (uint64_t m = longs; m; m &= m - 1ull) {
-            const uint32_t r = r0 + (uint32_t)__builtin_ctzll(m);
-            const int64_t b = ptr[r], e = ptr[r + 1];
-            if (t == 0) {
-                red[0] = ~0u;
-                red[1] = 0u;
-            }
-            __syncthreads();
-            uint32_t lo = ~0u, hi = 0u;
-            for (int64_t i = b + t; i < e; i += RT) {
-                const uint32_t f = list[i].y;
-                lo = f < lo ? f : lo;
-                hi = f > hi ? f : hi;
-            }
-            atomicMin(&red[0], lo);
-            atomicMax(&red[1], hi);
-            __syncthreads();
-            lo = red[0];
-            hi = red[1];
-            int64_t q0 = rowptr[r];
-            const uint32_t all = (hi - lo) / S + 1u;
-            for (uint32_t s0 = 0; s0 < all; s0 += LSLOTS) {
-                const uint32_t ns = all - s0 < LSLOTS ? all - s0 : LSLOTS;
-                const uint32_t nt = (ns + WAVE - 1u) / WAVE;
-                for (uint32_t i = t; i < nt * WAVE; i += RT) slot[i] = 0ull;
-                __syncthreads();
-                for (int64_t i = b + t; i < e; i += RT) {
-                    const uint4 x = list[i];
-                    const uint32_t k = (x.y - lo) / S - s0;
-                    if (k < ns) slot[k] = ((uint64_t)x.w << 32) | x.z;
-                }
-                __syncthreads();
-                for (uint32_t k = w; k < nt; k += RT / WAVE) {
-                    const uint64_t x = dev::wave_sum64((unsigned long long)__popcll(slot[k * WAVE + lane]));
-                    if (lane == 0) sum[k] = (uint32_t)x;
-                }
-                __syncthreads();
-                if (w == 0) {  // LSLOTS / WAVE tiles: one per lane
-                    static_assert(LSLOTS / WAVE == WAVE, "one tile per lane");
-                    const uint32_t x = lane < nt ? sum[lane] : 0u;
-                    sum[lane] = dev::wave_incl_scan(x);
-                }
-                __syncthreads();
-                for (uint32_t k = w; k < nt; k += RT / WAVE) {
-                    const uint64_t x = slot[k * WAVE + lane];
-                    const uint32_t c = (uint32_t)__popcll(x);
-                    const uint32_t before = (k ? sum[k - 1] : 0u) + dev::wave_incl_scan(c) - c;
-                    for (uint64_t some = __ballot(c != 0u); some; some &= some - 1ull) {
-                        const uint32_t i = (uint32_t)__builtin_ctzll(some);
-                        store_record(lane_mask((uint32_t)x, (uint32_t)(x >> 32), i), lo + (s0 + k * WAVE + i) * S, S,
-                                     lane, dst, q0 + (uint32_t)__builtin_amdgcn_readlane((int)before, (int)i), cap);
-                    }
-                }
-                q0 += sum[nt - 1];
-                __syncthreads();  // slots and sums are read
-            }
-            __syncthreads();  // red is read
-        }
-        __syncthreads();  // longs is read
+// The listed rows, one wave each.
+__global__ __launch_bounds__(RT) void k_rows_long(RowParams p, const int64_t* ptr, const uint4* list,
+                                                  const int64_t* rowptr, int32_t* dst, int64_t cap) {
+    __shared__ uint64_t slots[RT / WAVE][LSLOTS];
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t count = *p.long_count, step = gridDim.x * (RT / WAVE);
+    for (uint32_t i = blockIdx.x * (RT / WAVE) + w; i < count; i += step) {
+        const uint32_t r = p.long_rows[i];
+        row_by_slots(p.slots, list, ptr[r], ptr[r + 1], dst, rowptr[r], cap, slots[w]);
     }
 }
 
@@ -365,11 +437,10 @@ hipError_t launch_rows(const RowParams& p, hipStream_t s) {
     if (groups == 0) return hipSuccess;
     hipLaunchKernelGGL(k_rows_by_source, dim3(groups * p.words), dim3(RT), 0, s, p, 0u, p.U_rowptr, p.U_col, p.U_cap);
     hipLaunchKernelGGL(k_rec_lists, dim3(groups), dim3(RT), 0, s, p, 1u, p.cntL, p.R_ptr, p.list);
-    const uint32_t wb = (uint32_t)std::min<int64_t>((p.n + RT / WAVE - 1) / (RT / WAVE), 8192);
+    const int64_t per = (int64_t)(RT / WAVE) * (WAVE / SUB);
+    const uint32_t wb = (uint32_t)std::min<int64_t>((p.n + per - 1) / per, 8192);
     hipLaunchKernelGGL(k_rows_by_target, dim3(wb), dim3(RT), 0, s, p, p.R_ptr, p.list, p.L_rowptr, p.L_col, p.L_cap);
-    const uint32_t lb = (uint32_t)std::min<int64_t>((p.n + LROWS - 1) / LROWS, 8192);
-    hipLaunchKernelGGL(k_rows_by_target_long, dim3(lb), dim3(RT), 0, s, p, p.R_ptr, p.list, p.L_rowptr, p.L_col,
-                       p.L_cap);
+    hipLaunchKernelGGL(k_rows_long, dim3(LGRID), dim3(RT), 0, s, p, p.R_ptr, p.list, p.L_rowptr, p.L_col, p.L_cap);
     return hipGetLastError();
 }
 

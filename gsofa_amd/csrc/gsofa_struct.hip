@@ -6,6 +6,8 @@
 // with_space_optimization/symbfact.cuh:2126) and has only a stub for
 // supernodes (with_space_optimization/with_supernodes/symbfact.cuh:1087-1101);
 // the outputs here are defined by the fill-path sets themselves.
+#include <algorithm>
+
 #include "gsofa_device.h"
 #include "gsofa_internal.h"
 
@@ -38,6 +40,13 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t count, uint32_t v) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
          i += (uint64_t)gridDim.x * blockDim.x)
         p[i] = v;
+}
+
+// Clears up to ZeroSpans::MAX arrays of 32-bit words in one launch.
+__global__ void k_zero(ZeroSpans z) {
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+    for (int k = 0; k < z.count; k++)
+        for (uint64_t i = t; i < z.words[k]; i += step) z.p[k][i] = 0u;
 }
 
 __global__ void k_add_i32(int32_t* p, uint64_t count, int32_t d) {
@@ -450,11 +459,6 @@ struct OpAdd {
     __device__ static int64_t apply(int64_t a, int64_t b) { return a + b; }
     __device__ static int64_t identity() { return 0; }
 };
-struct OpMax {
-    __device__ static int64_t apply(int64_t a, int64_t b) { return a > b ? a : b; }
-    __device__ static int64_t identity() { return INT64_MIN; }
-};
-
 template <class Op>
 __global__ __launch_bounds__(SB) void k_scan_tiles(int64_t* a, int64_t len, int64_t* sums) {
     __shared__ int64_t sh[SB];
@@ -520,50 +524,136 @@ __global__ void k_u32_to_i64_shift(const uint32_t* in, int64_t* out, int64_t n) 
 // traversal from i passes through i-1), |U_i| = |U_{i-1}| - 1, and the
 // supernode holds fewer than max_size rows.  The cap splits a maximal run of
 // joining rows into consecutive pieces of max_size rows.
-__global__ void k_sn_flags(SuperParams p, int64_t* key) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p.n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        bool join = false;
-        if (i > 0) {
-            bool pass;
-            if (p.pass) {
-                pass = p.pass[i] != 0u;
-            } else {
-                const int64_t lb = p.L_rowptr[i], le = p.L_rowptr[i + 1];
-                pass = le > lb && p.L_col[le - 1] == (int32_t)(i - 1);
-            }
-            const int64_t ui = p.U_rowptr[i + 1] - p.U_rowptr[i];
-            const int64_t up = p.U_rowptr[i] - p.U_rowptr[i - 1];
-            join = pass && (ui == up - 1);
-        }
+// Three launches over tiles of SCAN_TILE rows; each block adds up what the
+// tiles before its own left (thousands at most), so no scan launches lie
+// between: on small matrices a launch's 5 us are all its time.
+__device__ __forceinline__ int64_t block_max(int64_t x, int64_t* sh) {
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int64_t y = __shfl_xor(x, d, WAVE);
+        x = y > x ? y : x;
+    }
+    if ((t & (WAVE - 1)) == 0) sh[t / WAVE] = x;
+    __syncthreads();
+    x = sh[0];
+    for (int k = 1; k < SB / WAVE; k++) x = sh[k] > x ? sh[k] : x;
+    __syncthreads();
+    return x;
+}
+
+// Exclusive prefix over the block (Op: max from -1, or sum from 0) of one value
+// per thread; the block's total in *all.
+template <bool MAX>
+__device__ __forceinline__ int64_t block_prefix(int64_t x, int64_t* sh, int64_t* all) {
+    const int t = threadIdx.x, lane = t & (WAVE - 1), w = t / WAVE;
+    int64_t incl = x;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int64_t y = __shfl_up(incl, d, WAVE);
+        if (lane >= d) incl = MAX ? (y > incl ? y : incl) : incl + y;
+    }
+    if (lane == WAVE - 1) sh[w] = incl;
+    __syncthreads();
+    int64_t pre = MAX ? -1 : 0, tot = pre;
+    for (int k = 0; k < SB / WAVE; k++) {
+        const int64_t v = sh[k];
+        if (k < w) pre = MAX ? (v > pre ? v : pre) : pre + v;
+        tot = MAX ? (v > tot ? v : tot) : tot + v;
+    }
+    __syncthreads();
+    const int64_t left = __shfl_up(incl, 1, WAVE);
+    if (lane > 0) pre = MAX ? (left > pre ? left : pre) : pre + left;
+    *all = tot;
+    return pre;
+}
+
+__device__ __forceinline__ bool sn_join(const SuperParams& p, int64_t i) {
+    if (i <= 0) return false;
+    bool pass;
+    if (p.pass) {
+        pass = p.pass[i] != 0u;
+    } else {
+        const int64_t lb = p.L_rowptr[i], le = p.L_rowptr[i + 1];
+        pass = le > lb && p.L_col[le - 1] == (int32_t)(i - 1);
+    }
+    const int64_t u0 = p.U_rowptr[i - 1], u1 = p.U_rowptr[i], u2 = p.U_rowptr[i + 1];
+    return pass && u2 - u1 == u1 - u0 - 1;
+}
+
+// Join flags, and per tile the last row that starts a run (-1: none).
+__global__ __launch_bounds__(SB) void k_sn_joins(SuperParams p, int64_t* runs) {
+    __shared__ int64_t sh[SB / WAVE];
+    int64_t last = -1;
+    for (int k = 0; k < SCAN_ITEMS; k++) {
+        const int64_t i = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)k * SB + threadIdx.x;
+        if (i >= p.n) break;
+        const bool join = sn_join(p, i);
         p.flag[i] = join ? 1u : 0u;
-        key[i] = join ? 0 : i;  // run start via inclusive max-scan
+        if (!join) last = i;
     }
+    last = block_max(last, sh);
+    if (threadIdx.x == 0) runs[blockIdx.x] = last;
 }
 
-__global__ void k_sn_starts(SuperParams p, const int64_t* runstart, int64_t* cnt) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p.n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const bool join = p.flag[i] != 0u;
-        const int64_t pos = i - runstart[i];
-        const bool start = !join || (p.max_size > 0 && (pos % p.max_size) == 0);
+// Supernode starts (a run's first row, or max_size rows into it) in place of
+// the join flags, and per tile their count.
+__global__ __launch_bounds__(SB) void k_sn_starts(SuperParams p, const int64_t* runs, int64_t* counts) {
+    __shared__ int64_t sh[SB / WAVE];
+    int64_t pre = -1, all;
+    for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SB) pre = runs[t] > pre ? runs[t] : pre;
+    pre = block_max(pre, sh);
+    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    uint32_t join = 0;
+    int64_t mine = -1;
+    for (int k = 0; k < SCAN_ITEMS; k++) {
+        const int64_t i = base + k;
+        if (i >= p.n) break;
+        if (p.flag[i]) join |= 1u << k;
+        else mine = i;
+    }
+    int64_t run = block_prefix<true>(mine, sh, &all);
+    run = run > pre ? run : pre;
+    int64_t cnt = 0;
+    for (int k = 0; k < SCAN_ITEMS; k++) {
+        const int64_t i = base + k;
+        if (i >= p.n) break;
+        const bool j = (join >> k) & 1u;
+        if (!j) run = i;
+        const bool start = !j || (p.max_size > 0 && ((i - run) % p.max_size) == 0);
         p.flag[i] = start ? 1u : 0u;
-        cnt[i + 1] = start ? 1 : 0;
+        cnt += start;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) cnt[0] = 0;
+    block_prefix<false>(cnt, sh, &all);
+    if (threadIdx.x == 0) counts[blockIdx.x] = all;
 }
 
-__global__ void k_sn_write(SuperParams p, const int64_t* excl) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p.n;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t id = excl[i] + (int64_t)p.flag[i] - 1;
-        p.supno[i] = (int32_t)id;
-        if (p.flag[i]) p.super_start[excl[i]] = (int32_t)i;
+__global__ __launch_bounds__(SB) void k_sn_write(SuperParams p, const int64_t* counts) {
+    __shared__ int64_t sh[SB / WAVE];
+    if (p.n <= 0) {
+        if (threadIdx.x == 0) {
+            *p.n_super = 0;
+            p.super_start[0] = 0;
+        }
+        return;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const int32_t ns = (int32_t)excl[p.n];
-        *p.n_super = ns;
-        p.super_start[ns] = p.n;
+    int64_t sum = 0, pre, all;
+    for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SB) sum += counts[t];
+    block_prefix<false>(sum, sh, &pre);
+    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+    uint32_t start = 0;
+    for (int k = 0; k < SCAN_ITEMS; k++)
+        if (base + k < p.n && p.flag[base + k]) start |= 1u << k;
+    int64_t id = pre + block_prefix<false>((int64_t)__popc(start), sh, &all) - 1;
+    for (int k = 0; k < SCAN_ITEMS; k++) {
+        const int64_t i = base + k;
+        if (i >= p.n) break;
+        if ((start >> k) & 1u) p.super_start[++id] = (int32_t)i;
+        p.supno[i] = (int32_t)id;
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        *p.n_super = (int32_t)(pre + all);
+        p.super_start[pre + all] = p.n;
     }
 }
 
@@ -690,6 +780,14 @@ hipError_t launch_fill(uint32_t* p, uint64_t count, uint32_t value, hipStream_t 
     return hipGetLastError();
 }
 
+hipError_t launch_zero(const ZeroSpans& z, hipStream_t s) {
+    uint64_t most = 0;
+    for (int k = 0; k < z.count; k++) most = std::max(most, z.words[k]);
+    if (most == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_zero, grid_for((int64_t)most, SB, 4096), dim3(SB), 0, s, z);
+    return hipGetLastError();
+}
+
 size_t scan_tmp_words(int64_t n) {
     size_t words = 0;
     int64_t len = n + 1;
@@ -735,20 +833,14 @@ hipError_t launch_sort_segments(const int64_t* rowptr, const int32_t* src, int32
 }
 
 hipError_t launch_supernodes(const SuperParams& p, hipStream_t s) {
-    if (p.n <= 0) {
-        hipLaunchKernelGGL(k_sn_write, dim3(1), dim3(SB), 0, s, p, p.tmp64);
-        return hipGetLastError();
+    const uint32_t tiles = p.n > 0 ? (uint32_t)(((int64_t)p.n + SCAN_TILE - 1) / SCAN_TILE) : 1u;
+    int64_t* runs = p.tmp64;            // tiles
+    int64_t* counts = p.tmp64 + tiles;  // tiles
+    if (p.n > 0) {
+        hipLaunchKernelGGL(k_sn_joins, dim3(tiles), dim3(SB), 0, s, p, runs);
+        hipLaunchKernelGGL(k_sn_starts, dim3(tiles), dim3(SB), 0, s, p, runs, counts);
     }
-    int64_t* key = p.tmp64;             // n
-    int64_t* cnt = p.tmp64 + p.n;       // n+1
-    int64_t* scratch = cnt + p.n + 1;   // scan temporaries
-    hipLaunchKernelGGL(k_sn_flags, grid_for(p.n), dim3(SB), 0, s, p, key);
-    hipError_t e = inclusive_scan<OpMax>(key, p.n, scratch, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_sn_starts, grid_for(p.n), dim3(SB), 0, s, p, key, cnt);
-    e = inclusive_scan<OpAdd>(cnt + 1, p.n, scratch, s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_sn_write, grid_for(p.n), dim3(SB), 0, s, p, cnt);
+    hipLaunchKernelGGL(k_sn_write, dim3(tiles), dim3(SB), 0, s, p, counts);
     return hipGetLastError();
 }
 
