@@ -214,16 +214,17 @@ def _options(n_virtual_gpu=1, virtual_gpu_id=-1, mem_gb=0.0, mem_budget_bytes=0,
 
 
 class _Owner:
-    """Holds a library-owned gsofa_result and releases it (gsofa_result_free)
-    when the last array viewing its memory is gone."""
+    """Holds a library-owned result and releases it (gsofa_result_free, or the
+    given function) when the last array viewing its memory is gone."""
 
-    def __init__(self, r):
+    def __init__(self, r, free="gsofa_result_free"):
         self.r = r
+        self.free = free
 
     def __del__(self):
         if self.r is not None:
             try:
-                _lib.lib().gsofa_result_free(C.byref(self.r))
+                getattr(_lib.lib(), self.free)(C.byref(self.r))
             except Exception:  # interpreter shutdown: the process releases it
                 pass
             self.r = None
@@ -287,27 +288,28 @@ class SymbfactResult:
             self.supno = None
 
 
-def _carr(ptr, cnt, ct, dt):
-    if cnt <= 0:
-        return np.zeros(0, dt)
-    return np.ctypeslib.as_array(C.cast(ptr, C.POINTER(ct)), shape=(cnt,)).copy()
-
-
 class SupernodalResult:
     """Supernodal hand-off (include/gsofa.h, gsofa_supernodal): supernode
-    starts and ids, per-supernode subscripts, and L and U by columns."""
+    starts and ids, per-supernode subscripts, and L and U by columns.
+
+    Takes ownership of the library result `h`: the arrays are views of its
+    memory (no copy), released with the last of them."""
 
     def __init__(self, h):
+        owner = _Owner(h, "gsofa_supernodal_free")
+
+        def arr(ptr, cnt, dt):
+            return np.asarray(_View(ptr, cnt, dt, owner)) if cnt > 0 else np.zeros(0, dt)
         n, ns = int(h.n), int(h.n_super)
         self.n, self.n_super = n, ns
-        self.xsup = _carr(h.xsup, ns + 1, C.c_int32, np.int32)
-        self.supno = _carr(h.supno, n, C.c_int32, np.int32)
-        self.xsub = _carr(h.xsub, ns + 1, C.c_int64, np.int64)
-        self.sub = _carr(h.sub, int(self.xsub[-1]), C.c_int32, np.int32)
-        self.xlcol = _carr(h.xlcol, n + 1, C.c_int64, np.int64)
-        self.lrow = _carr(h.lrow, int(self.xlcol[-1]), C.c_int32, np.int32)
-        self.xucol = _carr(h.xucol, n + 1, C.c_int64, np.int64)
-        self.urow = _carr(h.urow, int(self.xucol[-1]), C.c_int32, np.int32)
+        self.xsup = arr(h.xsup, ns + 1, np.int32)
+        self.supno = arr(h.supno, n, np.int32)
+        self.xsub = arr(h.xsub, ns + 1, np.int64)
+        self.sub = arr(h.sub, int(self.xsub[-1]), np.int32)
+        self.xlcol = arr(h.xlcol, n + 1, np.int64)
+        self.lrow = arr(h.lrow, int(self.xlcol[-1]), np.int32)
+        self.xucol = arr(h.xucol, n + 1, np.int64)
+        self.urow = arr(h.urow, int(self.xucol[-1]), np.int32)
 
 
 def symbfact(A, **kw):
@@ -363,10 +365,7 @@ class Plan:
         every share, structure built)."""
         h = _lib.Supernodal()
         _check(_lib.lib().gsofa_plan_fetch_supernodal(self._h, C.byref(h)), "plan_fetch_supernodal")
-        try:
-            return SupernodalResult(h)
-        finally:
-            _lib.lib().gsofa_supernodal_free(C.byref(h))
+        return SupernodalResult(h)
 
     def close(self):
         if getattr(self, "_h", None):

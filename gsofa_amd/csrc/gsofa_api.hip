@@ -149,7 +149,6 @@ struct gsofa_plan {
     int64_t nnzL = 0, nnzU = 0;
     int32_t* d_supno = nullptr;
     int32_t* d_sstart = nullptr;
-    int32_t* d_nsuper = nullptr;
     int64_t* d_sn64 = nullptr;
     uint32_t* d_snflag = nullptr;
 
@@ -175,7 +174,17 @@ struct gsofa_plan {
     hipGraphExec_t graph_exec = nullptr;
     bool graph_failed = false;  // capture was refused: executes run eagerly
     bool capturing = false;     // the stream is being captured: no event records
+    struct Piece {
+        void** where;
+        size_t bytes;
+    };
+    std::vector<Piece> pieces;  // of the slab, while gathered
+    bool gather = false;
+    char* slab = nullptr;
+    size_t slab_bytes = 0;
     Ctrl* h_ctrl = nullptr;     // pinned copy of the device counters
+    int32_t n_super = 0;
+    bool nsuper_known = false;
     bool last_replayed = false; // the last execute replayed the graph
     // arena (request server worker): capacities of the buffers a batch
     // fills, host copies the uploads read from, and supernode arrays' size
@@ -254,10 +263,36 @@ struct DevScratch {
     }
 };
 
+// A plan's device arrays.  Where all sizes are known at creation they are
+// pieces of one allocation (gather, then take_slab): twelve of 8 MB cost
+// 3.4 ms to make and release, one of 96 MB 0.6.
 template <class T>
-void dfree(T*& p) {
-    if (p) (void)hipFree(p);
+int palloc(gsofa_plan* P, T** p, size_t count) {
+    if (!P->gather) return dalloc(p, count);
+    *p = nullptr;
+    P->pieces.push_back({(void**)p, (sizeof(T) * std::max<size_t>(count, 1) + 511) & ~(size_t)511});
+    return GSOFA_OK;
+}
+
+template <class T>
+void pfree(gsofa_plan* P, T*& p) {
+    const char* a = (const char*)p;
+    if (a && !(P->slab && a >= P->slab && a < P->slab + P->slab_bytes)) (void)hipFree(p);
     p = nullptr;
+}
+
+int take_slab(gsofa_plan* P) {
+    P->gather = false;
+    P->slab_bytes = 0;
+    for (const gsofa_plan::Piece& x : P->pieces) P->slab_bytes += x.bytes;
+    const int e = dalloc(&P->slab, P->slab_bytes);
+    size_t off = 0;
+    for (const gsofa_plan::Piece& x : P->pieces) {
+        if (!e) *x.where = P->slab + off;
+        off += x.bytes;
+    }
+    P->pieces.clear();
+    return e;
 }
 
 int validate(const gsofa_matrix* A) {
@@ -322,12 +357,12 @@ uint64_t label_words(int32_t n, int32_t N, int32_t C, int32_t gid_lo, int32_t gi
 // fills, L and U entries of the rows it processes (every share, one share, or
 // for a spilled run the largest share).  rp/ci: packed rows.  bits > 0 (reach
 // mode): also the records of one pass, for groups of so many sources.
-void output_need(const gsofa_options& o, int32_t n, const int32_t* rp, const int32_t* ci, uint64_t* need_fill,
-                 uint64_t* need_L, uint64_t* need_U, int bits = 0, const std::vector<uint32_t>* mat_base = nullptr,
-                 uint64_t* need_rec = nullptr) {
+void output_need(const gsofa_options& o, int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT,
+                 const int32_t* ciT, uint64_t* need_fill, uint64_t* need_L, uint64_t* need_U, int bits = 0,
+                 const std::vector<uint32_t>* mat_base = nullptr, uint64_t* need_rec = nullptr) {
     std::vector<int64_t> Lb, Ub;
     std::vector<int32_t> parent;
-    lu_row_bounds(n, rp, ci, Lb, Ub, bits ? &parent : nullptr);
+    lu_row_bounds(n, rp, ci, rpT, ciT, Lb, Ub, bits ? &parent : nullptr);
     if (bits) *need_rec = reach_record_bound(*mat_base, parent, Ub, bits);
     const int32_t N = std::max(1, o.n_virtual_gpu);
     std::vector<uint64_t> fs((size_t)N, 0), ls((size_t)N, 0), us((size_t)N, 0);
@@ -508,27 +543,27 @@ void advance_state(gsofa_plan* P, int32_t gid) {
 // entries (list: records of the A^T pass, at most).
 int alloc_stream(gsofa_plan* P, uint64_t list) {
     if (P->mode != GSOFA_MODE_REACH) {
-        dfree(P->d_fills);
-        return dalloc(&P->d_fills, (size_t)P->fill_cap);
+        pfree(P, P->d_fills);
+        return palloc(P, &P->d_fills, (size_t)P->fill_cap);
     }
-    dfree(P->d_rec);
-    dfree(P->d_list);
+    pfree(P, P->d_rec);
+    pfree(P, P->d_list);
     P->list_cap = std::max<uint64_t>(list, 1);
-    if (dalloc(&P->d_rec, (size_t)P->fill_cap) || dalloc(&P->d_list, (size_t)P->list_cap)) return GSOFA_ERR_ALLOC;
+    if (palloc(P, &P->d_rec, (size_t)P->fill_cap) || palloc(P, &P->d_list, (size_t)P->list_cap)) return GSOFA_ERR_ALLOC;
     return GSOFA_OK;
 }
 
 void release_quot(gsofa_plan* P) {
     QuotParams& q = P->quot;
-    dfree(P->d_qtab);
-    dfree(q.comp);
-    dfree(q.info);
-    dfree(q.infoT);
-    dfree(q.ncnt);
-    dfree(q.blist);
-    dfree(q.nmap);
-    dfree(q.eb);
-    dfree(q.ctl);
+    pfree(P, P->d_qtab);
+    pfree(P, q.comp);
+    pfree(P, q.info);
+    pfree(P, q.infoT);
+    pfree(P, q.ncnt);
+    pfree(P, q.blist);
+    pfree(P, q.nmap);
+    pfree(P, q.eb);
+    pfree(P, q.ctl);
     q = QuotParams{};
     P->qcap = gsofa_plan::QuotCaps{};
 }
@@ -544,7 +579,7 @@ uint32_t quot_wanted(int64_t n, int64_t nnz, uint32_t W, int64_t room) {
 
 // The range table and device arrays of `levels` levels for the plan's matrices
 // (P->h_mat_base, n, nnz); d_ci and d_ciT hold quot_ext entries more.  Arrays
-// that are large enough stay (arenas).  The table's upload is queued.
+// that are large enough stay (arenas).
 int setup_quot(gsofa_plan* P, uint32_t levels) {
     QuotParams& q = P->quot;
     q.levels = levels;
@@ -558,42 +593,43 @@ int setup_quot(gsofa_plan* P, uint32_t levels) {
     gsofa_plan::QuotCaps& c = P->qcap;
     int e = 0;
     if (c.tab < P->h_qtab.size()) {
-        dfree(P->d_qtab);
-        dfree(q.ncnt);
-        e |= dalloc(&P->d_qtab, P->h_qtab.size());
-        dfree(q.blist);
-        e |= dalloc(&q.ncnt, P->h_qtab.size());
-        e |= dalloc(&q.blist, P->h_qtab.size());
+        pfree(P, P->d_qtab);
+        pfree(P, q.ncnt);
+        e |= palloc(P, &P->d_qtab, P->h_qtab.size());
+        pfree(P, q.blist);
+        e |= palloc(P, &q.ncnt, P->h_qtab.size());
+        e |= palloc(P, &q.blist, P->h_qtab.size());
         c.tab = P->h_qtab.size();
     }
     if (c.ln < ln) {
-        dfree(q.comp);
-        dfree(q.info);
-        dfree(q.infoT);
-        e |= dalloc(&q.comp, ln);
-        e |= dalloc(&q.info, ln);
-        e |= dalloc(&q.infoT, ln);
+        pfree(P, q.comp);
+        pfree(P, q.info);
+        pfree(P, q.infoT);
+        e |= palloc(P, &q.comp, ln);
+        e |= palloc(P, &q.info, ln);
+        e |= palloc(P, &q.infoT, ln);
         c.ln = ln;
     }
     if (c.n < n) {
-        dfree(q.nmap);
-        e |= dalloc(&q.nmap, 2 * n);
+        pfree(P, q.nmap);
+        e |= palloc(P, &q.nmap, 2 * n);
         c.n = n;
     }
     if (c.eb < (size_t)P->nnz) {
-        dfree(q.eb);
-        e |= dalloc(&q.eb, (size_t)P->nnz);
+        pfree(P, q.eb);
+        e |= palloc(P, &q.eb, (size_t)P->nnz);
         c.eb = (size_t)P->nnz;
     }
-    if (!q.ctl) e |= dalloc(&q.ctl, 1);
+    if (!q.ctl) e |= palloc(P, &q.ctl, 1);
     if (e) return GSOFA_ERR_ALLOC;
-    q.tab = P->d_qtab;
-    if (hipMemcpyAsync(P->d_qtab, P->h_qtab.data(), sizeof(uint2) * P->h_qtab.size(), hipMemcpyHostToDevice,
-                       P->stream) != hipSuccess) {
-        (void)hipGetLastError();
-        return GSOFA_ERR_HIP;
-    }
     return GSOFA_OK;
+}
+
+// The range table's upload joins the caller's.
+void upload_quot(gsofa_plan* P, std::vector<HostCopy>& up) {
+    if (P->quot.levels == 0) return;
+    P->quot.tab = P->d_qtab;
+    up.push_back({P->h_qtab.data(), P->d_qtab, sizeof(uint2) * P->h_qtab.size()});
 }
 
 // Bytes of setup_quot's arrays at their capacities (the class rows in d_ci and
@@ -603,200 +639,88 @@ int64_t quot_held(const gsofa_plan::QuotCaps& c) {
 }
 
 void release_device(gsofa_plan* P) {
-    dfree(P->d_rp);
-    dfree(P->d_ci);
-    dfree(P->d_lab);
-    dfree(P->d_mark);
-    dfree(P->d_orphan);
-    dfree(P->d_q0);
-    dfree(P->d_q1);
-    dfree(P->d_fills);
-    dfree(P->d_rec);
-    dfree(P->d_grp);
-    dfree(P->d_cnt64);
-    dfree(P->d_list);
-    dfree(P->d_rptr);
-    dfree(P->d_ctrl);
-    dfree(P->d_cntL);
-    dfree(P->d_cntU);
-    dfree(P->d_Lrp);
-    dfree(P->d_Urp);
-    dfree(P->d_rowfill);
-    dfree(P->d_scan);
-    dfree(P->d_Lcol);
-    dfree(P->d_Ucol);
-    dfree(P->d_Ltmp);
-    dfree(P->d_Utmp);
-    dfree(P->d_supno);
-    dfree(P->d_sstart);
-    dfree(P->d_nsuper);
-    dfree(P->d_sn64);
-    dfree(P->d_snflag);
-    dfree(P->d_sp_lcnt);
-    dfree(P->d_sp_ucnt);
-    dfree(P->d_sp_pass);
-    dfree(P->d_mask);
-    dfree(P->d_qgv);
-    dfree(P->d_bstate);
-    dfree(P->d_mat_base);
-    dfree(P->d_chunks);
-    dfree(P->d_row_te);
-    dfree(P->d_hlab);
-    dfree(P->d_row_reach);
-    dfree(P->d_row_fk);
-    dfree(P->d_rpT);
-    dfree(P->d_ciT);
-    dfree(P->d_vis);
-    dfree(P->d_rmask);
-    dfree(P->d_mat_te);
-    dfree(P->d_mat_reach);
+    pfree(P, P->d_rp);
+    pfree(P, P->d_ci);
+    pfree(P, P->d_lab);
+    pfree(P, P->d_mark);
+    pfree(P, P->d_orphan);
+    pfree(P, P->d_q0);
+    pfree(P, P->d_q1);
+    pfree(P, P->d_fills);
+    pfree(P, P->d_rec);
+    pfree(P, P->d_grp);
+    pfree(P, P->d_cnt64);
+    pfree(P, P->d_list);
+    pfree(P, P->d_rptr);
+    pfree(P, P->d_ctrl);
+    pfree(P, P->d_cntL);
+    pfree(P, P->d_cntU);
+    pfree(P, P->d_Lrp);
+    pfree(P, P->d_Urp);
+    pfree(P, P->d_rowfill);
+    pfree(P, P->d_scan);
+    pfree(P, P->d_Lcol);
+    pfree(P, P->d_Ucol);
+    pfree(P, P->d_Ltmp);
+    pfree(P, P->d_Utmp);
+    pfree(P, P->d_supno);
+    pfree(P, P->d_sstart);
+    pfree(P, P->d_sn64);
+    pfree(P, P->d_snflag);
+    pfree(P, P->d_sp_lcnt);
+    pfree(P, P->d_sp_ucnt);
+    pfree(P, P->d_sp_pass);
+    pfree(P, P->d_mask);
+    pfree(P, P->d_qgv);
+    pfree(P, P->d_bstate);
+    pfree(P, P->d_mat_base);
+    pfree(P, P->d_chunks);
+    pfree(P, P->d_row_te);
+    pfree(P, P->d_hlab);
+    pfree(P, P->d_row_reach);
+    pfree(P, P->d_row_fk);
+    pfree(P, P->d_rpT);
+    pfree(P, P->d_ciT);
+    pfree(P, P->d_vis);
+    pfree(P, P->d_rmask);
+    pfree(P, P->d_mat_te);
+    pfree(P, P->d_mat_reach);
     release_quot(P);
+    if (P->slab) (void)hipFree(P->slab);
+    P->slab = nullptr;
+}
+
+int alloc_supernodes(gsofa_plan* P) {
+    const size_t n = (size_t)P->n;
+    pfree(P, P->d_supno);
+    pfree(P, P->d_sstart);
+    pfree(P, P->d_sn64);
+    pfree(P, P->d_snflag);
+    int e = palloc(P, &P->d_supno, n);
+    e |= palloc(P, &P->d_sstart, n + 1);
+    e |= palloc(P, &P->d_sn64, scan_tmp_words((int32_t)n) + 2 * n + 8);
+    e |= palloc(P, &P->d_snflag, n);
+    if (!e) P->sn_cap = n;
+    return e;
 }
 
 int ensure_cols(gsofa_plan* P, int64_t nl, int64_t nu) {
     const bool staged = P->mode != GSOFA_MODE_REACH;  // columns sorted from a staging copy
     if (nl > P->Lcap) {
-        dfree(P->d_Lcol);
-        dfree(P->d_Ltmp);
+        pfree(P, P->d_Lcol);
+        pfree(P, P->d_Ltmp);
         int64_t cap = nl + nl / 8 + 1024;
-        if (dalloc(&P->d_Lcol, (size_t)cap) || (staged && dalloc(&P->d_Ltmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
+        if (palloc(P, &P->d_Lcol, (size_t)cap) || (staged && palloc(P, &P->d_Ltmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Lcap = cap;
     }
     if (nu > P->Ucap) {
-        dfree(P->d_Ucol);
-        dfree(P->d_Utmp);
+        pfree(P, P->d_Ucol);
+        pfree(P, P->d_Utmp);
         int64_t cap = nu + nu / 8 + 1024;
-        if (dalloc(&P->d_Ucol, (size_t)cap) || (staged && dalloc(&P->d_Utmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
+        if (palloc(P, &P->d_Ucol, (size_t)cap) || (staged && palloc(P, &P->d_Utmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Ucap = cap;
     }
     return GSOFA_OK;
-}
-
-// Device-to-host copies of large results go through pinned staging buffers
-// (a process-wide pool, kept until exit): the DMA of one chunk overlaps the
-// host copy of the previous one into the caller's (pageable) array.  That host
-// copy is what limits the rate: it first touches fresh pages (a few GB/s per
-// thread), so a large copy is split over up to kCopyParts threads, each with
-// two staging buffers of its own, and result arrays are allocated on 2 MB
-// boundaries with transparent huge pages requested (host_array).
-constexpr size_t kStageBytes = 16u << 20;
-constexpr size_t kStageMin = 8u << 20;    // smaller copies go direct
-constexpr size_t kPartMin = 64u << 20;    // bytes per copy thread, at least
-constexpr int kCopyParts = 4;
-constexpr size_t kHugePage = 2u << 20;
-std::mutex g_stage_mu;
-std::vector<void*> g_stage_free;
-
-void* stage_get() {
-    {
-        std::lock_guard<std::mutex> lk(g_stage_mu);
-        if (!g_stage_free.empty()) {
-            void* p = g_stage_free.back();
-            g_stage_free.pop_back();
-            return p;
-        }
-    }
-    void* p = nullptr;
-    if (hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return p;
-}
-
-void stage_put(void* p) {
-    if (!p) return;
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    g_stage_free.push_back(p);
-}
-
-// dst <- src through the staging buffers b0, b1: chunk k + 1's DMA runs while
-// chunk k is copied out.  Every DMA has ended when this returns.
-hipError_t copy_staged(void* dst, const void* src, size_t bytes, hipStream_t s, void* b0, void* b1) {
-    void* b[2] = {b0, b1};
-    hipEvent_t ev[2] = {nullptr, nullptr};
-    hipError_t e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
-    const size_t nch = (bytes + kStageBytes - 1) / kStageBytes;
-    auto issue = [&](size_t k) {
-        const size_t off = k * kStageBytes, len = std::min(kStageBytes, bytes - off);
-        hipError_t r = hipMemcpyAsync(b[k & 1], (const char*)src + off, len, hipMemcpyDeviceToHost, s);
-        return r == hipSuccess ? hipEventRecord(ev[k & 1], s) : r;
-    };
-    if (e == hipSuccess) e = issue(0);
-    for (size_t k = 0; k < nch && e == hipSuccess; k++) {
-        if (k + 1 < nch) e = issue(k + 1);  // its buffer was emptied in iteration k - 1
-        if (e == hipSuccess) e = hipEventSynchronize(ev[k & 1]);
-        if (e == hipSuccess) {
-            const size_t off = k * kStageBytes, len = std::min(kStageBytes, bytes - off);
-            memcpy((char*)dst + off, b[k & 1], len);
-        }
-    }
-    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // no copy left in flight into the buffers
-    for (hipEvent_t x : ev)
-        if (x) (void)hipEventDestroy(x);
-    return e;
-}
-
-// dst <- src (device), complete on return.  Work queued on s before the call
-// is ordered before the copy.
-hipError_t copy_d2h(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes == 0) return hipSuccess;
-    int parts = 0;
-    void* b[2 * kCopyParts] = {};
-    if (bytes >= kStageMin) {
-        const size_t want = std::min<size_t>(kCopyParts, std::max<size_t>(1, bytes / kPartMin));
-        for (; parts < (int)want; parts++) {
-            b[2 * parts] = stage_get();
-            b[2 * parts + 1] = stage_get();
-            if (!b[2 * parts] || !b[2 * parts + 1]) {
-                stage_put(b[2 * parts]);
-                stage_put(b[2 * parts + 1]);
-                b[2 * parts] = b[2 * parts + 1] = nullptr;
-                break;
-            }
-        }
-    }
-    if (parts == 0) {  // small, or no pinned memory: one direct copy
-        hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
-    }
-    // parts of whole staging chunks; the last takes the remainder
-    const size_t chunks = (bytes + kStageBytes - 1) / kStageBytes;
-    const size_t per = (chunks + parts - 1) / parts * kStageBytes;
-    std::vector<hipError_t> err((size_t)parts, hipSuccess);
-    std::vector<std::thread> th;
-    auto part = [&](int i) {
-        const size_t off = (size_t)i * per;
-        if (off >= bytes) return;
-        err[(size_t)i] = copy_staged((char*)dst + off, (const char*)src + off, std::min(per, bytes - off), s,
-                                     b[2 * i], b[2 * i + 1]);
-    };
-    for (int i = 1; i < parts; i++) {
-        try {
-            th.emplace_back(part, i);
-        } catch (...) {  // no thread: this one copies that part too
-            part(i);
-        }
-    }
-    part(0);
-    for (std::thread& t : th) t.join();
-    for (int i = 0; i < 2 * parts; i++) stage_put(b[i]);
-    for (hipError_t x : err)
-        if (x != hipSuccess) return x;
-    return hipSuccess;
-}
-
-// A host result array of `bytes`, released with free(): large ones start on
-// a 2 MB boundary with transparent huge pages requested, so that their first
-// touch (the staged copy above) faults once per 2 MB rather than per 4 KB.
-void* host_array(size_t bytes) {
-    if (bytes < kStageMin) return malloc(std::max<size_t>(bytes, 1));
-    const size_t len = (bytes + kHugePage - 1) / kHugePage * kHugePage;
-    void* p = nullptr;
-    if (posix_memalign(&p, kHugePage, len) != 0) return nullptr;
-    (void)madvise(p, len, MADV_HUGEPAGE);  // advice only: small pages if refused
-    return p;
 }
 
 float ev_ms(hipEvent_t a, hipEvent_t b) {
@@ -1143,15 +1067,16 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         int bits = 0;
         if (choose_bits(o, 1, (uint64_t)A->n, &bits) != GSOFA_OK) return -1;
         const uint64_t nchunks = ((uint64_t)A->n + bits - 1) / bits;
-        std::vector<int32_t> rp, ci;
+        std::vector<int32_t> rp, ci, rpT, ciT;
         pack_rows(A, rp, ci);
+        transpose_rows(A->n, rp.data(), ci.data(), rpT, ciT);
         uint64_t nf = 0, nl = 0, nu = 0;
         gsofa_options w = o;
         w.n_virtual_gpu = 1;
         w.virtual_gpu_id = -1;
         const std::vector<uint32_t> mb{0u, (uint32_t)A->n};
         uint64_t nr = 0;
-        output_need(w, A->n, rp.data(), ci.data(), &nf, &nl, &nu, bits, &mb, &nr);
+        output_need(w, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu, bits, &mb, &nr);
         nf = reach_reserve(nf, nl + nu, nr);
         uint32_t nb = 0;
         int threads = 0;
@@ -1174,10 +1099,11 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
     int64_t cols = -1;  // default: room for nnz + fc entries
     if (o.output_capacity <= 0) {  // what plan creation reserves from the row bounds
         if (validate(A) != GSOFA_OK) return -1;
-        std::vector<int32_t> rp, ci;
+        std::vector<int32_t> rp, ci, rpT, ciT;
         pack_rows(A, rp, ci);
+        transpose_rows(A->n, rp.data(), ci.data(), rpT, ciT);
         uint64_t nf = 0, nl = 0, nu = 0;
-        output_need(o, A->n, rp.data(), ci.data(), &nf, &nl, &nu);
+        output_need(o, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu);
         fc = std::max<uint64_t>(nf, 1);
         cols = (int64_t)(nl + nu);
     }
@@ -1245,15 +1171,16 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         return GSOFA_ERR_INVALID;
     }
     P->device = P->opt.device;
-    if (hipSetDevice(P->device) != hipSuccess || hipStreamCreate(&P->stream) != hipSuccess) {
+    if (hipSetDevice(P->device) != hipSuccess || stream_get(P->device, &P->stream) != hipSuccess) {
         (void)hipGetLastError();
         delete P;
         return GSOFA_ERR_HIP;
     }
-    std::vector<int32_t> ci;
+    std::vector<int32_t> ci, rpT, ciT;
     pack_rows(A, P->h_rp, ci);
     P->nnz = (int64_t)ci.size();
     const int32_t n = P->n;
+    if (reach || P->opt.output_capacity <= 0) transpose_rows(n, P->h_rp.data(), ci.data(), rpT, ciT);
 
     size_t freeb = 0, totalb = 0;
     (void)hipMemGetInfo(&freeb, &totalb);
@@ -1267,15 +1194,15 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         int bits = 0;
         rc = choose_bits(P->opt, n_mats, (uint64_t)n, &bits);
         if (rc) {
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return rc;
         }
         P->rbits = bits;
     }
     if (P->opt.output_capacity <= 0 && n > 0) {
-        output_need(P->opt, n, P->h_rp.data(), ci.data(), &need_fill, &need_L, &need_U, P->rbits, &P->h_mat_base,
-                    &need_rec);
+        output_need(P->opt, n, P->h_rp.data(), ci.data(), rpT.data(), ciT.data(), &need_fill, &need_L, &need_U,
+                    P->rbits, &P->h_mat_base, &need_rec);
         if (reach) need_fill = reach_reserve(need_fill, need_L + need_U, need_rec);
         const int64_t out_bytes = output_bytes(reach ? rch_fill_room(need_fill) : need_fill, need_L, need_U);
         if (out_bytes <= avail / 2) {
@@ -1293,7 +1220,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         if (P->opt.mode == GSOFA_MODE_AUTO && P->opt.top_sources <= 0 && n_mats == 1) {
             P->mode = GSOFA_MODE_GRID;
         } else {
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return GSOFA_ERR_TOO_LARGE;
         }
@@ -1317,13 +1244,13 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, P->device) != hipSuccess) {
         (void)hipGetLastError();
-        (void)hipStreamDestroy(P->stream);
+        stream_put(P->device, P->stream);
         delete P;
         return GSOFA_ERR_HIP;
     }
     int e = 0;
+    P->gather = reach && P->bounded;
     uint32_t qlev = 0;  // levels of classes (reach mode)
-    std::vector<int32_t> rpT, ciT;
     if (P->mode == GSOFA_MODE_REACH) {
         const int bits = P->rbits;
         P->S = (uint32_t)bits;
@@ -1342,7 +1269,6 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             P->h_chunks.swap(both);
             P->share_chunk_off.assign(2, 0);
             P->share_chunk_off[1] = (uint32_t)P->h_chunks.size();
-            transpose_rows(n, P->h_rp.data(), ci.data(), rpT, ciT);
             const int64_t tbytes = 4 * (int64_t)(n + 1) + 4 * P->nnz + 16 * (int64_t)n_mats;
             const int64_t room = std::max<int64_t>(avail - tbytes, 1 << 20);
             gsofa_options go = P->opt;
@@ -1353,25 +1279,25 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
                             &P->rthreads);
         }
         if (rc) {
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return rc;
         }
         P->C = (int32_t)(P->nblocks * P->S);
         const size_t nbw = (size_t)P->nblocks * (size_t)P->W;
-        e |= dalloc((uint64_t**)&P->d_vis, nbw * (size_t)(rch_visit_bytes(bits) / 8));
-        e |= dalloc((uint32_t**)&P->d_rmask, 2 * nbw * (size_t)(bits / 32));
-        e |= dalloc(&P->d_qgv, 2 * nbw);
-        e |= dalloc(&P->d_bstate, (size_t)P->nblocks);
-        e |= dalloc(&P->d_mat_base, (size_t)n_mats + 1);
-        e |= dalloc(&P->d_chunks, std::max<size_t>(P->h_chunks.size(), 1));
-        e |= dalloc(&P->d_grp, std::max<size_t>(P->h_chunks.size(), 1));
-        e |= dalloc(&P->d_cnt64, (size_t)n);
-        e |= dalloc(&P->d_rptr, (size_t)n + 1);
-        e |= dalloc(&P->d_mat_te, (size_t)n_mats);
-        e |= dalloc(&P->d_mat_reach, (size_t)n_mats);
-        e |= dalloc(&P->d_rpT, (size_t)n + 1);
-        e |= dalloc(&P->d_ciT, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
+        e |= palloc(P, (uint64_t**)&P->d_vis, nbw * (size_t)(rch_visit_bytes(bits) / 8));
+        e |= palloc(P, (uint32_t**)&P->d_rmask, 2 * nbw * (size_t)(bits / 32));
+        e |= palloc(P, &P->d_qgv, 2 * nbw);
+        e |= palloc(P, &P->d_bstate, (size_t)P->nblocks);
+        e |= palloc(P, &P->d_mat_base, (size_t)n_mats + 1);
+        e |= palloc(P, &P->d_chunks, std::max<size_t>(P->h_chunks.size(), 1));
+        e |= palloc(P, &P->d_grp, std::max<size_t>(P->h_chunks.size(), 1));
+        e |= palloc(P, &P->d_cnt64, (size_t)n);
+        e |= palloc(P, &P->d_rptr, (size_t)n + 1);
+        e |= palloc(P, &P->d_mat_te, (size_t)n_mats);
+        e |= palloc(P, &P->d_mat_reach, (size_t)n_mats);
+        e |= palloc(P, &P->d_rpT, (size_t)n + 1);
+        e |= palloc(P, &P->d_ciT, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
         e |= setup_quot(P, qlev);
     } else if (P->mode == GSOFA_MODE_BLOCK) {
         int S = 0;
@@ -1381,44 +1307,44 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         if (!rc) build_chunks(P);
         if (!rc) rc = size_block_mode(P, std::max<int64_t>(avail, 1 << 20));
         if (rc) {
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return rc;
         }
         const size_t slots = (size_t)P->nblocks * (size_t)P->S;
-        e |= dalloc(&P->d_lab, slots * (size_t)P->W);
-        e |= dalloc(&P->d_mask, (size_t)P->nblocks * 2 * (size_t)P->W);
-        e |= dalloc(&P->d_qgv, (size_t)P->nblocks * 2 * (size_t)P->W);
-        e |= dalloc(&P->d_bstate, 2 * (size_t)P->nblocks);
-        e |= dalloc(&P->d_mat_base, (size_t)n_mats + 1);
-        e |= dalloc(&P->d_chunks, std::max<size_t>(P->h_chunks.size(), 1));
-        e |= dalloc(&P->d_row_te, (size_t)n);
-        e |= dalloc(&P->d_row_reach, (size_t)n);
-        e |= dalloc(&P->d_row_fk, (size_t)n);
+        e |= palloc(P, &P->d_lab, slots * (size_t)P->W);
+        e |= palloc(P, &P->d_mask, (size_t)P->nblocks * 2 * (size_t)P->W);
+        e |= palloc(P, &P->d_qgv, (size_t)P->nblocks * 2 * (size_t)P->W);
+        e |= palloc(P, &P->d_bstate, 2 * (size_t)P->nblocks);
+        e |= palloc(P, &P->d_mat_base, (size_t)n_mats + 1);
+        e |= palloc(P, &P->d_chunks, std::max<size_t>(P->h_chunks.size(), 1));
+        e |= palloc(P, &P->d_row_te, (size_t)n);
+        e |= palloc(P, &P->d_row_reach, (size_t)n);
+        e |= palloc(P, &P->d_row_fk, (size_t)n);
         P->lab_words = slots * (size_t)P->W;
         if (P->hybrid) {
-            e |= dalloc(&P->d_hlab, (size_t)P->hlab_words);
-            e |= dalloc(&P->d_mark, (size_t)P->hC * (size_t)n);
-            e |= dalloc(&P->d_orphan, (size_t)P->hC * P->orphan_words);
-            e |= dalloc(&P->d_q0, (size_t)P->hQ);
-            e |= dalloc(&P->d_q1, (size_t)P->hQ);
+            e |= palloc(P, &P->d_hlab, (size_t)P->hlab_words);
+            e |= palloc(P, &P->d_mark, (size_t)P->hC * (size_t)n);
+            e |= palloc(P, &P->d_orphan, (size_t)P->hC * P->orphan_words);
+            e |= palloc(P, &P->d_q0, (size_t)P->hQ);
+            e |= palloc(P, &P->d_q1, (size_t)P->hQ);
         }
     } else {
         Sizing sz;
         rc = choose_sizing(A, &P->opt, P->nnz, std::max<int64_t>(avail, 1 << 20), &sz);
         if (rc) {
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return rc;
         }
         P->C = sz.C;
         P->Q = sz.Q;
         P->lab_words = sz.lab_words;
-        e |= dalloc(&P->d_lab, (size_t)P->lab_words);
-        e |= dalloc(&P->d_mark, (size_t)P->C * (size_t)n);
-        e |= dalloc(&P->d_orphan, (size_t)P->C * P->orphan_words);
-        e |= dalloc(&P->d_q0, (size_t)P->Q);
-        e |= dalloc(&P->d_q1, (size_t)P->Q);
+        e |= palloc(P, &P->d_lab, (size_t)P->lab_words);
+        e |= palloc(P, &P->d_mark, (size_t)P->C * (size_t)n);
+        e |= palloc(P, &P->d_orphan, (size_t)P->C * P->orphan_words);
+        e |= palloc(P, &P->d_q0, (size_t)P->Q);
+        e |= palloc(P, &P->d_q1, (size_t)P->Q);
     }
     P->fill_cap = P->opt.output_capacity > 0 ? (uint64_t)P->opt.output_capacity : default_fill_cap(P->nnz);
     if ((P->opt.flags & GSOFA_FLAG_SPILL) && P->opt.output_capacity <= 0)  // one share's fills at a time
@@ -1427,35 +1353,37 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         P->fill_cap = P->mode == GSOFA_MODE_REACH ? 2 * need_rec : std::max<uint64_t>(need_fill, 1);
         P->Lcap = (int64_t)need_L;
         P->Ucap = (int64_t)need_U;
-        e |= dalloc(&P->d_Lcol, (size_t)need_L);
-        e |= dalloc(&P->d_Ucol, (size_t)need_U);
+        e |= palloc(P, &P->d_Lcol, (size_t)need_L);
+        e |= palloc(P, &P->d_Ucol, (size_t)need_U);
         if (!reach) {
-            e |= dalloc(&P->d_Ltmp, (size_t)need_L);
-            e |= dalloc(&P->d_Utmp, (size_t)need_U);
+            e |= palloc(P, &P->d_Ltmp, (size_t)need_L);
+            e |= palloc(P, &P->d_Utmp, (size_t)need_U);
         }
     }
-    e |= dalloc(&P->d_rp, (size_t)n + 1);
-    e |= dalloc(&P->d_ci, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
+    e |= palloc(P, &P->d_rp, (size_t)n + 1);
+    e |= palloc(P, &P->d_ci, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
     if (!(P->opt.flags & GSOFA_FLAG_COUNTS_ONLY) || !reach) e |= alloc_stream(P, P->bounded ? need_rec : P->fill_cap);
-    e |= dalloc(&P->d_ctrl, 1);
-    e |= dalloc(&P->d_cntL, (size_t)n);
-    e |= dalloc(&P->d_cntU, (size_t)n);
-    e |= dalloc(&P->d_Lrp, (size_t)n + 1);
-    e |= dalloc(&P->d_Urp, (size_t)n + 1);
-    e |= dalloc(&P->d_rowfill, (size_t)n);
+    e |= palloc(P, &P->d_ctrl, 1);
+    e |= palloc(P, &P->d_cntL, (size_t)n);
+    e |= palloc(P, &P->d_cntU, (size_t)n);
+    e |= palloc(P, &P->d_Lrp, (size_t)n + 1);
+    e |= palloc(P, &P->d_Urp, (size_t)n + 1);
+    e |= palloc(P, &P->d_rowfill, (size_t)n);
     P->scan_words = scan_tmp_words(n) + 2 * (size_t)n + 8;
-    e |= dalloc(&P->d_scan, P->scan_words);
+    e |= palloc(P, &P->d_scan, P->scan_words);
+    if (P->gather && !(P->opt.flags & GSOFA_FLAG_COUNTS_ONLY)) e |= alloc_supernodes(P);
+    if (P->gather) e |= take_slab(P);
     if (e) {
         release_device(P);
-        (void)hipStreamDestroy(P->stream);
+        stream_put(P->device, P->stream);
         delete P;
         return GSOFA_ERR_ALLOC;
     }
-    bool ok = hipMemcpyAsync(P->d_rp, P->h_rp.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice,
-                             P->stream) == hipSuccess;
-    if (P->nnz)
-        ok = ok && hipMemcpyAsync(P->d_ci, ci.data(), sizeof(int32_t) * P->nnz, hipMemcpyHostToDevice,
-                                  P->stream) == hipSuccess;
+    std::vector<HostCopy> up;  // uploads, in one go
+    up.push_back({P->h_rp.data(), P->d_rp, sizeof(int32_t) * ((size_t)n + 1)});
+    up.push_back({ci.data(), P->d_ci, sizeof(int32_t) * (size_t)P->nnz});
+    upload_quot(P, up);
+    bool ok = true;
     if (P->mode == GSOFA_MODE_GRID || P->hybrid) {
         const size_t Cm = P->hybrid ? (size_t)P->hC : (size_t)P->C;
         ok = ok && hipMemsetAsync(P->d_mark, 0, sizeof(uint32_t) * Cm * n, P->stream) == hipSuccess;
@@ -1472,16 +1400,10 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         ok = ok && hipMemsetAsync(P->d_vis, 0, vb, P->stream) == hipSuccess;
         ok = ok && hipMemsetAsync(P->d_rmask, 0, mb, P->stream) == hipSuccess;
         ok = ok && hipMemsetAsync(P->d_bstate, 0, sizeof(uint32_t) * P->nblocks, P->stream) == hipSuccess;
-        ok = ok && hipMemcpyAsync(P->d_rpT, rpT.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice,
-                                  P->stream) == hipSuccess;
-        if (P->nnz)
-            ok = ok && hipMemcpyAsync(P->d_ciT, ciT.data(), sizeof(int32_t) * P->nnz, hipMemcpyHostToDevice,
-                                      P->stream) == hipSuccess;
-        ok = ok && hipMemcpyAsync(P->d_mat_base, P->h_mat_base.data(), sizeof(uint32_t) * (n_mats + 1),
-                                  hipMemcpyHostToDevice, P->stream) == hipSuccess;
-        if (!P->h_chunks.empty())
-            ok = ok && hipMemcpyAsync(P->d_chunks, P->h_chunks.data(), sizeof(BlkChunk) * P->h_chunks.size(),
-                                      hipMemcpyHostToDevice, P->stream) == hipSuccess;
+        up.push_back({rpT.data(), P->d_rpT, sizeof(int32_t) * ((size_t)n + 1)});
+        up.push_back({ciT.data(), P->d_ciT, sizeof(int32_t) * (size_t)P->nnz});
+        up.push_back({P->h_mat_base.data(), P->d_mat_base, sizeof(uint32_t) * ((size_t)n_mats + 1)});
+        up.push_back({P->h_chunks.data(), P->d_chunks, sizeof(BlkChunk) * P->h_chunks.size()});
     }
     std::vector<uint32_t> bst;
     if (P->mode == GSOFA_MODE_BLOCK) {
@@ -1491,19 +1413,16 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             bst[2 * b] = 0xFFFFFFFFu - P->W;
             bst[2 * b + 1] = 0;
         }
-        ok = ok && hipMemcpyAsync(P->d_bstate, bst.data(), sizeof(uint32_t) * bst.size(),
-                                  hipMemcpyHostToDevice, P->stream) == hipSuccess;
-        ok = ok && hipMemcpyAsync(P->d_mat_base, P->h_mat_base.data(), sizeof(uint32_t) * (n_mats + 1),
-                                  hipMemcpyHostToDevice, P->stream) == hipSuccess;
-        if (!P->h_chunks.empty())
-            ok = ok && hipMemcpyAsync(P->d_chunks, P->h_chunks.data(), sizeof(BlkChunk) * P->h_chunks.size(),
-                                      hipMemcpyHostToDevice, P->stream) == hipSuccess;
+        up.push_back({bst.data(), P->d_bstate, sizeof(uint32_t) * bst.size()});
+        up.push_back({P->h_mat_base.data(), P->d_mat_base, sizeof(uint32_t) * ((size_t)n_mats + 1)});
+        up.push_back({P->h_chunks.data(), P->d_chunks, sizeof(BlkChunk) * P->h_chunks.size()});
     }
+    ok = ok && copy_in(up, P->stream) == hipSuccess;
     ok = ok && hipStreamSynchronize(P->stream) == hipSuccess;
     if (!ok) {
         (void)hipGetLastError();
         release_device(P);
-        (void)hipStreamDestroy(P->stream);
+        stream_put(P->device, P->stream);
         delete P;
         return GSOFA_ERR_HIP;
     }
@@ -1520,7 +1439,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             occ <= 0) {
             (void)hipGetLastError();
             release_device(P);
-            (void)hipStreamDestroy(P->stream);
+            stream_put(P->device, P->stream);
             delete P;
             return GSOFA_ERR_HIP;
         }
@@ -1641,6 +1560,7 @@ static RowParams row_params(const gsofa_plan* P) {
     r.R_ptr = P->d_rptr;
     r.list = P->d_list;
     r.list_cap = (int64_t)P->list_cap;
+    r.ctrl = P->d_ctrl;
     r.long_rows = P->d_cntL;  // unused otherwise in reach mode
     r.long_count = &P->d_ctrl->cursor[0];
     r.L_col = P->d_Lcol;
@@ -1791,9 +1711,8 @@ static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t g
         P->totals_known = false;
     } else {
         int64_t tot[2] = {0, 0};
-        HIPCHK_OUT(hipMemcpyAsync(&tot[0], P->d_Lrp + n, sizeof(int64_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(&tot[1], P->d_Urp + n, sizeof(int64_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        HIPCHK_OUT(copy_out({{&tot[0], P->d_Lrp + n, sizeof(int64_t)}, {&tot[1], P->d_Urp + n, sizeof(int64_t)}},
+                            P->stream), P->stream);
         P->nnzL = tot[0];
         P->nnzU = tot[1];
         P->totals_known = true;
@@ -1814,17 +1733,37 @@ static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t g
     return GSOFA_OK;
 }
 
-// nnzL / nnzU of the last structure pass, read from the row pointers' ends.
+// nnzL, nnzU and the supernodes' number of the last structure pass: from the
+// counters where the pass wrote them there (row records), else from the row
+// pointers' ends.
 static int read_totals(gsofa_plan* P) {
-    if (P->totals_known || P->n == 0) return GSOFA_OK;
-    int64_t tot[2] = {0, 0};
-    HIPCHK_OUT(hipMemcpyAsync(&tot[0], P->d_Lrp + P->n, sizeof(int64_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-    HIPCHK_OUT(hipMemcpyAsync(&tot[1], P->d_Urp + P->n, sizeof(int64_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-    HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
-    if (tot[0] > P->Lcap || tot[1] > P->Ucap) return GSOFA_ERR_STATE;  // cannot happen: the bounds hold
+    if (P->n == 0 || (P->totals_known && (P->nsuper_known || !P->supernodes))) return GSOFA_OK;
+    int64_t tot[2] = {P->nnzL, P->nnzU};
+    std::vector<HostCopy> cp;
+    if (!P->totals_known) {
+        cp.push_back({&tot[0], P->d_Lrp + P->n, sizeof(int64_t)});
+        cp.push_back({&tot[1], P->d_Urp + P->n, sizeof(int64_t)});
+    }
+    if (P->supernodes) cp.push_back({&P->n_super, &P->d_ctrl->n_super, sizeof(int32_t)});
+    HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
+    if (!P->totals_known && (tot[0] > P->Lcap || tot[1] > P->Ucap)) return GSOFA_ERR_STATE;  // cannot happen: the bounds hold
     P->nnzL = tot[0];
     P->nnzU = tot[1];
     P->totals_known = true;
+    P->nsuper_known = P->supernodes;
+    return GSOFA_OK;
+}
+
+// The counters of a bounded pass have arrived in P->stats: its totals.
+static int take_totals(gsofa_plan* P) {
+    P->totals_known = !P->structure;
+    if (!P->structure || P->mode != GSOFA_MODE_REACH) return GSOFA_OK;
+    if (P->stats.nnz_L > P->Lcap || P->stats.nnz_U > P->Ucap) return GSOFA_ERR_STATE;  // cannot happen: the bounds hold
+    P->nnzL = P->stats.nnz_L;
+    P->nnzU = P->stats.nnz_U;
+    P->n_super = P->stats.n_super;
+    P->totals_known = true;
+    P->nsuper_known = P->supernodes;
     return GSOFA_OK;
 }
 
@@ -1832,21 +1771,7 @@ static int read_totals(gsofa_plan* P) {
 // per-row pass-through flags.
 static int build_supernodes(gsofa_plan* P, const uint32_t* pass) {
     const int32_t n = P->n;
-    if (!P->d_supno || P->sn_cap < (size_t)n) {
-        dfree(P->d_supno);
-        dfree(P->d_sstart);
-        dfree(P->d_nsuper);
-        dfree(P->d_sn64);
-        dfree(P->d_snflag);
-        int e = 0;
-        e |= dalloc(&P->d_supno, (size_t)n);
-        e |= dalloc(&P->d_sstart, (size_t)n + 1);
-        e |= dalloc(&P->d_nsuper, 1);
-        e |= dalloc(&P->d_sn64, scan_tmp_words(n) + 2 * (size_t)n + 8);
-        e |= dalloc(&P->d_snflag, (size_t)n);
-        if (e) return GSOFA_ERR_ALLOC;
-        P->sn_cap = (size_t)n;
-    }
+    if ((!P->d_supno || P->sn_cap < (size_t)n) && alloc_supernodes(P)) return GSOFA_ERR_ALLOC;
     SuperParams sp{};
     sp.n = n;
     sp.L_rowptr = P->d_Lrp;
@@ -1855,7 +1780,7 @@ static int build_supernodes(gsofa_plan* P, const uint32_t* pass) {
     sp.max_size = P->opt.max_supernode_size;
     sp.supno = P->d_supno;
     sp.super_start = P->d_sstart;
-    sp.n_super = P->d_nsuper;
+    sp.n_super = &P->d_ctrl->n_super;
     sp.tmp64 = P->d_sn64;
     sp.flag = P->d_snflag;
     sp.pass = pass;
@@ -1873,9 +1798,9 @@ static int execute_spill(gsofa_plan* P, const std::vector<int32_t>& shares) {
     const int32_t N = std::max(1, P->opt.n_virtual_gpu);
     if (!P->d_sp_lcnt) {
         int e = 0;
-        e |= dalloc(&P->d_sp_lcnt, (size_t)n);
-        e |= dalloc(&P->d_sp_ucnt, (size_t)n);
-        e |= dalloc(&P->d_sp_pass, (size_t)n);
+        e |= palloc(P, &P->d_sp_lcnt, (size_t)n);
+        e |= palloc(P, &P->d_sp_ucnt, (size_t)n);
+        e |= palloc(P, &P->d_sp_pass, (size_t)n);
         if (e) return GSOFA_ERR_ALLOC;
     }
     HIPCHK(launch_fill(P->d_sp_lcnt, (uint64_t)n, 0u, P->stream));
@@ -1899,9 +1824,9 @@ static int execute_spill(gsofa_plan* P, const std::vector<int32_t>& shares) {
             HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
             if (P->stats.abort) return GSOFA_ERR_DEVICE_TIMEOUT;
             if (P->stats.fill_pos <= P->fill_cap) break;
-            dfree(P->d_fills);
+            pfree(P, P->d_fills);
             P->fill_cap = P->stats.fill_pos + P->stats.fill_pos / 16 + 1024;
-            if (dalloc(&P->d_fills, (size_t)P->fill_cap)) return GSOFA_ERR_ALLOC;
+            if (palloc(P, &P->d_fills, (size_t)P->fill_cap)) return GSOFA_ERR_ALLOC;
         }
         if (P->stats.fill_pos > P->fill_cap) return GSOFA_ERR_ALLOC;
         int rc = build_structure(P, P->stats.fill_pos, N, gid);
@@ -1911,19 +1836,12 @@ static int execute_spill(gsofa_plan* P, const std::vector<int32_t>& shares) {
         SpillShare& h = P->sp[(size_t)gid];
         h.Lcol.resize((size_t)std::max<int64_t>(P->nnzL, 1));
         h.Ucol.resize((size_t)std::max<int64_t>(P->nnzU, 1));
-        HIPCHK_OUT(hipMemcpyAsync(lrp.data(), P->d_Lrp, sizeof(int64_t) * ((size_t)n + 1), hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(urp.data(), P->d_Urp, sizeof(int64_t) * ((size_t)n + 1), hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        if (P->nnzL)
-            HIPCHK_OUT(hipMemcpyAsync(h.Lcol.data(), P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL,
-                                      hipMemcpyDeviceToHost, P->stream), P->stream);
-        if (P->nnzU)
-            HIPCHK_OUT(hipMemcpyAsync(h.Ucol.data(), P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU,
-                                      hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(rowfill.data(), P->d_rowfill, sizeof(int64_t) * (size_t)n, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        HIPCHK_OUT(copy_out({{lrp.data(), P->d_Lrp, sizeof(int64_t) * ((size_t)n + 1)},
+                             {urp.data(), P->d_Urp, sizeof(int64_t) * ((size_t)n + 1)},
+                             {h.Lcol.data(), P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL},
+                             {h.Ucol.data(), P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU},
+                             {rowfill.data(), P->d_rowfill, sizeof(int64_t) * (size_t)n}},
+                            P->stream), P->stream);
         // the share's rows are the only non-empty ones: keep their offsets
         h.Loff.assign(1, 0);
         h.Uoff.assign(1, 0);
@@ -1962,18 +1880,14 @@ static int execute_spill(gsofa_plan* P, const std::vector<int32_t>& shares) {
     return GSOFA_OK;
 }
 
-// Reach mode, batches: per-matrix TE and |R| of the last execute to the host
-// (queued on the plan's stream; valid after the next synchronisation).
-static hipError_t fetch_mat_totals(gsofa_plan* P) {
-    if (P->mode != GSOFA_MODE_REACH || P->n_mats <= 1) return hipSuccess;
+// Reach mode, batches: per-matrix TE and |R| of the last execute, added to a
+// call's copies.
+static void fetch_mat_totals(gsofa_plan* P, std::vector<HostCopy>& cp) {
+    if (P->mode != GSOFA_MODE_REACH || P->n_mats <= 1) return;
     P->h_mat_te.resize((size_t)P->n_mats);
     P->h_mat_reach.resize((size_t)P->n_mats);
-    hipError_t e = hipMemcpyAsync(P->h_mat_te.data(), P->d_mat_te, sizeof(unsigned long long) * P->n_mats,
-                                  hipMemcpyDeviceToHost, P->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(P->h_mat_reach.data(), P->d_mat_reach, sizeof(unsigned long long) * P->n_mats,
-                           hipMemcpyDeviceToHost, P->stream);
-    return e;
+    cp.push_back({P->h_mat_te.data(), P->d_mat_te, sizeof(unsigned long long) * (size_t)P->n_mats});
+    cp.push_back({P->h_mat_reach.data(), P->d_mat_reach, sizeof(unsigned long long) * (size_t)P->n_mats});
 }
 
 // Traversal time per share and in total, and the whole execute's device time,
@@ -2010,7 +1924,10 @@ static int queue_bounded(gsofa_plan* P, const std::vector<int32_t>& shares, int3
         if (!rc && P->supernodes) rc = build_supernodes(P, nullptr);
         if (rc) return rc;
     }
-    HIPCHK_OUT(hipMemcpyAsync(stats, P->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, P->stream), P->stream);
+    if (stats == P->h_ctrl)  // pinned: written by a kernel
+        HIPCHK_OUT(launch_copy_words(stats, P->d_ctrl, sizeof(Ctrl) / 4, P->stream), P->stream);
+    else
+        HIPCHK_OUT(hipMemcpyAsync(stats, P->d_ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, P->stream), P->stream);
     if (!P->capturing) HIPCHK(hipEventRecord(P->ev[1], P->stream));
     return GSOFA_OK;
 }
@@ -2019,9 +1936,7 @@ static int queue_bounded(gsofa_plan* P, const std::vector<int32_t>& shares, int3
 // allocated every lazily sized buffer).  A refused capture leaves the plan
 // executing eagerly.
 static void capture_graph(gsofa_plan* P, const std::vector<int32_t>& shares, int32_t N, bool all_rows) {
-    if (!P->h_ctrl && hipHostMalloc((void**)&P->h_ctrl, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        P->h_ctrl = nullptr;
+    if (!P->h_ctrl) {
         P->graph_failed = true;
         return;
     }
@@ -2063,7 +1978,9 @@ int gsofa_plan_execute(gsofa_plan* P) {
     P->spilled = false;
     P->executed = false;
     P->host_valid = false;
+    P->nsuper_known = false;
     P->last_replayed = false;
+    if (!P->h_ctrl) P->h_ctrl = ctrl_get();
     memset(&P->stats, 0, sizeof(P->stats));
     if (n == 0) {
         P->executed = true;
@@ -2098,7 +2015,8 @@ int gsofa_plan_execute(gsofa_plan* P) {
             // the graph holds no events of its own: its whole replay is timed
             P->ms = ev_ms(P->ev[0], P->ev[1]);
             P->traverse_ms = P->share_min = P->share_max = 0;
-            P->totals_known = !P->structure;
+            const int rc = take_totals(P);
+            if (rc) return rc;
             P->last_replayed = true;
             P->executed = true;
             return GSOFA_OK;
@@ -2109,12 +2027,15 @@ int gsofa_plan_execute(gsofa_plan* P) {
         P->passes = 1;
         // one pass: traversal, structure and supernodes are queued back to
         // back; the host waits once, at the end
-        int rc = queue_bounded(P, shares, N, all_rows, &P->stats);
+        int rc = queue_bounded(P, shares, N, all_rows, P->h_ctrl ? P->h_ctrl : &P->stats);
         if (rc) return rc;
         HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        if (P->h_ctrl) P->stats = *P->h_ctrl;
         if (P->stats.abort) return GSOFA_ERR_DEVICE_TIMEOUT;
         if (!P->structure || P->stats.fill_pos <= P->fill_cap) {
             finish_timing(P, shares.size());
+            rc = take_totals(P);
+            if (rc) return rc;
             P->executed = true;
             if (graphable) capture_graph(P, shares, N, all_rows);
             return GSOFA_OK;
@@ -2193,17 +2114,19 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
     if (P->structure && !P->spilled) {
         const int rc = read_totals(P);
         if (rc) return rc;
+    } else if (P->structure && P->supernodes) {
+        HIPCHK_OUT(copy_out({{&P->n_super, &P->d_ctrl->n_super, sizeof(int32_t)}}, P->stream), P->stream);
     }
+    std::vector<HostCopy> cp;  // everything the call copies, in one go
     if (!P->structure) {
         // counts only: the block kernel's per-row fills, TE and |R|; the
         // reach kernels' per-row fills (grid and hybrid runs report totals only)
         if (P->mode == GSOFA_MODE_REACH) {
             r->row_fill = (int64_t*)malloc(sizeof(int64_t) * (size_t)n);
             if (!r->row_fill) return GSOFA_ERR_ALLOC;
-            HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
-                                      P->stream), P->stream);
-            HIPCHK_OUT(fetch_mat_totals(P), P->stream);
-            HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+            cp.push_back({r->row_fill, P->d_rowfill, sizeof(int64_t) * (size_t)n});
+            fetch_mat_totals(P, cp);
+            HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
             return GSOFA_OK;
         }
         if (P->mode != GSOFA_MODE_BLOCK || P->hybrid) return GSOFA_OK;
@@ -2214,30 +2137,25 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_row_fk, sizeof(int64_t) * n, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->row_te, P->d_row_te, sizeof(int64_t) * n, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->row_reach, P->d_row_reach, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        cp.push_back({r->row_fill, P->d_row_fk, sizeof(int64_t) * (size_t)n});
+        cp.push_back({r->row_te, P->d_row_te, sizeof(int64_t) * (size_t)n});
+        cp.push_back({r->row_reach, P->d_row_reach, sizeof(int64_t) * (size_t)n});
+        HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
         const int32_t N = std::max(1, P->opt.n_virtual_gpu), id = P->opt.virtual_gpu_id;
         for (int32_t i = 0; i < n; i++)
             if (id >= 0 && i % N != id) r->row_fill[i] = r->row_te[i] = r->row_reach[i] = -1;
         return GSOFA_OK;
     }
-    r->row_fill = (int64_t*)malloc(sizeof(int64_t) * (size_t)n);
-    r->L_rowptr = (int64_t*)malloc(sizeof(int64_t) * (size_t)(n + 1));
-    r->U_rowptr = (int64_t*)malloc(sizeof(int64_t) * (size_t)(n + 1));
+    r->row_fill = (int64_t*)host_array(sizeof(int64_t) * (size_t)n);
+    r->L_rowptr = (int64_t*)host_array(sizeof(int64_t) * (size_t)(n + 1));
+    r->U_rowptr = (int64_t*)host_array(sizeof(int64_t) * (size_t)(n + 1));
     r->L_col = (int32_t*)host_array(sizeof(int32_t) * (size_t)std::max<int64_t>(P->nnzL, 1));
     r->U_col = (int32_t*)host_array(sizeof(int32_t) * (size_t)std::max<int64_t>(P->nnzU, 1));
     if (!r->row_fill || !r->L_rowptr || !r->U_rowptr || !r->L_col || !r->U_col) {
         gsofa_result_free(r);
         return GSOFA_ERR_ALLOC;
     }
-    if (!P->spilled)
-        HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill, sizeof(int64_t) * n, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
+    if (!P->spilled) cp.push_back({r->row_fill, P->d_rowfill, sizeof(int64_t) * (size_t)n});
     if (P->mode == GSOFA_MODE_BLOCK && !P->hybrid) {
         r->row_te = (int64_t*)malloc(sizeof(int64_t) * (size_t)n);
         r->row_reach = (int64_t*)malloc(sizeof(int64_t) * (size_t)n);
@@ -2245,10 +2163,8 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        HIPCHK_OUT(hipMemcpyAsync(r->row_te, P->d_row_te, sizeof(int64_t) * n, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->row_reach, P->d_row_reach, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
+        cp.push_back({r->row_te, P->d_row_te, sizeof(int64_t) * (size_t)n});
+        cp.push_back({r->row_reach, P->d_row_reach, sizeof(int64_t) * (size_t)n});
     }
     if (P->spilled) {
         // rows in order, each from the share that built it (row i: share i mod N)
@@ -2271,36 +2187,27 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
             r->U_rowptr[i + 1] = uo;
         }
     } else {
-        HIPCHK_OUT(hipMemcpyAsync(r->L_rowptr, P->d_Lrp, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->U_rowptr, P->d_Urp, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(copy_d2h(r->L_col, P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL, P->stream), P->stream);
-        HIPCHK_OUT(copy_d2h(r->U_col, P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU, P->stream), P->stream);
+        cp.push_back({r->L_rowptr, P->d_Lrp, sizeof(int64_t) * ((size_t)n + 1)});
+        cp.push_back({r->U_rowptr, P->d_Urp, sizeof(int64_t) * ((size_t)n + 1)});
+        cp.push_back({r->L_col, P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL});
+        cp.push_back({r->U_col, P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU});
     }
-    if (r->row_te) {
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
-        for (int32_t i = 0; i < n; i++)
-            if (r->row_fill[i] < 0) r->row_te[i] = r->row_reach[i] = -1;
-    }
-    HIPCHK_OUT(fetch_mat_totals(P), P->stream);
+    fetch_mat_totals(P, cp);
     if (P->supernodes) {
-        int32_t ns = 0;
-        HIPCHK_OUT(hipMemcpyAsync(&ns, P->d_nsuper, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
-        r->n_super = ns;
-        r->super_start = (int32_t*)malloc(sizeof(int32_t) * (size_t)(ns + 1));
-        r->supno = (int32_t*)malloc(sizeof(int32_t) * (size_t)n);
+        r->n_super = P->n_super;
+        r->super_start = (int32_t*)host_array(sizeof(int32_t) * ((size_t)P->n_super + 1));
+        r->supno = (int32_t*)host_array(sizeof(int32_t) * (size_t)n);
         if (!r->super_start || !r->supno) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        HIPCHK_OUT(hipMemcpyAsync(r->super_start, P->d_sstart, sizeof(int32_t) * (ns + 1), hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->supno, P->d_supno, sizeof(int32_t) * n, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
+        cp.push_back({r->super_start, P->d_sstart, sizeof(int32_t) * ((size_t)P->n_super + 1)});
+        cp.push_back({r->supno, P->d_supno, sizeof(int32_t) * (size_t)n});
     }
-    HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+    HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
+    if (r->row_te)
+        for (int32_t i = 0; i < n; i++)
+            if (r->row_fill[i] < 0) r->row_te[i] = r->row_reach[i] = -1;
     return GSOFA_OK;
 }
 
@@ -2404,11 +2311,11 @@ void gsofa_plan_destroy(gsofa_plan* P) {
     (void)hipStreamSynchronize(P->stream);
     if (P->graph_exec) (void)hipGraphExecDestroy(P->graph_exec);
     if (P->graph) (void)hipGraphDestroy(P->graph);
-    if (P->h_ctrl) (void)hipHostFree(P->h_ctrl);
+    ctrl_put(P->h_ctrl);
     for (auto e : P->ev) (void)hipEventDestroy(e);
     gsofa_result_free(&P->host);
     release_device(P);
-    (void)hipStreamDestroy(P->stream);
+    stream_put(P->device, P->stream);
     delete P;
 }
 
@@ -2432,14 +2339,10 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
     if (P->n_mats != 1 || !P->structure || (!P->supernodes && P->n > 0) || P->spilled) return GSOFA_ERR_INVALID;
     const int32_t n = P->n;
     h->n = n;
-    int32_t ns = 0;
     HIPCHK_OUT(hipSetDevice(P->device), P->stream);
     const int trc = read_totals(P);
     if (trc) return trc;
-    if (n > 0) {
-        HIPCHK_OUT(hipMemcpyAsync(&ns, P->d_nsuper, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
-    }
+    const int32_t ns = n > 0 ? P->n_super : 0;
     h->n_super = ns;
     DevScratch T;  // device scratch for this call only
     int64_t *d_xl = nullptr, *d_xu = nullptr, *d_xs = nullptr;
@@ -2460,47 +2363,37 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
     if (ns > 0) {
         HIPCHK_OUT(supernode_sub_count(P->d_sstart, ns, P->d_Urp, P->d_cntL, P->stream), P->stream);
         HIPCHK_OUT(exclusive_scan_u32_to_i64(P->d_cntL, d_xs, ns, P->d_scan, P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(&nsub, d_xs + ns, sizeof(int64_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        HIPCHK_OUT(copy_out({{&nsub, d_xs + ns, sizeof(int64_t)}}, P->stream), P->stream);
         if (T.get(&d_sub, (size_t)nsub)) return GSOFA_ERR_ALLOC;
         HIPCHK_OUT(supernode_sub_write(P->d_sstart, ns, P->d_Urp, P->d_Ucol, d_xs, d_sub, P->stream), P->stream);
     }
     h->xsup = (int32_t*)malloc(sizeof(int32_t) * ((size_t)ns + 1));
     h->supno = (int32_t*)malloc(sizeof(int32_t) * std::max<size_t>((size_t)n, 1));
     h->xsub = (int64_t*)calloc((size_t)ns + 1, sizeof(int64_t));
-    h->sub = (int32_t*)malloc(sizeof(int32_t) * std::max<size_t>((size_t)nsub, 1));
+    h->sub = (int32_t*)host_array(sizeof(int32_t) * std::max<size_t>((size_t)nsub, 1));
     h->xlcol = (int64_t*)calloc((size_t)n + 1, sizeof(int64_t));
-    h->lrow = (int32_t*)malloc(sizeof(int32_t) * std::max<size_t>((size_t)P->nnzL, 1));
+    h->lrow = (int32_t*)host_array(sizeof(int32_t) * std::max<size_t>((size_t)P->nnzL, 1));
     h->xucol = (int64_t*)calloc((size_t)n + 1, sizeof(int64_t));
-    h->urow = (int32_t*)malloc(sizeof(int32_t) * std::max<size_t>((size_t)P->nnzU, 1));
+    h->urow = (int32_t*)host_array(sizeof(int32_t) * std::max<size_t>((size_t)P->nnzU, 1));
     if (!h->xsup || !h->supno || !h->xsub || !h->sub || !h->xlcol || !h->lrow || !h->xucol || !h->urow) {
         gsofa_supernodal_free(h);
         return GSOFA_ERR_ALLOC;
     }
     h->xsup[0] = 0;
+    std::vector<HostCopy> cp;
     if (n > 0) {
-        HIPCHK_OUT(hipMemcpyAsync(h->xsup, P->d_sstart, sizeof(int32_t) * ((size_t)ns + 1), hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(h->supno, P->d_supno, sizeof(int32_t) * (size_t)n, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(h->xlcol, d_xl, sizeof(int64_t) * ((size_t)n + 1), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(h->xucol, d_xu, sizeof(int64_t) * ((size_t)n + 1), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
+        cp.push_back({h->xsup, P->d_sstart, sizeof(int32_t) * ((size_t)ns + 1)});
+        cp.push_back({h->supno, P->d_supno, sizeof(int32_t) * (size_t)n});
+        cp.push_back({h->xlcol, d_xl, sizeof(int64_t) * ((size_t)n + 1)});
+        cp.push_back({h->xucol, d_xu, sizeof(int64_t) * ((size_t)n + 1)});
     }
-    if (P->nnzL)
-        HIPCHK_OUT(hipMemcpyAsync(h->lrow, d_lrow, sizeof(int32_t) * (size_t)P->nnzL, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-    if (P->nnzU)
-        HIPCHK_OUT(hipMemcpyAsync(h->urow, d_urow, sizeof(int32_t) * (size_t)P->nnzU, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
+    cp.push_back({h->lrow, d_lrow, sizeof(int32_t) * (size_t)P->nnzL});
+    cp.push_back({h->urow, d_urow, sizeof(int32_t) * (size_t)P->nnzU});
     if (ns > 0) {
-        HIPCHK_OUT(hipMemcpyAsync(h->xsub, d_xs, sizeof(int64_t) * ((size_t)ns + 1), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(h->sub, d_sub, sizeof(int32_t) * (size_t)nsub, hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
+        cp.push_back({h->xsub, d_xs, sizeof(int64_t) * ((size_t)ns + 1)});
+        cp.push_back({h->sub, d_sub, sizeof(int32_t) * (size_t)nsub});
     }
-    HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+    HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
     return GSOFA_OK;
 }
 
@@ -2508,10 +2401,11 @@ int gsofa_fill_bound(const gsofa_matrix* A, int64_t* row_fill_bound, uint64_t* f
                      uint64_t* U_bound) {
     const int rc = validate(A);
     if (rc) return rc;
-    std::vector<int32_t> rp, ci;
+    std::vector<int32_t> rp, ci, rpT, ciT;
     pack_rows(A, rp, ci);
+    transpose_rows(A->n, rp.data(), ci.data(), rpT, ciT);
     std::vector<int64_t> Lb, Ub;
-    lu_row_bounds(A->n, rp.data(), ci.data(), Lb, Ub);
+    lu_row_bounds(A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), Lb, Ub);
     uint64_t f = 0, l = 0, u = 0;
     for (int32_t i = 0; i < A->n; i++) {
         int64_t off = 0;  // A's own off-diagonal entries are not fills
@@ -2566,7 +2460,7 @@ int pack_matrix(const gsofa_matrix* A, PackedMatrix* M) {
     gsofa_options o;
     gsofa_options_default(&o);
     const std::vector<uint32_t> mb{0u, (uint32_t)M->n};
-    output_need(o, M->n, M->rp.data(), M->ci.data(), &M->need_fill, &M->need_L, &M->need_U, kArenaBits, &mb,
+    output_need(o, M->n, M->rp.data(), M->ci.data(), M->rpT.data(), M->ciT.data(), &M->need_fill, &M->need_L, &M->need_U, kArenaBits, &mb,
                 &M->need_rec);
     M->need_fill = reach_reserve(M->need_fill, M->need_L + M->need_U, M->need_rec);
     return GSOFA_OK;
@@ -2600,7 +2494,7 @@ int arena_create(const gsofa_options* opt, gsofa_plan** out) {
     P->mode = GSOFA_MODE_REACH;
     P->arena = true;
     P->device = P->opt.device;
-    if (hipSetDevice(P->device) != hipSuccess || hipStreamCreate(&P->stream) != hipSuccess) {
+    if (hipSetDevice(P->device) != hipSuccess || stream_get(P->device, &P->stream) != hipSuccess) {
         (void)hipGetLastError();
         delete P;
         return GSOFA_ERR_HIP;
@@ -2706,31 +2600,31 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     }
     int e = 0;
     if (c.rp < rows) {
-        dfree(P->d_rp);
-        dfree(P->d_rpT);
-        dfree(P->d_cntL);
-        dfree(P->d_cntU);
-        dfree(P->d_Lrp);
-        dfree(P->d_Urp);
-        dfree(P->d_rowfill);
-        dfree(P->d_cnt64);
-        dfree(P->d_rptr);
-        e |= dalloc(&P->d_rp, rows);
-        e |= dalloc(&P->d_rpT, rows);
-        e |= dalloc(&P->d_cntL, rows);
-        e |= dalloc(&P->d_cntU, rows);
-        e |= dalloc(&P->d_Lrp, rows);
-        e |= dalloc(&P->d_Urp, rows);
-        e |= dalloc(&P->d_rowfill, rows);
-        e |= dalloc(&P->d_cnt64, rows);
-        e |= dalloc(&P->d_rptr, rows);
+        pfree(P, P->d_rp);
+        pfree(P, P->d_rpT);
+        pfree(P, P->d_cntL);
+        pfree(P, P->d_cntU);
+        pfree(P, P->d_Lrp);
+        pfree(P, P->d_Urp);
+        pfree(P, P->d_rowfill);
+        pfree(P, P->d_cnt64);
+        pfree(P, P->d_rptr);
+        e |= palloc(P, &P->d_rp, rows);
+        e |= palloc(P, &P->d_rpT, rows);
+        e |= palloc(P, &P->d_cntL, rows);
+        e |= palloc(P, &P->d_cntU, rows);
+        e |= palloc(P, &P->d_Lrp, rows);
+        e |= palloc(P, &P->d_Urp, rows);
+        e |= palloc(P, &P->d_rowfill, rows);
+        e |= palloc(P, &P->d_cnt64, rows);
+        e |= palloc(P, &P->d_rptr, rows);
         c.rp = rows;
     }
     if (c.ci < ne) {
-        dfree(P->d_ci);
-        dfree(P->d_ciT);
-        e |= dalloc(&P->d_ci, ne);
-        e |= dalloc(&P->d_ciT, ne);
+        pfree(P, P->d_ci);
+        pfree(P, P->d_ciT);
+        e |= palloc(P, &P->d_ci, ne);
+        e |= palloc(P, &P->d_ciT, ne);
         c.ci = ne;
     }
     const size_t nfe = (size_t)(2 * nr);
@@ -2741,47 +2635,47 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     }
     const size_t nle = (size_t)std::max<uint64_t>(nl, 1), nue = (size_t)std::max<uint64_t>(nu, 1);
     if (c.L < nle) {
-        dfree(P->d_Lcol);
-        e |= dalloc(&P->d_Lcol, nle);
+        pfree(P, P->d_Lcol);
+        e |= palloc(P, &P->d_Lcol, nle);
         c.L = nle;
     }
     if (c.U < nue) {
-        dfree(P->d_Ucol);
-        e |= dalloc(&P->d_Ucol, nue);
+        pfree(P, P->d_Ucol);
+        e |= palloc(P, &P->d_Ucol, nue);
         c.U = nue;
     }
     P->scan_words = scan_tmp_words(n) + 2 * (size_t)n + 8;
     if (c.scan < P->scan_words) {
-        dfree(P->d_scan);
-        e |= dalloc(&P->d_scan, P->scan_words);
+        pfree(P, P->d_scan);
+        e |= palloc(P, &P->d_scan, P->scan_words);
         c.scan = P->scan_words;
     }
     if (c.mats < (size_t)count + 1) {
-        dfree(P->d_mat_base);
-        dfree(P->d_mat_te);
-        dfree(P->d_mat_reach);
-        e |= dalloc(&P->d_mat_base, (size_t)count + 1);
-        e |= dalloc(&P->d_mat_te, (size_t)count + 1);
-        e |= dalloc(&P->d_mat_reach, (size_t)count + 1);
+        pfree(P, P->d_mat_base);
+        pfree(P, P->d_mat_te);
+        pfree(P, P->d_mat_reach);
+        e |= palloc(P, &P->d_mat_base, (size_t)count + 1);
+        e |= palloc(P, &P->d_mat_te, (size_t)count + 1);
+        e |= palloc(P, &P->d_mat_reach, (size_t)count + 1);
         c.mats = (size_t)count + 1;
     }
     if (c.chunks < nchunks) {
-        dfree(P->d_chunks);
-        dfree(P->d_grp);
-        e |= dalloc(&P->d_grp, (size_t)nchunks);
-        e |= dalloc(&P->d_chunks, (size_t)nchunks);
+        pfree(P, P->d_chunks);
+        pfree(P, P->d_grp);
+        e |= palloc(P, &P->d_grp, (size_t)nchunks);
+        e |= palloc(P, &P->d_chunks, (size_t)nchunks);
         c.chunks = nchunks;
     }
-    if (!P->d_ctrl) e |= dalloc(&P->d_ctrl, 1);
+    if (!P->d_ctrl) e |= palloc(P, &P->d_ctrl, 1);
     e |= setup_quot(P, qlev);
     if (e) return GSOFA_ERR_ALLOC;
     // per-workgroup arrays: one stride (their capacity) for every batch,
     // cleared when they grow
     if (!P->d_vis || c.wg < W || c.nb < nb) {
-        dfree(P->d_vis);
-        dfree(P->d_rmask);
-        dfree(P->d_qgv);
-        dfree(P->d_bstate);
+        pfree(P, P->d_vis);
+        pfree(P, P->d_rmask);
+        pfree(P, P->d_qgv);
+        pfree(P, P->d_bstate);
         c.wg = std::max<size_t>(W, c.wg);
         c.nb = std::max<size_t>(nb, c.nb);
         if (reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64) > budget - fixed - qb) {  // exactly this batch's
@@ -2789,10 +2683,10 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
             c.nb = nb;
         }
         const size_t nbw = c.nb * c.wg;
-        e |= dalloc((uint4**)&P->d_vis, nbw);
-        e |= dalloc((uint64_t**)&P->d_rmask, 2 * nbw);
-        e |= dalloc(&P->d_qgv, 2 * nbw);
-        e |= dalloc(&P->d_bstate, c.nb);
+        e |= palloc(P, (uint4**)&P->d_vis, nbw);
+        e |= palloc(P, (uint64_t**)&P->d_rmask, 2 * nbw);
+        e |= palloc(P, &P->d_qgv, 2 * nbw);
+        e |= palloc(P, &P->d_bstate, c.nb);
         if (e) return GSOFA_ERR_ALLOC;
         HIPCHK(hipMemsetAsync(P->d_vis, 0, 16 * nbw, P->stream));
         HIPCHK(hipMemsetAsync(P->d_rmask, 0, 16 * nbw, P->stream));
@@ -2814,21 +2708,14 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         const long vsp = atol(sp);
         if (vsp >= 1 && vsp < (long)0xFFFFFFFFu) P->span_cap = (uint32_t)vsp;
     }
-    // uploads (the host copies stay in the plan until the next load)
-    HIPCHK(hipMemcpyAsync(P->d_rp, P->h_rp.data(), sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice,
-                          P->stream));
-    HIPCHK(hipMemcpyAsync(P->d_rpT, rpT.data(), sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice,
-                          P->stream));
-    if (nnz) {
-        HIPCHK(hipMemcpyAsync(P->d_ci, P->h_ci.data(), sizeof(int32_t) * (size_t)nnz, hipMemcpyHostToDevice,
-                              P->stream));
-        HIPCHK(hipMemcpyAsync(P->d_ciT, P->h_ciT.data(), sizeof(int32_t) * (size_t)nnz, hipMemcpyHostToDevice,
-                              P->stream));
-    }
-    HIPCHK(hipMemcpyAsync(P->d_mat_base, P->h_mat_base.data(), sizeof(uint32_t) * ((size_t)count + 1),
-                          hipMemcpyHostToDevice, P->stream));
-    HIPCHK(hipMemcpyAsync(P->d_chunks, P->h_chunks.data(), sizeof(BlkChunk) * nchunks, hipMemcpyHostToDevice,
-                          P->stream));
+    std::vector<HostCopy> up{{P->h_rp.data(), P->d_rp, sizeof(int32_t) * ((size_t)n + 1)},
+                    {rpT.data(), P->d_rpT, sizeof(int32_t) * ((size_t)n + 1)},
+                    {P->h_ci.data(), P->d_ci, sizeof(int32_t) * (size_t)nnz},
+                    {P->h_ciT.data(), P->d_ciT, sizeof(int32_t) * (size_t)nnz},
+                    {P->h_mat_base.data(), P->d_mat_base, sizeof(uint32_t) * ((size_t)count + 1)},
+                    {P->h_chunks.data(), P->d_chunks, sizeof(BlkChunk) * nchunks}};
+    upload_quot(P, up);
+    HIPCHK(copy_in(up, P->stream));
     P->executed = false;
     P->host_valid = false;
     return GSOFA_OK;
@@ -2853,17 +2740,12 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
     r->passes = P->passes;
     r->n_super = -1;
     unsigned long long te = 0, reach = 0;
-    HIPCHK_OUT(hipMemcpyAsync(&te, P->d_mat_te + index, sizeof(te), hipMemcpyDeviceToHost, P->stream), P->stream);
-    HIPCHK_OUT(hipMemcpyAsync(&reach, P->d_mat_reach + index, sizeof(reach), hipMemcpyDeviceToHost, P->stream),
-               P->stream);
-    r->te_alg = te;
-    r->reach = reach;
+    std::vector<HostCopy> cp{{&te, P->d_mat_te + index, sizeof(te)}, {&reach, P->d_mat_reach + index, sizeof(reach)}};
     r->row_fill = (int64_t*)malloc(sizeof(int64_t) * (size_t)std::max(nb, 1));
     if (!r->row_fill) return GSOFA_ERR_ALLOC;
     if (!P->structure) {  // counts only: the kernels' per-row tallies
-        HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill + b0, sizeof(int64_t) * (size_t)nb, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        cp.push_back({r->row_fill, P->d_rowfill + b0, sizeof(int64_t) * (size_t)nb});
+        HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
         r->te_alg = te;
         r->reach = reach;
         for (int32_t i = 0; i < nb; i++) r->fill_count += (uint64_t)r->row_fill[i];
@@ -2875,13 +2757,16 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
         gsofa_result_free(r);
         return GSOFA_ERR_ALLOC;
     }
-    HIPCHK_OUT(hipMemcpyAsync(r->L_rowptr, P->d_Lrp + b0, sizeof(int64_t) * ((size_t)nb + 1), hipMemcpyDeviceToHost,
-                              P->stream), P->stream);
-    HIPCHK_OUT(hipMemcpyAsync(r->U_rowptr, P->d_Urp + b0, sizeof(int64_t) * ((size_t)nb + 1), hipMemcpyDeviceToHost,
-                              P->stream), P->stream);
-    HIPCHK_OUT(hipMemcpyAsync(r->row_fill, P->d_rowfill + b0, sizeof(int64_t) * (size_t)nb, hipMemcpyDeviceToHost,
-                              P->stream), P->stream);
-    HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+    int32_t s0 = 0, s1 = 0;
+    cp.push_back({r->L_rowptr, P->d_Lrp + b0, sizeof(int64_t) * ((size_t)nb + 1)});
+    cp.push_back({r->U_rowptr, P->d_Urp + b0, sizeof(int64_t) * ((size_t)nb + 1)});
+    cp.push_back({r->row_fill, P->d_rowfill + b0, sizeof(int64_t) * (size_t)nb});
+    if (P->supernodes && nb > 0) {
+        cp.push_back({&s0, P->d_supno + b0, sizeof(int32_t)});
+        cp.push_back({&s1, P->d_supno + b1 - 1, sizeof(int32_t)});
+    }
+    HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
+    cp.clear();
     r->te_alg = te;
     r->reach = reach;
     const int64_t l0 = r->L_rowptr[0], l1 = r->L_rowptr[nb], u0 = r->U_rowptr[0], u1 = r->U_rowptr[nb];
@@ -2900,14 +2785,9 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
         HIPCHK_OUT(launch_add(P->d_Lcol + l0, (uint64_t)(l1 - l0), -(int32_t)b0, P->stream), P->stream);
         HIPCHK_OUT(launch_add(P->d_Ucol + u0, (uint64_t)(u1 - u0), -(int32_t)b0, P->stream), P->stream);
     }
-    HIPCHK_OUT(copy_d2h(r->L_col, P->d_Lcol + l0, sizeof(int32_t) * (size_t)(l1 - l0), P->stream), P->stream);
-    HIPCHK_OUT(copy_d2h(r->U_col, P->d_Ucol + u0, sizeof(int32_t) * (size_t)(u1 - u0), P->stream), P->stream);
+    cp.push_back({r->L_col, P->d_Lcol + l0, sizeof(int32_t) * (size_t)(l1 - l0)});
+    cp.push_back({r->U_col, P->d_Ucol + u0, sizeof(int32_t) * (size_t)(u1 - u0)});
     if (P->supernodes && nb > 0) {
-        int32_t s0 = 0, s1 = 0;
-        HIPCHK_OUT(hipMemcpyAsync(&s0, P->d_supno + b0, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(&s1, P->d_supno + b1 - 1, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream),
-                   P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
         // supernodes never cross matrices: (i-1) is never in L_i at a boundary
         r->n_super = s1 - s0 + 1;
         r->super_start = (int32_t*)malloc(sizeof(int32_t) * ((size_t)r->n_super + 1));
@@ -2916,16 +2796,15 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        HIPCHK_OUT(hipMemcpyAsync(r->super_start, P->d_sstart + s0, sizeof(int32_t) * (size_t)r->n_super,
-                                  hipMemcpyDeviceToHost, P->stream), P->stream);
-        HIPCHK_OUT(hipMemcpyAsync(r->supno, P->d_supno + b0, sizeof(int32_t) * (size_t)nb, hipMemcpyDeviceToHost,
-                                  P->stream), P->stream);
-        HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
+        cp.push_back({r->super_start, P->d_sstart + s0, sizeof(int32_t) * (size_t)r->n_super});
+        cp.push_back({r->supno, P->d_supno + b0, sizeof(int32_t) * (size_t)nb});
+    }
+    HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
+    if (r->supno) {
         for (int32_t s = 0; s < r->n_super; s++) r->super_start[s] -= (int32_t)b0;
         r->super_start[r->n_super] = nb;
         for (int32_t i = 0; i < nb; i++) r->supno[i] -= s0;
     }
-    HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
     return GSOFA_OK;
 }
 

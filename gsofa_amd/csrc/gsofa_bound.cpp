@@ -52,55 +52,44 @@ int32_t find_root(std::vector<int32_t>& anc, int32_t x) {
 
 }  // namespace
 
-// rp/ci: packed rows (sorted, duplicate-free), n rows.  On return
-// Lb[i] >= |L_i|, Ub[i] >= |U_i| (both strict, A's own entries included); the
-// elimination tree of A + A^T goes to *parent_out if given.
-void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int64_t>& Lb,
-                   std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out) {
+// rp/ci: packed rows (sorted, duplicate-free) of A, rpT/ciT of its transpose, n
+// rows.  On return Lb[i] >= |L_i|, Ub[i] >= |U_i| (both strict, A's own entries
+// included); the elimination tree of A + A^T goes to *parent_out if given.
+// S's rows are never built: row i of S is row i of A and row i of A^T, and an
+// entry met in both changes nothing the second time (its path to i is walked
+// and compressed, and j is no leaf of T_i twice).
+void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT, const int32_t* ciT,
+                   std::vector<int64_t>& Lb, std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out) {
     Lb.assign((size_t)n, 0);
     Ub.assign((size_t)n, 0);
     if (parent_out) parent_out->clear();
     if (n <= 0) return;
-    // S's strictly lower entries as (hi, lo) pairs, in two layouts:
-    // by hi (row hi's lower neighbours) and by lo (column lo's rows below)
-    std::vector<int64_t> cnt_hi((size_t)n + 1, 0), cnt_lo((size_t)n + 1, 0);
+    const int32_t* const rows[2] = {rp, rpT};
+    const int32_t* const cols[2] = {ci, ciT};
+    // elimination tree of S (Liu's ancestor algorithm with path compression);
+    // split[t][i]: row i's first entry above the diagonal
+    std::vector<int32_t> parent((size_t)n, -1), anc((size_t)n, -1), split[2];
+    split[0].resize((size_t)n);
+    split[1].resize((size_t)n);
     for (int32_t i = 0; i < n; i++)
-        for (int32_t p = rp[i]; p < rp[i + 1]; p++) {
-            const int32_t j = ci[p];
-            if (j == i) continue;
-            cnt_hi[(size_t)std::max(i, j) + 1]++;
-            cnt_lo[(size_t)std::min(i, j) + 1]++;
-        }
-    for (int32_t i = 0; i < n; i++) {
-        cnt_hi[(size_t)i + 1] += cnt_hi[(size_t)i];
-        cnt_lo[(size_t)i + 1] += cnt_lo[(size_t)i];
-    }
-    std::vector<int32_t> by_hi((size_t)cnt_hi[(size_t)n]), by_lo((size_t)cnt_lo[(size_t)n]);
-    {
-        std::vector<int64_t> ph(cnt_hi.begin(), cnt_hi.end() - 1), pl(cnt_lo.begin(), cnt_lo.end() - 1);
-        for (int32_t i = 0; i < n; i++)
-            for (int32_t p = rp[i]; p < rp[i + 1]; p++) {
-                const int32_t j = ci[p];
-                if (j == i) continue;
-                const int32_t hi = std::max(i, j), lo = std::min(i, j);
-                by_hi[(size_t)ph[(size_t)hi]++] = lo;
-                by_lo[(size_t)pl[(size_t)lo]++] = hi;
+        for (int t = 0; t < 2; t++) {
+            const int32_t* c = cols[t];
+            int32_t p = rows[t][i];
+            const int32_t e = rows[t][i + 1];
+            for (; p < e && c[p] < i; p++) {
+                int32_t r = c[p];
+                for (;;) {
+                    const int32_t a = anc[(size_t)r];
+                    if (a == i) break;
+                    anc[(size_t)r] = i;
+                    if (a < 0) {
+                        parent[(size_t)r] = i;
+                        break;
+                    }
+                    r = a;
+                }
             }
-    }
-    // elimination tree of S (Liu's ancestor algorithm with path compression)
-    std::vector<int32_t> parent((size_t)n, -1), anc((size_t)n, -1);
-    for (int32_t i = 0; i < n; i++)
-        for (int64_t p = cnt_hi[(size_t)i]; p < cnt_hi[(size_t)i + 1]; p++) {
-            int32_t r = by_hi[(size_t)p];
-            while (anc[(size_t)r] != -1 && anc[(size_t)r] != i) {
-                const int32_t t = anc[(size_t)r];
-                anc[(size_t)r] = i;
-                r = t;
-            }
-            if (anc[(size_t)r] == -1) {
-                anc[(size_t)r] = i;
-                parent[(size_t)r] = i;
-            }
+            split[t][(size_t)i] = p < e && c[p] == i ? p + 1 : p;
         }
     // depth (parents are numbered above their children) and a postorder
     std::vector<int32_t> depth((size_t)n, 0), head((size_t)n, -1), nxt((size_t)n, -1);
@@ -112,58 +101,57 @@ void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<
             head[(size_t)pj] = j;
         }
     }
-    std::vector<int32_t> post((size_t)n), stack;
+    std::vector<int32_t> post((size_t)n), first((size_t)n, -1);
     int32_t k = 0;
     for (int32_t root = 0; root < n; root++) {
         if (parent[(size_t)root] != -1) continue;
-        stack.push_back(root);
-        while (!stack.empty()) {
-            const int32_t v = stack.back();
+        // down to the next unvisited child, else number the vertex and go up
+        for (int32_t v = root;;) {
             const int32_t c = head[(size_t)v];
-            if (c >= 0) {  // descend into the next unvisited child
+            if (c >= 0) {
                 head[(size_t)v] = nxt[(size_t)c];
-                stack.push_back(c);
-            } else {
-                stack.pop_back();
-                post[(size_t)k++] = v;
+                v = c;
+                continue;
             }
+            if (first[(size_t)v] < 0) first[(size_t)v] = k;  // a leaf starts its subtree
+            post[(size_t)k++] = v;
+            const int32_t up = parent[(size_t)v];
+            if (up < 0) break;
+            if (first[(size_t)up] < 0) first[(size_t)up] = first[(size_t)v];
+            v = up;
         }
-    }
-    std::vector<int32_t> pnum((size_t)n), first((size_t)n, -1);
-    for (int32_t q = 0; q < n; q++) {
-        pnum[(size_t)post[(size_t)q]] = q;
-        for (int32_t v = post[(size_t)q]; v >= 0 && first[(size_t)v] < 0; v = parent[(size_t)v])
-            first[(size_t)v] = q;
     }
     // skeleton leaves, row counts and column-count weights, in postorder
     std::vector<int32_t> last_adj((size_t)n, -1), prev_leaf((size_t)n, -1), set((size_t)n);
-    std::vector<int64_t> w((size_t)n, 0);
+    int64_t* w = Ub.data();
     for (int32_t v = 0; v < n; v++) set[(size_t)v] = v;
     for (int32_t q = 0; q < n; q++) {
-        const int32_t j = post[(size_t)q];
-        for (int64_t p = cnt_lo[(size_t)j]; p < cnt_lo[(size_t)j + 1]; p++) {
-            const int32_t i = by_lo[(size_t)p];  // S(i, j) != 0 with i > j
-            const bool leaf = first[(size_t)j] > last_adj[(size_t)i];
-            last_adj[(size_t)i] = q;
-            if (!leaf) continue;
-            w[(size_t)j] += 1;
-            const int32_t pl = prev_leaf[(size_t)i];
-            int32_t top;  // where the path from j joins what row i already holds
-            if (pl < 0) {
-                top = i;
-                w[(size_t)i] -= 1;
-            } else {
-                top = find_root(set, pl);
-                w[(size_t)top] -= 1;
+        const int32_t j = post[(size_t)q], fj = first[(size_t)j], dj = depth[(size_t)j];
+        for (int t = 0; t < 2; t++) {
+            const int32_t e = rows[t][j + 1];
+            for (int32_t p = split[t][(size_t)j]; p < e; p++) {
+                const int32_t i = cols[t][p];  // S(i, j) != 0 with i > j
+                const bool leaf = fj > last_adj[(size_t)i];
+                last_adj[(size_t)i] = q;
+                if (!leaf) continue;
+                w[j] += 1;
+                const int32_t pl = prev_leaf[(size_t)i];
+                int32_t top;  // where the path from j joins what row i already holds
+                if (pl < 0) {
+                    top = i;
+                    w[i] -= 1;
+                } else {
+                    top = find_root(set, pl);
+                    w[top] -= 1;
+                }
+                Lb[(size_t)i] += dj - depth[(size_t)top];
+                prev_leaf[(size_t)i] = j;
             }
-            Lb[(size_t)i] += depth[(size_t)j] - depth[(size_t)top];
-            prev_leaf[(size_t)i] = j;
         }
         if (parent[(size_t)j] >= 0) set[(size_t)j] = parent[(size_t)j];
     }
     for (int32_t j = 0; j < n; j++)  // subtree sums: children precede parents
-        if (parent[(size_t)j] >= 0) w[(size_t)parent[(size_t)j]] += w[(size_t)j];
-    for (int32_t j = 0; j < n; j++) Ub[(size_t)j] = w[(size_t)j];
+        if (parent[(size_t)j] >= 0) w[parent[(size_t)j]] += w[j];
     if (parent_out) parent_out->swap(parent);
 }
 

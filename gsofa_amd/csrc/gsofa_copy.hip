@@ -1,0 +1,343 @@
+// gsofa_copy.hip -- copies between host arrays and the device through pinned
+// staging, and the small host-side pools behind them (host code, one kernel).
+//
+// Callers' arrays are pageable.  The runtime's own pageable copies take 115 us
+// for 256 KB and 400 us for 1 MB, where a pinned one takes 13 and 26, and each
+// copy is a call and a wait of its own.  So all arrays of a call go together:
+//   small totals (a matrix of thousands of rows) by one kernel between the
+//     arrays and one pinned buffer: the fetch of a 16 x 16 grid 160 -> 17 us,
+//     its upload 60 -> 19;
+//   the rest in chunks of at most 4 MB, each with its DMA in flight while the
+//     thread copies the previous one out.  A single thread that first touches
+//     the destination moves 14 GB/s, so larger totals take up to kThreads
+//     threads: 55 MB (33^3 grid) 9.5 -> 3.4 ms, 1.0 GB (48^3) 22.2 -> 18.9 ms
+//     (54 GB/s of the link's 57).  16 MB buffers instead of 4: 6.8 and 26 ms.
+// Result arrays start on 2 MB boundaries with transparent huge pages requested,
+// since their first touch is in this path.
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include <sys/mman.h>
+
+#include "gsofa_internal.h"
+
+namespace gsofa {
+
+namespace {
+
+constexpr size_t kStageBytes = 4u << 20;
+constexpr size_t kStageKeep = 64;          // idle staging buffers kept: four copies at once
+constexpr size_t kStageRest = 16;          // and after the last plan's release, one copy's (64 MB:
+                                           // making and releasing them takes over 1 ms)
+constexpr size_t kKernelMost = 512u << 10; // totals up to here: one kernel
+constexpr size_t kPerThread = 1u << 20;    // bytes per copy thread, at least
+constexpr int kThreads = 8;
+constexpr size_t kChunkMin = 256u << 10;
+constexpr size_t kHugePage = 2u << 20;
+constexpr size_t kHugeMin = 1u << 20;
+
+std::mutex g_mu;
+std::vector<void*> g_stage;                // idle staging buffers
+struct IdleStream {
+    int device;
+    hipStream_t s;
+};
+std::vector<IdleStream> g_streams;
+constexpr size_t kStreamKeep = 16;
+constexpr size_t kStreamRest = 2;
+size_t g_live = 0;                         // streams handed out: live plans
+std::vector<Ctrl*> g_ctrl;                 // idle pinned counter blocks, made a page at a time
+constexpr size_t kCtrlSlots = 4096 / sizeof(Ctrl);
+
+void* stage_get() {
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (!g_stage.empty()) {
+            void* p = g_stage.back();
+            g_stage.pop_back();
+            return p;
+        }
+    }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
+}
+
+void stage_put(void* p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (g_stage.size() < kStageKeep) {
+            g_stage.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
+struct Pieces {
+    static constexpr int MAX = 16;
+    uint32_t* dst[MAX];
+    const uint32_t* src[MAX];
+    uint32_t words[MAX];
+    int count;
+};
+
+__global__ void k_copy_pieces(Pieces p) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    for (int k = 0; k < p.count; k++)
+        for (uint32_t i = t; i < p.words[k]; i += step) p.dst[k][i] = p.src[k][i];
+}
+
+struct Chunk {
+    size_t first, count;  // pieces
+};
+
+// `out`: device to host, else host to device.
+hipError_t copy_small(const std::vector<HostCopy>& v, bool out, char* stage, hipStream_t s, size_t total) {
+    Pieces p{};
+    size_t off = 0;
+    for (const HostCopy& c : v) {
+        if (!c.bytes) continue;
+        if (!out) std::memcpy(stage + off, c.host, c.bytes);
+        p.dst[p.count] = reinterpret_cast<uint32_t*>(out ? stage + off : (char*)c.dev);
+        p.src[p.count] = reinterpret_cast<const uint32_t*>(out ? (char*)c.dev : stage + off);
+        p.words[p.count++] = (uint32_t)(c.bytes / 4);
+        off += (c.bytes + 15) & ~(size_t)15;
+    }
+    const uint32_t blocks = (uint32_t)std::min<size_t>((total / 4 + 255) / 256, 512);
+    hipLaunchKernelGGL(k_copy_pieces, dim3(std::max(blocks, 1u)), dim3(256), 0, s, p);
+    hipError_t e = hipGetLastError();
+    const hipError_t w = hipStreamSynchronize(s);  // in either case: nothing may still use the buffer
+    if (e == hipSuccess) e = w;
+    if (e != hipSuccess || !out) return e;
+    off = 0;
+    for (const HostCopy& c : v) {
+        if (c.bytes) std::memcpy(c.host, stage + off, c.bytes);
+        off += (c.bytes + 15) & ~(size_t)15;
+    }
+    return hipSuccess;
+}
+
+hipError_t copy_chunks(const std::vector<HostCopy>& pieces, const std::vector<Chunk>& chunks, bool out,
+                       hipStream_t s, std::atomic<size_t>& next, void* b0, void* b1, int device) {
+    (void)hipSetDevice(device);
+    char* buf[2] = {(char*)b0, (char*)b1};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    hipError_t e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
+    auto host_side = [&](size_t k, char* b) {
+        size_t off = 0;
+        for (size_t i = chunks[k].first; i < chunks[k].first + chunks[k].count; i++) {
+            const HostCopy& c = pieces[i];
+            if (out) std::memcpy(c.host, b + off, c.bytes);
+            else std::memcpy(b + off, c.host, c.bytes);
+            off += c.bytes;
+        }
+    };
+    auto dma = [&](size_t k, char* b, hipEvent_t x) {
+        size_t off = 0;
+        for (size_t i = chunks[k].first; i < chunks[k].first + chunks[k].count; i++) {
+            const HostCopy& c = pieces[i];
+            const hipError_t r = out ? hipMemcpyAsync(b + off, c.dev, c.bytes, hipMemcpyDeviceToHost, s)
+                                     : hipMemcpyAsync(c.dev, b + off, c.bytes, hipMemcpyHostToDevice, s);
+            if (r != hipSuccess) return r;
+            off += c.bytes;
+        }
+        return hipEventRecord(x, s);
+    };
+    const size_t none = ~(size_t)0;
+    size_t have[2] = {none, none};
+    for (int cur = 0; e == hipSuccess; cur ^= 1) {
+        size_t k = next.fetch_add(1);
+        if (k >= chunks.size()) k = none;
+        if (!out && have[cur] != none) {  // the buffer's previous chunk has left it
+            e = hipEventSynchronize(ev[cur]);
+            have[cur] = none;
+        }
+        if (e == hipSuccess && k != none) {
+            if (!out) host_side(k, buf[cur]);
+            e = dma(k, buf[cur], ev[cur]);
+            if (e == hipSuccess) have[cur] = k;
+        }
+        const int o = cur ^ 1;
+        if (e == hipSuccess && have[o] != none && (out || k == none)) {
+            e = hipEventSynchronize(ev[o]);
+            if (e == hipSuccess && out) host_side(have[o], buf[o]);
+            have[o] = none;
+        }
+        if (k == none) break;
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // no copy left in flight in the buffers
+    for (hipEvent_t x : ev)
+        if (x) (void)hipEventDestroy(x);
+    return e;
+}
+
+hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
+    size_t total = 0, used = 0;
+    for (const HostCopy& c : v) {
+        total += c.bytes;
+        used += c.bytes != 0;
+    }
+    if (total == 0) return hipSuccess;
+    void* buf[2 * kThreads] = {};
+    buf[0] = stage_get();
+    if (buf[0] && total <= kKernelMost && used <= (size_t)Pieces::MAX) {
+        const hipError_t e = copy_small(v, out, (char*)buf[0], s, total);
+        stage_put(buf[0]);
+        return e;
+    }
+    int threads = 0;
+    const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, total / kPerThread));
+    for (; threads < want; threads++) {
+        if (threads > 0) buf[2 * threads] = stage_get();
+        buf[2 * threads + 1] = stage_get();
+        if (!buf[2 * threads] || !buf[2 * threads + 1]) break;
+    }
+    if (threads == 0) {  // no pinned memory: direct copies
+        for (void* b : buf) stage_put(b);
+        hipError_t e = hipSuccess;
+        for (const HostCopy& c : v) {
+            if (!c.bytes || e != hipSuccess) continue;
+            e = out ? hipMemcpyAsync(c.host, c.dev, c.bytes, hipMemcpyDeviceToHost, s)
+                    : hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, s);
+        }
+        const hipError_t w = hipStreamSynchronize(s);
+        return e == hipSuccess ? w : e;
+    }
+    const size_t ch = std::min(kStageBytes, std::max(kChunkMin, total / (4 * (size_t)threads)));
+    std::vector<HostCopy> pieces;
+    std::vector<Chunk> chunks;
+    size_t room = 0;
+    for (const HostCopy& c : v)
+        for (size_t o = 0; o < c.bytes;) {
+            if (room == 0) {
+                chunks.push_back({pieces.size(), 0});
+                room = ch;
+            }
+            const size_t len = std::min(room, c.bytes - o);
+            pieces.push_back({(char*)c.host + o, (char*)c.dev + o, len});
+            chunks.back().count++;
+            room -= len;
+            o += len;
+        }
+    int device = 0;
+    (void)hipGetDevice(&device);
+    std::atomic<size_t> next{0};
+    std::vector<hipError_t> err((size_t)threads, hipSuccess);
+    std::vector<std::thread> th;
+    auto part = [&](int i) {
+        err[(size_t)i] = copy_chunks(pieces, chunks, out, s, next, buf[2 * i], buf[2 * i + 1], device);
+    };
+    for (int i = 1; i < threads; i++) {
+        try {
+            th.emplace_back(part, i);
+        } catch (...) {  // no thread: the others take its chunks
+            break;
+        }
+    }
+    part(0);
+    for (std::thread& t : th) t.join();
+    for (void* b : buf) stage_put(b);
+    for (hipError_t x : err)
+        if (x != hipSuccess) return x;
+    return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t copy_out(const std::vector<HostCopy>& v, hipStream_t s) { return copy_all(v, true, s); }
+hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s) { return copy_all(v, false, s); }
+
+hipError_t launch_copy_words(void* dst, const void* src, uint32_t words, hipStream_t s) {
+    Pieces p{};
+    p.dst[0] = static_cast<uint32_t*>(dst);
+    p.src[0] = static_cast<const uint32_t*>(src);
+    p.words[0] = words;
+    p.count = 1;
+    hipLaunchKernelGGL(k_copy_pieces, dim3(1), dim3(64), 0, s, p);
+    return hipGetLastError();
+}
+
+void* host_array(size_t bytes) {
+    if (bytes < kHugeMin) return malloc(std::max<size_t>(bytes, 1));
+    const size_t len = (bytes + kHugePage - 1) / kHugePage * kHugePage;
+    void* p = nullptr;
+    if (posix_memalign(&p, kHugePage, len) != 0) return nullptr;
+    (void)madvise(p, len, MADV_HUGEPAGE);  // advice only: small pages if refused
+    return p;
+}
+
+// Idle streams are kept (a stream's creation and release take 55 us, a tenth
+// of a small matrix's whole call); a returned one has no work left.  With the
+// last one's return only what a next single call takes up is left.
+hipError_t stream_get(int device, hipStream_t* s) {
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        for (size_t i = 0; i < g_streams.size(); i++)
+            if (g_streams[i].device == device) {
+                *s = g_streams[i].s;
+                g_streams.erase(g_streams.begin() + (ptrdiff_t)i);
+                g_live++;
+                return hipSuccess;
+            }
+    }
+    const hipError_t e = hipStreamCreate(s);
+    if (e == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_live++;
+    }
+    return e;
+}
+
+void stream_put(int device, hipStream_t s) {
+    if (!s) return;
+    // one with an error is not handed on
+    const bool idle = hipStreamSynchronize(s) == hipSuccess;
+    if (!idle) (void)hipGetLastError();
+    std::vector<hipStream_t> gone;
+    std::vector<void*> mem;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_live--;
+        if (idle) g_streams.insert(g_streams.begin(), {device, s});
+        else gone.push_back(s);
+        for (; g_streams.size() > (g_live ? kStreamKeep : kStreamRest); g_streams.pop_back())
+            gone.push_back(g_streams.back().s);
+        for (; g_live == 0 && g_stage.size() > kStageRest; g_stage.pop_back()) mem.push_back(g_stage.back());
+    }
+    for (hipStream_t x : gone) (void)hipStreamDestroy(x);
+    for (void* x : mem) (void)hipHostFree(x);
+}
+
+Ctrl* ctrl_get() {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (g_ctrl.empty()) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, sizeof(Ctrl) * kCtrlSlots, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        for (size_t i = 0; i < kCtrlSlots; i++) g_ctrl.push_back((Ctrl*)p + i);
+    }
+    Ctrl* c = g_ctrl.back();
+    g_ctrl.pop_back();
+    return c;
+}
+
+void ctrl_put(Ctrl* c) {
+    if (!c) return;
+    std::lock_guard<std::mutex> lk(g_mu);
+    g_ctrl.push_back(c);
+}
+
+}  // namespace gsofa

@@ -43,6 +43,12 @@ struct Ctrl {
     unsigned long long te_t;
     unsigned long long reach_t;
     unsigned long long expansions;
+    // reach mode: entries of L and U, and supernodes, as the structure and
+    // supernode passes leave them
+    int64_t nnz_L;
+    int64_t nnz_U;
+    int32_t n_super;
+    uint32_t pad2;
 };
 
 constexpr int32_t kMaxN = (1 << 25) - 1;      // wave-merge totals stay below 2^31
@@ -53,10 +59,10 @@ constexpr int64_t kMaxBlockNnz = 1ll << 30;  // block kernel: column byte offset
 int validate_matrix(const gsofa_matrix* A);
 
 // Per-row upper bounds of |L_i| and |U_i| (strict; A's own entries included)
-// from the elimination tree of A + A^T (gsofa_bound.cpp).  rp/ci are packed
-// rows, sorted and duplicate-free.
-void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int64_t>& Lb,
-                   std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out = nullptr);
+// from the elimination tree of A + A^T (gsofa_bound.cpp).  rp/ci and rpT/ciT are
+// packed rows of A and A^T, sorted and duplicate-free.
+void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT, const int32_t* ciT,
+                   std::vector<int64_t>& Lb, std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out = nullptr);
 uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
                             const std::vector<int64_t>& Ub, int bits);
 
@@ -237,6 +243,23 @@ struct TravParams {
     uint64_t spin_ticks;   // wall-clock ticks a barrier waits before aborting
 };
 
+// Host <-> device copies of a call's arrays together (gsofa_copy.hip), complete
+// on return; work queued on s before is ordered before them.  Sizes and device
+// addresses are multiples of 4 bytes.
+struct HostCopy {
+    void* host;
+    void* dev;
+    size_t bytes;
+};
+hipError_t copy_out(const std::vector<HostCopy>& v, hipStream_t s);
+hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s);
+hipError_t launch_copy_words(void* dst, const void* src, uint32_t words, hipStream_t s);  // pinned or device
+void* host_array(size_t bytes);  // a result array, released with free()
+hipError_t stream_get(int device, hipStream_t* s);
+void stream_put(int device, hipStream_t s);
+Ctrl* ctrl_get();  // a pinned counter block, or null
+void ctrl_put(Ctrl* c);
+
 // Launchers (gsofa_kernels.hip)
 hipError_t launch_traverse(const TravParams& p, hipStream_t s, int cooperative);
 int traverse_block_size();
@@ -301,6 +324,7 @@ struct RowParams {
     int64_t* R_ptr;        // n + 1: offsets of the rows' record lists
     uint4* list;           // the lists
     int64_t list_cap;
+    Ctrl* ctrl;            // nnz_L and nnz_U go there
     uint32_t* long_rows;   // n: rows of over 64 records
     uint32_t* long_count;  // zero on entry
     int32_t* L_col;

@@ -157,6 +157,10 @@ __global__ __launch_bounds__(RT) void k_row_ptrs(RowParams p) {
         p.L_rowptr[s + 1] = ol + cl[k];
         p.U_rowptr[s + 1] = ou + cu[k];
         p.R_ptr[s + 1] = orr + cr[k];
+        if (s + 1 == p.n) {
+            p.ctrl->nnz_L = ol + cl[k];
+            p.ctrl->nnz_U = ou + cu[k];
+        }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) p.L_rowptr[0] = p.U_rowptr[0] = p.R_ptr[0] = 0;
 }
