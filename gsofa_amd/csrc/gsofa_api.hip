@@ -356,13 +356,16 @@ uint64_t label_words(int32_t n, int32_t N, int32_t C, int32_t gid_lo, int32_t gi
 // Output one execute needs at most, from the row bounds of lu_row_bounds:
 // fills, L and U entries of the rows it processes (every share, one share, or
 // for a spilled run the largest share).  rp/ci: packed rows.  bits > 0 (reach
-// mode): also the records of one pass, for groups of so many sources.
+// mode): also the records of one pass, for groups of so many sources.  skew: also
+// the share's subtree_skew.
 void output_need(const gsofa_options& o, int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT,
                  const int32_t* ciT, uint64_t* need_fill, uint64_t* need_L, uint64_t* need_U, int bits = 0,
-                 const std::vector<uint32_t>* mat_base = nullptr, uint64_t* need_rec = nullptr) {
+                 const std::vector<uint32_t>* mat_base = nullptr, uint64_t* need_rec = nullptr,
+                 double* skew = nullptr) {
     std::vector<int64_t> Lb, Ub;
     std::vector<int32_t> parent;
-    lu_row_bounds(n, rp, ci, rpT, ciT, Lb, Ub, bits ? &parent : nullptr);
+    lu_row_bounds(n, rp, ci, rpT, ciT, Lb, Ub, bits || skew ? &parent : nullptr);
+    if (skew) *skew = subtree_skew(std::max(1, o.n_virtual_gpu), std::max(0, o.virtual_gpu_id), parent);
     if (bits) *need_rec = reach_record_bound(*mat_base, parent, Ub, bits);
     const int32_t N = std::max(1, o.n_virtual_gpu);
     std::vector<uint64_t> fs((size_t)N, 0), ls((size_t)N, 0), us((size_t)N, 0);
@@ -761,7 +764,17 @@ uint64_t default_fill_cap(int64_t nnz) { return std::max<uint64_t>(64 * (uint64_
 // small 2D meshes (where 8 is best) and the best on 3D meshes.  A single
 // matrix with nsrc sources takes the largest of 32, 16, 8 whose chunks still
 // give every co-resident workgroup one.
-int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots) {
+// A share (n_virtual_gpu > 1) is judged by `skew`, its largest subtree over the
+// mean.  Bands and naturally ordered grids (2.0 to 2.3) are done when all
+// workgroups are: the smallest slot count of at least 8 with up to four chunks
+// a CU; at 32 / 16 / 8 / 4 slots 10,000 sources of a band of 20,000 take 6.0 /
+// 3.7 / 5.1 / 9.5 ms, 4,133 of one of 12,397 2.9 / 1.9 / 1.6 / 2.7.  Nested
+// dissection (3.8 and more) is done when the deepest chunk is, and the fewer
+// its slots the sooner: 2, up to 16 chunks a CU.  At 16 / 8 / 4 / 2 slots a
+// quarter of a 21^3 grid takes 10.5 / 6.9 / 5.3 / 4.1 ms, half of a 24^3 25.2 /
+// 17.4 / 13.2 / 10.3, a third of a 128^2 40.4 / 21.2 / 14.9 / 10.8, an eighth
+// of a 12^3 1.34 / 0.82 / 0.71 / 0.61.
+int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots, double skew) {
     if (o.block_slots != 0) {
         if (!blk_slots_valid(o.block_slots)) return GSOFA_ERR_INVALID;
         *slots = o.block_slots;
@@ -775,6 +788,13 @@ int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slo
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess) {
         (void)hipGetLastError();
         return GSOFA_ERR_HIP;
+    }
+    if (o.n_virtual_gpu > 1 && skew > 0) {
+        const uint64_t most = (skew < 3.0 ? 4ull : 16ull) * (uint64_t)cus;
+        int S = skew < 3.0 ? 8 : 2;
+        while (S < kBlockSlots && (nsrc + S - 1) / S > most) S *= 2;
+        *slots = S;
+        return GSOFA_OK;
     }
     for (int S = kBlockSlots; S > 8; S /= 2) {
         int occ = 0;
@@ -796,7 +816,7 @@ int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slo
 // `device`.
 int resident_blocks(int slots, int device, uint32_t* out) {
     int occ = 0, cus = 0;
-    if (!blk_slots_valid(slots)) return GSOFA_ERR_INVALID;
+    if (!blk_slots_built(slots)) return GSOFA_ERR_INVALID;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, blk_kernel_ptr(slots), blk_block_size(), 0) !=
             hipSuccess ||
         occ <= 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
@@ -1090,23 +1110,25 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
     }
     const int32_t N = std::max(1, o.n_virtual_gpu);
     if (o.block_slots != 0 && !blk_slots_valid(o.block_slots)) return -1;
-    int S = 0;
-    if (choose_slots(o, 1, share_count(A->n, N, 0), &S) != GSOFA_OK) return -1;
-    const uint64_t nchunks = (share_count(A->n, N, 0) + S - 1) / S;
     uint64_t fc = o.output_capacity > 0 ? (uint64_t)o.output_capacity : default_fill_cap(A->nnz);
     if ((o.flags & GSOFA_FLAG_SPILL) && o.output_capacity <= 0)  // one share's fills at a time
         fc = std::max<uint64_t>(fc / (uint64_t)N, 1u << 20);
     int64_t cols = -1;  // default: room for nnz + fc entries
+    double skew = 0;
     if (o.output_capacity <= 0) {  // what plan creation reserves from the row bounds
         if (validate(A) != GSOFA_OK) return -1;
         std::vector<int32_t> rp, ci, rpT, ciT;
         pack_rows(A, rp, ci);
         transpose_rows(A->n, rp.data(), ci.data(), rpT, ciT);
         uint64_t nf = 0, nl = 0, nu = 0;
-        output_need(o, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu);
+        output_need(o, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu, 0, nullptr, nullptr,
+                    N > 1 ? &skew : nullptr);
         fc = std::max<uint64_t>(nf, 1);
         cols = (int64_t)(nl + nu);
     }
+    int S = 0;
+    if (choose_slots(o, 1, share_count(A->n, N, 0), &S, skew) != GSOFA_OK) return -1;
+    const uint64_t nchunks = (share_count(A->n, N, 0) + S - 1) / S;
     uint32_t nb = 0;
     if (block_grid(o, S, nchunks, (uint32_t)A->n, INT64_MAX / 4, &nb) != GSOFA_OK) return -1;
     return block_bytes(nb, (uint32_t)A->n, S) + block_fixed_bytes(A->n, A->nnz, 1, nchunks, fc, cols);
@@ -1190,6 +1212,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     // rows one execute processes (every share, one share, or for a spilled
     // run the largest share).
     uint64_t need_fill = 0, need_L = 0, need_U = 0, need_rec = 0;
+    double skew = 0;
     if (reach) {
         int bits = 0;
         rc = choose_bits(P->opt, n_mats, (uint64_t)n, &bits);
@@ -1202,7 +1225,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     }
     if (P->opt.output_capacity <= 0 && n > 0) {
         output_need(P->opt, n, P->h_rp.data(), ci.data(), rpT.data(), ciT.data(), &need_fill, &need_L, &need_U,
-                    P->rbits, &P->h_mat_base, &need_rec);
+                    P->rbits, &P->h_mat_base, &need_rec, !reach && P->opt.n_virtual_gpu > 1 ? &skew : nullptr);
         if (reach) need_fill = reach_reserve(need_fill, need_L + need_U, need_rec);
         const int64_t out_bytes = output_bytes(reach ? rch_fill_room(need_fill) : need_fill, need_L, need_U);
         if (out_bytes <= avail / 2) {
@@ -1302,7 +1325,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     } else if (P->mode == GSOFA_MODE_BLOCK) {
         int S = 0;
         const uint64_t nsrc = P->hybrid ? P->s_top : share_count(n, P->opt.n_virtual_gpu, 0);
-        rc = choose_slots(P->opt, n_mats, nsrc, &S);
+        rc = choose_slots(P->opt, n_mats, nsrc, &S, skew);
         P->S = (uint32_t)S;
         if (!rc) build_chunks(P);
         if (!rc) rc = size_block_mode(P, std::max<int64_t>(avail, 1 << 20));

@@ -4,8 +4,7 @@
 // (with_space_optimization/symbfact.cuh:883-1082) and seeding (:639-721), with
 // an execution model built for CDNA4:
 //
-// * Each workgroup (16 waves, one per CU) of a persistent grid owns SL source
-//   slots (32, 16 or 8; one kernel instance each) and runs a "mini-group" of
+// * Each workgroup (16 waves, one per CU) of a persistent grid owns //   slots (32, 16, 8, 4 or 2; one kernel instance each) and runs a "mini-group" of
 //   SL consecutive sources through all of their frontier levels by itself,
 //   synchronising only with __syncthreads.  The next mini-group comes from
 //   one global counter.  There is no grid-wide barrier and no hot global
@@ -86,11 +85,16 @@ constexpr uint32_t HOLE = 0xFFFFFFFFu;   // ent_m of an index that lost its inse
 // room for more targets.
 //   T  distinct targets per round, HB log2 of the hash slots (load <= 1/2),
 //   KR table entries relaxed together per lane group (<= SL),
-//   KV frontier vertices fetched together per lane group (<= SL).
+//   KV frontier vertices fetched together per lane group (<= SL),
+//   EPL edges of a row per lane: with 4 and 2 slots a step still takes 16.
+// With few slots the label lines of a workgroup stay in its XCD's L2 and a
+// vertex costs fewer cell updates: time goes as 8 + SL for the same vertices.
 template <int SL> struct Cfg;
-template <> struct Cfg<32> { static constexpr int T = 1024, HB = 11, KR = 16, KV = 4; };
-template <> struct Cfg<16> { static constexpr int T = 1792, HB = 12, KR = 16, KV = 4; };
-template <> struct Cfg<8> { static constexpr int T = 2048, HB = 12, KR = 8, KV = 4; };
+template <> struct Cfg<32> { static constexpr int T = 1024, HB = 11, KR = 16, KV = 4, EPL = 1; };
+template <> struct Cfg<16> { static constexpr int T = 1792, HB = 12, KR = 16, KV = 4, EPL = 1; };
+template <> struct Cfg<8> { static constexpr int T = 2048, HB = 12, KR = 8, KV = 4, EPL = 1; };
+template <> struct Cfg<4> { static constexpr int T = 3072, HB = 13, KR = 4, KV = 4, EPL = 4; };
+template <> struct Cfg<2> { static constexpr int T = 4096, HB = 13, KR = 2, KV = 2, EPL = 8; };
 
 template <int SL>
 struct Shape {
@@ -102,21 +106,26 @@ struct Shape {
     static constexpr int GPW = WAVE / SL;        // lane groups per wave
     static constexpr int NG = BW * GPW;          // lane groups per workgroup
     static constexpr uint32_t GM = SL == 32 ? 0xFFFFFFFFu : ((1u << SL) - 1u);  // a group's lanes
-    static_assert(SL == 8 || SL == 16 || SL == 32, "slots per workgroup");
+    static constexpr int EPL = Cfg<SL>::EPL;
+    static constexpr int EG = SL * EPL;          // edges of a row taken together
+    static constexpr uint32_t EM = EG == 32 ? 0xFFFFFFFFu : ((1u << EG) - 1u);
+    static_assert(SL == 2 || SL == 4 || SL == 8 || SL == 16 || SL == 32, "slots per workgroup");
     static_assert(KR <= SL && KV <= SL, "one entry / vertex per lane of a group");
+    static_assert(EG <= 32 && EG % 4 == 0, "edges fold in quads, their bits fill a word");
     static_assert(T <= H / 2, "hash load factor");
     static_assert(T % (GPW * KR) == 0, "relax batches tile the table");
-    static_assert((T + 1) * SL * 4 + H * 8 + T * 4 + NG * SL * 4 + 1024 <= 160 * 1024, "LDS of one CU");
+    static_assert((T + GPW) * SL * 4 + H * 8 + T * 4 + NG * EG * 4 + 1024 <= 160 * 1024, "LDS of one CU");
 };
 
 template <int SL>
 struct BlkLds {
     using Z = Shape<SL>;
-    uint32_t cell[Z::T + 1][SL];         // min cost per (round target, slot); INF = none.  Row T
-                                         // is a sink for the padding of edge quads, never read
+    uint32_t cell[Z::T + Z::GPW][SL];    // min cost per (round target, slot); INF = none.  Rows T ..
+                                         // take the padding of edge quads, one row for each lane
+                                         // group of a wave (distinct banks), never read
     unsigned long long hkey[Z::H];       // ((m + 1) << 32) | table index; 0 = empty
     uint32_t ent_m[Z::T];                // table index -> target (window-local) or HOLE
-    uint4 eidx[Z::NG][SL / 4];           // table index of each lane's edge (SL per group)
+    uint4 eidx[Z::NG][Z::EG / 4];        // table index of each edge of a lane group's row
     unsigned long long s_te[SL];         // per-slot TE of the current mini-group
     unsigned long long s_reach[SL];      // per-slot |R_<(s)|
     unsigned long long s_fill[SL];       // per-slot fills
@@ -223,9 +232,8 @@ __device__ __forceinline__ uint32_t from_lane(uint32_t x, uint32_t u) {
 // ballot bits, as a wave-uniform count.
 template <int SL>
 __device__ __forceinline__ uint32_t wave_top(uint64_t m) {
-    if constexpr (SL <= 16) m |= m >> 32;
-    if constexpr (SL <= 8) m |= m >> 16;
-    m |= m >> SL;
+#pragma unroll
+    for (int k = WAVE / 2; k >= SL; k /= 2) m |= m >> k;
     const uint32_t g = (uint32_t)m & Shape<SL>::GM;
     return g ? 32u - (uint32_t)__builtin_clz(g) : 0u;
 }
@@ -238,31 +246,31 @@ __device__ __forceinline__ uint32_t grp_ballot(bool x, uint32_t grp) {
 
 // Frontier vertices held by a lane group across rounds.  Lane k of the group
 // keeps vertex k's CSR cursor (pos, end) and its pending-edge mask for the
-// current SL-edge group; lane j keeps slot j's cost of every vertex and the
-// j-th edge target of its current group.
-template <int KV>
+// current group of EG = SL * EPL edges; lane j keeps slot j's cost of every
+// vertex and edges j, SL + j, ... of its current group.
+template <int KV, int EPL>
 struct GrpVtx {
     bool held;           // group-uniform: a batch is in progress
     bool done;           // group-uniform: the queue is exhausted for this level
     int32_t pos, end;    // lane k: vertex k's current group start, row end
     uint32_t pend;       // lane k: vertex k's edges of the group not yet folded
     uint32_t cost[KV];   // lane j: max(v_u + off, label_j(v_u)), INF if j not in v_u's mask
-    uint32_t civ[KV];    // lane j: target of edge j of v_u's current group (window-local)
+    uint32_t civ[KV][EPL];  // lane j: targets of edges i * SL + j of v_u's current group (window-local)
 };
 
 template <int SL>
 __device__ __forceinline__ uint32_t group_mask(int32_t left) {
-    return left >= SL ? Shape<SL>::GM : (left <= 0 ? 0u : ((1u << left) - 1u));
+    return left >= Shape<SL>::EG ? Shape<SL>::EM : (left <= 0 ? 0u : ((1u << left) - 1u));
 }
 
 // Phase A: pop frontier vertices (KV per lane group) and fold their edges'
 // costs into the table until the queue is exhausted or the table is full.
 // Wave-uniform control flow; the lane groups carry independent batches.
 template <int SL>
-__device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV>& hv, uint32_t cur,
+__device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV, Shape<SL>::EPL>& hv, uint32_t cur,
                               uint32_t size, TallyB& t) {
     using Z = Shape<SL>;
-    constexpr int KV = Z::KV;
+    constexpr int KV = Z::KV, EPL = Z::EPL, EG = Z::EG;
     const BlkParams& p = *B.p;
     const uint32_t lane = __lane_id();
     const uint32_t grp = lane / SL;
@@ -275,7 +283,11 @@ __device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV>
         for (int u = 0; u < KV; u++) {
             const uint32_t pu = from_lane<SL>(hv.pend, u);
             const int32_t pos = (int32_t)from_lane<SL>((uint32_t)hv.pos, u);
-            hv.civ[u] = ((pu >> j) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)j) << 2) - B.wb : 0u;
+#pragma unroll
+            for (int i = 0; i < EPL; i++) {
+                const uint32_t k = i * SL + j;
+                hv.civ[u][i] = ((pu >> k) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)k) << 2) - B.wb : 0u;
+            }
         }
     }
     for (;;) {
@@ -307,7 +319,11 @@ __device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV>
                 const int32_t pos = (int32_t)from_lane<SL>((uint32_t)hv.pos, u);
                 lv[u] = 0u;
                 if (fresh && vu != NONE) lv[u] = at(B.lab0, (vu * SL + j) << 2);
-                if (fresh) hv.civ[u] = ((pu >> j) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)j) << 2) - B.wb : 0u;
+#pragma unroll
+                for (int i = 0; i < EPL; i++) {
+                    const uint32_t k = i * SL + j;
+                    if (fresh) hv.civ[u][i] = ((pu >> k) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)k) << 2) - B.wb : 0u;
+                }
             }
             if (mine) {
                 at(maskc, q.x << 2) = 0u;  // consumed; this buffer is refilled two levels later
@@ -327,22 +343,27 @@ __device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV>
         // -- fold the held vertices' edges, vertex by vertex.  Bit k of each
         // group's share of longm: vertex k's row has more edge groups after
         // the current one (rare), so only those read back pos and end.
-        const uint64_t longm = __ballot(hv.held && j < (uint32_t)KV && hv.pos + SL < hv.end);
+        const uint64_t longm = __ballot(hv.held && j < (uint32_t)KV && hv.pos + EG < hv.end);
         bool full = false;
 #pragma unroll
         for (int u = 0; u < KV; u++) {
             uint32_t pu = hv.held ? from_lane<SL>(hv.pend, u) : 0u;
             while (pu) {  // group-uniform
-                const bool mine = (pu >> j) & 1u;
-                uint32_t idx = NONE;
-                if (mine) idx = tab_find<SL>(S, &S.tcnt[B.rb], hv.civ[u]);
-                const bool placed = mine && idx != FULL;
-                // unplaced edges (past the row end, or the table is full) fold
-                // into the sink row, so every group folds whole quads
-                reinterpret_cast<uint32_t*>(S.eidx[h])[j] = placed ? idx : (uint32_t)Z::T;
-                const uint64_t wm = __ballot(placed);
-                const uint32_t okm = (uint32_t)(wm >> (SL * grp)) & Z::GM;
-                const uint32_t nq = (wave_top<SL>(wm) + 3u) >> 2;  // wave-uniform
+                uint32_t okm = 0, top = 0;
+#pragma unroll
+                for (int i = 0; i < EPL; i++) {
+                    const bool mine = (pu >> (i * SL + j)) & 1u;
+                    uint32_t idx = NONE;
+                    if (mine) idx = tab_find<SL>(S, &S.tcnt[B.rb], hv.civ[u][i]);
+                    const bool placed = mine && idx != FULL;
+                    // unplaced edges (past the row end, or the table is full) fold
+                    // into the sink row, so every group folds whole quads
+                    reinterpret_cast<uint32_t*>(S.eidx[h])[i * SL + j] = placed ? idx : (uint32_t)Z::T + grp;
+                    const uint64_t wm = __ballot(placed);
+                    okm |= ((uint32_t)(wm >> (SL * grp)) & Z::GM) << (i * SL);
+                    if (wm) top = i * SL + wave_top<SL>(wm);
+                }
+                const uint32_t nq = (top + 3u) >> 2;  // wave-uniform
                 wave_sync();
                 if (hv.cost[u] != INF) {
                     const uint32_t cu = hv.cost[u];
@@ -365,11 +386,15 @@ __device__ void combine_phase(const Blk& B, BlkLds<SL>& S, GrpVtx<Shape<SL>::KV>
                 if ((longm >> (SL * grp + u)) & 1u) {  // group-uniform
                     int32_t pos = (int32_t)from_lane<SL>((uint32_t)hv.pos, u);
                     const int32_t end = (int32_t)from_lane<SL>((uint32_t)hv.end, u);
-                    if (pos + SL < end) {
-                        pos += SL;
+                    if (pos + EG < end) {
+                        pos += EG;
                         pu = group_mask<SL>(end - pos);
                         if (j == (uint32_t)u) hv.pos = pos;
-                        hv.civ[u] = ((pu >> j) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)j) << 2) - B.wb : 0u;
+#pragma unroll
+                        for (int i = 0; i < EPL; i++) {
+                            const uint32_t k = i * SL + j;
+                            hv.civ[u][i] = ((pu >> k) & 1u) ? at(p.ci, (uint32_t)(pos + (int32_t)k) << 2) - B.wb : 0u;
+                        }
                     }
                 }
             }
@@ -506,7 +531,7 @@ __global__ __launch_bounds__(BB) __attribute__((amdgpu_waves_per_eu(GSOFA_WPE, G
     uint32_t since = p.bstate[2 * blockIdx.x + 1];
     TallyB t{0, 0, 0, 0};
     unsigned long long levels = 0;
-    for (uint32_t i = tid; i < (uint32_t)((Z::T + 1) * SL); i += BB) (&S.cell[0][0])[i] = INF;
+    for (uint32_t i = tid; i < (uint32_t)((Z::T + Z::GPW) * SL); i += BB) (&S.cell[0][0])[i] = INF;
     for (uint32_t i = tid; i < (uint32_t)Z::H; i += BB) S.hkey[i] = 0ull;
     if (tid < 4) S.acc[tid] = 0;
     if (tid == 0) {
@@ -591,7 +616,7 @@ __global__ __launch_bounds__(BB) __attribute__((amdgpu_waves_per_eu(GSOFA_WPE, G
             __syncthreads();  // every thread has the size before it can change
             if (size == 0) break;
             const uint32_t nbuf = cur ^ 1u;
-            GrpVtx<Z::KV> hv;
+            GrpVtx<Z::KV, Z::EPL> hv;
             hv.held = false;
             hv.done = false;
             hv.pend = 0u;
@@ -656,11 +681,14 @@ __global__ __launch_bounds__(BB) __attribute__((amdgpu_waves_per_eu(GSOFA_WPE, G
 }  // namespace
 
 bool blk_slots_valid(int slots) { return slots == 32 || slots == 16 || slots == 8; }
+bool blk_slots_built(int slots) { return blk_slots_valid(slots) || slots == 4 || slots == 2; }
 int blk_block_size() { return BB; }
 const void* blk_kernel_ptr(int slots) {
     switch (slots) {
         case 16: return reinterpret_cast<const void*>(&k_traverse_blk<16>);
         case 8: return reinterpret_cast<const void*>(&k_traverse_blk<8>);
+        case 4: return reinterpret_cast<const void*>(&k_traverse_blk<4>);
+        case 2: return reinterpret_cast<const void*>(&k_traverse_blk<2>);
         default: return reinterpret_cast<const void*>(&k_traverse_blk<32>);
     }
 }
@@ -670,6 +698,8 @@ hipError_t launch_traverse_blk(const BlkParams& p, int slots, size_t lds_bytes, 
         case 32: hipLaunchKernelGGL(k_traverse_blk<32>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
         case 16: hipLaunchKernelGGL(k_traverse_blk<16>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
         case 8: hipLaunchKernelGGL(k_traverse_blk<8>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
+        case 4: hipLaunchKernelGGL(k_traverse_blk<4>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
+        case 2: hipLaunchKernelGGL(k_traverse_blk<2>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

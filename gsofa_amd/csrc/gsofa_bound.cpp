@@ -176,4 +176,20 @@ uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::ve
     return sum * (uint64_t)(bits > 64 ? bits / 64 : 1);
 }
 
+// Of the sources gid, gid + N, ...: the largest subtree of the elimination tree
+// (all that a source can reach below itself) over their mean.
+double subtree_skew(int32_t N, int32_t gid, const std::vector<int32_t>& parent) {
+    const int32_t n = (int32_t)parent.size();
+    std::vector<int32_t> below((size_t)n, 1);
+    for (int32_t i = 0; i < n; i++)
+        if (parent[(size_t)i] >= 0) below[(size_t)parent[(size_t)i]] += below[(size_t)i];
+    double sum = 0, most = 0;
+    int64_t count = 0;
+    for (int64_t i = gid; i < n; i += N, count++) {
+        sum += below[(size_t)i];
+        most = std::max<double>(most, below[(size_t)i]);
+    }
+    return sum > 0 ? most * (double)count / sum : 1;
+}
+
 }  // namespace gsofa

@@ -63,6 +63,7 @@ int validate_matrix(const gsofa_matrix* A);
 // packed rows of A and A^T, sorted and duplicate-free.
 void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT, const int32_t* ciT,
                    std::vector<int64_t>& Lb, std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out = nullptr);
+double subtree_skew(int32_t N, int32_t gid, const std::vector<int32_t>& parent);
 uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
                             const std::vector<int64_t>& Ub, int bits);
 
@@ -104,7 +105,8 @@ struct BlkParams {
 };
 int blk_block_size();
 bool blk_slots_valid(int slots);
-int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots);
+bool blk_slots_built(int slots);
+int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots, double skew = 0);
 // Block-mode sizing shared by plan creation, footprints and the server.
 int64_t block_bytes(uint32_t nb, uint32_t W, int slots);
 // cols: L + U column entries reserved (sorted + staging, 8 B each); < 0 means
