@@ -7,11 +7,16 @@
 //   small totals (a matrix of thousands of rows) by one kernel between the
 //     arrays and one pinned buffer: the fetch of a 16 x 16 grid 160 -> 17 us,
 //     its upload 60 -> 19;
-//   the rest in chunks of at most 4 MB, each with its DMA in flight while the
-//     thread copies the previous one out.  A single thread that first touches
-//     the destination moves 14 GB/s, so larger totals take up to kThreads
-//     threads: 55 MB (33^3 grid) 9.5 -> 3.4 ms, 1.0 GB (48^3) 22.2 -> 18.9 ms
-//     (54 GB/s of the link's 57).  16 MB buffers instead of 4: 6.8 and 26 ms.
+//   the rest in chunks of at most 4 MB, each moved by a kernel while the thread
+//     copies the previous one out.  (A copy of the runtime's is a kernel too,
+//     but 10 us apart from the next and one for each array.)  A single thread
+//     that first touches the destination moves 14 GB/s, so larger totals take
+//     up to kThreads threads.
+// Fetch us by pageable copies / this with the runtime's copies / with kernels:
+// 64 x 64 grid (2.2 MB) 230 / 250 / 97; band of 11,948 (9.9 MB) 2230 / 900 /
+// 310; 27^3 grid (49 MB) 4170 / 1570 / 1290; 33^3 (127 MB) 9490 / 3300 / 2900;
+// 48^3 (874 MB) 22200 / 18900 / 17200, 51 GB/s of the link's 57.  16 MB buffers
+// instead of 4: 33^3 6.8 ms; 1 MB a thread instead of 2: 64 x 64 128 us.
 // Result arrays start on 2 MB boundaries with transparent huge pages requested,
 // since their first touch is in this path.
 #include <algorithm>
@@ -35,9 +40,10 @@ constexpr size_t kStageKeep = 64;          // idle staging buffers kept: four co
 constexpr size_t kStageRest = 16;          // and after the last plan's release, one copy's (64 MB:
                                            // making and releasing them takes over 1 ms)
 constexpr size_t kKernelMost = 512u << 10; // totals up to here: one kernel
-constexpr size_t kPerThread = 1u << 20;    // bytes per copy thread, at least
+constexpr size_t kPerThread = 2u << 20;     // bytes per copy thread, at least
 constexpr int kThreads = 8;
-constexpr size_t kChunkMin = 256u << 10;
+constexpr size_t kChunkMin = 1u << 20;
+constexpr size_t kChunks = 4;              // chunks a thread, at least
 constexpr size_t kHugePage = 2u << 20;
 constexpr size_t kHugeMin = 1u << 20;
 
@@ -91,14 +97,43 @@ struct Pieces {
     int count;
 };
 
-__global__ void k_copy_pieces(Pieces p) {
+// Pieces whose two ends have the same alignment to 16 bytes move in 16-byte
+// words but for their ends, the others word by word.
+__global__ __launch_bounds__(256) void k_copy_pieces(Pieces p) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
-    for (int k = 0; k < p.count; k++)
-        for (uint32_t i = t; i < p.words[k]; i += step) p.dst[k][i] = p.src[k][i];
+    for (int k = 0; k < p.count; k++) {
+        uint32_t* d = p.dst[k];
+        const uint32_t* s = p.src[k];
+        const uint32_t n = p.words[k];
+        const uint32_t off = (uint32_t)(reinterpret_cast<uintptr_t>(d) >> 2) & 3u;
+        uint32_t head = n, body = 0;
+        if (((reinterpret_cast<uintptr_t>(d) ^ reinterpret_cast<uintptr_t>(s)) & 15u) == 0) {
+            head = (4u - off) & 3u;
+            head = head < n ? head : n;
+            body = (n - head) / 4u;
+        }
+        uint4* d4 = reinterpret_cast<uint4*>(d + head);
+        const uint4* s4 = reinterpret_cast<const uint4*>(s + head);
+        for (uint32_t i = t; i < body; i += step) d4[i] = s4[i];
+        for (uint32_t i = t; i < head; i += step) d[i] = s[i];
+        for (uint32_t i = head + 4u * body + t; i < n; i += step) d[i] = s[i];
+    }
+}
+
+hipError_t launch_pieces(const Pieces& p, size_t bytes, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)std::min<size_t>((bytes / 16 + 255) / 256, 512);
+    hipLaunchKernelGGL(k_copy_pieces, dim3(std::max(blocks, 1u)), dim3(256), 0, s, p);
+    return hipGetLastError();
 }
 
 struct Chunk {
-    size_t first, count;  // pieces
+    size_t first, count;  // pieces, at most Pieces::MAX
+};
+struct Piece {
+    char* host;
+    char* dev;
+    size_t bytes;
+    size_t off;  // in the chunk's buffer: aligned to 16 bytes as dev is
 };
 
 // `out`: device to host, else host to device.
@@ -113,9 +148,7 @@ hipError_t copy_small(const std::vector<HostCopy>& v, bool out, char* stage, hip
         p.words[p.count++] = (uint32_t)(c.bytes / 4);
         off += (c.bytes + 15) & ~(size_t)15;
     }
-    const uint32_t blocks = (uint32_t)std::min<size_t>((total / 4 + 255) / 256, 512);
-    hipLaunchKernelGGL(k_copy_pieces, dim3(std::max(blocks, 1u)), dim3(256), 0, s, p);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_pieces(p, total, s);
     const hipError_t w = hipStreamSynchronize(s);  // in either case: nothing may still use the buffer
     if (e == hipSuccess) e = w;
     if (e != hipSuccess || !out) return e;
@@ -127,7 +160,7 @@ hipError_t copy_small(const std::vector<HostCopy>& v, bool out, char* stage, hip
     return hipSuccess;
 }
 
-hipError_t copy_chunks(const std::vector<HostCopy>& pieces, const std::vector<Chunk>& chunks, bool out,
+hipError_t copy_chunks(const std::vector<Piece>& pieces, const std::vector<Chunk>& chunks, bool out,
                        hipStream_t s, std::atomic<size_t>& next, void* b0, void* b1, int device) {
     (void)hipSetDevice(device);
     char* buf[2] = {(char*)b0, (char*)b1};
@@ -135,24 +168,26 @@ hipError_t copy_chunks(const std::vector<HostCopy>& pieces, const std::vector<Ch
     hipError_t e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
     auto host_side = [&](size_t k, char* b) {
-        size_t off = 0;
         for (size_t i = chunks[k].first; i < chunks[k].first + chunks[k].count; i++) {
-            const HostCopy& c = pieces[i];
-            if (out) std::memcpy(c.host, b + off, c.bytes);
-            else std::memcpy(b + off, c.host, c.bytes);
-            off += c.bytes;
+            const Piece& c = pieces[i];
+            if (out) std::memcpy(c.host, b + c.off, c.bytes);
+            else std::memcpy(b + c.off, c.host, c.bytes);
         }
     };
     auto dma = [&](size_t k, char* b, hipEvent_t x) {
-        size_t off = 0;
+        Pieces p{};
+        size_t bytes = 0;
         for (size_t i = chunks[k].first; i < chunks[k].first + chunks[k].count; i++) {
-            const HostCopy& c = pieces[i];
-            const hipError_t r = out ? hipMemcpyAsync(b + off, c.dev, c.bytes, hipMemcpyDeviceToHost, s)
-                                     : hipMemcpyAsync(c.dev, b + off, c.bytes, hipMemcpyHostToDevice, s);
-            if (r != hipSuccess) return r;
-            off += c.bytes;
+            const Piece& c = pieces[i];
+            uint32_t* st = reinterpret_cast<uint32_t*>(b + c.off);
+            uint32_t* dv = reinterpret_cast<uint32_t*>(c.dev);
+            p.dst[p.count] = out ? st : dv;
+            p.src[p.count] = out ? dv : st;
+            p.words[p.count++] = (uint32_t)(c.bytes / 4);
+            bytes += c.bytes;
         }
-        return hipEventRecord(x, s);
+        const hipError_t r = launch_pieces(p, bytes, s);
+        return r != hipSuccess ? r : hipEventRecord(x, s);
     };
     const size_t none = ~(size_t)0;
     size_t have[2] = {none, none};
@@ -214,20 +249,22 @@ hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
         const hipError_t w = hipStreamSynchronize(s);
         return e == hipSuccess ? w : e;
     }
-    const size_t ch = std::min(kStageBytes, std::max(kChunkMin, total / (4 * (size_t)threads)));
-    std::vector<HostCopy> pieces;
+    const size_t ch = std::min(kStageBytes, std::max(kChunkMin, total / (kChunks * (size_t)threads)));
+    std::vector<Piece> pieces;
     std::vector<Chunk> chunks;
-    size_t room = 0;
+    size_t at = ch;  // bytes of the last chunk's buffer in use
     for (const HostCopy& c : v)
         for (size_t o = 0; o < c.bytes;) {
-            if (room == 0) {
+            char* dev = (char*)c.dev + o;
+            size_t off = ((at + 15) & ~(size_t)15) + ((uintptr_t)dev & 15u);
+            if (off + 4 > ch || chunks.back().count == (size_t)Pieces::MAX) {
                 chunks.push_back({pieces.size(), 0});
-                room = ch;
+                off = (uintptr_t)dev & 15u;
             }
-            const size_t len = std::min(room, c.bytes - o);
-            pieces.push_back({(char*)c.host + o, (char*)c.dev + o, len});
+            const size_t len = std::min((ch - off) & ~(size_t)3, c.bytes - o);
+            pieces.push_back({(char*)c.host + o, dev, len, off});
             chunks.back().count++;
-            room -= len;
+            at = off + len;
             o += len;
         }
     int device = 0;
