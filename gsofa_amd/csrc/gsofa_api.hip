@@ -2367,28 +2367,51 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
     if (trc) return trc;
     const int32_t ns = n > 0 ? P->n_super : 0;
     h->n_super = ns;
-    DevScratch T;  // device scratch for this call only
-    int64_t *d_xl = nullptr, *d_xu = nullptr, *d_xs = nullptr;
-    int32_t *d_lrow = nullptr, *d_urow = nullptr;
-    if (T.get(&d_xl, (size_t)n + 1) || T.get(&d_xu, (size_t)n + 1) || T.get(&d_xs, (size_t)ns + 1) ||
-        T.get(&d_lrow, (size_t)P->nnzL) || T.get(&d_urow, (size_t)P->nnzU))
-        return GSOFA_ERR_ALLOC;
-    // L and U by columns; the staging arrays of the structure pass are free now
-    int32_t *t_l = P->d_Ltmp, *t_u = P->d_Utmp;
-    if ((!t_l && T.get(&t_l, (size_t)P->nnzL)) || (!t_u && T.get(&t_u, (size_t)P->nnzU))) return GSOFA_ERR_ALLOC;
-    HIPCHK_OUT(transpose_structure(P->d_Lrp, P->d_Lcol, P->nnzL, n, P->d_cntL, d_xl, P->d_scan, t_l, d_lrow,
-                                   P->stream), P->stream);
-    HIPCHK_OUT(transpose_structure(P->d_Urp, P->d_Ucol, P->nnzU, n, P->d_cntU, d_xu, P->d_scan, t_u, d_urow,
-                                   P->stream), P->stream);
-    // supernode subscripts
-    int64_t nsub = 0;
-    int32_t* d_sub = nullptr;
+    // device scratch for this call only, in two pieces: what the subscripts'
+    // number takes, then the rest
+    DevScratch T;
+    int64_t *d_xl = nullptr, *d_xu = nullptr, *d_xs = nullptr, nsub = 0;
+    if (T.get(&d_xs, (size_t)ns + 1)) return GSOFA_ERR_ALLOC;
     if (ns > 0) {
         HIPCHK_OUT(supernode_sub_count(P->d_sstart, ns, P->d_Urp, P->d_cntL, P->stream), P->stream);
         HIPCHK_OUT(exclusive_scan_u32_to_i64(P->d_cntL, d_xs, ns, P->d_scan, P->stream), P->stream);
         HIPCHK_OUT(copy_out({{&nsub, d_xs + ns, sizeof(int64_t)}}, P->stream), P->stream);
-        if (T.get(&d_sub, (size_t)nsub)) return GSOFA_ERR_ALLOC;
+    }
+    // a reach-mode run's records give the columns as they gave the rows
+    const bool records = P->mode == GSOFA_MODE_REACH && n > 0;
+    const bool staged = !records && (!P->d_Ltmp || !P->d_Utmp);  // the structure pass left no staging arrays
+    const size_t nl = (size_t)P->nnzL, nu = (size_t)P->nnzU;
+    int32_t* mem = nullptr;
+    if (T.get(&mem, 4 * ((size_t)n + 1) + (nl + nu) * (staged ? 2 : 1) + (size_t)nsub)) return GSOFA_ERR_ALLOC;
+    d_xl = reinterpret_cast<int64_t*>(mem);
+    d_xu = d_xl + n + 1;
+    int32_t* const d_lrow = reinterpret_cast<int32_t*>(d_xu + n + 1);
+    int32_t* const d_urow = d_lrow + nl;
+    int32_t* const d_sub = d_urow + nu;
+    if (ns > 0)
         HIPCHK_OUT(supernode_sub_write(P->d_sstart, ns, P->d_Urp, P->d_Ucol, d_xs, d_sub, P->stream), P->stream);
+    if (records) {
+        RowParams r = row_params(P);
+        r.row_fill = nullptr;
+        r.ctrl = nullptr;
+        r.L_rowptr = d_xu;
+        r.L_col = d_urow;
+        r.L_cap = P->nnzU;
+        r.U_rowptr = d_xl;
+        r.U_col = d_lrow;
+        r.U_cap = P->nnzL;
+        ZeroSpans z{};
+        z.add(r.cntL, sizeof(unsigned long long) * (uint64_t)n);
+        z.add(r.long_count, sizeof(uint32_t));
+        HIPCHK_OUT(launch_zero(z, P->stream), P->stream);
+        HIPCHK_OUT(launch_columns(r, P->d_cntU, P->stream), P->stream);
+    } else {
+        int32_t* const t_l = staged ? d_sub + nsub : P->d_Ltmp;
+        int32_t* const t_u = staged ? t_l + nl : P->d_Utmp;
+        HIPCHK_OUT(transpose_structure(P->d_Lrp, P->d_Lcol, P->nnzL, n, P->d_cntL, d_xl, P->d_scan, t_l, d_lrow,
+                                       P->stream), P->stream);
+        HIPCHK_OUT(transpose_structure(P->d_Urp, P->d_Ucol, P->nnzU, n, P->d_cntU, d_xu, P->d_scan, t_u, d_urow,
+                                       P->stream), P->stream);
     }
     h->xsup = (int32_t*)malloc(sizeof(int32_t) * ((size_t)ns + 1));
     h->supno = (int32_t*)malloc(sizeof(int32_t) * std::max<size_t>((size_t)n, 1));

@@ -319,14 +319,14 @@ struct RowParams {
     const uint4* grp;
     const uint32_t* cntU;
     unsigned long long* cntL;
-    int64_t* row_fill;
+    int64_t* row_fill;     // null: columns
     int64_t* sums;         // row_sum_words(n) (null: counts only)
     int64_t* L_rowptr;
     int64_t* U_rowptr;
     int64_t* R_ptr;        // n + 1: offsets of the rows' record lists
     uint4* list;           // the lists
     int64_t list_cap;
-    Ctrl* ctrl;            // nnz_L and nnz_U go there
+    Ctrl* ctrl;            // nnz_L and nnz_U go there, unless null
     uint32_t* long_rows;   // n: rows of over 64 records
     uint32_t* long_count;  // zero on entry
     int32_t* L_col;
@@ -337,6 +337,7 @@ size_t row_sum_words(int64_t n);
 hipError_t launch_row_fills(const RowParams& p, hipStream_t s);
 hipError_t launch_row_ptrs(const RowParams& p, hipStream_t s);
 hipError_t launch_rows(const RowParams& p, hipStream_t s);
+hipError_t launch_columns(const RowParams& p, uint32_t* cnt_l, hipStream_t s);
 
 struct FinalParams {
     int32_t n;
