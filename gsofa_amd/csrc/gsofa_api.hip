@@ -356,17 +356,18 @@ uint64_t label_words(int32_t n, int32_t N, int32_t C, int32_t gid_lo, int32_t gi
 // Output one execute needs at most, from the row bounds of lu_row_bounds:
 // fills, L and U entries of the rows it processes (every share, one share, or
 // for a spilled run the largest share).  rp/ci: packed rows.  bits > 0 (reach
-// mode): also the records of one pass, for groups of so many sources.  skew: also
+// mode): also the records of one pass, for groups of so many sources, and the
+// largest group (reach_record_bound).  skew: also
 // the share's subtree_skew.
 void output_need(const gsofa_options& o, int32_t n, const int32_t* rp, const int32_t* ci, const int32_t* rpT,
                  const int32_t* ciT, uint64_t* need_fill, uint64_t* need_L, uint64_t* need_U, int bits = 0,
                  const std::vector<uint32_t>* mat_base = nullptr, uint64_t* need_rec = nullptr,
-                 double* skew = nullptr) {
+                 double* skew = nullptr, uint64_t* largest = nullptr) {
     std::vector<int64_t> Lb, Ub;
     std::vector<int32_t> parent;
     lu_row_bounds(n, rp, ci, rpT, ciT, Lb, Ub, bits || skew ? &parent : nullptr);
     if (skew) *skew = subtree_skew(std::max(1, o.n_virtual_gpu), std::max(0, o.virtual_gpu_id), parent);
-    if (bits) *need_rec = reach_record_bound(*mat_base, parent, Ub, bits);
+    if (bits) *need_rec = reach_record_bound(*mat_base, parent, Ub, bits, largest);
     const int32_t N = std::max(1, o.n_virtual_gpu);
     std::vector<uint64_t> fs((size_t)N, 0), ls((size_t)N, 0), us((size_t)N, 0);
     for (int32_t i = 0; i < n; i++) {
@@ -995,8 +996,9 @@ int reach_resident(int device, int threads, uint32_t* out) {
 }
 
 // As block_grid, for the reach kernel's per-workgroup arrays; also the
-// workgroup shape.  records: of one pass, at most (0: unknown).
-int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint32_t W, int64_t avail,
+// workgroup shape.  records: of one pass, at most (0: unknown);
+// largest: the largest group.
+int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint64_t largest, uint32_t W, int64_t avail,
                uint32_t* nb_out, int* threads_out) {
     if (o.workgroup_threads != 0 && !rch_threads_valid(o.workgroup_threads)) return GSOFA_ERR_INVALID;
     if (o.mem_budget_bytes > 0) avail = std::min<int64_t>(avail, o.mem_budget_bytes);
@@ -1008,7 +1010,7 @@ int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t reco
             return GSOFA_ERR_HIP;
         }
         const uint64_t groups = std::max<uint64_t>(nchunks / 2, 1) * (uint64_t)std::max(bits / 64, 1);
-        threads = reach_shape(nchunks, records ? records / groups : UINT64_MAX, W, bits, (uint32_t)cus, avail);
+        threads = reach_shape(nchunks, records ? records / groups : UINT64_MAX, largest, W, bits, (uint32_t)cus, avail);
     }
     *threads_out = threads;
     uint32_t nb = 0;
@@ -1095,12 +1097,13 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         w.n_virtual_gpu = 1;
         w.virtual_gpu_id = -1;
         const std::vector<uint32_t> mb{0u, (uint32_t)A->n};
-        uint64_t nr = 0;
-        output_need(w, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu, bits, &mb, &nr);
+        uint64_t nr = 0, largest = 0;
+        output_need(w, A->n, rp.data(), ci.data(), rpT.data(), ciT.data(), &nf, &nl, &nu, bits, &mb, &nr, nullptr,
+                    &largest);
         nf = reach_reserve(nf, nl + nu, nr);
         uint32_t nb = 0;
         int threads = 0;
-        if (reach_grid(o, bits, 2 * nchunks, nr, (uint32_t)A->n, INT64_MAX / 4, &nb, &threads) != GSOFA_OK) return -1;
+        if (reach_grid(o, bits, 2 * nchunks, nr, largest, (uint32_t)A->n, INT64_MAX / 4, &nb, &threads) != GSOFA_OK) return -1;
         const uint32_t ql = quot_wanted(A->n, (int64_t)ci.size(), (uint32_t)A->n,
                                         o.mem_budget_bytes > 0 ? o.mem_budget_bytes : INT64_MAX / 4);
         return reach_bytes(nb, (uint32_t)A->n, bits) +
@@ -1211,7 +1214,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     // Output reserve from the row bounds: the fills, L and U entries of the
     // rows one execute processes (every share, one share, or for a spilled
     // run the largest share).
-    uint64_t need_fill = 0, need_L = 0, need_U = 0, need_rec = 0;
+    uint64_t need_fill = 0, need_L = 0, need_U = 0, need_rec = 0, largest = 0;
     double skew = 0;
     if (reach) {
         int bits = 0;
@@ -1225,7 +1228,8 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     }
     if (P->opt.output_capacity <= 0 && n > 0) {
         output_need(P->opt, n, P->h_rp.data(), ci.data(), rpT.data(), ciT.data(), &need_fill, &need_L, &need_U,
-                    P->rbits, &P->h_mat_base, &need_rec, !reach && P->opt.n_virtual_gpu > 1 ? &skew : nullptr);
+                    P->rbits, &P->h_mat_base, &need_rec, !reach && P->opt.n_virtual_gpu > 1 ? &skew : nullptr,
+                    &largest);
         if (reach) need_fill = reach_reserve(need_fill, need_L + need_U, need_rec);
         const int64_t out_bytes = output_bytes(reach ? rch_fill_room(need_fill) : need_fill, need_L, need_U);
         if (out_bytes <= avail / 2) {
@@ -1298,7 +1302,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room);
             const int64_t qb = qlev ? quot_bytes(n, P->nnz, P->W) : 0;
             if (go.mem_budget_bytes > 0) go.mem_budget_bytes -= qb;
-            rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), need_rec, P->W, room - qb, &P->nblocks,
+            rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), need_rec, largest, P->W, room - qb, &P->nblocks,
                             &P->rthreads);
         }
         if (rc) {
@@ -2507,7 +2511,7 @@ int pack_matrix(const gsofa_matrix* A, PackedMatrix* M) {
     gsofa_options_default(&o);
     const std::vector<uint32_t> mb{0u, (uint32_t)M->n};
     output_need(o, M->n, M->rp.data(), M->ci.data(), M->rpT.data(), M->ciT.data(), &M->need_fill, &M->need_L, &M->need_U, kArenaBits, &mb,
-                &M->need_rec);
+                &M->need_rec, nullptr, &M->largest);
     M->need_fill = reach_reserve(M->need_fill, M->need_L + M->need_U, M->need_rec);
     return GSOFA_OK;
 }
@@ -2554,9 +2558,10 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     HIPCHK(hipSetDevice(P->device));
     int64_t n = 0, nnz = 0;
     uint32_t W = 1;
-    uint64_t nf = 0, nl = 0, nu = 0, nr = 0;
+    uint64_t nf = 0, nl = 0, nu = 0, nr = 0, largest = 0;
     for (int32_t b = 0; b < count; b++) {
         nr += mats[b]->need_rec;
+        largest = std::max(largest, mats[b]->largest);
         n += mats[b]->n;
         nnz += mats[b]->nnz;
         W = std::max<uint32_t>(W, (uint32_t)mats[b]->n);
@@ -2621,7 +2626,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     o.mem_budget_bytes = 0;
     const uint32_t qlev = quot_wanted(n, nnz, W, budget - fixed);
     const int64_t qb = qlev ? quot_bytes(n, nnz, W) : 0;
-    int rc = reach_grid(o, bits, nchunks, nr, W, budget - fixed - qb, &nb, &P->rthreads);
+    int rc = reach_grid(o, bits, nchunks, nr, largest, W, budget - fixed - qb, &nb, &P->rthreads);
     if (rc) return rc;
     gsofa_plan::Caps& c = P->cap;
     const size_t rows = (size_t)n + 1;

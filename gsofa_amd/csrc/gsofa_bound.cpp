@@ -160,16 +160,23 @@ void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, const int32_
 // itself; groups are cut from each matrix's last vertex down).  A source's
 // vertices above it lie in its column of C, and a column's entries but the
 // parent lie in the parent's column, so a group reaches its own vertices and
-// the columns of those whose parent is outside the group.
+// the columns of those whose parent is outside the group.  *largest: vertices
+// of the group with the longest such column, its own and that column's (for the
+// deep groups, whose columns mostly lie in one another, all they reach).
 uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
-                            const std::vector<int64_t>& Ub, int bits) {
+                            const std::vector<int64_t>& Ub, int bits, uint64_t* largest) {
     uint64_t sum = 0;
+    *largest = 0;
     for (size_t b = 0; b + 1 < mat_base.size(); b++) {
         for (int64_t hi = (int64_t)mat_base[b + 1]; hi > (int64_t)mat_base[b]; hi -= bits) {
             const int64_t lo = std::max<int64_t>(hi - bits, (int64_t)mat_base[b]);
-            uint64_t items = (uint64_t)(hi - lo);
+            uint64_t items = (uint64_t)(hi - lo), column = 0;
             for (int64_t j = lo; j < hi; j++)
-                if (parent[(size_t)j] < 0 || parent[(size_t)j] >= hi) items += (uint64_t)Ub[(size_t)j];
+                if (parent[(size_t)j] < 0 || parent[(size_t)j] >= hi) {
+                    items += (uint64_t)Ub[(size_t)j];
+                    column = std::max(column, (uint64_t)Ub[(size_t)j]);
+                }
+            *largest = std::max(*largest, (uint64_t)(hi - lo) + column);
             sum += items;
         }
     }

@@ -65,7 +65,7 @@ void lu_row_bounds(int32_t n, const int32_t* rp, const int32_t* ci, const int32_
                    std::vector<int64_t>& Lb, std::vector<int64_t>& Ub, std::vector<int32_t>* parent_out = nullptr);
 double subtree_skew(int32_t N, int32_t gid, const std::vector<int32_t>& parent);
 uint64_t reach_record_bound(const std::vector<uint32_t>& mat_base, const std::vector<int32_t>& parent,
-                            const std::vector<int64_t>& Ub, int bits);
+                            const std::vector<int64_t>& Ub, int bits, uint64_t* largest);
 
 constexpr int kBlockSlots = 32;      // largest source-slot count per workgroup in block mode
 constexpr int kBatchSlots = 16;      // slots per workgroup for batches of matrices by default
@@ -192,7 +192,7 @@ struct RchParams {
 };
 bool rch_threads_valid(int threads);  // a caller's choice of threads per reach workgroup: 1024 or 512
 bool rch_shape_valid(int threads);    // any shape there is: 256 too
-int reach_shape(uint64_t chunks, uint64_t reach, uint32_t W, int bits, uint32_t cus, int64_t room);
+int reach_shape(uint64_t chunks, uint64_t reach, uint64_t largest, uint32_t W, int bits, uint32_t cus, int64_t room);
 bool rch_bits_valid(int bits);
 const void* rch_kernel_ptr(int bits, int threads);
 int64_t reach_bytes(uint32_t nb, uint32_t W, int bits);
@@ -210,7 +210,7 @@ int resolve_mode(const gsofa_options& o);
 std::string tune_signature(int64_t n_max, int64_t nnz, int64_t n_total, int32_t n_mats);
 bool apply_tuned(gsofa_options* o, int64_t n_max, int64_t nnz, int64_t n_total, int32_t n_mats);
 int choose_bits(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* bits);
-int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint32_t W, int64_t avail,
+int reach_grid(const gsofa_options& o, int bits, uint64_t nchunks, uint64_t records, uint64_t largest, uint32_t W, int64_t avail,
                uint32_t* nb_out, int* threads_out);
 void transpose_rows(int32_t n, const int32_t* rp, const int32_t* ci, std::vector<int32_t>& rpT,
                     std::vector<int32_t>& ciT);
@@ -292,6 +292,7 @@ struct PackedMatrix {
     std::vector<int32_t> rp, ci, rpT, ciT;
     uint64_t need_fill = 0, need_L = 0, need_U = 0;
     uint64_t need_rec = 0;  // records of one pass
+    uint64_t largest = 0;   // vertices of its largest group
 };
 int pack_matrix(const gsofa_matrix* A, PackedMatrix* M);
 // Arena: a reach-mode plan that takes one batch after another in its own

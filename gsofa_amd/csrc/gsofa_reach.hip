@@ -17,14 +17,28 @@
 // nested-dissection grids).
 //
 // Execution model (CDNA4, persistent grid of co-resident workgroups: one of
-// 1024 threads per CU with the largest target table, or two of 512 threads
-// with half the table each, so one runs while the other waits at a barrier):
+// 1024 threads per CU with the largest tables, or two of 512 threads or four of
+// 256 with a part of it each, so one runs while another waits at a barrier):
 // * A workgroup owns MB source slots (32, 64, 128 or 256: the bits of a mask
 //   of one, two or four 64-bit words) and runs a mini-group of up to MB
 //   sources of one matrix, in one of the two passes, through all of its
 //   levels alone.  The next mini-group comes from one global counter over a
 //   work table that interleaves the passes' chunks, deepest first, so both
 //   passes share one launch and its tail.
+// * With 32 and 64 slots a mini-group's nodes (the vertices and classes that its
+//   sources reach, a few hundred on banded and 2D matrices, up to thousands on
+//   3D ones) are kept in an LDS table for its whole traversal, with their
+//   visited and pending bits (walk_nodes): a lane group pops a node, maps each
+//   edge's target to its node, ORs the new bits into it and queues it if it had
+//   none pending.  A level is one barrier, and per hop only the graph is read
+//   from memory: edges, their classes, new nodes' rows.  What bounds it: those
+//   three dependent reads, 2 to 3 us a level, and for wide levels the LDS
+//   operations per edge.  Execute ms, before -> now: 64^2 grid in natural order
+//   0.41 -> 0.33; 181^2 0.84 -> 0.64; 27^3 0.76 -> 0.59; 33^3 1.08 -> 0.79; band
+//   of 100,003 0.79 -> 0.70; 128 2D grids 11.1 -> 7.2; 48^3, whose deep groups
+//   do not fit, 2.30 -> 2.30.
+// * A mini-group whose nodes outgrow the table, and every one with more slots,
+//   keeps its state in memory, as follows.
 // * Per vertex, one word holds the MB slots' visited bits with the
 //   mini-group's stamp beside it; an older stamp reads as "nothing visited",
 //   so the array is never cleared between mini-groups (the reference's
@@ -305,11 +319,46 @@ constexpr int tab_slots(int threads) {
 // such vertices per level (any more are queued whole).
 constexpr uint32_t SPLIT_ROW = 192, SPLIT_PARTS = 32, SPLIT_MAX = 32;
 
-template <class M, int H>
+// A mini-group's nodes, all of them, in LDS (one- and two-word masks): node
+// table slots for the space of the target table at 64 slots, at most FT in use.
+template <class M>
+constexpr int node_slots(int threads) {
+    return ((threads == NT_WIDE ? NH_WIDE : threads == NT_PAIR ? NH_PAIR : NH_QUAD) * 14 - 8 * threads) /
+           (18 + 2 * (int)sizeof(M)) / WAVE * WAVE;
+}
+constexpr uint32_t node_room(uint32_t slots) { return slots / 8u * 7u; }  // nodes, at most
+
+// Rows of over two steps are walked in parts, by as many lane groups as there
+// are parts: a level of few nodes, as most are once classes stand for the
+// vertices, would otherwise last as long as its longest row.
+constexpr uint32_t PART_STEPS = 2, PART_ROWS = 64;  // such rows of a level, at most
+template <class M, int F, int NT>
+struct RNodes {
+    M vis[F];                            // sources that have visited the node
+    M pend[F];                           // of those, the ones it is still to be expanded for
+    uint2 row[F];                        // a queued node's row; at the group's end a bitmap and its prefix
+    uint32_t key[F];                     // node + 1; 0 = empty
+    uint16_t q[2][F];                    // queues, by level parity
+    uint16_t ent[F];                     // slots in use, in the order of insertion
+    M pmask[PART_ROWS];                  // masks of this level's rows in parts
+    uint32_t plen[2][PART_ROWS];         // edges of a part, by level parity
+    uint16_t pnode[2][PART_ROWS];        // their nodes
+    uint16_t part[2][NT];                // the parts: (row << 10) | part of it
+};
+
+template <class M, int H, int F, int NT>
 struct RLds {
-    uint32_t hkey[H];                    // target + 1 (window-local); 0 = empty
-    M hmask[H];                          // OR of the masks folded into the target this round
-    uint16_t ent[H];                     // occupied hash slots in insertion order
+    union {
+        struct {                         // all zero between rounds but for ent
+            uint32_t hkey[H];            // target + 1 (window-local); 0 = empty
+            M hmask[H];                  // OR of the masks folded into the target this round
+            uint16_t ent[H];             // occupied hash slots in insertion order
+        };
+        RNodes<M, F, NT> n;                 // vis, pend and key zero between mini-groups
+    };
+    uint32_t nq[3], ncur[3];             // queue sizes and cursors, by level modulo 3
+    uint32_t nrow[3], npart[3];          // rows in parts and parts, likewise
+    uint32_t used, over[3];              // nodes in the table; it ran full in a level
     uint32_t s_cnt[MaskOps<M>::BITS];    // A pass: U entries per slot
     uint32_t wsum[16];                   // per-wave sums of a block scan
     uint32_t nup, tmax;                  // vertices above the group reached so far; the largest
@@ -328,8 +377,8 @@ struct RLds {
 
 // Hash slot of window-local target m, inserting it if new; FULLI when it is
 // new and the round already holds T targets.  Linear probing.
-template <class M, int H>
-__device__ __forceinline__ uint32_t rtab_find(RLds<M, H>& S, uint32_t* tcnt, uint32_t m) {
+template <class M, int H, int F, int NT>
+__device__ __forceinline__ uint32_t rtab_find(RLds<M, H, F, NT>& S, uint32_t* tcnt, uint32_t m) {
     constexpr int T = H / 2;
     const uint32_t key = m + 1u;
     uint32_t s = (uint32_t)(((uint64_t)(m * 2654435761u) * (uint32_t)H) >> 32);
@@ -403,6 +452,21 @@ struct RCur {
         const uint32_t h = 31u - (uint32_t)__builtin_clz((m >> kQuotShift) ^ jb);
         return h < top ? h : top;
     }
+    // row and (vertices, row lengths) of a node
+    __device__ __forceinline__ uint2 row(uint32_t m) const {
+        if (m < below) {
+            const uint4 in = info[(uint64_t)level_of(m) * cn + wb + m];
+            return make_uint2(in.x, in.y);
+        }
+        return make_uint2((uint32_t)rp[wb + m], (uint32_t)rp[wb + m + 1u]);
+    }
+    __device__ __forceinline__ uint2 weight(uint32_t m) const {
+        if (m < below) {
+            const uint4 in = info[(uint64_t)level_of(m) * cn + wb + m];
+            return make_uint2(in.z, in.w);
+        }
+        return make_uint2(1u, (uint32_t)rp[wb + m + 1u] - (uint32_t)rp[wb + m]);
+    }
     // the node (local) that stands for local vertex m
     __device__ __forceinline__ uint32_t node(uint32_t m) const {
         return m < below ? (uint32_t)comp[(uint64_t)level_of(m) * cn + wb + m] - wb : m;
@@ -415,8 +479,8 @@ struct RCur {
 // first fold).  Each target is found or inserted in the table and the
 // vertex's mask folded into it, until the queue is exhausted or the table is
 // full.  Wave-uniform control flow; the groups hold independent vertices.
-template <int H, int G, int E, class M>
-__device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, const uint4* qc, uint32_t qsize,
+template <int H, int F, int G, int E, class M, int NT>
+__device__ void rcombine(RLds<M, H, F, NT>& S, RGrp<M>& hv, const RCur& c, M* maskc, const uint4* qc, uint32_t qsize,
                          uint32_t size, const uint4* sp, uint32_t* cursor, uint32_t rb, RTally& t) {
     using O = MaskOps<M>;
     constexpr int T = H / 2;
@@ -497,7 +561,7 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
 #pragma unroll
             for (int k = 0; k < E; k++) {
                 if (m[k] != FULLI) {
-                    const uint32_t hs = rtab_find<M, H>(S, &S.tcnt[rb], m[k]);
+                    const uint32_t hs = rtab_find(S, &S.tcnt[rb], m[k]);
                     if (hs == FULLI) left |= 1u << k;
                     else mask_or(&S.hmask[hs], hv.vm);
                 }
@@ -515,14 +579,340 @@ __device__ void rcombine(RLds<M, H>& S, RGrp<M>& hv, const RCur& c, M* maskc, co
     }
 }
 
-template <int RB, int H, int G, int E, class M>
-__global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
+// Table slot of node m, inserting it if new; FULLI (and *over set) when the
+// table is full.
+template <class M, int H, int F, int NT>
+__device__ __forceinline__ uint32_t node_find(RLds<M, H, F, NT>& S, uint32_t* over, uint32_t m) {
+    constexpr uint32_t FT = node_room((uint32_t)F);
+    const uint32_t key = m + 1u;
+    uint32_t s = (uint32_t)(((uint64_t)(m * 2654435761u) * (uint32_t)F) >> 32);
+    for (int probe = 0; probe < F; probe++) {
+        const uint32_t cur = S.n.key[s];
+        if (cur == key) return s;
+        if (cur == 0u) {
+            if (S.used >= FT) break;
+            const uint32_t prev = atomicCAS(&S.n.key[s], 0u, key);
+            if (prev == 0u) {
+                S.n.ent[atomicAdd(&S.used, 1u)] = (uint16_t)s;  // at most F keys are ever inserted
+                return s;
+            }
+            if (prev == key) return s;
+        }
+        s = s + 1u == (uint32_t)F ? 0u : s + 1u;
+    }
+    *over = 1u;
+    return FULLI;
+}
+
+__device__ __forceinline__ uint32_t mask_or_rtn(uint32_t* p, uint32_t v) { return atomicOr(p, v); }
+__device__ __forceinline__ uint64_t mask_or_rtn(uint64_t* p, uint64_t v) {
+    return atomicOr(reinterpret_cast<unsigned long long*>(p), (unsigned long long)v);
+}
+__device__ __forceinline__ uint32_t mask_take(uint32_t* p) { return atomicExch(p, 0u); }
+__device__ __forceinline__ uint64_t mask_take(uint64_t* p) {
+    return atomicExch(reinterpret_cast<unsigned long long*>(p), 0ull);
+}
+
+// A mini-group's whole traversal on the node table.  A popped node's bits go
+// straight to its targets' visited words; who sets a pending bit of a node with
+// none queues it.  So a level is one phase and one barrier and nothing but the
+// graph itself is read from memory: edges, their classes, the new nodes' rows.
+// Returns false, with the table to be cleared, if it ran full.
+template <int RB, int H, int F, int G, int E, class M>
+__device__ bool walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsigned long long& levels) {
+    using O = MaskOps<M>;
+    const uint32_t tid = threadIdx.x, lane = __lane_id();
+    const uint32_t grp = lane / G, j = lane % G;
+    RTally own{0, 0, 0, 0, 0};
+    // a row of over PART edges to level lv's parts; false: no room left
+    constexpr uint32_t STEP = (uint32_t)(G * E), PART = PART_STEPS * STEP;
+    auto in_parts = [&](uint32_t lv, uint32_t node, uint32_t len, M mask) {
+        uint32_t per = (len + RB / 4u - 1u) / (RB / 4u);
+        per = per < PART ? PART : (per + STEP - 1u) / STEP * STEP;
+        const uint32_t parts = (len + per - 1u) / per, q = lv & 1u;
+        const uint32_t r = atomicAdd(&S.nrow[lv % 3u], 1u);
+        if (r >= PART_ROWS) return false;
+        const uint32_t o = atomicAdd(&S.npart[lv % 3u], parts);
+        const bool fits = o + parts <= (uint32_t)RB;
+        for (uint32_t k = 0; k < parts && o + k < (uint32_t)RB; k++)
+            S.n.part[q][o + k] = fits ? (uint16_t)((r << 10) | k) : (uint16_t)0xFFFF;
+        S.n.pnode[q][r] = (uint16_t)(fits ? node : 0xFFFFu);
+        S.n.plen[q][r] = per;
+        if (mask) S.n.pmask[r] = mask;
+        return fits;
+    };
+    if (tid < 3u) S.nq[tid] = tid == 0 ? c.count : 0u;
+    if (tid >= 3u && tid < 6u) S.ncur[tid - 3u] = 0;
+    if (tid >= 6u && tid < 9u) S.nrow[tid - 6u] = 0;
+    if (tid >= 9u && tid < 12u) S.npart[tid - 9u] = 0;
+    if (tid >= 12u && tid < 15u) S.over[tid - 12u] = 0;
+    __syncthreads();
+    if (tid < c.count) {  // level 0: the sources, each for its own slot
+        const uint32_t sg = c.first - tid * c.stride;
+        const uint32_t k = node_find(S, &S.over[2], sg - c.wb);  // distinct, and far fewer than slots
+        const uint32_t r0 = (uint32_t)c.rp[sg], r1 = (uint32_t)c.rp[sg + 1];
+        S.n.vis[k] = O::bit(tid);
+        S.n.row[k] = make_uint2(r0, r1);
+        S.n.q[0][tid] = (uint16_t)(r1 - r0 > PART && in_parts(0u, k, r1 - r0, O::bit(tid)) ? 0xFFFFu : k);
+        own.te = r1 - r0;
+    }
+    uint32_t lev = 0;
+    bool full;
+    for (;; lev++) {
+        __syncthreads();
+        const uint32_t b = lev % 3u, nb = (lev + 1u) % 3u;
+        const uint32_t qsize = S.nq[b], nrow = S.nrow[b] < PART_ROWS ? S.nrow[b] : PART_ROWS;
+        const uint32_t size = qsize + (S.npart[b] < (uint32_t)RB ? S.npart[b] : (uint32_t)RB);
+        full = S.over[(lev + 2u) % 3u] != 0u;  // in the level before: this one's flag may be set by now
+        if (size == 0u || full) break;
+        if (tid == 0) {  // the counters of the level after the next: last read a barrier ago
+            const uint32_t z = (lev + 2u) % 3u;
+            S.nq[z] = S.ncur[z] = S.nrow[z] = S.npart[z] = 0;
+        }
+        const uint16_t* qc = S.n.q[lev & 1u];
+        uint16_t* qn = S.n.q[(lev + 1u) & 1u];
+        const uint32_t par = lev & 1u;
+        if (nrow && lev) {
+            if (tid < nrow && S.n.pnode[par][tid] != 0xFFFFu) S.n.pmask[tid] = mask_take(&S.n.pend[S.n.pnode[par][tid]]);
+            __syncthreads();
+        }
+        bool held = false, done = false;
+        uint32_t pos = 0, end = 0;
+        M vm = (M)0;
+        for (;;) {
+            const bool want = !held && !done;
+            const uint64_t wl = __ballot(want && j == 0u);
+            if (wl) {
+                uint32_t base = 0;
+                if (lane == 0) base = atomicAdd(&S.ncur[b], (uint32_t)__popcll(wl));
+                base = bcast0(base);
+                if (want) {
+                    const uint32_t idx = base + (uint32_t)__popcll(wl & ((1ull << (G * grp)) - 1ull));
+                    if (idx >= size) {
+                        done = true;
+                    } else if (idx < qsize) {
+                        const uint32_t k = qc[idx];
+                        if (k != 0xFFFFu) {  // not one that is walked in parts
+                            const uint2 r = S.n.row[k];
+                            pos = r.x;
+                            end = r.y;
+                            M m = (M)0;
+                            if (j == 0u) m = lev ? mask_take(&S.n.pend[k]) : O::bit(idx);
+                            vm = __shfl(m, 0, G);
+                            held = pos < end;
+                            if (j == 0u) own.expansions++;
+                        }
+                    } else {
+                        const uint32_t x = S.n.part[par][idx - qsize];
+                        if (x != 0xFFFFu) {
+                            const uint32_t per = S.n.plen[par][x >> 10];
+                            const uint2 r = S.n.row[S.n.pnode[par][x >> 10]];
+                            pos = r.x + (x & 1023u) * per;
+                            end = r.y - pos > per ? pos + per : r.y;
+                            vm = S.n.pmask[x >> 10];
+                            held = true;
+                            if ((x & 1023u) == 0u && j == 0u) own.expansions++;
+                        }
+                    }
+                }
+            }
+            if (!__ballot(held)) {
+                if (__ballot(!done)) continue;
+                break;
+            }
+            // one step of every group that holds a node
+            uint32_t m[E];
+#pragma unroll
+            for (int k = 0; k < E; k++) {
+                const uint32_t ek = pos + j + (uint32_t)(G * k);
+                m[k] = held && ek < end ? (uint32_t)c.ci[ek] - c.wb : FULLI;
+            }
+#pragma unroll
+            for (int k = 0; k < E; k++)
+                if (m[k] != FULLI) m[k] = c.node(m[k]);
+            uint32_t push[E];
+            uint2 row[E];
+#pragma unroll
+            for (int k = 0; k < E; k++) {
+                push[k] = FULLI;
+                if (m[k] == FULLI) continue;
+                const uint32_t sl = node_find(S, &S.over[b], m[k]);
+                if (sl == FULLI) continue;
+                M nw = vm & ~S.n.vis[sl];
+                if (!nw) continue;
+                nw = nw & ~mask_or_rtn(&S.n.vis[sl], nw);
+                if (!nw) continue;
+                const M bl = nw & above_mask<M>(m[k] + c.wb, c.first, c.stride, c.count);
+                if (lev) own.fills += O::popc(nw & ~bl);
+                if (bl && !mask_or_rtn(&S.n.pend[sl], bl)) push[k] = sl;
+            }
+#pragma unroll
+            for (int k = 0; k < E; k++)
+                if (push[k] != FULLI) row[k] = c.row(m[k]);
+#pragma unroll
+            for (int k = 0; k < E; k++) {
+                bool enq = push[k] != FULLI;
+                if (enq) {
+                    S.n.row[push[k]] = row[k];
+                    const uint32_t len = row[k].y - row[k].x;
+                    if (len > PART && in_parts(lev + 1u, push[k], len, (M)0)) enq = false;
+                }
+                const uint64_t em = __ballot(enq);
+                if (em) {
+                    uint32_t qb = 0;
+                    if (lane == 0) qb = atomicAdd(&S.nq[nb], (uint32_t)__popcll(em));
+                    qb = bcast0(qb);
+                    if (enq) qn[qb + rank_in(em)] = (uint16_t)push[k];
+                }
+            }
+            if (held) {
+                pos += (uint32_t)(G * E);
+                held = pos < end;
+            }
+        }
+    }
+    if (full) return false;
+    // TE and |R|: every node below a source that visited it, with its weights
+    const uint32_t fl = c.first - c.wb, used = S.used;
+    for (uint32_t x = tid; x < used; x += RB) {
+        const uint32_t i = S.n.ent[x], m = S.n.key[i] - 1u;
+        if (m > fl) continue;
+        const M bl = S.n.vis[i] & above_mask<M>(m + c.wb, c.first, c.stride, c.count);
+        if (!bl) continue;
+        const uint2 w = c.weight(m);
+        own.reach += (unsigned long long)O::popc(bl) * w.x;
+        own.te += (unsigned long long)O::popc(bl) * w.y;
+    }
+    t.fills += own.fills;
+    t.expansions += own.expansions;
+    t.te += own.te;
+    t.reach += own.reach;
+    t.checks += own.te;  // every node once for every source that visits it
+    levels += tid == 0 ? lev : 0u;
+    return true;
+}
+
+// The group's entries from the node table, which is cleared: records in order
+// of the vertex by ranks in an LDS bitmap over the vertices above the group,
+// a window of 32 F of them at a time; counts per row.
+template <int RB, int H, int F, class M>
+__device__ void emit_nodes(RLds<M, H, F, RB>& S, const RCur& c, const RchParams& p, uint32_t ck) {
+    using O = MaskOps<M>;
+    static_assert(sizeof(M) <= 8, "one record word");
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / WAVE;
+    const uint32_t fl = c.first - c.wb, lo = fl - (c.count - 1u), used = S.used;
+    const bool rec = p.rec_cap != 0ull;
+    uint32_t* bm = reinterpret_cast<uint32_t*>(S.n.row);
+    uint32_t* before = bm + F;
+    uint32_t nup = 0, top = 0;
+    for (uint32_t x = tid; x < used; x += RB) {
+        const uint32_t m = S.n.key[S.n.ent[x]] - 1u;
+        if (m <= fl) continue;
+        nup++;
+        top = m > top ? m : top;
+    }
+    nup = dev::wave_incl_scan(nup);
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const uint32_t o = __shfl_xor(top, d, WAVE);
+        top = o > top ? o : top;
+    }
+    if (lane == WAVE - 1 && nup) {
+        atomicAdd(&S.nup, nup);
+        atomicMax(&S.tmax, top);
+    }
+    __syncthreads();
+    const uint32_t items = c.count + S.nup;
+    const uint32_t all = rec && S.nup ? ((S.tmax - fl - 1u) >> 5) + 1u : 0u;
+    if (rec && tid == 0) {
+        const unsigned long long o = aadd64(&p.ctrl->fill_pos, (unsigned long long)items);
+        const bool fits = o + (unsigned long long)items <= p.rec_cap;
+        S.rbase = fits ? o : ~0ull;
+        p.grp[ck] = make_uint4((uint32_t)o, (uint32_t)(o >> 32), fits ? items : 0u, 0u);
+    }
+    uint32_t acc = 0, sorted = c.count;
+    for (uint32_t w0 = 0; w0 == 0u || w0 < all; w0 += F) {
+        const uint32_t nw = all - w0 < (uint32_t)F ? all - w0 : (uint32_t)F;
+        if (rec) {
+            for (uint32_t i = tid; i < nw; i += RB) bm[i] = 0u;
+            __syncthreads();
+            for (uint32_t x = tid; x < used; x += RB) {
+                const uint32_t m = S.n.key[S.n.ent[x]] - 1u, o = m - fl - 1u;
+                if (m > fl && (o >> 5) - w0 < nw) atomicOr(&bm[(o >> 5) - w0], 1u << (o & 31u));
+            }
+            __syncthreads();
+            const uint32_t per = (nw + RB - 1u) / RB;
+            const uint32_t b0 = tid * per < nw ? tid * per : nw;
+            const uint32_t b1 = b0 + per < nw ? b0 + per : nw;
+            uint32_t cnt = 0;
+            for (uint32_t b = b0; b < b1; b++) cnt += (uint32_t)__popc(bm[b]);
+            const uint32_t incl = wave_incl_scan(cnt);
+            if (lane == WAVE - 1) S.wsum[w] = incl;
+            __syncthreads();
+            uint32_t pos = sorted + incl - cnt;
+            for (uint32_t k = 0; k < (uint32_t)(RB / WAVE); k++) {
+                if (k < w) pos += S.wsum[k];
+                sorted += S.wsum[k];
+            }
+            for (uint32_t b = b0; b < b1; b++) {
+                before[b] = pos;
+                pos += (uint32_t)__popc(bm[b]);
+            }
+            __syncthreads();
+        }
+        const uint64_t r0 = rec ? S.rbase : ~0ull;
+        for (uint32_t x0 = w * WAVE; x0 < used; x0 += RB) {
+            const uint32_t i = x0 + lane < used ? S.n.ent[x0 + lane] : 0u;
+            const uint32_t m = x0 + lane < used ? S.n.key[i] - 1u : 0u, o = m - fl - 1u;
+            bool in = false;
+            uint32_t at = 0;
+            M mk = (M)0;
+            if (m > fl) {
+                in = !rec || (o >> 5) - w0 < nw;
+                if (in) {
+                    mk = S.n.vis[i];
+                    if (rec) at = before[(o >> 5) - w0] + (uint32_t)__popc(bm[(o >> 5) - w0] & ((1u << (o & 31u)) - 1u));
+                }
+            } else if (x0 + lane < used && m >= lo && w0 == 0u) {
+                in = true;
+                at = m - lo;
+                mk = S.n.vis[i] & ~O::prefix(c.count - at);  // sources below the vertex
+            }
+            const uint64_t wd = mask_word(mk, 0);
+            if (in && r0 != ~0ull) p.rec[r0 + at] = make_uint4(c.wb + m, c.first, (uint32_t)wd, (uint32_t)(wd >> 32));
+            if (!__ballot(wd != 0ull)) continue;
+            if (c.tpass) {
+                if (wd) aadd64(&p.cntL[c.wb + m], (1ull << 32) | (unsigned long long)__popcll(wd));
+            } else {
+#pragma unroll
+                for (int j = 0; j < O::BITS; j++) {
+                    const uint32_t n = (uint32_t)__popcll(__ballot((wd >> j) & 1ull));
+                    if (lane == (uint32_t)j) acc += n;
+                }
+            }
+        }
+        __syncthreads();  // the window's ranks are read
+    }
+    if (!c.tpass && acc) atomicAdd(&S.s_cnt[lane], acc);
+    for (uint32_t x = tid; x < used; x += RB) {
+        const uint32_t i = S.n.ent[x];
+        S.n.key[i] = 0u;
+        S.n.vis[i] = S.n.pend[i] = (M)0;
+    }
+    __syncthreads();
+    if (tid == 0) S.used = 0;
+    if (!c.tpass && tid < c.count) p.cntU[c.first - tid * c.stride] = S.s_cnt[tid];
+}
+
+template <int RB, int H, int F, int G, int E, class M>
+__global__ __launch_bounds__(RB, sizeof(M) <= 16 ? 4 : 1) void k_reach_blk(RchParams p) {
     static_assert(H / 2 + RB <= H, "insert overshoot stays within the entry list");
     static_assert(H <= 65536, "entries are 16-bit slot numbers");
     static_assert(WAVE % G == 0 && G < 32 && E >= 1 && E < 32, "lane groups tile a wave; a lane's edges fit its pending bits");
     using O = MaskOps<M>;
     using VW = typename O::V;
-    __shared__ RLds<M, H> S;
+    using Lds = RLds<M, H, F, RB>;
+    __shared__ Lds S;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = __lane_id();
     const uint32_t w = tid / WAVE;
@@ -533,10 +923,14 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
     uint32_t epoch = p.bstate[blockIdx.x];
     RTally t{0, 0, 0, 0, 0};
     unsigned long long levels = 0;
-    for (uint32_t i = tid; i < (uint32_t)H; i += RB) {
-        S.hkey[i] = 0u;
-        S.hmask[i] = (M)0;
-    }
+    constexpr bool NODES = sizeof(M) <= 8;
+    constexpr uint32_t TAB_WORDS = (uint32_t)(offsetof(Lds, nq) / 4);
+    auto clear_tables = [&] {
+        for (uint32_t i = tid; i < TAB_WORDS; i += RB) reinterpret_cast<uint32_t*>(&S)[i] = 0u;
+    };
+    uint32_t wait = 0;  // mini-groups to go before the node table is tried again
+    clear_tables();
+    if (tid == 0) S.used = 0;
     if (tid < 8) S.acc[tid] = 0;
     if (tid == 0) {
         S.qcnt[0] = S.qcnt[1] = 0;
@@ -572,13 +966,35 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
         c.top = p.quot.levels - 1u;
         c.jb = classes ? (c.first - (c.count - 1u) * c.stride - c.wb) >> kQuotShift : 0u;
         c.below = c.jb << kQuotShift;
+        bool nodes = false;  // the node table holds the whole group
+        if constexpr (NODES) {
+            if (wait == 0u) {
+                nodes = walk_nodes<RB, H, F, G, E, M>(S, c, t, levels);
+                if (!nodes) {
+                    // the sizes of neighbouring groups are alike
+                    wait = 8u;
+                    __syncthreads();
+                    clear_tables();
+                    if (tid == 0) S.used = 0;
+                    __syncthreads();
+                }
+            }
+        }
+        // No vertex above the group is ever queued, so the queue arrays' entries
+        // past the group's largest source hold the list of those reached (in
+        // the first array) and its sorted copy (in the second).
+        const uint32_t fl = c.first - c.wb;
+        uint32_t* const ulist = reinterpret_cast<uint32_t*>(q0 + fl + 1u);
+        uint32_t* const slist = reinterpret_cast<uint32_t*>(q0 + W + fl + 1u);
+        uint32_t stamp = 0;
+        if (!nodes) {
         if (epoch >= p.loops) {  // stamps exhausted: clear this workgroup's visited words
             for (uint32_t i = tid; i < W; i += RB) vis[i] = O::make((M)0, 0u);
             epoch = 0;
             __syncthreads();  // cleared before the sources are stamped
         }
         epoch++;
-        const uint32_t stamp = epoch;
+        stamp = epoch;
         // level 0: the sources themselves, each visited by and queued for its own slot
         if (tid < c.count) {
             const uint32_t sg = c.first - tid * c.stride;
@@ -591,12 +1007,6 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             t.te += r1 - r0;
         }
         if (tid == 0) S.qcnt[0] = c.count;
-        // No vertex above the group is ever queued, so the queue arrays' entries
-        // past the group's largest source hold the list of those reached (in
-        // the first array) and its sorted copy (in the second).
-        const uint32_t fl = c.first - c.wb;
-        uint32_t* const ulist = reinterpret_cast<uint32_t*>(q0 + fl + 1u);
-        uint32_t* const slist = reinterpret_cast<uint32_t*>(q0 + W + fl + 1u);
         __syncthreads();
 
         uint32_t cur = 0;
@@ -631,7 +1041,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             hv.pos = hv.end = 0u;
             hv.vm = (M)0;
             for (;;) {  // rounds, two barriers each
-                rcombine<H, G, E, M>(S, hv, c, maskc, qc, qsize, size, S.sp[cur], cursor, rb, t);
+                rcombine<H, F, G, E, M>(S, hv, c, maskc, qc, qsize, size, S.sp[cur], cursor, rb, t);
                 if (hv.held && (lane % G) == 0u) atomicOr(&S.held[rb], 1u);
                 __syncthreads();
                 // final for this round: the cursor moves only in phase A
@@ -737,6 +1147,7 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             cur = nxt;
             levels++;
         }
+        }
         // the mini-group's TE and |R| (per matrix for the A pass); counts-only
         // fills per source row
         const unsigned long long te = wave_sum64(t.te), rc = wave_sum64(t.reach);
@@ -752,6 +1163,12 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             if (!c.tpass && p.mat_te) {
                 aadd64(&p.mat_te[c.mat], S.cte);
                 aadd64(&p.mat_reach[c.mat], S.creach);
+            }
+        }
+        if constexpr (NODES) {
+            if (nodes) {
+                emit_nodes<RB, H, F, M>(S, c, p, ck);
+                continue;
             }
         }
         // ---- the group's entries, from the final visited words: items are the
@@ -839,6 +1256,10 @@ __global__ __launch_bounds__(RB) void k_reach_blk(RchParams p) {
             if (tid < c.count) p.cntU[c.first - tid * c.stride] = S.s_cnt[tid];
         }
         __syncthreads();
+        if (NODES && wait && --wait == 0u) {
+            clear_tables();
+            __syncthreads();
+        }
     }
     if (t.fills) atomicAdd(&S.acc[0], t.fills);
     if (t.checks) atomicAdd(&S.acc[1], t.checks);
@@ -867,22 +1288,31 @@ bool rch_shape_valid(int threads) { return rch_threads_valid(threads) || threads
 
 // The shape for `chunks` mini-groups (both passes) of matrices of up to W
 // vertices, whose groups reach `reach` vertices at or above themselves on
-// average (from the record bound), on `cus` CUs:
-//   wide  while every mini-group has a CU of its own;
+// average (from the record bound) and the largest of them `largest`, on `cus`
+// CUs:
 //   quad  where several mini-groups queue per CU and they are narrow;
+//   wide  where the largest group's nodes fit only its table;
 //   pair  otherwise.
-// More workgroups hold more per-vertex arrays, so a shape is taken only while
-// those stay within `room` bytes (quad 8 GiB, pair half the room and 32 GiB);
-// pair's 256-slot kernel has registers for one workgroup per CU.  Execute ms at wide /
-// pair / quad: 64^2 grid (256 mini-groups) 0.50 / 0.56 / 0.68; 181^2 grid
-// (1,024) 1.10 / 0.83 / 0.90; 33^3 (1,124) 1.70 / 1.42 / 1.85; 48^3 (3,456 of
-// about 1,600 vertices) 3.69 / 2.89 / 3.53; band n = 100,003 (3,126 of about
-// 400) 1.54 / 1.23 / 1.18; 128 2D grids (64,800 of about 250) 32.9 / 17.1 /
-// 13.6.
-int reach_shape(uint64_t chunks, uint64_t reach, uint32_t W, int bits, uint32_t cus, int64_t room) {
-    if (chunks <= cus) return NT_WIDE;
+// With 128 and 256 slots, which use no node table, wide while every mini-group
+// has a CU of its own.  More workgroups hold more per-vertex arrays, so a shape
+// is taken only while those stay within `room` bytes (quad 8 GiB, pair half the
+// room and 32 GiB); pair's 256-slot kernel has registers for one workgroup per
+// CU.  Execute ms at 64 slots, wide / pair / quad where taken: 16^2 grid 0.162 /
+// 0.156; 64^2 grid 0.346 / 0.332; band n = 11,948 0.32 / 0.30; 181^2 grid 0.77 /
+// 0.64; 33^3 grid (largest group about 3,000) 0.79 / 1.06; 48^3 (6,000 and
+// more) 2.8 / 2.3; band n = 100,003 1.02 / 0.73 / 0.70; 128 2D grids 17.6 / 9.3
+// / 7.2.
+int reach_shape(uint64_t chunks, uint64_t reach, uint64_t largest, uint32_t W, int bits, uint32_t cus, int64_t room) {
+    if (bits > 64 && chunks <= cus) return NT_WIDE;
     const int64_t quad = reach_bytes((uint32_t)std::min<uint64_t>(4ull * cus, chunks), W, bits);
     if (chunks >= 8ull * cus && reach <= 512 && quad <= std::min<int64_t>(room, 8ll << 30)) return NT_QUAD;
+    if (bits <= 64) {
+        const uint64_t need = largest + 256;  // with the nodes below the group
+        const bool m64 = bits == 64;
+        const uint64_t in_pair = node_room((uint32_t)(m64 ? node_slots<uint64_t>(NT_PAIR) : node_slots<uint32_t>(NT_PAIR)));
+        const uint64_t in_wide = node_room((uint32_t)(m64 ? node_slots<uint64_t>(NT_WIDE) : node_slots<uint32_t>(NT_WIDE)));
+        if (need > in_pair && need <= in_wide) return NT_WIDE;
+    }
     const int64_t pair = reach_bytes((uint32_t)std::min<uint64_t>(2ull * cus, chunks), W, bits);
     return bits < 256 && pair <= std::min<int64_t>(room / 2, 32ll << 30) ? NT_PAIR : NT_WIDE;
 }
@@ -891,11 +1321,11 @@ namespace {
 template <int NT, class M>
 const void* kptr() {
     return reinterpret_cast<const void*>(
-        &k_reach_blk<NT, tab_slots<M>(NT), lanes_per_vertex<NT>(), edges_per_lane<NT>(), M>);
+        &k_reach_blk<NT, tab_slots<M>(NT), node_slots<M>(NT), lanes_per_vertex<NT>(), edges_per_lane<NT>(), M>);
 }
 template <int NT, class M>
 void klaunch(const RchParams& p, hipStream_t s) {
-    hipLaunchKernelGGL((k_reach_blk<NT, tab_slots<M>(NT), lanes_per_vertex<NT>(), edges_per_lane<NT>(), M>),
+    hipLaunchKernelGGL((k_reach_blk<NT, tab_slots<M>(NT), node_slots<M>(NT), lanes_per_vertex<NT>(), edges_per_lane<NT>(), M>),
                        dim3(p.nblocks), dim3(NT), 0, s, p);
 }
 template <int NT>
