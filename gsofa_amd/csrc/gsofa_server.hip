@@ -15,9 +15,10 @@
 // of the device budget, loads them into its arena (one upload), runs them as
 // one persistent launch plus the structure and supernode passes, and copies
 // each request's rows straight from the device into its result.  A worker in
-// steady state makes no device allocation, so batches of different workers
-// overlap on the device: requests that arrive while others run start as soon
-// as a worker (slot) and its share of memory are free.
+// steady state makes no device allocation.  One batch loads and runs at a time,
+// beside the copies of those before it, which take several times as long (48^3
+// grid: 6 and 11 ms): what arrives meanwhile shares the next launch instead of
+// the device.
 //
 // Admission: each worker owns budget / max_inflight bytes.  A batch's bytes
 // are its fixed arrays (CSR of A and A^T, per-row arrays, and the fill stream
@@ -75,6 +76,7 @@ struct gsofa_server {
     std::condition_variable cv_done;  // a request became final
     std::condition_variable cv_idle;  // no batch in flight
     int32_t running = 0;              // batches in flight
+    bool loading = false;             // a batch is being loaded or run on the device
     bool exclusive = false;           // a request is waiting for or using the whole budget
     std::deque<Request*> waiting;
     std::unordered_map<int64_t, Request*> live;  // every request not yet taken
@@ -184,6 +186,11 @@ void run_arena(gsofa_server* S, int32_t worker, std::vector<Request*>& batch, in
     for (size_t i = 0; i < batch.size(); i++) mats[i] = &batch[i]->pm;
     if (rc == GSOFA_OK) rc = gsofa::arena_load(A, mats.data(), (int32_t)mats.size(), S->share);
     if (rc == GSOFA_OK) rc = gsofa_plan_execute(A);
+    {  // the next batch, of all that waits by now, beside this one's copies
+        std::lock_guard<std::mutex> lk(S->mu);
+        S->loading = false;
+    }
+    S->cv_work.notify_all();  // one takes what waits; on shutdown all look again
     if (rc == GSOFA_OK) {
         for (size_t i = 0; i < batch.size(); i++) {
             st[i] = gsofa::arena_fetch(A, (int32_t)i, &res[i]);
@@ -230,7 +237,9 @@ void worker_main(gsofa_server* S, int32_t worker) {
     if (hipSetDevice(S->opt.device) != hipSuccess) (void)hipGetLastError();
     std::unique_lock<std::mutex> lk(S->mu);
     for (;;) {
-        S->cv_work.wait(lk, [&] { return (S->stop || !S->waiting.empty()) && !S->exclusive; });
+        S->cv_work.wait(lk, [&] {
+            return (S->stop && S->waiting.empty()) || (!S->waiting.empty() && !S->exclusive && !S->loading);
+        });
         if (S->waiting.empty()) break;  // stopping and drained
         std::vector<Request*> batch;
         int64_t sum_n = 0, sum_nnz = 0;
@@ -274,6 +283,7 @@ void worker_main(gsofa_server* S, int32_t worker) {
                 r->t_start = Clock::now();
                 finish(S, r, GSOFA_ERR_BUDGET);
                 S->cv_done.notify_all();
+                S->cv_work.notify_all();
                 continue;
             }
             // it fits the whole budget (in core or spilled): run it alone once
@@ -292,7 +302,7 @@ void worker_main(gsofa_server* S, int32_t worker) {
         const Clock::time_point t0 = Clock::now();
         for (Request* r : batch) r->t_start = t0;
         S->running++;
-        if (!alone && !S->waiting.empty()) S->cv_work.notify_one();  // another worker may take the rest
+        S->loading = !alone;
         lk.unlock();
         if (alone) run_alone(S, batch[0], id, budget, spill);
         else run_arena(S, worker, batch, id);
