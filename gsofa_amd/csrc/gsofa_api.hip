@@ -2216,8 +2216,8 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
     } else {
         cp.push_back({r->L_rowptr, P->d_Lrp, sizeof(int64_t) * ((size_t)n + 1)});
         cp.push_back({r->U_rowptr, P->d_Urp, sizeof(int64_t) * ((size_t)n + 1)});
-        cp.push_back({r->L_col, P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL});
-        cp.push_back({r->U_col, P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU});
+        cp.push_back({r->L_col, P->d_Lcol, sizeof(int32_t) * (size_t)P->nnzL, true});
+        cp.push_back({r->U_col, P->d_Ucol, sizeof(int32_t) * (size_t)P->nnzU, true});
     }
     fetch_mat_totals(P, cp);
     if (P->supernodes) {
@@ -2228,8 +2228,8 @@ int gsofa_plan_fetch(gsofa_plan* P, gsofa_result* r) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        cp.push_back({r->super_start, P->d_sstart, sizeof(int32_t) * ((size_t)P->n_super + 1)});
-        cp.push_back({r->supno, P->d_supno, sizeof(int32_t) * (size_t)n});
+        cp.push_back({r->super_start, P->d_sstart, sizeof(int32_t) * ((size_t)P->n_super + 1), true});
+        cp.push_back({r->supno, P->d_supno, sizeof(int32_t) * (size_t)n, true});
     }
     HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
     if (r->row_te)
@@ -2432,16 +2432,16 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
     h->xsup[0] = 0;
     std::vector<HostCopy> cp;
     if (n > 0) {
-        cp.push_back({h->xsup, P->d_sstart, sizeof(int32_t) * ((size_t)ns + 1)});
-        cp.push_back({h->supno, P->d_supno, sizeof(int32_t) * (size_t)n});
+        cp.push_back({h->xsup, P->d_sstart, sizeof(int32_t) * ((size_t)ns + 1), true});
+        cp.push_back({h->supno, P->d_supno, sizeof(int32_t) * (size_t)n, true});
         cp.push_back({h->xlcol, d_xl, sizeof(int64_t) * ((size_t)n + 1)});
         cp.push_back({h->xucol, d_xu, sizeof(int64_t) * ((size_t)n + 1)});
     }
-    cp.push_back({h->lrow, d_lrow, sizeof(int32_t) * (size_t)P->nnzL});
-    cp.push_back({h->urow, d_urow, sizeof(int32_t) * (size_t)P->nnzU});
+    cp.push_back({h->lrow, d_lrow, sizeof(int32_t) * (size_t)P->nnzL, true});
+    cp.push_back({h->urow, d_urow, sizeof(int32_t) * (size_t)P->nnzU, true});
     if (ns > 0) {
         cp.push_back({h->xsub, d_xs, sizeof(int64_t) * ((size_t)ns + 1)});
-        cp.push_back({h->sub, d_sub, sizeof(int32_t) * (size_t)nsub});
+        cp.push_back({h->sub, d_sub, sizeof(int32_t) * (size_t)nsub, true});
     }
     HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
     return GSOFA_OK;
@@ -2836,8 +2836,8 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
         HIPCHK_OUT(launch_add(P->d_Lcol + l0, (uint64_t)(l1 - l0), -(int32_t)b0, P->stream), P->stream);
         HIPCHK_OUT(launch_add(P->d_Ucol + u0, (uint64_t)(u1 - u0), -(int32_t)b0, P->stream), P->stream);
     }
-    cp.push_back({r->L_col, P->d_Lcol + l0, sizeof(int32_t) * (size_t)(l1 - l0)});
-    cp.push_back({r->U_col, P->d_Ucol + u0, sizeof(int32_t) * (size_t)(u1 - u0)});
+    cp.push_back({r->L_col, P->d_Lcol + l0, sizeof(int32_t) * (size_t)(l1 - l0), true});
+    cp.push_back({r->U_col, P->d_Ucol + u0, sizeof(int32_t) * (size_t)(u1 - u0), true});
     if (P->supernodes && nb > 0) {
         // supernodes never cross matrices: (i-1) is never in L_i at a boundary
         r->n_super = s1 - s0 + 1;
@@ -2847,8 +2847,8 @@ int arena_fetch(gsofa_plan* P, int32_t index, gsofa_result* r) {
             gsofa_result_free(r);
             return GSOFA_ERR_ALLOC;
         }
-        cp.push_back({r->super_start, P->d_sstart + s0, sizeof(int32_t) * (size_t)r->n_super});
-        cp.push_back({r->supno, P->d_supno + b0, sizeof(int32_t) * (size_t)nb});
+        cp.push_back({r->super_start, P->d_sstart + s0, sizeof(int32_t) * (size_t)r->n_super, true});
+        cp.push_back({r->supno, P->d_supno + b0, sizeof(int32_t) * (size_t)nb, true});
     }
     HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
     if (r->supno) {

@@ -12,11 +12,17 @@
 //     but 10 us apart from the next and one for each array.)  A single thread
 //     that first touches the destination moves 14 GB/s, so larger totals take
 //     up to kThreads threads.
-// Fetch us by pageable copies / this with the runtime's copies / with kernels:
-// 64 x 64 grid (2.2 MB) 230 / 250 / 97; band of 11,948 (9.9 MB) 2230 / 900 /
-// 310; 27^3 grid (49 MB) 4170 / 1570 / 1290; 33^3 (127 MB) 9490 / 3300 / 2900;
-// 48^3 (874 MB) 22200 / 18900 / 17200, 51 GB/s of the link's 57.  16 MB buffers
-// instead of 4: 33^3 6.8 ms; 1 MB a thread instead of 2: 64 x 64 128 us.
+// Vertex numbers make up nearly all of a result, and neighbouring ones are
+// close: rows are sorted and follow each other.  They cross the link as 16-bit
+// offsets, 64 to a base, and the thread that would copy them adds the base
+// (host rate of either: 120 GB/s at eight threads, twice the link's); a block of
+// a wider range, as where a row of far-spread columns ends, crosses as it is.
+// Fetch us by pageable copies / through pinned buffers by the runtime's copies /
+// by kernels / as 16-bit offsets: 64 x 64 grid (2.2 MB) 230 / 250 / 97 / 77;
+// band of 11,948 (9.9 MB) 2230 / 900 / 310 / 220; 27^3 grid (49 MB) 4170 / 1570
+// / 1290 / 1110; 33^3 (127 MB) 9490 / 3300 / 2900 / 2250; 48^3 (874 MB) 22200 /
+// 18900 / 17200 / 10000, where the link alone took 15300.  Eight threads instead
+// of 12: 2.40 and 11.3 ms; 16: the same.  16 MB buffers: 33^3 6.8 ms.
 // Result arrays start on 2 MB boundaries with transparent huge pages requested,
 // since their first touch is in this path.
 #include <algorithm>
@@ -35,13 +41,16 @@ namespace gsofa {
 
 namespace {
 
-constexpr size_t kStageBytes = 4u << 20;
-constexpr size_t kStageKeep = 64;          // idle staging buffers kept: four copies at once
-constexpr size_t kStageRest = 16;          // and after the last plan's release, one copy's (64 MB:
-                                           // making and releasing them takes over 1 ms)
+constexpr uint32_t kBlock = 64;             // indexes that share a base
+constexpr size_t kChunkMost = 4u << 20;    // bytes of result in a chunk, and what they take as
+                                           // bases, 16-bit offsets and room for whole blocks
+constexpr size_t kStageBytes = kChunkMost / (4 * kBlock) * (4 + 6 * kBlock) + (16u << 10);
+constexpr size_t kStageKeep = 48;          // idle staging buffers kept: two large copies at once
+constexpr size_t kStageRest = 24;          // and after the last plan's release, one copy's (146 MB:
+                                           // making and releasing them takes over 2 ms)
 constexpr size_t kKernelMost = 512u << 10; // totals up to here: one kernel
 constexpr size_t kPerThread = 2u << 20;     // bytes per copy thread, at least
-constexpr int kThreads = 8;
+constexpr int kThreads = 12;
 constexpr size_t kChunkMin = 1u << 20;
 constexpr size_t kChunks = 4;              // chunks a thread, at least
 constexpr size_t kHugePage = 2u << 20;
@@ -94,8 +103,82 @@ struct Pieces {
     uint32_t* dst[MAX];
     const uint32_t* src[MAX];
     uint32_t words[MAX];
+    bool index[MAX];  // packed on the way out: dst is the piece's bases
     int count;
 };
+
+// An index piece in a staging buffer: a word for every block (its smallest
+// value, or WIDE), then the blocks' 16-bit offsets, then their places as they
+// are, used by blocks of a wider range only.
+constexpr uint32_t WIDE = 0x80000000u;
+__host__ __device__ constexpr uint32_t blocks_of(uint32_t words) { return (words + kBlock - 1) / kBlock; }
+__host__ __device__ constexpr size_t offsets_at(uint32_t words) { return ((size_t)blocks_of(words) * 4 + 15) & ~(size_t)15; }
+__host__ __device__ constexpr size_t wide_at(uint32_t words) {
+    return offsets_at(words) + (size_t)blocks_of(words) * kBlock * 2;
+}
+constexpr size_t index_bytes(uint32_t words) { return wide_at(words) + (size_t)blocks_of(words) * kBlock * 4; }
+
+struct __attribute__((packed, aligned(4))) Quad {
+    uint32_t x, y, z, w;
+};
+
+// Eight lanes a block, eight values a lane.
+__device__ void pack_piece(uint32_t* bases, const uint32_t* src, uint32_t words, uint32_t t, uint32_t step) {
+    char* const b = reinterpret_cast<char*>(bases);
+    uint4* const offs = reinterpret_cast<uint4*>(b + offsets_at(words));
+    uint4* const wide = reinterpret_cast<uint4*>(b + wide_at(words));
+    const uint32_t lanes = blocks_of(words) * (kBlock / 8u);
+    for (uint32_t i = t; i < lanes; i += step) {  // the lanes of a block stay together
+        const uint32_t e = i * 8u;
+        uint32_t v[8];
+        if (e + 8u <= words) {
+            const Quad a = *reinterpret_cast<const Quad*>(src + e), c = *reinterpret_cast<const Quad*>(src + e + 4u);
+            v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+            v[4] = c.x, v[5] = c.y, v[6] = c.z, v[7] = c.w;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; k++) v[k] = e + k < words ? src[e + k] : src[words - 1u];
+        }
+        uint32_t lo = v[0], hi = v[0];
+#pragma unroll
+        for (uint32_t k = 1; k < 8u; k++) {
+            lo = v[k] < lo ? v[k] : lo;
+            hi = v[k] > hi ? v[k] : hi;
+        }
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) {
+            const uint32_t ol = __shfl_xor(lo, d, 8), oh = __shfl_xor(hi, d, 8);
+            lo = ol < lo ? ol : lo;
+            hi = oh > hi ? oh : hi;
+        }
+        const bool fits = hi - lo < 65536u;
+        if ((i & 7u) == 0u) bases[i >> 3] = fits ? lo : WIDE;
+        if (fits) {
+            offs[i] = make_uint4((v[0] - lo) | ((v[1] - lo) << 16), (v[2] - lo) | ((v[3] - lo) << 16),
+                                 (v[4] - lo) | ((v[5] - lo) << 16), (v[6] - lo) | ((v[7] - lo) << 16));
+        } else {
+            wide[2u * i] = make_uint4(v[0], v[1], v[2], v[3]);
+            wide[2u * i + 1u] = make_uint4(v[4], v[5], v[6], v[7]);
+        }
+    }
+}
+
+void unpack_piece(uint32_t* dst, const char* b, uint32_t words) {
+    const uint32_t* bases = reinterpret_cast<const uint32_t*>(b);
+    const uint16_t* offs = reinterpret_cast<const uint16_t*>(b + offsets_at(words));
+    const uint32_t* wide = reinterpret_cast<const uint32_t*>(b + wide_at(words));
+    for (uint32_t k = 0, e = 0; e < words; k++, e += kBlock) {
+        const uint32_t lo = bases[k];
+        const uint16_t* o = offs + e;
+        uint32_t* d = dst + e;
+        if (lo == WIDE) std::memcpy(d, wide + e, 4 * std::min(kBlock, words - e));
+        else if (words - e >= kBlock)
+            for (uint32_t j = 0; j < kBlock; j++) d[j] = lo + o[j];
+        else
+            for (uint32_t j = 0; j < words - e; j++) d[j] = lo + o[j];
+    }
+}
+
 
 // Pieces whose two ends have the same alignment to 16 bytes move in 16-byte
 // words but for their ends, the others word by word.
@@ -105,6 +188,10 @@ __global__ __launch_bounds__(256) void k_copy_pieces(Pieces p) {
         uint32_t* d = p.dst[k];
         const uint32_t* s = p.src[k];
         const uint32_t n = p.words[k];
+        if (p.index[k]) {
+            pack_piece(d, s, n, t, step);
+            continue;
+        }
         const uint32_t off = (uint32_t)(reinterpret_cast<uintptr_t>(d) >> 2) & 3u;
         uint32_t head = n, body = 0;
         if (((reinterpret_cast<uintptr_t>(d) ^ reinterpret_cast<uintptr_t>(s)) & 15u) == 0) {
@@ -133,7 +220,8 @@ struct Piece {
     char* host;
     char* dev;
     size_t bytes;
-    size_t off;  // in the chunk's buffer: aligned to 16 bytes as dev is
+    size_t off;  // in the chunk's buffer: aligned to 16 bytes, unless packed as dev is
+    bool index;  // packed
 };
 
 // `out`: device to host, else host to device.
@@ -170,7 +258,8 @@ hipError_t copy_chunks(const std::vector<Piece>& pieces, const std::vector<Chunk
     auto host_side = [&](size_t k, char* b) {
         for (size_t i = chunks[k].first; i < chunks[k].first + chunks[k].count; i++) {
             const Piece& c = pieces[i];
-            if (out) std::memcpy(c.host, b + c.off, c.bytes);
+            if (c.index) unpack_piece(reinterpret_cast<uint32_t*>(c.host), b + c.off, (uint32_t)(c.bytes / 4));
+            else if (out) std::memcpy(c.host, b + c.off, c.bytes);
             else std::memcpy(b + c.off, c.host, c.bytes);
         }
     };
@@ -183,6 +272,7 @@ hipError_t copy_chunks(const std::vector<Piece>& pieces, const std::vector<Chunk
             uint32_t* dv = reinterpret_cast<uint32_t*>(c.dev);
             p.dst[p.count] = out ? st : dv;
             p.src[p.count] = out ? dv : st;
+            p.index[p.count] = c.index;
             p.words[p.count++] = (uint32_t)(c.bytes / 4);
             bytes += c.bytes;
         }
@@ -249,22 +339,25 @@ hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
         const hipError_t w = hipStreamSynchronize(s);
         return e == hipSuccess ? w : e;
     }
-    const size_t ch = std::min(kStageBytes, std::max(kChunkMin, total / (kChunks * (size_t)threads)));
+    const size_t ch = std::min(kChunkMost, std::max(kChunkMin, total / (kChunks * (size_t)threads)));
     std::vector<Piece> pieces;
     std::vector<Chunk> chunks;
-    size_t at = ch;  // bytes of the last chunk's buffer in use
+    size_t room = 0, at = 0;  // of the last chunk: bytes of result left, bytes of its buffer in use
     for (const HostCopy& c : v)
         for (size_t o = 0; o < c.bytes;) {
             char* dev = (char*)c.dev + o;
-            size_t off = ((at + 15) & ~(size_t)15) + ((uintptr_t)dev & 15u);
-            if (off + 4 > ch || chunks.back().count == (size_t)Pieces::MAX) {
+            if (room < 4 || chunks.back().count == (size_t)Pieces::MAX) {
                 chunks.push_back({pieces.size(), 0});
-                off = (uintptr_t)dev & 15u;
+                room = ch;
+                at = 0;
             }
-            const size_t len = std::min((ch - off) & ~(size_t)3, c.bytes - o);
-            pieces.push_back({(char*)c.host + o, dev, len, off});
+            const bool index = out && c.index;
+            const size_t len = std::min(room & ~(size_t)3, c.bytes - o);
+            const size_t off = ((at + 15) & ~(size_t)15) + (index ? 0 : (uintptr_t)dev & 15u);
+            pieces.push_back({(char*)c.host + o, dev, len, off, index});
             chunks.back().count++;
-            at = off + len;
+            at = off + (index ? index_bytes((uint32_t)(len / 4)) : len);
+            room -= len;
             o += len;
         }
     int device = 0;

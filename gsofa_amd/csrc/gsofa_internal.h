@@ -252,6 +252,7 @@ struct HostCopy {
     void* host;
     void* dev;
     size_t bytes;
+    bool index = false;  // 4-byte values from 0 to 2^31 - 1: may cross as 16-bit offsets
 };
 hipError_t copy_out(const std::vector<HostCopy>& v, hipStream_t s);
 hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s);

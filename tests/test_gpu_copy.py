@@ -48,6 +48,28 @@ def test_result_sizes(n, b):
     np.testing.assert_array_equal(h.xlcol[1:], np.cumsum(np.bincount(key // n, minlength=n)))
 
 
+def test_wide_ranges():
+    """Columns further apart than 16 bits, within rows and where rows meet."""
+    import gsofa_amd as g
+    n = 140003
+    rng = np.random.default_rng(8)
+    i = np.arange(n, dtype=np.int64)
+    f = i[::3]
+    rows = np.concatenate([i, i, f, np.minimum(f + 1, n - 1), i[-400:]])
+    cols = np.concatenate([i, np.minimum(i + 1, n - 1), n - 1 - f % 37, f, rng.integers(0, n - 400, 400)])
+    key = np.unique(rows * n + cols)
+    end = np.cumsum(np.bincount(key // n, minlength=n))
+    A = g.CsrMatrix(n, np.concatenate([[0], end[:-1]]), end, key % n)
+    o = _oracle(A)
+    assert np.abs(np.diff(o.U_col)).max() > 65536
+    assert_same_structure(g.symbfact(A), o)
+    with g.Plan(A) as plan:
+        plan.execute()
+        h = plan.fetch_supernodal()
+    key = np.sort(np.asarray(o.U_col, np.int64) * n + np.repeat(np.arange(n), np.diff(o.U_rowptr)))
+    np.testing.assert_array_equal(h.urow, (key % n).astype(np.int32))
+
+
 def test_concurrent_results():
     import gsofa_amd as g
     mats = [_full_band(n, b) for n, b in SIZES[2:7]]
