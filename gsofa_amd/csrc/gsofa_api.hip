@@ -765,17 +765,21 @@ uint64_t default_fill_cap(int64_t nnz) { return std::max<uint64_t>(64 * (uint64_
 // small 2D meshes (where 8 is best) and the best on 3D meshes.  A single
 // matrix with nsrc sources takes the largest of 32, 16, 8 whose chunks still
 // give every co-resident workgroup one.
-// A share (n_virtual_gpu > 1) is judged by `skew`, its largest subtree over the
-// mean.  Bands and naturally ordered grids (2.0 to 2.3) are done when all
-// workgroups are: the smallest slot count of at least 8 with up to four chunks
-// a CU; at 32 / 16 / 8 / 4 slots 10,000 sources of a band of 20,000 take 6.0 /
-// 3.7 / 5.1 / 9.5 ms, 4,133 of one of 12,397 2.9 / 1.9 / 1.6 / 2.7.  Nested
-// dissection (3.8 and more) is done when the deepest chunk is, and the fewer
-// its slots the sooner: 2, up to 16 chunks a CU.  At 16 / 8 / 4 / 2 slots a
-// quarter of a 21^3 grid takes 10.5 / 6.9 / 5.3 / 4.1 ms, half of a 24^3 25.2 /
-// 17.4 / 13.2 / 10.3, a third of a 128^2 40.4 / 21.2 / 14.9 / 10.8, an eighth
-// of a 12^3 1.34 / 0.82 / 0.71 / 0.61.
-int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots, double skew) {
+// A share (n_virtual_gpu > 1) is judged by whether its labels fit LDS and by
+// `skew`, its largest subtree over the mean.
+//  In LDS: bands and naturally ordered grids (skew 2.0 to 2.3) are done when all
+//  workgroups are: 4 slots, 2 with few sources or where 4 do not fit.  At 8 / 4 /
+//  2 / 1 slots 750 sources of a band of 3,000 take 0.31 / 0.24 / 0.20 / 0.24 ms,
+//  1,800 of a 60^2 grid 0.53 / 0.46 / 0.60 / 0.88, 4,133 of a band of 12,397 (2
+//  and 1 fit) 1.57 / - / 1.24 / 1.78.  Nested dissection (3.8 and more) is done
+//  when the deepest group is: one source each, two where there are many and two
+//  fit.  At 4 / 2 / 1 a quarter of a 21^3 grid takes 5.5 / 0.92 / 0.78, an eighth
+//  of a 12^3 0.33 / 0.25 / 0.20, half of a 17^3 0.68 / 0.53 / 0.56, half of a 24^3
+//  (1 fits) 12.8 / 10.2 / 2.6, a third of a 128^2 (1 fits) 15.0 / 10.9 / 2.6.
+//  In memory: with little skew the smallest slot count of at least 8 with up to
+//  four chunks a CU (10,000 sources of a band of 20,000 at 32 / 16 / 8 / 4: 6.0 /
+//  3.7 / 5.1 / 9.5 ms), else from 2 up to 16 chunks a CU.
+int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, uint32_t W, int* slots, double skew) {
     if (o.block_slots != 0) {
         if (!blk_slots_valid(o.block_slots)) return GSOFA_ERR_INVALID;
         *slots = o.block_slots;
@@ -791,8 +795,16 @@ int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slo
         return GSOFA_ERR_HIP;
     }
     if (o.n_virtual_gpu > 1 && skew > 0) {
-        const uint64_t most = (skew < 3.0 ? 4ull : 16ull) * (uint64_t)cus;
-        int S = skew < 3.0 ? 8 : 2;
+        const bool level = skew < 3.0;
+        int S = level ? (nsrc <= 4ull * cus ? 2 : 4) : (nsrc <= 10ull * cus ? 1 : 2);
+        if (S == 4 && !blk_in_lds(4, W)) S = 2;
+        if (S == 2 && !level && !blk_in_lds(2, W)) S = 1;
+        if (blk_in_lds(S, W)) {
+            *slots = S;
+            return GSOFA_OK;
+        }
+        const uint64_t most = (level ? 4ull : 16ull) * (uint64_t)cus;
+        S = level ? 8 : 2;
         while (S < kBlockSlots && (nsrc + S - 1) / S > most) S *= 2;
         *slots = S;
         return GSOFA_OK;
@@ -1130,7 +1142,7 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         cols = (int64_t)(nl + nu);
     }
     int S = 0;
-    if (choose_slots(o, 1, share_count(A->n, N, 0), &S, skew) != GSOFA_OK) return -1;
+    if (choose_slots(o, 1, share_count(A->n, N, 0), (uint32_t)A->n, &S, skew) != GSOFA_OK) return -1;
     const uint64_t nchunks = (share_count(A->n, N, 0) + S - 1) / S;
     uint32_t nb = 0;
     if (block_grid(o, S, nchunks, (uint32_t)A->n, INT64_MAX / 4, &nb) != GSOFA_OK) return -1;
@@ -1329,7 +1341,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     } else if (P->mode == GSOFA_MODE_BLOCK) {
         int S = 0;
         const uint64_t nsrc = P->hybrid ? P->s_top : share_count(n, P->opt.n_virtual_gpu, 0);
-        rc = choose_slots(P->opt, n_mats, nsrc, &S, skew);
+        rc = choose_slots(P->opt, n_mats, nsrc, P->W, &S, skew);
         P->S = (uint32_t)S;
         if (!rc) build_chunks(P);
         if (!rc) rc = size_block_mode(P, std::max<int64_t>(avail, 1 << 20));

@@ -4,7 +4,8 @@
 // (with_space_optimization/symbfact.cuh:883-1082) and seeding (:639-721), with
 // an execution model built for CDNA4:
 //
-// * Each workgroup (16 waves, one per CU) of a persistent grid owns //   slots (32, 16, 8, 4 or 2; one kernel instance each) and runs a "mini-group" of
+// * Each workgroup (16 waves, one per CU) of a persistent grid owns //   slots (32, 16, 8, 4 or 2; one kernel instance each; what fits is run in LDS
+//   alone, k_traverse_lds) and runs a "mini-group" of
 //   SL consecutive sources through all of their frontier levels by itself,
 //   synchronising only with __syncthreads.  The next mini-group comes from
 //   one global counter.  There is no grid-wide barrier and no hot global
@@ -678,22 +679,282 @@ __global__ __launch_bounds__(BB) __attribute__((amdgpu_waves_per_eu(GSOFA_WPE, G
     }
 }
 
+// ---- the same traversal with all its state in LDS
+//
+// Where a matrix's labels for SL slots fit a CU's LDS, with a byte of pending
+// slots and two queue places a vertex, an edge needs no target table and no
+// relax phase: it lowers its target's label by an LDS atomic min, and who sets
+// a pending bit of a vertex with none queues the vertex.  A level is one
+// barrier and two dependent reads of memory (row, edges).  Fills, TE and |R|
+// are read off the final labels: 0 marks A's own neighbours, 1 + max id the
+// others, so a vertex below the source is an L entry iff its label is at most
+// its own number, one above it a U entry iff it has a label.
+// What bounds it: the two reads of a level and the deepest group's levels; few
+// slots keep a group's levels narrow and let larger matrices in (1: 18,000
+// vertices, 2: 12,500, 4: 7,700, 8: 4,400).  Traversal ms against labels in
+// memory at the same slots: quarter of a 21^3 grid, 2 slots, 3.9 -> 0.70; half of
+// a 60^2 in natural order, 8, 1.27 -> 0.44; band of 3,000, 8, 0.44 -> 0.23.
+struct LShare {
+    uint32_t nq[3], ncur[3];        // queue sizes and cursors, by level modulo 3
+    uint32_t chunk;
+    uint32_t wsum[BW];
+    unsigned long long te[8], reach[8], fill[8];  // by slot
+    unsigned long long acc[4];
+    unsigned long long base;
+};
+
+template <int SL>
+constexpr uint32_t lds_words(uint32_t W) { return W * SL + (W + 3u) / 4u + (2u * W + 1u) / 2u + 1u; }
+
+template <int SL>
+__global__ __launch_bounds__(BB) void k_traverse_lds(BlkParams p) {
+    constexpr int G = 4, E = 3;     // lanes per vertex, edges per lane and step
+    extern __shared__ uint32_t dyn[];
+    __shared__ LShare S;
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / WAVE;
+    const uint32_t grp = lane / G, j = lane % G;
+    uint32_t* const lab = dyn;
+    uint32_t* const pm = lab + p.W * SL;
+    uint16_t* const qs = reinterpret_cast<uint16_t*>(pm + (p.W + 3u) / 4u);
+    unsigned long long checks = 0, levels = 0;
+    if (tid < 4) S.acc[tid] = 0;
+    // adds slots `bits` to vertex m's pending ones; true if it had none
+    auto pend = [&](uint32_t m, uint32_t bits) {
+        const uint32_t sh = 8u * (m & 3u);
+        return ((atomicOr(&pm[m >> 2], bits << sh) >> sh) & 0xFFu) == 0u;
+    };
+    for (;;) {
+        if (tid == 0) {
+            S.chunk = atomicAdd(&p.ctrl->src_next, 1u);
+            for (int k = 0; k < 3; k++) S.nq[k] = S.ncur[k] = 0;
+        }
+        if (tid < 8) S.te[tid] = S.reach[tid] = S.fill[tid] = 0;
+        __syncthreads();
+        const uint32_t ck = S.chunk;
+        if (ck >= p.n_chunks) break;
+        const BlkChunk C = p.chunks[ck];
+        const uint32_t nsrc = C.count;
+        const uint32_t wb = p.mat_base[C.mat], nv = p.mat_base[C.mat + 1u] - wb;
+        uint32_t src[SL];  // window-local; slots past nsrc never get a bit
+#pragma unroll
+        for (int k = 0; k < SL; k++) src[k] = (uint32_t)k < nsrc ? C.first - (uint32_t)k * C.stride - wb : 0u;
+        for (uint32_t i = tid; i < nv * SL; i += BB) lab[i] = INF;
+        for (uint32_t i = tid; i < (nv + 3u) / 4u; i += BB) pm[i] = 0u;
+        __syncthreads();
+        // level 0: the sources' neighbours, those below queued
+#pragma unroll
+        for (int k = 0; k < SL; k++) {
+            if ((uint32_t)k >= nsrc) continue;
+            const uint32_t b = (uint32_t)p.rp[wb + src[k]], e = (uint32_t)p.rp[wb + src[k] + 1u];
+            if (tid == 0) {
+                lab[src[k] * SL + k] = 0u;
+                checks += e - b;
+            }
+            for (uint32_t i = b + tid; i < e; i += BB) {
+                const uint32_t m = (uint32_t)p.ci[i] - wb;
+                lab[m * SL + k] = 0u;
+                if (m < src[k] && pend(m, 1u << k)) qs[atomicAdd(&S.nq[0], 1u)] = (uint16_t)m;
+            }
+        }
+        for (uint32_t lev = 0;; lev++) {
+            __syncthreads();
+            const uint32_t size = S.nq[lev % 3u], nb = (lev + 1u) % 3u;
+            if (size == 0u) break;
+            levels += tid == 0 ? 1u : 0u;
+            if (tid == 0) S.nq[(lev + 2u) % 3u] = S.ncur[(lev + 2u) % 3u] = 0;  // last read a barrier ago
+            const uint16_t* qc = qs + (lev & 1u) * p.W;
+            uint16_t* qn = qs + ((lev + 1u) & 1u) * p.W;
+            bool held = false, done = false;
+            uint32_t pos = 0, end = 0, cost[SL];
+            for (;;) {
+                const bool want = !held && !done;
+                const uint64_t wl = __ballot(want && j == 0u);
+                if (wl) {
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(&S.ncur[lev % 3u], (uint32_t)__popcll(wl));
+                    base = bcast0(base);
+                    if (want) {
+                        const uint32_t idx = base + (uint32_t)__popcll(wl & ((1ull << (G * grp)) - 1ull));
+                        if (idx >= size) {
+                            done = true;
+                        } else {
+                            const uint32_t v = qc[idx], sh = 8u * (v & 3u);
+                            pos = (uint32_t)p.rp[wb + v];
+                            end = (uint32_t)p.rp[wb + v + 1u];
+                            uint32_t M = 0;
+                            if (j == 0u) M = (atomicAnd(&pm[v >> 2], ~(0xFFu << sh)) >> sh) & 0xFFu;
+                            M = __shfl(M, 0, G);
+#pragma unroll
+                            for (int k = 0; k < SL; k++) {  // symbfact.cuh:924
+                                const uint32_t l = lab[v * SL + k];
+                                cost[k] = (M >> k) & 1u ? (v + 1u > l ? v + 1u : l) : INF;
+                            }
+                            if (j == 0u) checks += (unsigned long long)(end - pos) * (uint32_t)__popc(M);
+                            held = pos < end;
+                        }
+                    }
+                }
+                if (!__ballot(held)) {
+                    if (__ballot(!done)) continue;
+                    break;
+                }
+                uint32_t m[E];
+#pragma unroll
+                for (int q = 0; q < E; q++) {
+                    const uint32_t e = pos + j + (uint32_t)(G * q);
+                    m[q] = held && e < end ? (uint32_t)p.ci[e] - wb : INF;
+                }
+#pragma unroll
+                for (int q = 0; q < E; q++) {
+                    bool enq = false;
+                    if (m[q] != INF) {
+                        uint32_t bits = 0;
+#pragma unroll
+                        for (int k = 0; k < SL; k++) {
+                            if (cost[k] == INF) continue;
+                            uint32_t* const at = &lab[m[q] * SL + k];
+                            const uint32_t l = *at;
+                            if (m[q] > src[k]) {  // above: any label will do (symbfact.cuh:992-1009)
+                                if (l == INF) *at = cost[k];
+                            } else if (l > cost[k] && atomicMin(at, cost[k]) > cost[k]) {  // :1018-1063
+                                bits |= 1u << k;
+                            }
+                        }
+                        enq = bits && pend(m[q], bits);
+                    }
+                    const uint64_t em = __ballot(enq);
+                    if (em) {
+                        uint32_t qb = 0;
+                        if (lane == 0) qb = atomicAdd(&S.nq[nb], (uint32_t)__popcll(em));
+                        qb = bcast0(qb);
+                        if (enq) qn[qb + rank_in(em)] = (uint16_t)m[q];
+                    }
+                }
+                if (held) {
+                    pos += (uint32_t)(G * E);
+                    held = pos < end;
+                }
+            }
+        }
+        // the final labels: per slot TE, |R_<(s)| and fills; each thread's fills
+        // take places in its order of vertices
+        uint32_t mine = 0;
+        auto is_fill = [&](uint32_t m, int k, uint32_t l) {
+            return l != 0u && l != INF && (m > src[k] || l < m + 1u);
+        };
+#pragma unroll
+        for (int k = 0; k < SL; k++) {
+            if ((uint32_t)k >= nsrc) continue;
+            unsigned long long te = 0, reach = 0;
+            uint32_t fill = 0;
+            for (uint32_t m = tid; m < nv; m += BB) {
+                const uint32_t l = lab[m * SL + k];
+                if (l == INF) continue;
+                fill += is_fill(m, k, l) ? 1u : 0u;
+                if (m < src[k]) {
+                    reach++;
+                    te += (uint32_t)(p.rp[wb + m + 1u] - p.rp[wb + m]);
+                }
+            }
+            mine += fill;
+            te = wave_sum64(te);
+            reach = wave_sum64(reach);
+            const unsigned long long f = wave_sum64(fill);
+            if (lane == 0) {
+                if (te) atomicAdd(&S.te[k], te);
+                if (reach) atomicAdd(&S.reach[k], reach);
+                if (f) atomicAdd(&S.fill[k], f);
+            }
+        }
+        const uint32_t incl = wave_incl_scan(mine);
+        if (lane == WAVE - 1) S.wsum[w] = incl;
+        __syncthreads();
+        if (tid < nsrc) {
+            const uint32_t s = C.first - tid * C.stride;
+            const unsigned long long te = S.te[tid] + (uint32_t)(p.rp[s + 1] - p.rp[s]);
+            p.row_te[s] = te;
+            p.row_reach[s] = S.reach[tid];
+            p.row_fills[s] = S.fill[tid];
+            atomicAdd(&S.acc[0], S.fill[tid]);
+            atomicAdd(&S.acc[1], te);
+            atomicAdd(&S.acc[2], S.reach[tid]);
+        }
+        if (p.fill_cap != 0ull) {
+            uint32_t before = incl - mine, all = 0;
+            for (uint32_t k = 0; k < (uint32_t)BW; k++) {
+                if (k < w) before += S.wsum[k];
+                all += S.wsum[k];
+            }
+            if (tid == 0 && all) S.base = aadd64(&p.ctrl->fill_pos, all);
+            __syncthreads();
+            uint64_t at = S.base + before;
+#pragma unroll
+            for (int k = 0; k < SL; k++) {
+                if ((uint32_t)k >= nsrc) continue;
+                const uint64_t row = (uint64_t)(src[k] + wb) << 32;
+                for (uint32_t m = tid; m < nv; m += BB) {
+                    if (!is_fill(m, k, lab[m * SL + k])) continue;
+                    if (at < p.fill_cap) p.fills[at] = row | (m + wb);
+                    at++;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (checks) atomicAdd(&S.acc[3], checks);
+    __syncthreads();
+    if (tid == 0) {
+        if (S.acc[0]) aadd64(&p.ctrl->fill_count, S.acc[0]);
+        if (S.acc[1]) aadd64(&p.ctrl->te, S.acc[1]);
+        if (S.acc[2]) aadd64(&p.ctrl->reach, S.acc[2]);
+        if (S.acc[3]) aadd64(&p.ctrl->edge_checks, S.acc[3]);
+        aadd64(&p.ctrl->levels, levels);
+    }
+}
+
+constexpr uint32_t LDS_MOST = (160u * 1024u - (uint32_t)sizeof(LShare) - 64u) / 4u * 4u;
+
+// Dynamic LDS of k_traverse_lds for `slots` slots and matrices of up to W
+// vertices; 0 where that is not built or does not fit a CU.
+uint32_t lds_state_bytes(int slots, uint32_t W) {
+    if (W >= 65536u) return 0;
+    const uint32_t words = slots == 1 ? lds_words<1>(W) : slots == 2 ? lds_words<2>(W) : slots == 4 ? lds_words<4>(W) : slots == 8 ? lds_words<8>(W) : ~0u / 4u;
+    return words <= LDS_MOST / 4u ? words * 4u : 0u;
+}
+
+template <int SL>
+hipError_t launch_lds(const BlkParams& p, uint32_t bytes, hipStream_t s) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_traverse_lds<SL>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_MOST);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_traverse_lds<SL>, dim3(p.nblocks), dim3(BB), bytes, s, p);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 bool blk_slots_valid(int slots) { return slots == 32 || slots == 16 || slots == 8; }
-bool blk_slots_built(int slots) { return blk_slots_valid(slots) || slots == 4 || slots == 2; }
+bool blk_slots_built(int slots) { return blk_slots_valid(slots) || slots == 4 || slots == 2 || slots == 1; }
+bool blk_in_lds(int slots, uint32_t W) { return lds_state_bytes(slots, W) != 0; }
 int blk_block_size() { return BB; }
 const void* blk_kernel_ptr(int slots) {
     switch (slots) {
         case 16: return reinterpret_cast<const void*>(&k_traverse_blk<16>);
         case 8: return reinterpret_cast<const void*>(&k_traverse_blk<8>);
         case 4: return reinterpret_cast<const void*>(&k_traverse_blk<4>);
+        case 1:  // runs in LDS only: one workgroup a CU, as this one
         case 2: return reinterpret_cast<const void*>(&k_traverse_blk<2>);
         default: return reinterpret_cast<const void*>(&k_traverse_blk<32>);
     }
 }
 
 hipError_t launch_traverse_blk(const BlkParams& p, int slots, size_t lds_bytes, hipStream_t s) {
+    if (const uint32_t state = lds_state_bytes(slots, p.W)) {
+        if (slots == 1) return launch_lds<1>(p, state, s);
+        if (slots == 2) return launch_lds<2>(p, state, s);
+        if (slots == 4) return launch_lds<4>(p, state, s);
+        return launch_lds<8>(p, state, s);
+    }
     switch (slots) {
         case 32: hipLaunchKernelGGL(k_traverse_blk<32>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;
         case 16: hipLaunchKernelGGL(k_traverse_blk<16>, dim3(p.nblocks), dim3(BB), lds_bytes, s, p); break;

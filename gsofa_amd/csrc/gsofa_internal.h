@@ -106,7 +106,8 @@ struct BlkParams {
 int blk_block_size();
 bool blk_slots_valid(int slots);
 bool blk_slots_built(int slots);
-int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, int* slots, double skew = 0);
+bool blk_in_lds(int slots, uint32_t W);
+int choose_slots(const gsofa_options& o, int32_t n_mats, uint64_t nsrc, uint32_t W, int* slots, double skew = 0);
 // Block-mode sizing shared by plan creation, footprints and the server.
 int64_t block_bytes(uint32_t nb, uint32_t W, int slots);
 // cols: L + U column entries reserved (sorted + staging, 8 B each); < 0 means

@@ -102,7 +102,7 @@ typedef struct gsofa_options {
                                   /* groups (GSOFA_MODE_HYBRID); 0 = none                   */
     int32_t block_slots;          /* block mode: sources per workgroup, 32, 16 or 8; 0 =    */
                                   /* chosen (one share: 32, or fewer with few chunks; a     */
-                                  /* share of several: also 4 and 2, by its subtrees).  Reach */
+                                  /* share of several: also 4 to 1, by its subtrees).  Reach  */
                                   /* mode: 32, 64, 128 or 256 (bits of a visited word);      */
                                   /* 0 = 64, or 32 when fewer chunks than workgroups        */
     int32_t workgroup_threads;    /* reach mode: threads per workgroup, 1024 (one per CU,   */
