@@ -82,3 +82,12 @@ def test_windows(bits):
     for threads in (0, 512):
         print("case", bits, threads, A.nnz, flush=True)
         assert_same_structure(g.symbfact(A, mode="reach", block_slots=bits, workgroup_threads=threads), o)
+
+
+@pytest.mark.parametrize("bits", [32, 64, 256])
+@pytest.mark.parametrize("n,band,lam", [(1500, 200, 12.0), (6011, 250, 9.0), (5000, 2500, 14.0)])
+def test_shared_targets(n, band, lam, bits):
+    """Classes whose members share targets, which their rows hold once."""
+    import gsofa_amd as g
+    A = g.gen_band(n, band, lam, n)
+    assert_same_structure(g.symbfact(A, mode="reach", block_slots=bits), _oracle(A))
