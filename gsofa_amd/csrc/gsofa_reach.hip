@@ -10,11 +10,10 @@
 // So one kernel answers both: over A it yields U rows, |R| and TE exactly as
 // the reference's traversal does for U (with_space_optimization/
 // symbfact.cuh:883-1082, the "m > src" branch at :992-1009); over A^T it
-// yields L columns, written to the fill stream as (row, column) pairs so the
-// structure pass builds the same sorted rows.  Each (vertex, source) pair is
-// expanded at most once, where the reference's max-id labels re-expand a
-// vertex each time its label drops (2-10 times per pair on 3D
-// nested-dissection grids).
+// yields L columns, from whose records the same sorted rows are built.  Each
+// (vertex, source) pair is expanded at most once, where the reference's max-id
+// labels re-expand a vertex each time its label drops (2-10 times per pair on
+// 3D nested-dissection grids).
 //
 // Execution model (CDNA4, persistent grid of co-resident workgroups: one of
 // 1024 threads per CU with the largest tables, or two of 512 threads or four of

@@ -9,7 +9,7 @@
 //
 // max_inflight worker threads each own an arena: a reach-mode plan with its
 // own HIP stream whose device buffers (CSR of A and A^T, per-workgroup
-// visited words, masks and queues, fill stream, L/U columns, per-row arrays)
+// visited words, masks and queues, records, L/U columns, per-row arrays)
 // grow to the largest batch the worker has run and then stay.  A free worker
 // admits the waiting requests, oldest first, while the batch fits its share
 // of the device budget, loads them into its arena (one upload), runs them as
@@ -21,7 +21,7 @@
 // the device.
 //
 // Admission: each worker owns budget / max_inflight bytes.  A batch's bytes
-// are its fixed arrays (CSR of A and A^T, per-row arrays, and the fill stream
+// are its fixed arrays (CSR of A and A^T, per-row arrays, and the records
 // and output columns sized from the requests' bounds; reach_fixed_bytes) plus
 // its traversal workgroups, which take what the fixed part leaves of the share
 // (reach_grid).  A request is added while at least one workgroup still fits.

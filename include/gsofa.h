@@ -190,7 +190,7 @@ void gsofa_result_free(gsofa_result* r);
  *   row_fill_bound  n entries (caller-owned, may be NULL): >= row_fill[i]
  *   fill_bound      >= fill_count;  L_bound >= nnz(L);  U_bound >= nnz(U)
  * All equal the exact values when A is structurally symmetric.  Plans size
- * their fill stream and output from these, so no traversal is repeated. */
+ * their records or fill stream and output from these, so no traversal is repeated. */
 int gsofa_fill_bound(const gsofa_matrix* A, int64_t* row_fill_bound, uint64_t* fill_bound,
                      uint64_t* L_bound, uint64_t* U_bound);
 
@@ -281,11 +281,12 @@ void gsofa_supernodal_free(gsofa_supernodal* s);
  * No counterpart in the reference (one matrix per process run).  Requests are
  * submitted one at a time from any host thread; the server copies the matrix
  * and returns a ticket.  max_inflight worker threads each own a HIP stream:
- * whenever a worker is free it admits the waiting requests, oldest first, up
+ * whenever a worker and the device are free it admits the waiting requests, oldest first, up
  * to max_batch and while the device bytes of all in-flight batches stay within
  * mem_budget_bytes, runs them as one batch plan (one persistent launch) and
- * publishes every request's result.  Batches of different workers overlap on
- * the device.  Each result equals the request's stand-alone result.
+ * publishes every request's result.  One batch loads and runs at a time, beside
+ * the copies of those before it.  Each result equals the request's stand-alone
+ * result.
  * gsofa_server_submit checks the request as gsofa_plan_create would (index
  * ranges, size limits) and returns any error to its caller alone.  A request
  * whose own footprint exceeds budget / max_inflight runs alone once the
