@@ -27,7 +27,7 @@
 // dependent gathers (row, column, class, class of the class) and barriers,
 // 15-20 us of one workgroup whatever its nodes, up to 50 us with rows of
 // thousands of targets.  So a range's nodes are closed as a bit matrix
-// (2.2 us for 64 nodes, 10 us for 128, 35 us for 256), lanes that share a row
+// (2.4 us for 64 nodes, 8 us for 128, 22 us for 240), lanes that share a row
 // step its cursor once, rows of a level lie where the matrix's rows lie (no
 // allocation), and the vertices' classes of one level are written behind the
 // ranges of the next.
@@ -70,7 +70,7 @@ constexpr uint32_t QSIFT = 2048;
 static_assert(QSEEN >= 2u * QCAP, "a place and a target name the row");
 constexpr int ROUNDS = 4, ITERS = 96;  // label rounds of a range and iterations of a round, at most
 constexpr int QB = 1 << kQuotShift;  // vertices of a block
-constexpr int QNT = QB, QNT_LEVEL = 512, QNT_BIG = 1024;
+constexpr int QNT = 512, QNT_LEVEL = 512, QNT_BIG = 1024;
 static_assert(QB <= QN && QB % WAVE == 0, "a block's vertices are the nodes of one bit matrix");
 
 template <int N>
@@ -132,58 +132,108 @@ __device__ __forceinline__ void each_row(uint32_t m, Row row, F f) {
 
 // Strongly connected classes of m <= 64 NW nodes from their adjacency bits
 // S.u.c.adj (rows of nodes at or above m empty): Warshall's closure, 64 pivots
-// at a time.  Thread i of the first 64 NW holds row i as dwords; the wave of
-// the pivots closes its own rows by lane broadcasts (one and-or per dword and
-// pivot), publishes them, and the other rows take them from LDS.  root[i]: the
-// smallest node that i reaches and that reaches i.  Called by the whole
-// workgroup.
-template <int NW, int N>
+// at a time.  Wave w of the first NW holds columns 64 w .. of every row, row
+// 64 g + lane as r[g].  The pivots' wave closes its columns by lane broadcasts
+// (two and-ors per pivot and row), publishes them, and the others add the
+// pivots' rows to the rows that the closed bits name.  root[i]: the smallest
+// node that i reaches and that reaches i.  Called by the whole workgroup.
+//
+// Bound by instruction issue of the few waves that work, and by fetching code
+// that a workgroup runs once: a lane per row with every pivot unrolled (NW * 64
+// pivots of 17 instructions at NW = 4) took 35 us for 256 nodes, and its code
+// evicted the other phases'.  Loops over the pivots below m and columns split
+// over the waves take 22; 9.4 -> 7.5 us at 128 nodes.  Pivots taken in pairs
+// need fewer steps in sequence and more instructions: 10.4.  With the base
+// blocks at 512 threads in place of 128, execute ms before -> after: 181^2 grid
+// 0.64 -> 0.57, 128 2D grids 7.25 -> 6.90, n = 11,948 0.278 -> 0.253, 64^2
+// 0.345 -> 0.326, 16^2 0.159 -> 0.146, band n = 659,033 4.30 -> 4.09.
+template <int NW, int N, int NT>
 __device__ __forceinline__ void closure_classes(QLds<N>& S, uint32_t m) {
-    constexpr int ND = 2 * NW, QD = QN / 32;
-    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = tid / WAVE;
-    const bool row = tid < (uint32_t)(64 * NW);
+    constexpr int QD = QN / 32;
+    constexpr uint32_t CW = 64u * NW / (NT / WAVE);  // columns that a wave transposes
+    static_assert(CW >= 1u && CW <= 32u && 32u % CW == 0u && NT / WAVE >= NW, "a wave's columns are in one dword");
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / WAVE));
     uint32_t(*adj)[QD] = reinterpret_cast<uint32_t(*)[QD]>(S.u.c.adj);
-    uint32_t r[ND];
+    uint32_t r[NW][2];
+    // r |= the rows of block b's pivots, in o, that the bits c name
+    auto pivots = [&](int b, const uint32_t (&o)[2], const uint32_t (&c)[NW][2]) {
 #pragma unroll
-    for (int q = 0; q < ND; q++) r[q] = row ? adj[tid][q] : 0u;
+        for (int h = 0; h < 2; h++) {
+            const uint32_t k0 = 64u * (uint32_t)b + 32u * (uint32_t)h;
+            const uint32_t n = m <= k0 ? 0u : m - k0 < 32u ? m - k0 : 32u;
+#pragma unroll 4
+            for (uint32_t k = 0; k < n; k++) {
+                const uint32_t p0 = (uint32_t)__builtin_amdgcn_readlane((int)o[0], (int)(32u * h + k));
+                const uint32_t p1 = (uint32_t)__builtin_amdgcn_readlane((int)o[1], (int)(32u * h + k));
+#pragma unroll
+                for (int g = 0; g < NW; g++) {
+                    const uint32_t has = (uint32_t)__builtin_amdgcn_sbfe((int)c[g][h], k, 1u);
+                    r[g][0] |= p0 & has;
+                    r[g][1] |= p1 & has;
+                }
+            }
+        }
+    };
+    if (w < (uint32_t)NW) {
+#pragma unroll
+        for (int g = 0; g < NW; g++) {
+            r[g][0] = adj[64 * g + (int)lane][2u * w];
+            r[g][1] = adj[64 * g + (int)lane][2u * w + 1u];
+        }
+    }
 #pragma unroll
     for (int b = 0; b < NW; b++) {
         if (w == (uint32_t)b) {
+            pivots(b, r[b], r);
 #pragma unroll
-            for (int k = 0; k < 64; k++) {
-                const uint32_t has = 0u - ((r[2 * b + (k >> 5)] >> (k & 31)) & 1u);
-#pragma unroll
-                for (int q = 0; q < ND; q++) r[q] |= (uint32_t)__builtin_amdgcn_readlane((int)r[q], k) & has;
-            }
-            if (NW > 1) {
-#pragma unroll
-                for (int q = 0; q < ND; q++) adj[tid][q] = r[q];
+            for (int g = 0; g < NW; g++) {
+                adj[64 * g + (int)lane][2 * b] = r[g][0];
+                adj[64 * g + (int)lane][2 * b + 1] = r[g][1];
             }
         }
-        if (NW > 1) {
-            __syncthreads();
-            if (row && w != (uint32_t)b) {
-#pragma unroll 8
-                for (int k = 0; k < 64; k++) {
-                    const uint32_t has = 0u - ((r[2 * b + (k >> 5)] >> (k & 31)) & 1u);
+        if (NW == 1) break;
+        __syncthreads();
+        if (w < (uint32_t)NW && w != (uint32_t)b) {
+            uint32_t c[NW][2];
 #pragma unroll
-                    for (int q = 0; q < ND; q++) r[q] |= adj[64 * b + k][q] & has;
-                }
+            for (int g = 0; g < NW; g++) {
+                c[g][0] = adj[64 * g + (int)lane][2 * b];
+                c[g][1] = adj[64 * g + (int)lane][2 * b + 1];
             }
-            // the next block's pivots write their own rows of adj only
+            const uint32_t o[2] = {r[b][0], r[b][1]};
+            pivots(b, o, c);
+        }
+        // the next block's wave writes its own columns only
+    }
+    if (NW > 1 && w + 1u < (uint32_t)NW) {  // the last wave's columns are complete
+#pragma unroll
+        for (int g = 0; g < NW; g++) {
+            adj[64 * g + (int)lane][2u * w] = r[g][0];
+            adj[64 * g + (int)lane][2u * w + 1u] = r[g][1];
         }
     }
-    // transpose: the ballot of bit 64 q + k over wave w is word w of row 64 q + k
-    if (row) {
+    __syncthreads();
+    // transpose, by all waves: the ballot of bit c over rows 64 g .. is word g of row c
+    {
+        const uint32_t c0 = w * CW;
+        uint32_t x[NW];
+        uint64_t mine[NW];
 #pragma unroll
-        for (int q = 0; q < NW; q++) {
-            uint64_t mine = 0;
+        for (int g = 0; g < NW; g++) {
+            x[g] = adj[64 * g + (int)lane][c0 >> 5];
+            mine[g] = 0;
+        }
+#pragma unroll 2
+        for (uint32_t k = 0; k < CW; k++) {
 #pragma unroll
-            for (int k = 0; k < 64; k++) {
-                const uint64_t bal = __ballot((r[2 * q + (k >> 5)] >> (k & 31)) & 1u);
-                if (lane == (uint32_t)k) mine = bal;
+            for (int g = 0; g < NW; g++) {
+                const uint64_t bal = __ballot((x[g] >> ((c0 & 31u) + k)) & 1u);
+                if (lane == k) mine[g] = bal;
             }
-            S.u.c.tr[64 * q + (int)lane][w] = mine;
+        }
+        if (lane < CW) {
+#pragma unroll
+            for (int g = 0; g < NW; g++) S.u.c.tr[c0 + lane][g] = mine[g];
         }
     }
     __syncthreads();
@@ -191,7 +241,7 @@ __device__ __forceinline__ void closure_classes(QLds<N>& S, uint32_t m) {
         uint32_t c = tid;
 #pragma unroll
         for (int q = NW - 1; q >= 0; q--) {
-            const uint64_t both = (((uint64_t)r[2 * q + 1] << 32) | r[2 * q]) & S.u.c.tr[tid][q];
+            const uint64_t both = S.u.c.adj[tid][q] & S.u.c.tr[tid][q];
             if (both) {
                 const uint32_t j = 64u * (uint32_t)q + (uint32_t)__builtin_ctzll(both);
                 c = j < c ? j : c;
@@ -453,12 +503,12 @@ __device__ bool range_classes(QLds<N>& S, const QuotParams& p, uint32_t lev, uin
     });
     __syncthreads();
     if constexpr (BASE) {
-        closure_classes<QB / 64>(S, nl);
+        closure_classes<QB / 64, N, NT>(S, nl);
     } else {
         if (N > QN && !bits) label_classes<N, NT>(S, nl, S.ne, eb);
-        else if (nl <= 64u) closure_classes<1>(S, nl);
-        else if (nl <= 128u) closure_classes<2>(S, nl);
-        else closure_classes<QN / 64>(S, nl);
+        else if (nl <= 64u) closure_classes<1, N, NT>(S, nl);
+        else if (nl <= 128u) closure_classes<2, N, NT>(S, nl);
+        else closure_classes<QN / 64, N, NT>(S, nl);
     }
     __syncthreads();
     for (uint32_t c = tid; c < nl; c += NT) {

@@ -49,6 +49,34 @@ def test_few_classes(lam, threads):
     _check(g.gen_band(20011, 200, lam, 7), block_slots=64, workgroup_threads=threads)
 
 
+@pytest.mark.parametrize("nodes", [2, 63, 64, 65, 127, 128, 129, 193, 255, 256])
+def test_closure_sizes(nodes):
+    """Ranges of two blocks of 128 with that many nodes: in each block the last
+    vertices are one cycle, the others have edges to later ones only, and sparse
+    edges between the blocks close cycles of every length among the nodes."""
+    rng = np.random.default_rng(nodes)
+    n, half = 2048 + 77, 128
+    rows, cols = [], []
+    for b in range(n // half):
+        m = nodes // 2 if b % 2 == 0 else nodes - nodes // 2
+        first = m - 1 if m < half else half  # of the cycle
+        c = b * half + np.arange(first, half)
+        if len(c) > 1:
+            rows.append(c), cols.append(np.roll(c, -1))
+        u = rng.integers(0, half, (2, 40))
+        u = np.sort(u[:, u.max(axis=0) < first], axis=0)
+        rows.append(b * half + u[0]), cols.append(b * half + u[1])
+        v = rng.integers(0, half, (2, 48))
+        v[0, 0] = v[1, 0] = 0
+        rows.append(b * half + v[0]), cols.append((b ^ 1) * half + v[1])
+    u = rng.integers(0, n, (2, 600))
+    rows.append(u[0]), cols.append(u[1])
+    rows, cols = np.concatenate(rows), np.concatenate(cols)
+    keep = cols < n
+    for bits in (32, 64, 256):
+        _check(_from_edges(n, rows[keep], cols[keep]), block_slots=bits)
+
+
 def test_too_many_nodes():
     """Ranges of over 256 live nodes keep their halves' classes: pairs (2i, 2i+1)
     are strongly connected, the pairs form an acyclic chain of chains."""
