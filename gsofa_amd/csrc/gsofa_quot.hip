@@ -60,6 +60,11 @@ constexpr int QM = 4096;             // nodes of a range, at most, if its halves
 // they go to a few large workgroups that take up to QCAP by label rounds.
 constexpr int QCAP = 2048;
 constexpr uint32_t QBIG_LEVEL = 4, QBIG_GRID = 256;
+// Up to one range per CU, a range gets 1,024 threads: 181^2 grid 0.564 -> 0.549
+// ms, 48^3 2.28 -> 2.24, 33^3 0.780 -> 0.769.  More ranges share the CUs, which
+// hold two workgroups of 512 threads for one of 1,024: 128 2D grids at 1,024
+// threads 6.90 -> 7.36, band n = 659,033 4.09 -> 4.29.
+constexpr uint32_t QFEW = 256;
 constexpr uint32_t QSEEN = 4096;     // a power of two, at least two rows for every node
 // Where merged classes' rows have so many entries, and 16 for every node, their
 // members share targets (a band's class of 1,024 vertices has 2,000 entries and
@@ -657,7 +662,8 @@ __device__ __forceinline__ void map_level(const QuotParams& p, uint32_t lev, uin
 // The ranges of a level, one workgroup each.  The blocks behind them write the
 // classes of the level below (lev >= 2), which this level's own look-ups take
 // in two steps instead.
-__global__ __launch_bounds__(QNT_LEVEL) void k_quot_level(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ctab0,
+template <int NT>
+__global__ __launch_bounds__(NT) void k_quot_level(QuotParams p, uint32_t lev, uint32_t tab0, uint32_t ctab0,
                                                           uint32_t ranges, uint32_t cranges) {
     __shared__ QLds<QN> S;
     if (lev > p.judge && quot_off(p)) return;
@@ -665,7 +671,7 @@ __global__ __launch_bounds__(QNT_LEVEL) void k_quot_level(QuotParams p, uint32_t
         map_level(p, lev - 1u, ctab0, cranges, blockIdx.x - ranges, gridDim.x - ranges);
         return;
     }
-    if (!range_classes<QN, QNT_LEVEL, false>(S, p, lev, tab0, ctab0, blockIdx.x, lev <= QBIG_LEVEL) &&
+    if (!range_classes<QN, NT, false>(S, p, lev, tab0, ctab0, blockIdx.x, lev <= QBIG_LEVEL) &&
         threadIdx.x == 0)
         p.blist[atomicAdd(&p.ctl->big[lev], 1u)] = blockIdx.x;
 }
@@ -735,8 +741,9 @@ hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hi
     for (; h < p.levels && off[h + 1] > off[h]; h++) {
         const uint32_t ranges = off[h + 1] - off[h], below = off[h] - off[h - 1];
         const uint32_t mb = h >= 2 ? map_blocks((uint64_t)below << (kQuotShift + h - 1)) : 0u;
-        hipLaunchKernelGGL(k_quot_level, dim3(ranges + mb), dim3(QNT_LEVEL), 0, s, p, h, off[h], off[h - 1], ranges,
-                           below);
+        auto* level = ranges <= QFEW ? k_quot_level<QNT_BIG> : k_quot_level<QNT_LEVEL>;
+        hipLaunchKernelGGL(level, dim3(ranges + mb), dim3(ranges <= QFEW ? QNT_BIG : QNT_LEVEL), 0, s, p, h, off[h],
+                           off[h - 1], ranges, below);
         if (h <= QBIG_LEVEL)
             hipLaunchKernelGGL(k_quot_big, dim3(std::min(ranges, QBIG_GRID)), dim3(QNT_BIG), 0, s, p, h, off[h],
                                off[h - 1]);
