@@ -572,28 +572,35 @@ void release_quot(gsofa_plan* P) {
     P->qcap = gsofa_plan::QuotCaps{};
 }
 
-// Levels of classes for a reach-mode run within `room` bytes: all that the
-// largest matrix has, or none where their arrays would take over an eighth of
-// the room or class rows would pass 32-bit entry numbers.
-uint32_t quot_wanted(int64_t n, int64_t nnz, uint32_t W, int64_t room) {
-    const uint32_t L = quot_levels(W);
-    if (L == 0 || nnz + (int64_t)quot_ext((uint64_t)nnz, L) >= (int64_t)UINT32_MAX) return 0;
-    return quot_bytes(n, nnz, W) <= room / 8 ? L : 0;
+// Levels of classes for a reach-mode run within `room` bytes, from blocks of
+// 2^*shift vertices: all that the largest matrix has, or none where their arrays
+// would take over an eighth of the room or class rows would pass 32-bit entry
+// numbers.  Blocks of kQuotShift, one level less, where only those fit.
+uint32_t quot_wanted(int64_t n, int64_t nnz, uint32_t W, int64_t room, const int32_t* rp, const int32_t* ci,
+                     uint32_t* shift) {
+    for (*shift = quot_shift(W, n, rp, ci);; *shift = kQuotShift) {
+        const uint32_t L = quot_levels(W, *shift);
+        if (L != 0 && nnz + (int64_t)quot_ext((uint64_t)nnz, L) < (int64_t)UINT32_MAX &&
+            quot_bytes(n, nnz, W, *shift) <= room / 8)
+            return L;
+        if (*shift == kQuotShift) return 0;
+    }
 }
 
 // The range table and device arrays of `levels` levels for the plan's matrices
 // (P->h_mat_base, n, nnz); d_ci and d_ciT hold quot_ext entries more.  Arrays
 // that are large enough stay (arenas).
-int setup_quot(gsofa_plan* P, uint32_t levels) {
+int setup_quot(gsofa_plan* P, uint32_t levels, uint32_t shift) {
     QuotParams& q = P->quot;
     q.levels = levels;
+    q.shift = shift;
     if (levels == 0) return GSOFA_OK;
     const size_t n = (size_t)P->n, ln = (size_t)levels * n;
     q.n = (uint32_t)n;
     q.ext0 = (uint32_t)P->nnz;
-    quot_table(P->h_mat_base, levels, P->h_qtab, P->h_qoff);
-    q.judge = std::min(kQuotJudge, levels - 1u);
-    q.judged = (P->h_qoff[q.judge + 1] - P->h_qoff[q.judge]) << (kQuotShift + q.judge);
+    quot_table(P->h_mat_base, levels, shift, P->h_qtab, P->h_qoff);
+    q.judge = std::min(kQuotJudge - shift, levels - 1u);
+    q.judged = (P->h_qoff[q.judge + 1] - P->h_qoff[q.judge]) << (shift + q.judge);
     gsofa_plan::QuotCaps& c = P->qcap;
     int e = 0;
     if (c.tab < P->h_qtab.size()) {
@@ -1116,10 +1123,12 @@ int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
         uint32_t nb = 0;
         int threads = 0;
         if (reach_grid(o, bits, 2 * nchunks, nr, largest, (uint32_t)A->n, INT64_MAX / 4, &nb, &threads) != GSOFA_OK) return -1;
+        uint32_t shift = 0;
         const uint32_t ql = quot_wanted(A->n, (int64_t)ci.size(), (uint32_t)A->n,
-                                        o.mem_budget_bytes > 0 ? o.mem_budget_bytes : INT64_MAX / 4);
+                                        o.mem_budget_bytes > 0 ? o.mem_budget_bytes : INT64_MAX / 4, rp.data(),
+                                        ci.data(), &shift);
         return reach_bytes(nb, (uint32_t)A->n, bits) +
-               (ql ? quot_bytes(A->n, (int64_t)ci.size(), (uint32_t)A->n) : 0) +
+               (ql ? quot_bytes(A->n, (int64_t)ci.size(), (uint32_t)A->n, shift) : 0) +
                block_fixed_bytes(A->n, (int64_t)ci.size(), 1, nchunks, rch_fill_room(nf), (int64_t)(nl + nu)) +
                4 * (int64_t)(A->n + 1) + 4 * (int64_t)ci.size();
     }
@@ -1289,7 +1298,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     }
     int e = 0;
     P->gather = reach && P->bounded;
-    uint32_t qlev = 0;  // levels of classes (reach mode)
+    uint32_t qlev = 0, qshift = 0;  // levels of classes (reach mode)
     if (P->mode == GSOFA_MODE_REACH) {
         const int bits = P->rbits;
         P->S = (uint32_t)bits;
@@ -1311,8 +1320,9 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             const int64_t tbytes = 4 * (int64_t)(n + 1) + 4 * P->nnz + 16 * (int64_t)n_mats;
             const int64_t room = std::max<int64_t>(avail - tbytes, 1 << 20);
             gsofa_options go = P->opt;
-            qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room);
-            const int64_t qb = qlev ? quot_bytes(n, P->nnz, P->W) : 0;
+            qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room,
+                               P->h_rp.data(), ci.data(), &qshift);
+            const int64_t qb = qlev ? quot_bytes(n, P->nnz, P->W, qshift) : 0;
             if (go.mem_budget_bytes > 0) go.mem_budget_bytes -= qb;
             rc = reach_grid(go, bits, std::max<uint64_t>(P->h_chunks.size(), 1), need_rec, largest, P->W, room - qb, &P->nblocks,
                             &P->rthreads);
@@ -1337,7 +1347,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         e |= palloc(P, &P->d_mat_reach, (size_t)n_mats);
         e |= palloc(P, &P->d_rpT, (size_t)n + 1);
         e |= palloc(P, &P->d_ciT, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
-        e |= setup_quot(P, qlev);
+        e |= setup_quot(P, qlev, qshift);
     } else if (P->mode == GSOFA_MODE_BLOCK) {
         int S = 0;
         const uint64_t nsrc = P->hybrid ? P->s_top : share_count(n, P->opt.n_virtual_gpu, 0);
@@ -2636,8 +2646,9 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     o.mode = GSOFA_MODE_AUTO;  // the tuned grid for this batch's signature (slots stay 64)
     if (!apply_tuned(&o, W, nnz, n, count) || resolve_mode(o) != GSOFA_MODE_REACH) o = P->opt;
     o.mem_budget_bytes = 0;
-    const uint32_t qlev = quot_wanted(n, nnz, W, budget - fixed);
-    const int64_t qb = qlev ? quot_bytes(n, nnz, W) : 0;
+    uint32_t qshift = 0;
+    const uint32_t qlev = quot_wanted(n, nnz, W, budget - fixed, P->h_rp.data(), P->h_ci.data(), &qshift);
+    const int64_t qb = qlev ? quot_bytes(n, nnz, W, qshift) : 0;
     int rc = reach_grid(o, bits, nchunks, nr, largest, W, budget - fixed - qb, &nb, &P->rthreads);
     if (rc) return rc;
     gsofa_plan::Caps& c = P->cap;
@@ -2730,7 +2741,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         c.chunks = nchunks;
     }
     if (!P->d_ctrl) e |= palloc(P, &P->d_ctrl, 1);
-    e |= setup_quot(P, qlev);
+    e |= setup_quot(P, qlev, qshift);
     if (e) return GSOFA_ERR_ALLOC;
     // per-workgroup arrays: one stride (their capacity) for every batch,
     // cleared when they grow

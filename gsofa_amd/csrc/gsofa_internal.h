@@ -122,12 +122,9 @@ hipError_t launch_traverse_blk(const BlkParams& p, int slots, size_t lds_bytes, 
 
 // Classes of vertex ranges (gsofa_quot.hip), built on the device at the start
 // of every reach-mode execute.
-// log2 of a block's vertices.  A source walks up to a block of single
-// vertices; each halving of the block adds a level of ranges to build.
-// Execute ms at blocks of 64 / 128 / 256: 48^3 grid 2.47 / 2.52 / 2.61, 128 2D
-// grids 11.4 / 11.6 / 12.9, 27^3 0.91 / 0.91 / 1.01, n = 11,948 band 0.40 /
-// 0.38 / 0.42, band n = 659,033 - / 4.83 / 4.67.
-constexpr uint32_t kQuotShift = 7;
+// log2 of a block's vertices (quot_shift chooses).  A source walks up to a block
+// of single vertices; each halving of the block adds a level of ranges to build.
+constexpr uint32_t kQuotShift = 7, kQuotShiftChain = 6;
 struct QuotCtl {
     unsigned long long nodes;          // classes of the judged level's ranges
     uint32_t big[8];                   // ranges of a low level left to large workgroups
@@ -140,6 +137,7 @@ struct QuotParams {
     uint32_t n;          // all vertices (stride of the per-level arrays)
     uint32_t ext0;
     uint32_t levels;
+    uint32_t shift;      // log2 of a block's vertices
     uint32_t judge;      // the level by whose classes quot_off judges
     uint32_t judged;     // vertices of its ranges
     const uint2* tab;
@@ -152,15 +150,17 @@ struct QuotParams {
     uint32_t* eb;        // nnz: edge lists of those ranges
     QuotCtl* ctl;
 };
-// Classes do not pay where ranges of 2^(kQuotShift + kQuotJudge) vertices keep
+// Classes do not pay where ranges of 2^kQuotJudge vertices keep
 // over half of them as classes: the traversal then walks plain vertices.
 // (Smaller ranges say little: a banded matrix has few edges within them.)
-constexpr uint32_t kQuotJudge = 3;
+constexpr uint32_t kQuotJudge = 10;
 __device__ __forceinline__ bool quot_off(const QuotParams& p) { return 2ull * p.ctl->nodes > (unsigned long long)p.judged; }
-uint32_t quot_levels(uint32_t W);
+uint32_t quot_shift(uint32_t W, int64_t n, const int32_t* rp, const int32_t* ci);
+uint32_t quot_levels(uint32_t W, uint32_t shift);
 uint64_t quot_ext(uint64_t nnz, uint32_t levels);
-int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W);
-void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vector<uint2>& tab, std::vector<uint32_t>& off);
+int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W, uint32_t shift);
+void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, uint32_t shift, std::vector<uint2>& tab,
+                std::vector<uint32_t>& off);
 hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hipStream_t s);
 
 // Reach mode (gsofa_reach.hip): one launch over a work table whose chunks

@@ -9,7 +9,7 @@
 // TE, is exactly what the walk over single vertices gives.
 //
 // Each matrix's vertices are cut into blocks of
-// 2^kQuotShift.  Level h holds the
+// 128 (or 64, see quot_shift).  Level h holds the
 // complete, aligned ranges of 2^h blocks; a range's classes are found in the
 // subgraph of its own vertices, from its two halves' classes (level 0: from
 // single vertices).  A source in block j uses the ranges of j's binary
@@ -56,10 +56,10 @@ constexpr uint32_t MID_ROW = 256;    // rows up to here: one wave each; longer o
 constexpr int QN = 256;              // live nodes whose reachability is closed as a bit matrix
 constexpr int QM = 4096;             // nodes of a range, at most, if its halves' classes are to be merged
 // Ranges with more live nodes are rare where classes pay at all: sparse bands
-// near the bottom, before their main class forms.  At levels up to QBIG_LEVEL
+// near the bottom, before their main class forms.  Up to 2^QBIG_SHIFT vertices
 // they go to a few large workgroups that take up to QCAP by label rounds.
 constexpr int QCAP = 2048;
-constexpr uint32_t QBIG_LEVEL = 4, QBIG_GRID = 256;
+constexpr uint32_t QBIG_SHIFT = 11, QBIG_GRID = 256;
 // Up to one range per CU, a range gets 1,024 threads: 181^2 grid 0.564 -> 0.549
 // ms, 48^3 2.28 -> 2.24, 33^3 0.780 -> 0.769.  More ranges share the CUs, which
 // hold two workgroups of 512 threads for one of 1,024: 128 2D grids at 1,024
@@ -74,9 +74,10 @@ constexpr uint32_t QSEEN = 4096;     // a power of two, at least two rows for ev
 constexpr uint32_t QSIFT = 2048;
 static_assert(QSEEN >= 2u * QCAP, "a place and a target name the row");
 constexpr int ROUNDS = 4, ITERS = 96;  // label rounds of a range and iterations of a round, at most
-constexpr int QB = 1 << kQuotShift;  // vertices of a block
+constexpr int QB = 1 << kQuotShift;  // vertices of a block, at most
 constexpr int QNT = 512, QNT_LEVEL = 512, QNT_BIG = 1024;
-static_assert(QB <= QN && QB % WAVE == 0, "a block's vertices are the nodes of one bit matrix");
+static_assert(QB <= QN && QB == 2 * WAVE && 2 << kQuotShiftChain == QB,
+              "a block's vertices are the nodes of one bit matrix");
 
 template <int N>
 struct QLds {
@@ -372,7 +373,7 @@ __device__ bool range_classes(QLds<N>& S, const QuotParams& p, uint32_t lev, uin
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint64_t ln = p.n;
     const uint2 R = p.tab[tab0 + range];
-    const uint32_t size = 1u << (kQuotShift + lev), x = R.x, xr = x + size / 2u;
+    const uint32_t size = 1u << (p.shift + lev), x = R.x, xr = x + size / 2u;
     const uint4* info_prev = BASE ? nullptr : p.info + (lev - 1u) * ln;
     const uint4* infoT_prev = BASE ? nullptr : p.infoT + (lev - 1u) * ln;
     uint4* info_cur = p.info + lev * ln;
@@ -508,7 +509,8 @@ __device__ bool range_classes(QLds<N>& S, const QuotParams& p, uint32_t lev, uin
     });
     __syncthreads();
     if constexpr (BASE) {
-        closure_classes<QB / 64, N, NT>(S, nl);
+        if (nl <= 64u) closure_classes<1, N, NT>(S, nl);
+        else closure_classes<2, N, NT>(S, nl);
     } else {
         if (N > QN && !bits) label_classes<N, NT>(S, nl, S.ne, eb);
         else if (nl <= 64u) closure_classes<1, N, NT>(S, nl);
@@ -648,7 +650,7 @@ __global__ __launch_bounds__(QNT) void k_quot_base(QuotParams p) {
 // `blocks` blocks from `block` on share the work.
 __device__ __forceinline__ void map_level(const QuotParams& p, uint32_t lev, uint32_t tab0, uint32_t ranges,
                                           uint32_t block, uint32_t blocks) {
-    const uint32_t sh = kQuotShift + lev;
+    const uint32_t sh = p.shift + lev;
     const uint64_t total = (uint64_t)ranges << sh;
     const int32_t* prev = p.comp + (uint64_t)(lev - 1u) * p.n;
     const int32_t* map = p.nmap + (uint64_t)(lev & 1u) * p.n;
@@ -671,7 +673,7 @@ __global__ __launch_bounds__(NT) void k_quot_level(QuotParams p, uint32_t lev, u
         map_level(p, lev - 1u, ctab0, cranges, blockIdx.x - ranges, gridDim.x - ranges);
         return;
     }
-    if (!range_classes<QN, NT, false>(S, p, lev, tab0, ctab0, blockIdx.x, lev <= QBIG_LEVEL) &&
+    if (!range_classes<QN, NT, false>(S, p, lev, tab0, ctab0, blockIdx.x, p.shift + lev <= QBIG_SHIFT) &&
         threadIdx.x == 0)
         p.blist[atomicAdd(&p.ctl->big[lev], 1u)] = blockIdx.x;
 }
@@ -693,10 +695,33 @@ __global__ __launch_bounds__(QNT_LEVEL) void k_quot_map(QuotParams p, uint32_t l
 
 }  // namespace
 
+// Blocks of 64 where most vertices i have an entry with i - 1 or i + 1, as grids
+// do, else of 128: such a block holds long paths, and walks in a source's own
+// block, one step of a path at a time, bound small matrices.  Where neighbours
+// are rarely coupled a walk takes few steps and the level more is all that
+// blocks of 64 bring.  (Looks at up to 1,024 rows, 64 entries of each.)
+// Execute ms at blocks of 128 -> 64: 64^2 grid 0.326 -> 0.283, 16^2 0.145 ->
+// 0.132, 300 x 200 grid 0.79 -> 0.70, 128 2D grids 6.89 -> 6.67, 48^3 2.24 ->
+// 2.21, narrow band n = 60,000 0.72 -> 0.64; 33^3 0.764 -> 0.777 and 24^3 0.339
+// -> 0.345 are the worst.  Bands of 256, which stay: n = 659,033 4.09 -> 4.25,
+// n = 100,003 0.61 -> 0.65, n = 11,948 0.251 -> 0.258.
+uint32_t quot_shift(uint32_t W, int64_t n, const int32_t* rp, const int32_t* ci) {
+    if (W <= 1u << kQuotShift) return kQuotShift;
+    const int64_t step = std::max<int64_t>(n / 1024, 1);
+    int64_t rows = 0, hits = 0;
+    for (int64_t i = 0; i < n; i += step, rows++)
+        for (int32_t k = rp[i], e = k + std::min(rp[i + 1] - k, 64); k < e; k++)
+            if (ci[k] == i - 1 || ci[k] == i + 1) {
+                hits++;
+                break;
+            }
+    return 2 * hits > rows ? kQuotShiftChain : kQuotShift;
+}
+
 // Levels of the largest matrix: a source's block index is at most blocks - 1,
 // and only complete blocks are contracted.
-uint32_t quot_levels(uint32_t W) {
-    const uint32_t last = W == 0u ? 0u : (W - 1u) >> kQuotShift;
+uint32_t quot_levels(uint32_t W, uint32_t shift) {
+    const uint32_t last = W == 0u ? 0u : (W - 1u) >> shift;
     uint32_t l = 0;
     while (last >> l) l++;
     return l;
@@ -704,16 +729,17 @@ uint32_t quot_levels(uint32_t W) {
 
 uint64_t quot_ext(uint64_t nnz, uint32_t levels) { return nnz * levels; }
 
-int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W) {
-    const int64_t L = quot_levels(W);
+int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W, uint32_t shift) {
+    const int64_t L = quot_levels(W, shift);
     if (L == 0) return 0;
     return L * n * (4 + 32) + 8 * n + 4 * nnz + 8 * (int64_t)quot_ext((uint64_t)nnz, (uint32_t)L) +
-           16 * ((n >> kQuotShift) * 2 + L + 1) + (int64_t)sizeof(QuotCtl) + 4096;
+           16 * ((n >> shift) * 2 + L + 1) + (int64_t)sizeof(QuotCtl) + 4096;
 }
 
 // Ranges of every level: tab[off[h] ..] = (first vertex, entry of the first
 // half among level h - 1's); the halves' entries are neighbours.
-void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vector<uint2>& tab, std::vector<uint32_t>& off) {
+void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, uint32_t shift, std::vector<uint2>& tab,
+                std::vector<uint32_t>& off) {
     tab.clear();
     off.assign((size_t)levels + 1, 0);
     std::vector<uint32_t> child(mat_base.size(), 0), mine(mat_base.size(), 0);
@@ -721,10 +747,10 @@ void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, std::vec
         off[h] = (uint32_t)tab.size();
         for (size_t b = 0; b + 1 < mat_base.size(); b++) {
             const uint32_t nb = mat_base[b + 1] - mat_base[b];
-            const uint32_t cnt = (nb == 0u ? 0u : (nb - 1u) >> kQuotShift) >> h;
+            const uint32_t cnt = (nb == 0u ? 0u : (nb - 1u) >> shift) >> h;
             mine[b] = (uint32_t)tab.size() - off[h];
             for (uint32_t q = 0; q < cnt; q++)
-                tab.push_back(make_uint2(mat_base[b] + (q << (kQuotShift + h)), child[b] + 2u * q));
+                tab.push_back(make_uint2(mat_base[b] + (q << (shift + h)), child[b] + 2u * q));
         }
         child = mine;
     }
@@ -740,17 +766,17 @@ hipError_t launch_quot(const QuotParams& p, const std::vector<uint32_t>& off, hi
     uint32_t h = 1;
     for (; h < p.levels && off[h + 1] > off[h]; h++) {
         const uint32_t ranges = off[h + 1] - off[h], below = off[h] - off[h - 1];
-        const uint32_t mb = h >= 2 ? map_blocks((uint64_t)below << (kQuotShift + h - 1)) : 0u;
+        const uint32_t mb = h >= 2 ? map_blocks((uint64_t)below << (p.shift + h - 1)) : 0u;
         auto* level = ranges <= QFEW ? k_quot_level<QNT_BIG> : k_quot_level<QNT_LEVEL>;
         hipLaunchKernelGGL(level, dim3(ranges + mb), dim3(ranges <= QFEW ? QNT_BIG : QNT_LEVEL), 0, s, p, h, off[h],
                            off[h - 1], ranges, below);
-        if (h <= QBIG_LEVEL)
+        if (p.shift + h <= QBIG_SHIFT)
             hipLaunchKernelGGL(k_quot_big, dim3(std::min(ranges, QBIG_GRID)), dim3(QNT_BIG), 0, s, p, h, off[h],
                                off[h - 1]);
     }
     if (h >= 2) {
         const uint32_t ranges = off[h] - off[h - 1];
-        hipLaunchKernelGGL(k_quot_map, dim3(map_blocks((uint64_t)ranges << (kQuotShift + h - 1))), dim3(QNT_LEVEL), 0,
+        hipLaunchKernelGGL(k_quot_map, dim3(map_blocks((uint64_t)ranges << (p.shift + h - 1))), dim3(QNT_LEVEL), 0,
                            s, p, h - 1u, off[h - 1], ranges);
     }
     return hipGetLastError();

@@ -444,11 +444,11 @@ struct RCur {
     // sources all lie at or above it
     const int32_t* comp;
     const uint4* info;
-    uint32_t jb, below, top;
+    uint32_t jb, below, top, shift;
     uint64_t cn;  // stride of the per-level arrays
 
     __device__ __forceinline__ uint32_t level_of(uint32_t m) const {
-        const uint32_t h = 31u - (uint32_t)__builtin_clz((m >> kQuotShift) ^ jb);
+        const uint32_t h = 31u - (uint32_t)__builtin_clz((m >> shift) ^ jb);
         return h < top ? h : top;
     }
     // row and (vertices, row lengths) of a node
@@ -963,8 +963,9 @@ __global__ __launch_bounds__(RB, sizeof(M) <= 16 ? 4 : 1) void k_reach_blk(RchPa
         c.info = c.tpass ? p.quot.infoT : p.quot.info;
         c.cn = p.quot.n;
         c.top = p.quot.levels - 1u;
-        c.jb = classes ? (c.first - (c.count - 1u) * c.stride - c.wb) >> kQuotShift : 0u;
-        c.below = c.jb << kQuotShift;
+        c.shift = p.quot.shift;
+        c.jb = classes ? (c.first - (c.count - 1u) * c.stride - c.wb) >> c.shift : 0u;
+        c.below = c.jb << c.shift;
         bool nodes = false;  // the node table holds the whole group
         if constexpr (NODES) {
             if (wait == 0u) {

@@ -77,6 +77,20 @@ def test_closure_sizes(nodes):
         _check(_from_edges(n, rows[keep], cols[keep]), block_slots=bits)
 
 
+@pytest.mark.parametrize("n", [128, 129, 192, 193, 256, 257, 1024, 1025, 2111, 4161])
+def test_chain_blocks(n):
+    """Rows mostly coupled to their neighbours take blocks of 64 vertices: one
+    direction, both, and every third link cut, with a few long entries."""
+    rng = np.random.default_rng(n)
+    i = np.arange(n - 1)
+    far = rng.integers(0, n, (2, n // 16))
+    for links, back in ((i, i[::2]), (i, i), (i[i % 3 != 0], i[:0]), (i[:0], i)):
+        rows = np.concatenate([links, back + 1, far[0]])
+        cols = np.concatenate([links + 1, back, far[1]])
+        for bits in (32, 64, 128):
+            _check(_from_edges(n, rows, cols), block_slots=bits)
+
+
 def test_too_many_nodes():
     """Ranges of over 256 live nodes keep their halves' classes: pairs (2i, 2i+1)
     are strongly connected, the pairs form an acyclic chain of chains."""
