@@ -8,9 +8,8 @@
 // (|R| and TE count every vertex).  Reachability, and with it L, U, |R| and
 // TE, is exactly what the walk over single vertices gives.
 //
-// Each matrix's vertices are cut into blocks of
-// 128 (or 64, see quot_shift).  Level h holds the
-// complete, aligned ranges of 2^h blocks; a range's classes are found in the
+// Each matrix's vertices are cut into blocks of 128 (or 64, see quot_shift).
+// Level h holds the complete, aligned ranges of 2^h blocks; a range's classes are found in the
 // subgraph of its own vertices, from its two halves' classes (level 0: from
 // single vertices).  A source in block j uses the ranges of j's binary
 // decomposition: the vertices below block j are covered by one range per set
@@ -33,11 +32,10 @@
 // ranges of the next.
 //
 // Measured, traversal of one execute walking vertices -> classes (the
-// classes' construction included): band n = 659,033 780 -> 4.0 ms, band
-// n = 100,003 32.3 -> 0.71, 48^3 grid 64.9 -> 1.57, 128 2D grids 278 -> 10.0,
-// 181^2 grid 16.4 -> 0.68, n = 11,948 1.13 -> 0.24.  The construction with
-// label rounds for every range and two launches a level took 0.73 ms at 48^3,
-// now 0.36; at the 128 grids 1.8, now 0.8; at the band 1.45, now 0.45.
+// classes' construction included): band n = 659,033 780 -> 3.1 ms, band
+// n = 100,003 32.3 -> 0.59, 48^3 grid 64.9 -> 1.56, 181^2 grid 16.4 -> 0.45,
+// n = 11,948 1.13 -> 0.22.  The construction with label rounds for every range
+// and two launches a level took 0.73 ms at 48^3, now 0.36.
 #include <algorithm>
 
 #include "gsofa_device.h"
