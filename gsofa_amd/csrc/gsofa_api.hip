@@ -178,6 +178,7 @@ struct gsofa_plan {
         void** where;
         size_t bytes;
     };
+    int fail_alloc = 0;         // see alloc_fails
     std::vector<Piece> pieces;  // of the slab, while gathered
     bool gather = false;
     char* slab = nullptr;
@@ -263,13 +264,20 @@ struct DevScratch {
     }
 };
 
+// GSOFA_FAIL_ALLOC=k in the environment when a plan (a server worker's too) is
+// made: its k-th device allocation fails, once, so tests reach what follows.
+void read_fail_alloc(gsofa_plan* P) {
+    if (const char* f = getenv("GSOFA_FAIL_ALLOC")) P->fail_alloc = atoi(f);
+}
+bool alloc_fails(gsofa_plan* P) { return P->fail_alloc > 0 && --P->fail_alloc == 0; }
+
 // A plan's device arrays.  Where all sizes are known at creation they are
 // pieces of one allocation (gather, then take_slab): twelve of 8 MB cost
 // 3.4 ms to make and release, one of 96 MB 0.6.
 template <class T>
 int palloc(gsofa_plan* P, T** p, size_t count) {
-    if (!P->gather) return dalloc(p, count);
     *p = nullptr;
+    if (!P->gather) return alloc_fails(P) ? GSOFA_ERR_ALLOC : dalloc(p, count);
     P->pieces.push_back({(void**)p, (sizeof(T) * std::max<size_t>(count, 1) + 511) & ~(size_t)511});
     return GSOFA_OK;
 }
@@ -285,7 +293,7 @@ int take_slab(gsofa_plan* P) {
     P->gather = false;
     P->slab_bytes = 0;
     for (const gsofa_plan::Piece& x : P->pieces) P->slab_bytes += x.bytes;
-    const int e = dalloc(&P->slab, P->slab_bytes);
+    const int e = alloc_fails(P) ? GSOFA_ERR_ALLOC : dalloc(&P->slab, P->slab_bytes);
     size_t off = 0;
     for (const gsofa_plan::Piece& x : P->pieces) {
         if (!e) *x.where = P->slab + off;
@@ -544,7 +552,13 @@ void advance_state(gsofa_plan* P, int32_t gid) {
 }
 
 // The fill stream, or reach mode's records and record lists, of P->fill_cap
-// entries (list: records of the A^T pass, at most).
+// entries (list: records of the A^T pass, at most).  After a failure some are
+// missing, and the next execute asks for them again.
+bool stream_missing(const gsofa_plan* P) {
+    if (P->mode == GSOFA_MODE_REACH) return !P->d_rec || !P->d_list;
+    return !P->d_fills;
+}
+
 int alloc_stream(gsofa_plan* P, uint64_t list) {
     if (P->mode != GSOFA_MODE_REACH) {
         pfree(P, P->d_fills);
@@ -707,6 +721,7 @@ int alloc_supernodes(gsofa_plan* P) {
     pfree(P, P->d_sstart);
     pfree(P, P->d_sn64);
     pfree(P, P->d_snflag);
+    P->sn_cap = 0;
     int e = palloc(P, &P->d_supno, n);
     e |= palloc(P, &P->d_sstart, n + 1);
     e |= palloc(P, &P->d_sn64, scan_tmp_words((int32_t)n) + 2 * n + 8);
@@ -720,6 +735,7 @@ int ensure_cols(gsofa_plan* P, int64_t nl, int64_t nu) {
     if (nl > P->Lcap) {
         pfree(P, P->d_Lcol);
         pfree(P, P->d_Ltmp);
+        P->Lcap = 0;
         int64_t cap = nl + nl / 8 + 1024;
         if (palloc(P, &P->d_Lcol, (size_t)cap) || (staged && palloc(P, &P->d_Ltmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Lcap = cap;
@@ -727,6 +743,7 @@ int ensure_cols(gsofa_plan* P, int64_t nl, int64_t nu) {
     if (nu > P->Ucap) {
         pfree(P, P->d_Ucol);
         pfree(P, P->d_Utmp);
+        P->Ucap = 0;
         int64_t cap = nu + nu / 8 + 1024;
         if (palloc(P, &P->d_Ucol, (size_t)cap) || (staged && palloc(P, &P->d_Utmp, (size_t)cap))) return GSOFA_ERR_ALLOC;
         P->Ucap = cap;
@@ -1173,6 +1190,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     else gsofa_options_default(&P->opt);
     P->n_mats = n_mats;
     P->h_mat_base.assign(mat_base, mat_base + n_mats + 1);
+    read_fail_alloc(P);
     P->W = 1;
     for (int32_t b = 0; b < n_mats; b++) P->W = std::max<uint32_t>(P->W, mat_base[b + 1] - mat_base[b]);
     if (n_mats > 1) {  // batches: one share, reach or block mode
@@ -1820,7 +1838,7 @@ static int take_totals(gsofa_plan* P) {
 // per-row pass-through flags.
 static int build_supernodes(gsofa_plan* P, const uint32_t* pass) {
     const int32_t n = P->n;
-    if ((!P->d_supno || P->sn_cap < (size_t)n) && alloc_supernodes(P)) return GSOFA_ERR_ALLOC;
+    if (P->sn_cap < (size_t)n && alloc_supernodes(P)) return GSOFA_ERR_ALLOC;
     SuperParams sp{};
     sp.n = n;
     sp.L_rowptr = P->d_Lrp;
@@ -1845,7 +1863,10 @@ static int build_supernodes(gsofa_plan* P, const uint32_t* pass) {
 static int execute_spill(gsofa_plan* P, const std::vector<int32_t>& shares) {
     const int32_t n = P->n;
     const int32_t N = std::max(1, P->opt.n_virtual_gpu);
-    if (!P->d_sp_lcnt) {
+    if (!P->d_sp_lcnt || !P->d_sp_ucnt || !P->d_sp_pass) {
+        pfree(P, P->d_sp_lcnt);
+        pfree(P, P->d_sp_ucnt);
+        pfree(P, P->d_sp_pass);
         int e = 0;
         e |= palloc(P, &P->d_sp_lcnt, (size_t)n);
         e |= palloc(P, &P->d_sp_ucnt, (size_t)n);
@@ -2042,6 +2063,9 @@ int gsofa_plan_execute(gsofa_plan* P) {
         HIPCHK(hipEventCreate(&e));
         P->ev.push_back(e);
     }
+    // a call before this one failed to grow it
+    if (P->structure && stream_missing(P) && alloc_stream(P, std::max<uint64_t>(P->list_cap, P->fill_cap)))
+        return GSOFA_ERR_ALLOC;
     if (P->structure && (P->opt.flags & GSOFA_FLAG_SPILL)) {
         P->spilled = true;
         P->passes = 1;
@@ -2565,6 +2589,7 @@ int arena_create(const gsofa_options* opt, gsofa_plan** out) {
     P->opt.flags &= ~(GSOFA_FLAG_SPILL | GSOFA_FLAG_GRAPH);
     P->mode = GSOFA_MODE_REACH;
     P->arena = true;
+    read_fail_alloc(P);
     P->device = P->opt.device;
     if (hipSetDevice(P->device) != hipSuccess || stream_get(P->device, &P->stream) != hipSuccess) {
         (void)hipGetLastError();
@@ -2575,8 +2600,23 @@ int arena_create(const gsofa_options* opt, gsofa_plan** out) {
     return GSOFA_OK;
 }
 
-int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, int64_t budget) {
-    if (!P || !P->arena || !mats || count < 1) return GSOFA_ERR_INVALID;
+// Gives back all the arena's device memory: it starts over with the next batch.
+static void arena_reset(gsofa_plan* P) {
+    (void)hipStreamSynchronize(P->stream);
+    release_device(P);
+    P->cap = gsofa_plan::Caps();
+    P->sn_cap = 0;
+    P->held = 0;
+}
+
+// Device bytes of an arena's buffers at these capacities.
+static int64_t caps_bytes(const gsofa_plan::Caps& c, const gsofa_plan::QuotCaps& q) {
+    return (int64_t)(c.rp * (4 + 4 + 4 + 4 + 8 + 8 + 8 + 8 + 8) + c.ci * 8 + c.fills * 24 + c.L * 4 + c.U * 4 +
+                     c.scan * 8 + c.mats * 20 + c.chunks * (sizeof(BlkChunk) + 16) + sizeof(Ctrl)) +
+           quot_held(q) + reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, kArenaBits);
+}
+
+static int load_batch(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, int64_t budget) {
     HIPCHK(hipSetDevice(P->device));
     int64_t n = 0, nnz = 0;
     uint32_t W = 1;
@@ -2656,21 +2696,45 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     const size_t ne = (size_t)std::max<int64_t>(nnz + (int64_t)quot_ext((uint64_t)nnz, qlev), 1);
     // The arena keeps each buffer at the largest size seen.  If keeping them
     // and growing the rest would exceed the budget, it starts over with
-    // exactly this batch's sizes (the only path that frees device memory).
+    // exactly this batch's sizes.
     {
-        auto mx = [](size_t a, uint64_t b) { return (int64_t)std::max<uint64_t>(a, std::max<uint64_t>(b, 1)); };
-        gsofa_plan::QuotCaps qc = P->qcap;
-        qc.ln = std::max(qc.ln, (size_t)qlev * (size_t)n);
-        const int64_t keep = quot_held(qc) + 48 * mx(c.rp, rows) + 8 * mx(c.ci, (uint64_t)ne) + 24 * mx(c.fills, 2 * nr) +
-                             4 * mx(c.L, nl) + 4 * mx(c.U, nu) + 8 * mx(c.scan, scan_tmp_words(n) + 2 * (size_t)n + 8) +
-                             reach_bytes((uint32_t)std::max<size_t>(c.nb, nb), (uint32_t)std::max<size_t>(c.wg, W), 64);
-        if (keep > budget && P->held > 0) {
-            HIPCHK_OUT(hipStreamSynchronize(P->stream), P->stream);
-            release_device(P);
-            P->cap = gsofa_plan::Caps();
-            P->sn_cap = 0;
-            P->held = 0;
+        gsofa_plan::Caps one;  // this batch alone
+        one.rp = rows;
+        one.ci = ne;
+        one.fills = (size_t)(2 * nr);
+        one.L = (size_t)std::max<uint64_t>(nl, 1);
+        one.U = (size_t)std::max<uint64_t>(nu, 1);
+        one.scan = scan_tmp_words(n) + 2 * (size_t)n + 8;
+        one.mats = (size_t)count + 1;
+        one.chunks = nchunks;
+        one.wg = W;
+        one.nb = nb;
+        gsofa_plan::QuotCaps qone;
+        if (qlev) {
+            qone.tab = 2 * (size_t)(n >> qshift);  // each level at most half of the one below
+            qone.ln = (size_t)qlev * (size_t)n;
+            qone.n = (size_t)n;
+            qone.eb = (size_t)nnz;
         }
+        gsofa_plan::Caps all = one;
+        gsofa_plan::QuotCaps qall = qone;
+        auto raise = [](size_t& a, size_t b) { a = std::max(a, b); };
+        raise(all.rp, c.rp);
+        raise(all.ci, c.ci);
+        raise(all.fills, c.fills);
+        raise(all.L, c.L);
+        raise(all.U, c.U);
+        raise(all.scan, c.scan);
+        raise(all.mats, c.mats);
+        raise(all.chunks, c.chunks);
+        raise(all.wg, c.wg);
+        raise(all.nb, c.nb);
+        raise(qall.tab, P->qcap.tab);
+        raise(qall.ln, P->qcap.ln);
+        raise(qall.n, P->qcap.n);
+        raise(qall.eb, P->qcap.eb);
+        const int64_t keep = caps_bytes(all, qall);
+        if (keep > budget && keep > caps_bytes(one, qone)) arena_reset(P);
     }
     int e = 0;
     if (c.rp < rows) {
@@ -2766,9 +2830,7 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
         HIPCHK(hipMemsetAsync(P->d_rmask, 0, 16 * nbw, P->stream));
         HIPCHK(hipMemsetAsync(P->d_bstate, 0, sizeof(uint32_t) * c.nb, P->stream));
     }
-    P->held = (int64_t)(c.rp * (4 + 4 + 4 + 4 + 8 + 8 + 8 + 8 + 8) + c.ci * 8 + c.fills * 24 + c.L * 4 + c.U * 4 +
-                        c.scan * 8 + c.mats * 20 + c.chunks * (sizeof(BlkChunk) + 16) + sizeof(Ctrl)) +
-              quot_held(P->qcap) + reach_bytes((uint32_t)c.nb, (uint32_t)c.wg, 64);
+    P->held = caps_bytes(c, P->qcap);
     P->W = (uint32_t)c.wg;  // the kernels' per-workgroup stride
     P->nblocks = nb;
     P->C = (int32_t)(nb * P->S);
@@ -2793,6 +2855,15 @@ int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, in
     P->executed = false;
     P->host_valid = false;
     return GSOFA_OK;
+}
+
+// After an error the capacities may stand for arrays that are not there: the
+// arena gives everything back, and the next batch starts over.
+int arena_load(gsofa_plan* P, const PackedMatrix* const* mats, int32_t count, int64_t budget) {
+    if (!P || !P->arena || !mats || count < 1) return GSOFA_ERR_INVALID;
+    const int rc = load_batch(P, mats, count, budget);
+    if (rc == GSOFA_ERR_ALLOC || rc == GSOFA_ERR_HIP) arena_reset(P);
+    return rc;
 }
 
 // Matrix `index` of the last execute, in its own numbering, copied straight

@@ -310,6 +310,7 @@ hipError_t copy_chunks(const std::vector<Piece>& pieces, const std::vector<Chunk
 hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
     size_t total = 0, used = 0;
     for (const HostCopy& c : v) {
+        if (c.bytes && (!c.host || !c.dev)) return hipErrorInvalidValue;  // the kernels would fault
         total += c.bytes;
         used += c.bytes != 0;
     }
