@@ -551,13 +551,35 @@ void advance_state(gsofa_plan* P, int32_t gid) {
     advance_groups(P, gid, P->C, 0, (cnt + P->C - 1) / P->C);
 }
 
-// The fill stream, or reach mode's records and record lists, of P->fill_cap
-// entries (list: records of the A^T pass, at most).  After a failure some are
-// missing, and the next execute asks for them again.
-bool stream_missing(const gsofa_plan* P) {
-    if (P->mode == GSOFA_MODE_REACH) return !P->d_rec || !P->d_list;
-    return !P->d_fills;
+// After a failure to grow the stream it is missing, and the next execute asks
+// for it again.
+bool stream_missing(const gsofa_plan* P) { return P->mode == GSOFA_MODE_REACH ? !P->d_rec : !P->d_fills; }
+
+// Entries that a run not sized from its row bounds starts with: fills of 8 bytes,
+// or in reach mode records of 16 in as many bytes, and no more than the bounds
+// allow (need_rec: of one pass; 0: not known).
+uint64_t first_stream(const gsofa_options& o, bool reach, int64_t nnz, uint64_t need_rec) {
+    uint64_t fills = o.output_capacity > 0 ? (uint64_t)o.output_capacity : default_fill_cap(nnz);
+    if ((o.flags & GSOFA_FLAG_SPILL) && o.output_capacity <= 0)  // one share's fills at a time
+        fills = std::max<uint64_t>(fills / (uint64_t)std::max(1, o.n_virtual_gpu), 1u << 20);
+    if (!reach) return fills;
+    const uint64_t rec = std::max<uint64_t>(fills / 2, 1);
+    return need_rec ? std::min(rec, 2 * need_rec) : rec;
 }
+
+// The record lists (reach mode): `list` records of the pass they are made of.
+int ensure_list(gsofa_plan* P, uint64_t list) {
+    if (list <= P->list_cap) return GSOFA_OK;
+    pfree(P, P->d_list);
+    P->list_cap = 0;
+    if (palloc(P, &P->d_list, (size_t)list)) return GSOFA_ERR_ALLOC;
+    P->list_cap = list;
+    return GSOFA_OK;
+}
+
+// The fill stream, or reach mode's records, of P->fill_cap entries.  list:
+// records of the A^T pass at most, 0 where they are not bounded and the lists
+// are made once the traversal has counted them.
 
 int alloc_stream(gsofa_plan* P, uint64_t list) {
     if (P->mode != GSOFA_MODE_REACH) {
@@ -566,9 +588,9 @@ int alloc_stream(gsofa_plan* P, uint64_t list) {
     }
     pfree(P, P->d_rec);
     pfree(P, P->d_list);
-    P->list_cap = std::max<uint64_t>(list, 1);
-    if (palloc(P, &P->d_rec, (size_t)P->fill_cap) || palloc(P, &P->d_list, (size_t)P->list_cap)) return GSOFA_ERR_ALLOC;
-    return GSOFA_OK;
+    P->list_cap = 0;
+    if (palloc(P, &P->d_rec, (size_t)P->fill_cap)) return GSOFA_ERR_ALLOC;
+    return ensure_list(P, list);
 }
 
 void release_quot(gsofa_plan* P) {
@@ -1336,7 +1358,12 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
             P->share_chunk_off.assign(2, 0);
             P->share_chunk_off[1] = (uint32_t)P->h_chunks.size();
             const int64_t tbytes = 4 * (int64_t)(n + 1) + 4 * P->nnz + 16 * (int64_t)n_mats;
-            const int64_t room = std::max<int64_t>(avail - tbytes, 1 << 20);
+            // workgroups beside the first stream, if it grows on demand (to them
+            // goes half of the room at least: a longer stream fails by itself)
+            const int64_t stream = P->bounded || (P->opt.flags & GSOFA_FLAG_COUNTS_ONLY)
+                                       ? 0
+                                       : 16 * (int64_t)std::min<uint64_t>(first_stream(P->opt, true, P->nnz, need_rec), 1ull << 40);
+            const int64_t room = std::max<int64_t>(avail - tbytes - std::min(stream, avail / 2), 1 << 20);
             gsofa_options go = P->opt;
             qlev = quot_wanted(n, P->nnz, P->W, go.mem_budget_bytes > 0 ? std::min(room, go.mem_budget_bytes) : room,
                                P->h_rp.data(), ci.data(), &qshift);
@@ -1413,9 +1440,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
         e |= palloc(P, &P->d_q0, (size_t)P->Q);
         e |= palloc(P, &P->d_q1, (size_t)P->Q);
     }
-    P->fill_cap = P->opt.output_capacity > 0 ? (uint64_t)P->opt.output_capacity : default_fill_cap(P->nnz);
-    if ((P->opt.flags & GSOFA_FLAG_SPILL) && P->opt.output_capacity <= 0)  // one share's fills at a time
-        P->fill_cap = std::max<uint64_t>(P->fill_cap / (uint64_t)std::max(1, P->opt.n_virtual_gpu), 1u << 20);
+    P->fill_cap = first_stream(P->opt, reach, P->nnz, need_rec);
     if (P->bounded) {
         P->fill_cap = P->mode == GSOFA_MODE_REACH ? 2 * need_rec : std::max<uint64_t>(need_fill, 1);
         P->Lcap = (int64_t)need_L;
@@ -1429,7 +1454,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
     }
     e |= palloc(P, &P->d_rp, (size_t)n + 1);
     e |= palloc(P, &P->d_ci, (size_t)(P->nnz + (int64_t)quot_ext((uint64_t)P->nnz, qlev)));
-    if (!(P->opt.flags & GSOFA_FLAG_COUNTS_ONLY) || !reach) e |= alloc_stream(P, P->bounded ? need_rec : P->fill_cap);
+    if (!(P->opt.flags & GSOFA_FLAG_COUNTS_ONLY) || !reach) e |= alloc_stream(P, P->bounded ? need_rec : 0);
     e |= palloc(P, &P->d_ctrl, 1);
     e |= palloc(P, &P->d_cntL, (size_t)n);
     e |= palloc(P, &P->d_cntU, (size_t)n);
@@ -1777,13 +1802,15 @@ static int build_structure(gsofa_plan* P, uint64_t n_fills, int32_t N, int32_t g
     if (on_device) {
         P->totals_known = false;
     } else {
-        int64_t tot[2] = {0, 0};
-        HIPCHK_OUT(copy_out({{&tot[0], P->d_Lrp + n, sizeof(int64_t)}, {&tot[1], P->d_Urp + n, sizeof(int64_t)}},
-                            P->stream), P->stream);
+        int64_t tot[3] = {0, 0, 0};  // L, U and the A^T pass's records
+        std::vector<HostCopy> cp{{&tot[0], P->d_Lrp + n, sizeof(int64_t)}, {&tot[1], P->d_Urp + n, sizeof(int64_t)}};
+        if (reach) cp.push_back({&tot[2], P->d_rptr + n, sizeof(int64_t)});
+        HIPCHK_OUT(copy_out(cp, P->stream), P->stream);
         P->nnzL = tot[0];
         P->nnzU = tot[1];
         P->totals_known = true;
         int rc = ensure_cols(P, P->nnzL, P->nnzU);
+        if (!rc) rc = ensure_list(P, (uint64_t)tot[2]);
         if (rc) return rc;
     }
     if (reach) {
@@ -2064,7 +2091,7 @@ int gsofa_plan_execute(gsofa_plan* P) {
         P->ev.push_back(e);
     }
     // a call before this one failed to grow it
-    if (P->structure && stream_missing(P) && alloc_stream(P, std::max<uint64_t>(P->list_cap, P->fill_cap)))
+    if (P->structure && stream_missing(P) && alloc_stream(P, 0))
         return GSOFA_ERR_ALLOC;
     if (P->structure && (P->opt.flags & GSOFA_FLAG_SPILL)) {
         P->spilled = true;
@@ -2132,7 +2159,7 @@ int gsofa_plan_execute(gsofa_plan* P) {
         if (!P->structure || P->stats.fill_pos <= P->fill_cap) break;
         // the stream outgrew its reserve: grow to the exact size and rerun
         P->fill_cap = P->stats.fill_pos + P->stats.fill_pos / 16 + 1024;
-        if (alloc_stream(P, P->fill_cap)) return GSOFA_ERR_ALLOC;
+        if (alloc_stream(P, 0)) return GSOFA_ERR_ALLOC;
     }
     if (P->structure && P->stats.fill_pos > P->fill_cap) return GSOFA_ERR_ALLOC;
 
@@ -2427,8 +2454,10 @@ int gsofa_plan_fetch_supernodal(gsofa_plan* P, gsofa_supernodal* h) {
         HIPCHK_OUT(exclusive_scan_u32_to_i64(P->d_cntL, d_xs, ns, P->d_scan, P->stream), P->stream);
         HIPCHK_OUT(copy_out({{&nsub, d_xs + ns, sizeof(int64_t)}}, P->stream), P->stream);
     }
-    // a reach-mode run's records give the columns as they gave the rows
-    const bool records = P->mode == GSOFA_MODE_REACH && n > 0;
+    // a reach-mode run's records give the columns as they gave the rows, if the
+    // lists have room for the other pass's
+    const bool records = P->mode == GSOFA_MODE_REACH && n > 0 &&
+                         (P->bounded || ensure_list(P, P->stats.fill_pos) == GSOFA_OK);
     const bool staged = !records && (!P->d_Ltmp || !P->d_Utmp);  // the structure pass left no staging arrays
     const size_t nl = (size_t)P->nnzL, nu = (size_t)P->nnzU;
     int32_t* mem = nullptr;

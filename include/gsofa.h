@@ -93,7 +93,9 @@ typedef struct gsofa_options {
     int32_t wave_block_threshold; /* row length from which a whole workgroup expands a row  */
     int32_t device;               /* HIP device ordinal                                     */
     int64_t queue_capacity;       /* frontier pairs per queue; 0 = automatic                */
-    int64_t output_capacity;      /* fill entries reserved; 0 = automatic (grown on demand) */
+    int64_t output_capacity;      /* fill entries reserved, 8 bytes each (reach mode: as    */
+                                  /* many bytes of its records); grown on demand; 0 =       */
+                                  /* automatic                                              */
     int32_t flags;                /* GSOFA_FLAG_*                                            */
     int32_t grid_blocks;          /* persistent grid size; 0 = occupancy-bounded maximum    */
     int32_t mode;                 /* GSOFA_MODE_*                                           */

@@ -2,6 +2,9 @@
 GSOFA_FAIL_ALLOC=k, read when a plan or a server worker's arena is made, fails
 its k-th allocation once; whatever runs next on the same plan or server must
 find every array it needs."""
+import ctypes as C
+
+import numpy as np
 import pytest
 
 from gpu_util import assert_same_structure
@@ -74,3 +77,66 @@ def test_plan_after_a_failed_execute(cases, monkeypatch, kw):
                 p.execute()
             assert_same_structure(p.fetch(), o)
     assert failed >= 3
+
+
+def _free_bytes():
+    from gsofa_amd import _lib
+    free, total = C.c_size_t(), C.c_size_t()
+    assert _lib.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _columns(p):
+    h = p.fetch_supernodal()
+    return [getattr(h, k) for k in ("xsup", "supno", "xsub", "sub", "xlcol", "lrow", "xucol", "urow")]
+
+
+@pytest.mark.parametrize("mode", ["reach", "block"])
+def test_given_capacity_is_what_is_reserved(cases, mode):
+    """output_capacity reserves 8 bytes an entry in every mode; all else of this
+    plan is some 40 allocations of under 2 MB each."""
+    import gsofa_amd as g
+    A, o = cases[1]
+    cap = 1 << 28
+    with g.Plan(A) as p:
+        p.execute()
+        want = _columns(p)
+    before = _free_bytes()
+    with g.Plan(A, mode=mode, output_capacity=cap) as p:
+        assert before - _free_bytes() <= 8 * cap + (128 << 20)
+        p.execute()
+        r = p.fetch()
+        assert r.passes == 1
+        assert_same_structure(r, o)
+        for a, b in zip(_columns(p), want):
+            np.testing.assert_array_equal(a, b)
+
+
+def test_columns_without_room_for_the_lists(cases, monkeypatch):
+    """The allocation that fails is, from some k on, that of the hand-off's longer
+    record lists: the columns then come from the rows."""
+    import gsofa_amd as g
+    A, _ = cases[1]
+    with g.Plan(A) as p:
+        p.execute()
+        want = _columns(p)
+    for k in range(30, 50):
+        print("case: hand-off, allocation", k, flush=True)
+        monkeypatch.setenv("GSOFA_FAIL_ALLOC", str(k))
+        try:
+            p = g.Plan(A, mode="reach", output_capacity=1 << 16)
+        except g.GsofaError as e:
+            assert e.code == ERR_ALLOC
+            continue
+        with p:
+            try:
+                p.execute()
+            except g.GsofaError as e:
+                assert e.code == ERR_ALLOC
+                p.execute()
+            for _ in range(2):
+                for a, b in zip(_columns(p), want):
+                    np.testing.assert_array_equal(a, b)
+            p.execute()
+            for a, b in zip(_columns(p), want):
+                np.testing.assert_array_equal(a, b)
