@@ -784,6 +784,9 @@ __global__ __launch_bounds__(BB) void k_traverse_lds(BlkParams p) {
                             uint32_t M = 0;
                             if (j == 0u) M = (atomicAnd(&pm[v >> 2], ~(0xFFu << sh)) >> sh) & 0xFFu;
                             M = __shfl(M, 0, G);
+                            // the labels are read after the bits are taken: what
+                            // lowers one later finds no bit and queues the vertex
+                            wave_sync();
 #pragma unroll
                             for (int k = 0; k < SL; k++) {  // symbfact.cuh:924
                                 const uint32_t l = lab[v * SL + k];
