@@ -616,8 +616,7 @@ uint32_t quot_wanted(int64_t n, int64_t nnz, uint32_t W, int64_t room, const int
                      uint32_t* shift) {
     for (*shift = quot_shift(W, n, rp, ci);; *shift = kQuotShift) {
         const uint32_t L = quot_levels(W, *shift);
-        if (L != 0 && nnz + (int64_t)quot_ext((uint64_t)nnz, L) < (int64_t)UINT32_MAX &&
-            quot_bytes(n, nnz, W, *shift) <= room / 8)
+        if (L != 0 && quot_fits((uint64_t)nnz, L) && quot_bytes(n, nnz, W, *shift) <= room / 8)
             return L;
         if (*shift == kQuotShift) return 0;
     }

@@ -158,6 +158,7 @@ __device__ __forceinline__ bool quot_off(const QuotParams& p) { return 2ull * p.
 uint32_t quot_shift(uint32_t W, int64_t n, const int32_t* rp, const int32_t* ci);
 uint32_t quot_levels(uint32_t W, uint32_t shift);
 uint64_t quot_ext(uint64_t nnz, uint32_t levels);
+bool quot_fits(uint64_t nnz, uint32_t levels);
 int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W, uint32_t shift);
 void quot_table(const std::vector<uint32_t>& mat_base, uint32_t levels, uint32_t shift, std::vector<uint2>& tab,
                 std::vector<uint32_t>& off);

@@ -727,6 +727,16 @@ uint32_t quot_levels(uint32_t W, uint32_t shift) {
 
 uint64_t quot_ext(uint64_t nnz, uint32_t levels) { return nnz * levels; }
 
+// Whether entry numbers of the matrix's and the classes' rows fit 32 bits, also
+// where a loop steps past a row's end: up to four steps of a workgroup here, and
+// a lane group's step in the traversal.  (A number that wrapped would read as
+// one before the row's end, and the loop would go on.)
+bool quot_fits(uint64_t nnz, uint32_t levels) {
+    constexpr uint64_t past = 1ull << 16;
+    static_assert(past >= 8ull * QNT_BIG, "a loop's last step and its lanes");
+    return nnz + quot_ext(nnz, levels) + past <= (1ull << 32);
+}
+
 int64_t quot_bytes(int64_t n, int64_t nnz, uint32_t W, uint32_t shift) {
     const int64_t L = quot_levels(W, shift);
     if (L == 0) return 0;
