@@ -45,9 +45,15 @@ constexpr uint32_t kBlock = 64;             // indexes that share a base
 constexpr size_t kChunkMost = 4u << 20;    // bytes of result in a chunk, and what they take as
                                            // bases, 16-bit offsets and room for whole blocks
 constexpr size_t kStageBytes = kChunkMost / (4 * kBlock) * (4 + 6 * kBlock) + (16u << 10);
-constexpr size_t kStageKeep = 48;          // idle staging buffers kept: two large copies at once
-constexpr size_t kStageRest = 24;          // and after the last plan's release, one copy's (146 MB:
-                                           // making and releasing them takes over 2 ms)
+// Making and releasing the buffers of one large copy takes over 2 ms, so they
+// are kept and no copy makes more than it must: with kStageMost out (four large
+// copies') a further one has a single thread's two.  So at most
+// kStageMost + 1 + 2 * callers exist, all kept while plans live for up to 15
+// callers at a time (a server has 16 workers at most); after the last plan's
+// release kStageRest, one copy's (153 MB).
+constexpr size_t kStageMost = 96;
+constexpr size_t kStageKeep = kStageMost + 32;
+constexpr size_t kStageRest = 24;
 constexpr size_t kKernelMost = 512u << 10; // totals up to here: one kernel
 constexpr size_t kPerThread = 2u << 20;     // bytes per copy thread, at least
 constexpr int kThreads = 12;
@@ -58,6 +64,8 @@ constexpr size_t kHugeMin = 1u << 20;
 
 std::mutex g_mu;
 std::vector<void*> g_stage;                // idle staging buffers
+size_t g_out = 0;                          // buffers in use
+uint64_t g_made = 0;                       // made so far
 struct IdleStream {
     int device;
     hipStream_t s;
@@ -69,18 +77,25 @@ size_t g_live = 0;                         // streams handed out: live plans
 std::vector<Ctrl*> g_ctrl;                 // idle pinned counter blocks, made a page at a time
 constexpr size_t kCtrlSlots = 4096 / sizeof(Ctrl);
 
-void* stage_get() {
+// A buffer; null if none can be made, or for one that the call can do without
+// (`more`) when enough are out.
+void* stage_get(bool more) {
     {
         std::lock_guard<std::mutex> lk(g_mu);
+        if (more && g_out >= kStageMost) return nullptr;
+        g_out++;
         if (!g_stage.empty()) {
             void* p = g_stage.back();
             g_stage.pop_back();
             return p;
         }
+        g_made++;
     }
     void* p = nullptr;
     if (hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_out--;
         return nullptr;
     }
     return p;
@@ -90,6 +105,7 @@ void stage_put(void* p) {
     if (!p) return;
     {
         std::lock_guard<std::mutex> lk(g_mu);
+        g_out--;
         if (g_stage.size() < kStageKeep) {
             g_stage.push_back(p);
             return;
@@ -316,7 +332,7 @@ hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
     }
     if (total == 0) return hipSuccess;
     void* buf[2 * kThreads] = {};
-    buf[0] = stage_get();
+    buf[0] = stage_get(false);
     if (buf[0] && total <= kKernelMost && used <= (size_t)Pieces::MAX) {
         const hipError_t e = copy_small(v, out, (char*)buf[0], s, total);
         stage_put(buf[0]);
@@ -325,12 +341,15 @@ hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
     int threads = 0;
     const int want = (int)std::min<size_t>(kThreads, std::max<size_t>(1, total / kPerThread));
     for (; threads < want; threads++) {
-        if (threads > 0) buf[2 * threads] = stage_get();
-        buf[2 * threads + 1] = stage_get();
-        if (!buf[2 * threads] || !buf[2 * threads + 1]) break;
+        void*(&b)[2] = reinterpret_cast<void*(&)[2]>(buf[2 * threads]);
+        if (threads > 0) b[0] = stage_get(true);
+        if (b[0]) b[1] = stage_get(threads > 0);
+        if (b[0] && b[1]) continue;
+        stage_put(b[0]);
+        b[0] = nullptr;
+        break;
     }
     if (threads == 0) {  // no pinned memory: direct copies
-        for (void* b : buf) stage_put(b);
         hipError_t e = hipSuccess;
         for (const HostCopy& c : v) {
             if (!c.bytes || e != hipSuccess) continue;
@@ -385,6 +404,11 @@ hipError_t copy_all(const std::vector<HostCopy>& v, bool out, hipStream_t s) {
 }
 
 }  // namespace
+
+uint64_t stage_made() {
+    std::lock_guard<std::mutex> lk(g_mu);
+    return g_made;
+}
 
 hipError_t copy_out(const std::vector<HostCopy>& v, hipStream_t s) { return copy_all(v, true, s); }
 hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s) { return copy_all(v, false, s); }

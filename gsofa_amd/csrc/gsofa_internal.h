@@ -258,6 +258,7 @@ struct HostCopy {
 };
 hipError_t copy_out(const std::vector<HostCopy>& v, hipStream_t s);
 hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s);
+uint64_t stage_made();  // pinned staging buffers made so far
 hipError_t launch_copy_words(void* dst, const void* src, uint32_t words, hipStream_t s);  // pinned or device
 void* host_array(size_t bytes);  // a result array, released with free()
 hipError_t stream_get(int device, hipStream_t* s);

@@ -221,6 +221,10 @@ int gsofa_counts_noalloc(int32_t n, int64_t nnz, const int32_t* d_rowptr, const 
                          int64_t* d_row_fill, int64_t* d_row_te, int64_t* d_row_reach, uint64_t* d_totals,
                          int32_t device, void* stream);
 
+/* Results come through pinned staging buffers of 6.4 MB, which calls make as
+ * they need them (24 for one of over 24 MB) and the library keeps: up to 128
+ * while plans or servers live, 24 (153 MB) after the last one's release. */
+
 /* ---- device-resident plan ---------------------------------------------------
  * create: validate, upload the CSR and size the workspace (no traversal).
  * execute: traversal + L/U structure + supernodes on the device; the inputs
