@@ -24,8 +24,8 @@ from . import _lib
 from ._lib import GSOFA_FLAG_COUNTS_ONLY, GSOFA_FLAG_GRAPH, GSOFA_FLAG_SPILL
 
 __all__ = ["CsrMatrix", "SymbfactResult", "GsofaError", "Plan", "Server", "symbfact", "gen_grid",
-           "gen_band", "read_ascii", "write_ascii", "footprint", "GSOFA_FLAG_COUNTS_ONLY", "GSOFA_FLAG_SPILL",
-           "GSOFA_FLAG_GRAPH"]
+           "gen_band", "read_ascii", "write_ascii", "footprint", "release_memory",
+           "GSOFA_FLAG_COUNTS_ONLY", "GSOFA_FLAG_SPILL", "GSOFA_FLAG_GRAPH"]
 
 
 class GsofaError(RuntimeError):
@@ -325,6 +325,12 @@ def footprint(A, **kw):
     m = A.to_c()
     o = _options(**kw)
     return int(_lib.lib().gsofa_plan_footprint(C.byref(m), C.byref(o)))
+
+
+def release_memory():
+    """Gives back the memory that the library keeps between calls and does not
+    use: device memory of released plans, staging buffers, streams."""
+    _lib.lib().gsofa_release_memory()
 
 
 class Plan:

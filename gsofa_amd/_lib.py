@@ -119,6 +119,8 @@ def lib():
     L.gsofa_supernodal_free.argtypes = [P(Supernodal)]
     L.gsofa_plan_footprint.argtypes = [P(Matrix), P(Options)]
     L.gsofa_plan_footprint.restype = C.c_int64
+    L.gsofa_release_memory.argtypes = []
+    L.gsofa_release_memory.restype = None
     L.gsofa_order_nd.argtypes = [P(Matrix), C.c_int32, C.c_void_p]
     L.gsofa_order_nd.restype = C.c_int
     L.gsofa_permute.argtypes = [P(Matrix), C.c_void_p, P(Csr)]

@@ -235,14 +235,9 @@ const char* kErr[] = {"ok",
 
 template <class T>
 int dalloc(T** p, size_t count) {
-    *p = nullptr;
     if (count == 0) count = 1;
-    if (hipMalloc((void**)p, count * sizeof(T)) != hipSuccess) {
-        (void)hipGetLastError();
-        *p = nullptr;
-        return GSOFA_ERR_ALLOC;
-    }
-    return GSOFA_OK;
+    *p = (T*)device_alloc(count * sizeof(T));
+    return *p ? GSOFA_OK : GSOFA_ERR_ALLOC;
 }
 
 // Device allocations released together when the holder goes out of scope.
@@ -253,11 +248,8 @@ struct DevScratch {
     }
     template <class T>
     int get(T** out, size_t count) {
-        void* q = nullptr;
-        if (hipMalloc(&q, sizeof(T) * std::max<size_t>(count, 1)) != hipSuccess) {
-            (void)hipGetLastError();
-            return GSOFA_ERR_ALLOC;
-        }
+        void* q = device_alloc(sizeof(T) * std::max<size_t>(count, 1));
+        if (!q) return GSOFA_ERR_ALLOC;
         p.push_back(q);
         *out = (T*)q;
         return GSOFA_OK;
@@ -272,8 +264,9 @@ void read_fail_alloc(gsofa_plan* P) {
 bool alloc_fails(gsofa_plan* P) { return P->fail_alloc > 0 && --P->fail_alloc == 0; }
 
 // A plan's device arrays.  Where all sizes are known at creation they are
-// pieces of one allocation (gather, then take_slab): twelve of 8 MB cost
-// 3.4 ms to make and release, one of 96 MB 0.6.
+// pieces of one allocation (gather, then take_slab), which is kept for the next
+// plan when this one is released: twelve of 8 MB cost 3.4 ms to make and
+// release, one of 96 MB 0.6.
 template <class T>
 int palloc(gsofa_plan* P, T** p, size_t count) {
     *p = nullptr;
@@ -293,7 +286,8 @@ int take_slab(gsofa_plan* P) {
     P->gather = false;
     P->slab_bytes = 0;
     for (const gsofa_plan::Piece& x : P->pieces) P->slab_bytes += x.bytes;
-    const int e = alloc_fails(P) ? GSOFA_ERR_ALLOC : dalloc(&P->slab, P->slab_bytes);
+    if (!alloc_fails(P)) P->slab = (char*)slab_get(P->device, &P->slab_bytes);
+    const int e = P->slab ? GSOFA_OK : GSOFA_ERR_ALLOC;
     size_t off = 0;
     for (const gsofa_plan::Piece& x : P->pieces) {
         if (!e) *x.where = P->slab + off;
@@ -732,7 +726,9 @@ void release_device(gsofa_plan* P) {
     pfree(P, P->d_mat_te);
     pfree(P, P->d_mat_reach);
     release_quot(P);
-    if (P->slab) (void)hipFree(P->slab);
+    // kept for another plan's stream: nothing of this one's may still use it
+    if (P->slab && hipStreamSynchronize(P->stream) == hipSuccess) slab_put(P->device, P->slab, P->slab_bytes);
+    else if (P->slab) (void)hipFree(P->slab);
     P->slab = nullptr;
 }
 
@@ -1128,6 +1124,11 @@ void gsofa_result_free(gsofa_result* r) {
     memset(r, 0, sizeof(*r));
 }
 
+void gsofa_release_memory(void) {
+    (void)slabs_release();
+    host_idle_release();
+}
+
 int64_t gsofa_plan_footprint(const gsofa_matrix* A, const gsofa_options* opt) {
     gsofa_options o;
     if (opt) o = *opt;
@@ -1269,6 +1270,7 @@ static int plan_create_impl(const gsofa_matrix* A, const uint32_t* mat_base, int
 
     size_t freeb = 0, totalb = 0;
     (void)hipMemGetInfo(&freeb, &totalb);
+    freeb += slabs_idle(P->device);
     int64_t avail = (int64_t)((double)freeb * 0.80) - 8 * (int64_t)(n + 1 + P->nnz) -
                     64ll * (n + 1) - (64ll << 20);
     // Output reserve from the row bounds: the fills, L and U entries of the

@@ -474,6 +474,144 @@ void stream_put(int device, hipStream_t s) {
     for (void* x : mem) (void)hipHostFree(x);
 }
 
+// Idle slabs: the device memory of released plans, the longest idle first.
+// Never destroyed: plans may be released while the process ends.
+namespace {
+
+constexpr size_t kSlabShare = 16;        // of a device's memory, at most this part is kept idle
+constexpr size_t kSlabSpare = 16u << 20;
+
+struct Slabs {
+    struct Idle {
+        int device;
+        void* p;
+        size_t bytes;
+    };
+    std::mutex mu;
+    std::vector<Idle> idle;
+    uint64_t made = 0;
+};
+Slabs& slabs() {
+    static Slabs* s = new Slabs();
+    return *s;
+}
+
+size_t idle_bytes(const Slabs& s, int device) {
+    size_t sum = 0;
+    for (const Slabs::Idle& x : s.idle)
+        if (x.device == device) sum += x.bytes;
+    return sum;
+}
+
+}  // namespace
+
+// Device memory of at least *bytes for the current device, which is `device`;
+// *bytes becomes its size: the smallest idle slab of up to twice as much, else a
+// new one.  Its contents are any.  Null when there is none.
+//
+// A plan's memory is mostly its workgroups' arrays (63^3 grid: 8.2 of 9.9 GB), and
+// memory that has been in use once is cleared by the driver before it is given
+// out again, at 42 GB/s and beside nothing else: a stream of one-shot calls that
+// made and released it, 67 GB in 0.27 s of calls, ran at that rate with calls of
+// up to 1.7 s among it once it had gone through the card's 288 GB.  32 such calls,
+// s a round over seven rounds: 0.26 to 4.5; with slabs kept 0.25 to 0.28 (the first
+// round and one other 1.1 and 0.5 where another process had left the card's memory
+// in use).
+void* slab_get(int device, size_t* bytes) {
+    Slabs& s = slabs();
+    {
+        std::lock_guard<std::mutex> lk(s.mu);
+        size_t best = s.idle.size();
+        for (size_t i = s.idle.size(); i-- > 0;)  // of equal ones the last released
+            if (s.idle[i].device == device && s.idle[i].bytes >= *bytes && s.idle[i].bytes <= 2 * *bytes + kSlabSpare &&
+                (best == s.idle.size() || s.idle[i].bytes < s.idle[best].bytes))
+                best = i;
+        if (best < s.idle.size()) {
+            void* p = s.idle[best].p;
+            *bytes = s.idle[best].bytes;
+            s.idle.erase(s.idle.begin() + (ptrdiff_t)best);
+            return p;
+        }
+        s.made++;
+    }
+    return device_alloc(*bytes);
+}
+
+// p: of slab_get, with no work on it left.  Slabs beyond the bound go, the
+// longest idle first.
+void slab_put(int device, void* p, size_t bytes) {
+    if (!p) return;
+    size_t total = 0;
+    if (hipDeviceTotalMem(&total, device) != hipSuccess) {
+        (void)hipGetLastError();
+        total = 0;
+    }
+    std::vector<void*> gone;
+    Slabs& s = slabs();
+    {
+        std::lock_guard<std::mutex> lk(s.mu);
+        s.idle.push_back({device, p, bytes});
+        size_t sum = idle_bytes(s, device);
+        for (size_t i = 0; i < s.idle.size() && sum > total / kSlabShare;) {
+            if (s.idle[i].device != device) {
+                i++;
+                continue;
+            }
+            gone.push_back(s.idle[i].p);
+            sum -= s.idle[i].bytes;
+            s.idle.erase(s.idle.begin() + (ptrdiff_t)i);
+        }
+    }
+    for (void* x : gone) (void)hipFree(x);
+}
+
+// Bytes that slabs_release would give back on `device`.
+size_t slabs_idle(int device) {
+    Slabs& s = slabs();
+    std::lock_guard<std::mutex> lk(s.mu);
+    return idle_bytes(s, device);
+}
+
+bool slabs_release() {
+    std::vector<Slabs::Idle> gone;
+    Slabs& s = slabs();
+    {
+        std::lock_guard<std::mutex> lk(s.mu);
+        gone.swap(s.idle);
+    }
+    for (const Slabs::Idle& x : gone) (void)hipFree(x.p);
+    return !gone.empty();
+}
+
+uint64_t slabs_made() {
+    Slabs& s = slabs();
+    std::lock_guard<std::mutex> lk(s.mu);
+    return s.made;
+}
+
+// hipMalloc; what idle slabs hold is given back before it fails.
+void* device_alloc(size_t bytes) {
+    for (;;) {
+        void* p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        if (!slabs_release()) return nullptr;
+    }
+}
+
+// Idle staging buffers and streams.
+void host_idle_release() {
+    std::vector<IdleStream> gone;
+    std::vector<void*> mem;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        gone.swap(g_streams);
+        mem.swap(g_stage);
+    }
+    for (const IdleStream& x : gone) (void)hipStreamDestroy(x.s);
+    for (void* x : mem) (void)hipHostFree(x);
+}
+
 Ctrl* ctrl_get() {
     std::lock_guard<std::mutex> lk(g_mu);
     if (g_ctrl.empty()) {

@@ -261,6 +261,13 @@ hipError_t copy_in(const std::vector<HostCopy>& v, hipStream_t s);
 uint64_t stage_made();  // pinned staging buffers made so far
 hipError_t launch_copy_words(void* dst, const void* src, uint32_t words, hipStream_t s);  // pinned or device
 void* host_array(size_t bytes);  // a result array, released with free()
+void* device_alloc(size_t bytes);
+void* slab_get(int device, size_t* bytes);
+void slab_put(int device, void* p, size_t bytes);
+size_t slabs_idle(int device);
+bool slabs_release();
+uint64_t slabs_made();
+void host_idle_release();
 hipError_t stream_get(int device, hipStream_t* s);
 void stream_put(int device, hipStream_t s);
 Ctrl* ctrl_get();  // a pinned counter block, or null

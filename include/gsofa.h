@@ -221,9 +221,16 @@ int gsofa_counts_noalloc(int32_t n, int64_t nnz, const int32_t* d_rowptr, const 
                          int64_t* d_row_fill, int64_t* d_row_te, int64_t* d_row_reach, uint64_t* d_totals,
                          int32_t device, void* stream);
 
-/* Results come through pinned staging buffers of 6.4 MB, which calls make as
- * they need them (24 for one of over 24 MB) and the library keeps: up to 128
- * while plans or servers live, 24 (153 MB) after the last one's release. */
+/* What the library keeps between calls, for all plans and servers of the process:
+ *  - device memory of released plans, for the plans after them: at most a
+ *    sixteenth of the device's (it goes when an allocation of the library fails
+ *    otherwise, and counts as free where the library sizes by free memory);
+ *  - pinned staging buffers of 6.4 MB that results come through (24 for a result
+ *    of over 24 MB): up to 128 while plans or servers live, 24 (153 MB) after the
+ *    last one's release;
+ *  - a few idle streams.
+ * gsofa_release_memory gives back all of it that is idle, from any thread. */
+void gsofa_release_memory(void);
 
 /* ---- device-resident plan ---------------------------------------------------
  * create: validate, upload the CSR and size the workspace (no traversal).
