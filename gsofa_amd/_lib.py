@@ -17,7 +17,7 @@ MODE_AUTO, MODE_BLOCK, MODE_GRID, MODE_HYBRID, MODE_REACH = 0, 1, 2, 3, 4
 
 # Every entry point include/gsofa.h declares (kept in sync by a CPU test).
 EXPORTS = [
-    "gsofa_strerror", "gsofa_csr_free", "gsofa_options_default", "gsofa_result_free",
+    "gsofa_strerror", "gsofa_csr_free", "gsofa_options_default", "gsofa_release_memory", "gsofa_result_free",
     "gsofa_symbfact", "gsofa_plan_create", "gsofa_plan_execute", "gsofa_plan_fetch",
     "gsofa_plan_destroy", "gsofa_plan_footprint", "gsofa_read_ascii", "gsofa_write_ascii",
     "gsofa_gen_grid", "gsofa_gen_band", "gsofa_gen_side_loguniform", "gsofa_gen_uniform_int",
