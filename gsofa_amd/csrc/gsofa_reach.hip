@@ -35,9 +35,9 @@
 //   operations per edge.  Execute ms, before -> now: 64^2 grid in natural order
 //   0.41 -> 0.33; 181^2 0.84 -> 0.64; 27^3 0.76 -> 0.59; 33^3 1.08 -> 0.79; band
 //   of 100,003 0.79 -> 0.70; 128 2D grids 11.1 -> 7.2; 48^3, whose deep groups
-//   do not fit, 2.30 -> 2.30.
-// * A mini-group whose nodes outgrow the table, and every one with more slots,
-//   keeps its state in memory, as follows.
+//   outgrow it, 2.30 -> 2.13.
+// * A mini-group goes on in memory from where its nodes outgrow the table
+//   (nodes_to_memory), and every one with more slots starts there, as follows.
 // * Per vertex, one word holds the MB slots' visited bits with the
 //   mini-group's stamp beside it; an older stamp reads as "nothing visited",
 //   so the array is never cleared between mini-groups (the reference's
@@ -616,9 +616,12 @@ __device__ __forceinline__ uint64_t mask_take(uint64_t* p) {
 // straight to its targets' visited words; who sets a pending bit of a node with
 // none queues it.  So a level is one phase and one barrier and nothing but the
 // graph itself is read from memory: edges, their classes, the new nodes' rows.
-// Returns false, with the table to be cleared, if it ran full.
+// If the table ran full: in level 0, the group starts again elsewhere; later, it
+// goes on from what the table holds (nodes_to_memory), where every node that the
+// level walked is pending again with all its bits, since its edges may be lost.
+enum class Walk { DONE, FULL_AT_ONCE, OUTGREW };
 template <int RB, int H, int F, int G, int E, class M>
-__device__ bool walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsigned long long& levels) {
+__device__ Walk walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsigned long long& levels) {
     using O = MaskOps<M>;
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t grp = lane / G, j = lane % G;
@@ -770,7 +773,23 @@ __device__ bool walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsig
             }
         }
     }
-    if (full) return false;
+    if (full && lev < 2u) return Walk::FULL_AT_ONCE;
+    t.fills += own.fills;
+    t.expansions += own.expansions;
+    t.te += own.te;
+    t.checks += own.te;
+    levels += tid == 0 ? lev : 0u;
+    if (full) {
+        const uint32_t b = (lev + 2u) % 3u, par = (lev + 1u) & 1u, qsize = S.nq[b];
+        const uint32_t nrow = S.nrow[b] < PART_ROWS ? S.nrow[b] : PART_ROWS;
+        for (uint32_t x = tid; x < qsize + nrow; x += RB) {  // a node is in the queue or in parts
+            const uint32_t k = x < qsize ? S.n.q[par][x] : S.n.pnode[par][x - qsize];
+            if (k != 0xFFFFu)
+                S.n.pend[k] |= S.n.vis[k] & above_mask<M>(S.n.key[k] - 1u + c.wb, c.first, c.stride, c.count);
+        }
+        __syncthreads();
+        return Walk::OUTGREW;
+    }
     // TE and |R|: every node below a source that visited it, with its weights
     const uint32_t fl = c.first - c.wb, used = S.used;
     for (uint32_t x = tid; x < used; x += RB) {
@@ -779,16 +798,73 @@ __device__ bool walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsig
         const M bl = S.n.vis[i] & above_mask<M>(m + c.wb, c.first, c.stride, c.count);
         if (!bl) continue;
         const uint2 w = c.weight(m);
-        own.reach += (unsigned long long)O::popc(bl) * w.x;
-        own.te += (unsigned long long)O::popc(bl) * w.y;
+        t.reach += (unsigned long long)O::popc(bl) * w.x;
+        t.te += (unsigned long long)O::popc(bl) * w.y;
+        t.checks += (unsigned long long)O::popc(bl) * w.y;  // every node once for every source that visits it
     }
-    t.fills += own.fills;
-    t.expansions += own.expansions;
-    t.te += own.te;
-    t.reach += own.reach;
-    t.checks += own.te;  // every node once for every source that visits it
-    levels += tid == 0 ? lev : 0u;
-    return true;
+    return Walk::DONE;
+}
+
+// A group that outgrew its table goes on in memory: its nodes' visited words, the
+// pending ones as level `cur` = 0's queue, those above the group on their list.
+// Starting it again there instead walked up to the whole group twice.  Traversal
+// ms again -> on (with no table at all): directed cycle of 5,000 19.1 -> 12.1
+// (12.2), one-directional band of 60,000 with 2,000 entries back 6.9 -> 4.9 (4.5),
+// hubs n = 8,000 2.06 -> 1.76 (6.2), 48^3 grid 1.44 -> 1.33.
+template <int RB, int H, int F, class M>
+__device__ void nodes_to_memory(RLds<M, H, F, RB>& S, const RCur& c, typename MaskOps<M>::V* vis, M* nmask0, uint4* q0,
+                                uint32_t* ulist, uint32_t stamp, RTally& t) {
+    using O = MaskOps<M>;
+    static_assert(merges<M>(), "masks side by side");
+    const uint32_t lane = __lane_id(), fl = c.first - c.wb, used = S.used;
+    for (uint32_t x0 = threadIdx.x - lane; x0 < used; x0 += RB) {
+        bool up = false, enq = false;
+        uint32_t m = 0;
+        uint4 e = make_uint4(0u, 0u, 0u, 0u);
+        if (x0 + lane < used) {
+            const uint32_t i = S.n.ent[x0 + lane];
+            m = S.n.key[i] - 1u;
+            const M v = S.n.vis[i], pd = S.n.pend[i];
+            vis[m] = O::make(v, stamp);
+            const M bl = v & above_mask<M>(m + c.wb, c.first, c.stride, c.count);
+            up = m > fl;
+            if (bl) {
+                const uint2 w = c.weight(m);
+                t.reach += (unsigned long long)O::popc(bl) * w.x;
+                t.te += (unsigned long long)O::popc(bl) * w.y;
+                t.checks += (unsigned long long)O::popc(bl & ~pd) * w.y;
+                if (pd) {
+                    const uint2 r = S.n.row[i];
+                    nmask0[2u * m] = pd;
+                    e = make_uint4(m, r.x, r.y, w.y);
+                    enq = true;
+                    if (r.y - r.x > SPLIT_ROW) {
+                        const uint32_t k = atomicAdd(&S.spn[0], 1u);
+                        if (k < SPLIT_MAX) {
+                            S.sp[0][k] = e;
+                            enq = false;
+                        }
+                    }
+                }
+            }
+        }
+        const uint64_t em = __ballot(enq), um = __ballot(up);
+        if (em) {
+            uint32_t qb = 0;
+            if (lane == 0) qb = atomicAdd(&S.qcnt[0], (uint32_t)__popcll(em));
+            qb = bcast0(qb);
+            if (enq) q0[qb + rank_in(em)] = e;
+        }
+        if (um) {
+            uint32_t ub = 0;
+            if (lane == 0) ub = atomicAdd(&S.nup, (uint32_t)__popcll(um));
+            ub = bcast0(ub);
+            if (up) {
+                ulist[ub + rank_in(um)] = m;
+                atomicMax(&S.tmax, m);
+            }
+        }
+    }
 }
 
 // The group's entries from the node table, which is cleared: records in order
@@ -967,17 +1043,13 @@ __global__ __launch_bounds__(RB, sizeof(M) <= 16 ? 4 : 1) void k_reach_blk(RchPa
         c.jb = classes ? (c.first - (c.count - 1u) * c.stride - c.wb) >> c.shift : 0u;
         c.below = c.jb << c.shift;
         bool nodes = false;  // the node table holds the whole group
+        bool part = false;   // or its first levels
         if constexpr (NODES) {
             if (wait == 0u) {
-                nodes = walk_nodes<RB, H, F, G, E, M>(S, c, t, levels);
-                if (!nodes) {
-                    // the sizes of neighbouring groups are alike
-                    wait = 8u;
-                    __syncthreads();
-                    clear_tables();
-                    if (tid == 0) S.used = 0;
-                    __syncthreads();
-                }
+                const Walk r = walk_nodes<RB, H, F, G, E, M>(S, c, t, levels);
+                nodes = r == Walk::DONE;
+                part = r == Walk::OUTGREW;
+                if (!nodes) wait = 8u;  // the sizes of neighbouring groups are alike
             }
         }
         // No vertex above the group is ever queued, so the queue arrays' entries
@@ -995,8 +1067,17 @@ __global__ __launch_bounds__(RB, sizeof(M) <= 16 ? 4 : 1) void k_reach_blk(RchPa
         }
         epoch++;
         stamp = epoch;
+        if constexpr (NODES) {
+            if (wait == 8u) {  // the table is left
+                if (part) nodes_to_memory<RB>(S, c, vis, nmask0, q0, ulist, stamp, t);
+                __syncthreads();
+                clear_tables();
+                if (tid == 0) S.used = 0;
+                __syncthreads();
+            }
+        }
         // level 0: the sources themselves, each visited by and queued for its own slot
-        if (tid < c.count) {
+        if (!part && tid < c.count) {
             const uint32_t sg = c.first - tid * c.stride;
             const uint32_t s = sg - c.wb;
             const M bit = O::bit(tid);
@@ -1006,11 +1087,11 @@ __global__ __launch_bounds__(RB, sizeof(M) <= 16 ? 4 : 1) void k_reach_blk(RchPa
             q0[tid] = make_uint4(s, r0, r1, r1 - r0);
             t.te += r1 - r0;
         }
-        if (tid == 0) S.qcnt[0] = c.count;
+        if (!part && tid == 0) S.qcnt[0] = c.count;
         __syncthreads();
 
         uint32_t cur = 0;
-        for (uint32_t lev = 0;; lev++) {
+        for (uint32_t lev = part ? 2u : 0u;; lev++) {  // level 0 alone is told apart; cur is its parity
             // final since the last barrier; reset during this level's relax
             const uint32_t nxt = cur ^ 1u;
             const uint32_t qsize = S.qcnt[cur];
