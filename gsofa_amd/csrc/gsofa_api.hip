@@ -574,7 +574,6 @@ int ensure_list(gsofa_plan* P, uint64_t list) {
 // The fill stream, or reach mode's records, of P->fill_cap entries.  list:
 // records of the A^T pass at most, 0 where they are not bounded and the lists
 // are made once the traversal has counted them.
-
 int alloc_stream(gsofa_plan* P, uint64_t list) {
     if (P->mode != GSOFA_MODE_REACH) {
         pfree(P, P->d_fills);

@@ -1,10 +1,12 @@
-// gsofa_block.hip -- block-resident multi-source traversal (default mode).
+// gsofa_block.hip -- block-resident multi-source traversal (block mode: single
+// shares, spilled runs and callers that ask for it).
 //
 // Same per-source arithmetic as the reference's warp-centric level kernel
 // (with_space_optimization/symbfact.cuh:883-1082) and seeding (:639-721), with
 // an execution model built for CDNA4:
 //
-// * Each workgroup (16 waves, one per CU) of a persistent grid owns //   slots (32, 16, 8, 4 or 2; one kernel instance each; what fits is run in LDS
+// * Each workgroup (16 waves, one per CU) of a persistent grid owns SL source
+//   slots (32, 16, 8, 4 or 2; one kernel instance each; what fits is run in LDS
 //   alone, k_traverse_lds) and runs a "mini-group" of
 //   SL consecutive sources through all of their frontier levels by itself,
 //   synchronising only with __syncthreads.  The next mini-group comes from

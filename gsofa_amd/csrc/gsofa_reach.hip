@@ -808,7 +808,7 @@ __device__ Walk walk_nodes(RLds<M, H, F, RB>& S, const RCur& c, RTally& t, unsig
 // A group that outgrew its table goes on in memory: its nodes' visited words, the
 // pending ones as level `cur` = 0's queue, those above the group on their list.
 // Starting it again there instead walked up to the whole group twice.  Traversal
-// ms again -> on (with no table at all): directed cycle of 5,000 19.1 -> 12.1
+// ms again -> on (before there was a table): directed cycle of 5,000 19.1 -> 12.1
 // (12.2), one-directional band of 60,000 with 2,000 entries back 6.9 -> 4.9 (4.5),
 // hubs n = 8,000 2.06 -> 1.76 (6.2), 48^3 grid 1.44 -> 1.33.
 template <int RB, int H, int F, class M>
